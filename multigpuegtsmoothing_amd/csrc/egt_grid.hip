@@ -253,40 +253,184 @@ __global__ void __launch_bounds__(BLK) k_morton_points(const float4* __restrict_
     if (mcloud) mcloud[m] = scloud[s];
 }
 
-__global__ void __launch_bounds__(BLK) k_level_flags(const uint32_t* __restrict__ code,
-                                                      const int32_t* __restrict__ mcloud, int64_t n, int shift,
-                                                      uint32_t* __restrict__ flag) {
-    const int64_t m = (int64_t)blockIdx.x * BLK + threadIdx.x;
-    if (m >= n) return;
-    bool first = m == 0 || (code[m] >> shift) != (code[m - 1] >> shift);
-    if (mcloud && m > 0) first = first || mcloud[m] != mcloud[m - 1];
-    flag[m] = first ? 1u : 0u;
+// ---- Level tables ---------------------------------------------------------------------------------------
+// Level l groups 2^l fine cells per axis (Morton code >> 3 l). Position m is the first of its level-l cell for
+// every l below first_levels(m): the highest bit in which its code differs from the previous position's tells
+// all levels at once, so one pass over the codes serves the whole pyramid. The counting and ranking kernels
+// walk tiles of LV_TILE positions, position base + 256 r + thread, so a group of 64 positions is one wave's
+// round r and a level's ranks come from ballots.
+//
+// Bound: launches on small clouds, the inserts' random lines on large ones. A flag pass, a scan (one to three
+// launches), a starts pass and an insert pass per level were 45-80 launches per grid build, now 4-5. Whole calls:
+// 1,500 points 2.45 -> 2.26 ms, 100,000 points (k=40, 150 iterations) 4.80 -> 4.58, 1M points (k=16, 50
+// iterations, normals) 8.85 -> 8.31, 192 clouds of 20M points 145.8 -> 138.8.
+constexpr int LV_ITEMS = 8;
+constexpr int LV_TILE = BLK * LV_ITEMS;  // 2048
+constexpr int LV_GROUPS = LV_TILE / 64;  // 32
+
+__device__ inline int first_levels(const uint32_t* __restrict__ code, const int32_t* __restrict__ mcloud, int64_t m,
+                                   int64_t n, int nl) {
+    if (m >= n) return 0;
+    if (m == 0 || (mcloud && mcloud[m] != mcloud[m - 1])) return nl;
+    const uint32_t x = code[m] ^ code[m - 1];
+    return x ? min(nl, (31 - __builtin_clz(x)) / 3 + 1) : 0;
 }
 
-__global__ void __launch_bounds__(BLK) k_level_starts(const uint32_t* __restrict__ flag,
-                                                       const uint32_t* __restrict__ seg, int64_t n,
+// Cells that start in each tile: cnt[l * nb + tile].
+__global__ void __launch_bounds__(BLK) k_level_count(const uint32_t* __restrict__ code,
+                                                      const int32_t* __restrict__ mcloud, int64_t n, int nl, int nb,
+                                                      uint32_t* __restrict__ cnt) {
+    __shared__ uint32_t s[EGT_MAX_LEVELS];
+    if (threadIdx.x < EGT_MAX_LEVELS) s[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * LV_TILE + threadIdx.x;
+    int fl[LV_ITEMS];
+#pragma unroll
+    for (int r = 0; r < LV_ITEMS; ++r) fl[r] = first_levels(code, mcloud, base + r * BLK, n, nl);
+    for (int l = 0; l < nl; ++l) {
+        uint32_t c = 0;
+#pragma unroll
+        for (int r = 0; r < LV_ITEMS; ++r) c += (uint32_t)__popcll(__ballot(fl[r] > l));
+        if (__lane_id() == 0) atomicAdd(&s[l], c);
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nl) cnt[(int64_t)threadIdx.x * nb + blockIdx.x] = s[threadIdx.x];
+}
+
+// Exclusive prefix over the tiles of each level, in place (one block per level); the level's cell count goes
+// to total[l * stride].
+constexpr int LVS_BLK = 1024;
+__global__ void __launch_bounds__(LVS_BLK) k_level_scan(uint32_t* __restrict__ cnt, int nb, uint32_t* __restrict__ total,
+                                                         int stride) {
+    __shared__ uint32_t ws[LVS_BLK / 64];
+    uint32_t* c = cnt + (int64_t)blockIdx.x * nb;
+    const int lane = __lane_id(), wid = threadIdx.x / 64;
+    uint32_t run = 0;
+    for (int b0 = 0; b0 < nb; b0 += LVS_BLK) {
+        const int i = b0 + (int)threadIdx.x;
+        const uint32_t v = i < nb ? c[i] : 0u;
+        uint32_t x = v;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(x, d, 64);
+            if (lane >= d) x += o;
+        }
+        if (lane == 63) ws[wid] = x;
+        __syncthreads();
+        uint32_t off = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < LVS_BLK / 64; ++w) {
+            if (w < wid) off += ws[w];
+            all += ws[w];
+        }
+        if (i < nb) c[i] = run + off + x - v;
+        run += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) total[(int64_t)blockIdx.x * stride] = run;
+}
+
+// First position of every cell of every level: starts + soff[l], in Morton order.
+struct LevelStarts {
+    uint64_t soff[EGT_MAX_LEVELS];
+};
+__global__ void __launch_bounds__(BLK) k_level_starts(const uint32_t* __restrict__ code,
+                                                       const int32_t* __restrict__ mcloud, int64_t n, int nl, int nb,
+                                                       const uint32_t* __restrict__ pre, LevelStarts S,
                                                        uint32_t* __restrict__ starts) {
-    const int64_t m = (int64_t)blockIdx.x * BLK + threadIdx.x;
-    if (m >= n) return;
-    if (flag[m]) starts[seg[m]] = (uint32_t)m;
+    __shared__ uint32_t g[EGT_MAX_LEVELS][LV_GROUPS];
+    const int lane = __lane_id(), wid = threadIdx.x / 64;
+    const int64_t base = (int64_t)blockIdx.x * LV_TILE + threadIdx.x;
+    int fl[LV_ITEMS];
+#pragma unroll
+    for (int r = 0; r < LV_ITEMS; ++r) fl[r] = first_levels(code, mcloud, base + r * BLK, n, nl);
+    for (int l = 0; l < nl; ++l) {
+#pragma unroll
+        for (int r = 0; r < LV_ITEMS; ++r) {
+            const uint32_t c = (uint32_t)__popcll(__ballot(fl[r] > l));
+            if (lane == 0) g[l][r * (BLK / 64) + wid] = c;
+        }
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nl) {
+        uint32_t run = pre[(int64_t)threadIdx.x * nb + blockIdx.x];
+        for (int i = 0; i < LV_GROUPS; ++i) {
+            const uint32_t c = g[threadIdx.x][i];
+            g[threadIdx.x][i] = run;
+            run += c;
+        }
+    }
+    __syncthreads();
+    const uint64_t lt = (1ull << lane) - 1ull;
+    for (int l = 0; l < nl; ++l) {
+#pragma unroll
+        for (int r = 0; r < LV_ITEMS; ++r) {
+            const uint64_t b = __ballot(fl[r] > l);
+            if (fl[r] > l)
+                starts[S.soff[l] + g[l][r * (BLK / 64) + wid] + (uint32_t)__popcll(b & lt)] =
+                    (uint32_t)(base + r * BLK);
+        }
+    }
 }
 
-__global__ void __launch_bounds__(BLK) k_level_insert(const uint32_t* __restrict__ starts, int64_t cells,
-                                                       int64_t n, const uint32_t* __restrict__ code,
-                                                       const int32_t* __restrict__ mcloud, int shift,
-                                                       uint4* __restrict__ tab, uint64_t offset, uint32_t log2cap,
+// Running cell count of every level at each cloud's first position, one wave per cloud:
+// out[l * (nclouds + 2) + 1 + c] (entry 0 of a level holds its total, entry nclouds + 1 gets it again).
+__global__ void __launch_bounds__(64) k_cells_at_bases(const uint32_t* __restrict__ code,
+                                                        const int32_t* __restrict__ mcloud, int64_t n, int nl, int nb,
+                                                        const uint32_t* __restrict__ pre,
+                                                        const CloudDev* __restrict__ clouds, int nclouds,
+                                                        uint32_t* __restrict__ out) {
+    const int c = blockIdx.x, lane = threadIdx.x;
+    if (c == nclouds) {
+        if (lane < nl) out[(int64_t)lane * (nclouds + 2) + 1 + c] = out[(int64_t)lane * (nclouds + 2)];
+        return;
+    }
+    const int64_t base = clouds[c].base, t0 = base / LV_TILE * LV_TILE;
+    uint32_t v[EGT_MAX_LEVELS] = {};
+    for (int64_t m0 = t0; m0 < base; m0 += 64) {
+        const int64_t m = m0 + lane;
+        const int fl = m < base ? first_levels(code, mcloud, m, n, nl) : 0;
+#pragma unroll
+        for (int l = 0; l < EGT_MAX_LEVELS; ++l) v[l] += (uint32_t)__popcll(__ballot(fl > l));
+    }
+#pragma unroll
+    for (int l = 0; l < EGT_MAX_LEVELS; ++l)
+        if (l < nl && lane == 0) out[(int64_t)l * (nclouds + 2) + 1 + c] = pre[(int64_t)l * nb + t0 / LV_TILE] + v[l];
+}
+
+// Inserts the cells of every level (thread i: cell i - first[l] of the level l whose range holds i), one CAS
+// per cell into a random slot. The level's largest cell is kept by one atomic per wave, and only by a wave that
+// exceeds the value read first: with one unconditional atomic per wave, every wave of a level queued at one
+// address (1M points: 411 us for the 11 levels, 158 us now; 4M points: 905 -> 347).
+struct LevelInsert {
+    int64_t first[EGT_MAX_LEVELS + 1];  // first thread of each level; first[nl] = all cells
+    uint64_t soff[EGT_MAX_LEVELS];      // the level's cell starts
+    uint64_t offset[EGT_MAX_LEVELS];    // the level's table
+    uint32_t log2cap[EGT_MAX_LEVELS];
+    int nl;
+};
+__device__ inline void max_if_larger(int* p, int v) {
+    if (v > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p, v);
+}
+__global__ void __launch_bounds__(BLK) k_level_insert(LevelInsert P, const uint32_t* __restrict__ starts, int64_t n,
+                                                       const uint32_t* __restrict__ code,
+                                                       const int32_t* __restrict__ mcloud, uint4* __restrict__ tab,
                                                        int* __restrict__ maxc) {
-    const int64_t c = (int64_t)blockIdx.x * BLK + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * BLK + threadIdx.x;
+    int l = 0;
+    for (int j = 1; j < P.nl; ++j) l += i >= P.first[j] ? 1 : 0;
     int cnt = 0;
-    if (c < cells) {
-        const uint32_t st = starts[c];
-        const uint32_t en = c + 1 < cells ? starts[c + 1] : (uint32_t)n;
-        const unsigned long long cc = cell_key(mcloud ? (uint32_t)mcloud[st] : 0u, code[st] >> shift);
-        const uint32_t mask = (1u << log2cap) - 1u;
+    if (i < P.first[P.nl]) {
+        const int64_t c = i - P.first[l];
+        const uint32_t* st_l = starts + P.soff[l];
+        const uint32_t st = st_l[c];
+        const uint32_t en = i + 1 < P.first[l + 1] ? st_l[c + 1] : (uint32_t)n;
+        const unsigned long long cc = cell_key(mcloud ? (uint32_t)mcloud[st] : 0u, code[st] >> (3 * l));
+        const uint32_t log2cap = P.log2cap[l], mask = (1u << log2cap) - 1u;
         uint32_t s = hash_slot(cc, log2cap);
         // a table has at least twice as many slots as cells, so an empty slot is always found
         for (;;) {
-            uint4* e = &tab[offset + s];
+            uint4* e = &tab[P.offset[l] + s];
             const unsigned long long prev =
                 atomicCAS(reinterpret_cast<unsigned long long*>(e), (unsigned long long)HASH_EMPTY, cc);
             if (prev == HASH_EMPTY) {
@@ -297,19 +441,15 @@ __global__ void __launch_bounds__(BLK) k_level_insert(const uint32_t* __restrict
         }
         cnt = (int)(en - st);
     }
-    // largest cell of the level: one atomic per wave (every cell used to hit the one address)
+    // levels ascend with the thread, so a wave that starts and ends in one level lies in it
+    const int l0 = __shfl(l, 0, 64);
+    if (__shfl(l, 63, 64) == l0) {
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) cnt = max(cnt, __shfl_xor(cnt, d, 64));
-    if (__lane_id() == 0) atomicMax(maxc, cnt);
-}
-
-// seg value at each cloud's first Morton position (running cell count), plus the total at the end.
-__global__ void __launch_bounds__(BLK) k_cells_at_bases(const uint32_t* __restrict__ seg, const CloudDev* __restrict__ clouds,
-                                                         int nclouds, const uint32_t* __restrict__ total,
-                                                         uint32_t* __restrict__ out) {
-    const int c = blockIdx.x * BLK + threadIdx.x;
-    if (c < nclouds) out[c] = seg[clouds[c].base];
-    if (c == nclouds) out[c] = *total;
+        for (int d = 32; d >= 1; d >>= 1) cnt = max(cnt, __shfl_xor(cnt, d, 64));
+        if (__lane_id() == 0) max_if_larger(&maxc[l0], cnt);
+    } else {
+        max_if_larger(&maxc[l], cnt);
+    }
 }
 
 __global__ void __launch_bounds__(BLK) k_fill_u64(uint64_t* __restrict__ p, uint64_t n, uint64_t v) {
@@ -568,35 +708,31 @@ void build_search_structure(egt_ctx* h) {
     LAUNCH_CHECK();
     const int32_t* mcl = batch ? h->mcloud.p : nullptr;
 
-    // level tables: level l groups 2^l fine cells per axis (Morton code >> 3l), per cloud. Counting pass, level
-    // by level without a host wait: a flag per Morton position (first of its cell), a scan whose total stays on
-    // the device, the cells' first positions (kept for the inserts) and, for a batch, the running count at
-    // each cloud's first position. One read-back of every level's counts then sizes the tables.
+    // level tables: every level's cells are counted, ranked and (below) inserted together; one read-back of the
+    // counts of the levels (and, in a batch, of the running counts at each cloud's first position) sizes the tables
     h->nlev = log2B + 1;
     const int nc = h->nclouds, nl = h->nlev;
-    DBuf<uint32_t>& flag = sc.bufs[9];
-    DBuf<uint32_t>& seg = sc.bufs[10];
-    flag.alloc(n);
-    seg.alloc(n);
     // room for the starts of every level: at most min(n, cells of the level's grid over all clouds) each
     std::vector<size_t> soff(nl + 1, 0);
+    LevelStarts ls{};
     for (int l = 0; l < nl; ++l) {
         const double grid_cells = (double)nc * std::pow((double)(h->B >> l), 3.0);
         soff[l + 1] = soff[l] + (size_t)std::min<double>((double)n, grid_cells);
+        ls.soff[l] = soff[l];
     }
     uint32_t* starts = sc.get<uint32_t>(38, soff[nl]);
+    const int nb = ceil_div(n, LV_TILE);
+    uint32_t* tiles = sc.get<uint32_t>(9, (size_t)nl * nb);
     uint32_t* dtot = sc.get<uint32_t>(23, (size_t)nl * (nc + 2));  // per level: total, then the cloud bases
-    for (int l = 0; l < nl; ++l) {
-        k_level_flags<<<ceil_div(n, BLK), BLK, 0, s>>>(h->mcode.p, mcl, n, 3 * l, flag.p);
+    k_level_count<<<nb, BLK, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles);
+    LAUNCH_CHECK();
+    k_level_scan<<<nl, LVS_BLK, 0, s>>>(tiles, nb, dtot, nc + 2);
+    LAUNCH_CHECK();
+    k_level_starts<<<nb, BLK, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles, ls, starts);
+    LAUNCH_CHECK();
+    if (batch) {
+        k_cells_at_bases<<<nc + 1, 64, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles, h->dclouds.p, nc, dtot);
         LAUNCH_CHECK();
-        uint32_t* tl = dtot + (size_t)l * (nc + 2);
-        exclusive_scan_u32_dev(flag.p, seg.p, n, s, sc, tl);
-        k_level_starts<<<ceil_div(n, BLK), BLK, 0, s>>>(flag.p, seg.p, n, starts + soff[l]);
-        LAUNCH_CHECK();
-        if (batch) {
-            k_cells_at_bases<<<ceil_div(nc + 1, BLK), BLK, 0, s>>>(seg.p, h->dclouds.p, nc, tl, tl + 1);
-            LAUNCH_CHECK();
-        }
     }
     std::vector<uint32_t> ht((size_t)nl * (nc + 2));
     HIP_CHECK(hipMemcpyAsync(ht.data(), dtot, ht.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
@@ -627,12 +763,17 @@ void build_search_structure(egt_ctx* h) {
     DBuf<uint32_t>& dmax = sc.bufs[14];
     dmax.alloc(nl);
     HIP_CHECK(hipMemsetAsync(dmax.p, 0, nl * sizeof(uint32_t), s));
+    LevelInsert li{};
+    li.nl = nl;
     for (int l = 0; l < nl; ++l) {
-        k_level_insert<<<std::max(1, ceil_div(cells[l], BLK)), BLK, 0, s>>>(
-            starts + soff[l], cells[l], n, h->mcode.p, mcl, 3 * l, h->htab.p, h->lev[l].offset, h->lev[l].log2cap,
-            reinterpret_cast<int*>(dmax.p) + l);
-        LAUNCH_CHECK();
+        li.first[l + 1] = li.first[l] + cells[l];
+        li.soff[l] = soff[l];
+        li.offset[l] = h->lev[l].offset;
+        li.log2cap[l] = h->lev[l].log2cap;
     }
+    k_level_insert<<<ceil_div(li.first[nl], BLK), BLK, 0, s>>>(li, starts, n, h->mcode.p, mcl, h->htab.p,
+                                                               reinterpret_cast<int*>(dmax.p));
+    LAUNCH_CHECK();
     std::vector<int32_t> mx(nl);
     HIP_CHECK(hipMemcpyAsync(mx.data(), dmax.p, nl * sizeof(int32_t), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
