@@ -95,7 +95,8 @@ struct KnnParams {
     unsigned long long* __restrict__ queue;  // work-queue counter (persistent launch) or null
     int32_t* __restrict__ knn;             // rows, cloud after cloud, local sorted indices
     float* __restrict__ kth;               // per sorted point: k-th distance of valid rows, else -1
-    unsigned long long* __restrict__ counters;  // [0] candidates, [1] invalid rows, [2] learned, [3] fallbacks,
+    unsigned long long* __restrict__ counters;  // null: no statistics; else, followed by STAT_SLOTS copies of the
+                                                // statistics (see stat_slot): [0] candidates, [1] invalid rows, [2] learned, [3] fallbacks,
                                                 // [4] cells looked up, [5] work queue, [6] queries handed
                                                 // back (retry list length), [7] keys inserted into the lists,
                                                 // [8] most candidates of a query, [9] long queries handed on
@@ -114,6 +115,37 @@ struct KnnParams {
     uint32_t bigmask;  // levels holding a cell with >= maxc points (any cloud)
     float a, ba;
 };
+
+// Statistics of a search: every wave adds its sums to one of STAT_SLOTS copies of the counters (a 128-byte line
+// each, chosen by workgroup), and k_stats_sum folds the copies once per search. With one shared copy, the waves'
+// atomics on the same few addresses were served one after another, 37 ns a wave whatever the wave did, which
+// bound every search of short waves: one query per wave took 37 ms per million queries on every cloud and k, and
+// the pass over 650,000 queries handed back on a 16M-point cluster mixture 24.2 of the call's 182 ms.
+constexpr int STAT_SLOTS = 512, STAT_WORDS = 16;
+__device__ inline unsigned long long* stat_slot(const KnnParams& P) {
+    return P.counters ? P.counters + (size_t)(1 + (blockIdx.x & (STAT_SLOTS - 1))) * STAT_WORDS : nullptr;
+}
+__global__ void __launch_bounds__(STAT_SLOTS) k_stats_sum(const unsigned long long* __restrict__ slots,
+                                                           unsigned long long* __restrict__ counters) {
+    __shared__ unsigned long long part[STAT_SLOTS / 64][STAT_WORDS];
+    const int lane = __lane_id(), wid = threadIdx.x / 64;
+    for (int i = 0; i < 10; ++i) {
+        if (i == 5 || i == 6) continue;  // work queue and hand-back list: kept in the counters themselves
+        unsigned long long v = slots[(size_t)threadIdx.x * STAT_WORDS + i];
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) {
+            const unsigned long long o = __shfl_xor(v, d, 64);
+            v = i == 8 ? (o > v ? o : v) : v + o;
+        }
+        if (lane == 0) part[wid][i] = v;
+    }
+    __syncthreads();
+    const int i = threadIdx.x;
+    if (i >= 10 || i == 5 || i == 6) return;
+    unsigned long long v = 0;
+    for (int w = 0; w < STAT_SLOTS / 64; ++w) v = i == 8 ? (part[w][i] > v ? part[w][i] : v) : v + part[w][i];
+    counters[i] = v;
+}
 
 // FP64 min / max as single instructions. The keys are never NaN, so the quieting the compiler adds to keep
 // IEEE minNum semantics for arbitrary inputs (one more v_max_f64 per operand) is not needed.
@@ -555,7 +587,7 @@ __global__ void __launch_bounds__(KBLK)
         }
     }
     }
-    // one atomic per wave
+    // one atomic per wave and statistic
     unsigned long long c0 = cand;
     uint32_t c1 = invalid_row, c2 = learned, c3 = fallback, c4 = cells, c7 = inserted, c8 = most, c9 = nlong;
 #pragma unroll
@@ -569,15 +601,16 @@ __global__ void __launch_bounds__(KBLK)
         c2 += __shfl_xor(c2, d, 64);
         c3 += __shfl_xor(c3, d, 64);
     }
-    if (__lane_id() == 0) {
-        if (c0) atomicAdd(&P.counters[0], c0);
-        if (c1) atomicAdd(&P.counters[1], (unsigned long long)c1);
-        if (c2) atomicAdd(&P.counters[2], (unsigned long long)c2);
-        if (c3) atomicAdd(&P.counters[3], (unsigned long long)c3);
-        if (c4) atomicAdd(&P.counters[4], (unsigned long long)c4);
-        if (c7) atomicAdd(&P.counters[7], (unsigned long long)c7);
-        if (c8) atomicMax(&P.counters[8], (unsigned long long)c8);
-        if (c9) atomicAdd(&P.counters[9], (unsigned long long)c9);
+    unsigned long long* const st = stat_slot(P);
+    if (st && __lane_id() == 0) {
+        if (c0) atomicAdd(&st[0], c0);
+        if (c1) atomicAdd(&st[1], (unsigned long long)c1);
+        if (c2) atomicAdd(&st[2], (unsigned long long)c2);
+        if (c3) atomicAdd(&st[3], (unsigned long long)c3);
+        if (c4) atomicAdd(&st[4], (unsigned long long)c4);
+        if (c7) atomicAdd(&st[7], (unsigned long long)c7);
+        if (c8) atomicMax(&st[8], (unsigned long long)c8);
+        if (c9) atomicAdd(&st[9], (unsigned long long)c9);
     }
 }
 
@@ -1015,14 +1048,15 @@ __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) 
     uint32_t c4 = ncells;
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) c4 += __shfl_xor(c4, d, 64);
-    if (lane == 0) {
-        if (ncand) atomicAdd(&P.counters[0], (unsigned long long)ncand);
-        if (ninvalid) atomicAdd(&P.counters[1], (unsigned long long)ninvalid);
-        if (nlearned) atomicAdd(&P.counters[2], (unsigned long long)nlearned);
-        if (nfallback) atomicAdd(&P.counters[3], (unsigned long long)nfallback);
-        if (c4) atomicAdd(&P.counters[4], (unsigned long long)c4);
-        if (nins) atomicAdd(&P.counters[7], (unsigned long long)nins);
-        if (most) atomicMax(&P.counters[8], (unsigned long long)most);
+    unsigned long long* const st = stat_slot(P);
+    if (st && lane == 0) {
+        if (ncand) atomicAdd(&st[0], (unsigned long long)ncand);
+        if (ninvalid) atomicAdd(&st[1], (unsigned long long)ninvalid);
+        if (nlearned) atomicAdd(&st[2], (unsigned long long)nlearned);
+        if (nfallback) atomicAdd(&st[3], (unsigned long long)nfallback);
+        if (c4) atomicAdd(&st[4], (unsigned long long)c4);
+        if (nins) atomicAdd(&st[7], (unsigned long long)nins);
+        if (most) atomicMax(&st[8], (unsigned long long)most);
     }
 }
 
@@ -1210,7 +1244,9 @@ KnnParams knn_params(egt_ctx* h, bool scratch = true) {
     P.mcloud = h->nclouds > 1 ? h->mcloud.p : nullptr;
     P.knn = h->knn.p;
     P.kth = scratch ? h->scratch.get<float>(15, h->n) : nullptr;
-    P.counters = scratch ? reinterpret_cast<unsigned long long*>(h->scratch.get<uint64_t>(14, 10)) : nullptr;
+    P.counters = scratch ? reinterpret_cast<unsigned long long*>(
+                               h->scratch.get<uint64_t>(14, (size_t)STAT_WORDS * (STAT_SLOTS + 1)))
+                         : nullptr;
     P.queue = nullptr;
     P.bigmask = 0;
     for (int l = 0; l < h->nlev; ++l)
@@ -1232,6 +1268,17 @@ KnnParams knn_params(egt_ctx* h, bool scratch = true) {
     P.ba = (1.0f + h->eps) - P.a;
     P.stride = 1;
     return P;
+}
+
+// Clears a search's statistics, and reads them back (10 counters; synchronizes the stream).
+void clear_stats(const KnnParams& P, hipStream_t s) {
+    HIP_CHECK(hipMemsetAsync(P.counters, 0, (size_t)STAT_WORDS * (STAT_SLOTS + 1) * sizeof(uint64_t), s));
+}
+void read_stats(const KnnParams& P, uint64_t (&hc)[10], hipStream_t s) {
+    k_stats_sum<<<1, STAT_SLOTS, 0, s>>>(P.counters + STAT_WORDS, P.counters);
+    LAUNCH_CHECK();
+    HIP_CHECK(hipMemcpyAsync(hc, P.counters, sizeof(hc), hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipStreamSynchronize(s));
 }
 
 // Work lists per neighbour-count class: chunks of 64 Morton-consecutive queries that never straddle two
@@ -1290,7 +1337,7 @@ void run_knn_clouds(egt_ctx* h) {
     KnnParams P = knn_params(h);
     const std::vector<WorkClass> classes = build_work_lists(h, h->work_lists);
     h->work_classes = classes;
-    HIP_CHECK(hipMemsetAsync(P.counters, 0, 10 * sizeof(uint64_t), s));
+    clear_stats(P, s);
     Event e0, e1;
     HIP_CHECK(hipEventRecord(e0, s));
     int64_t handed_back = 0;
@@ -1301,8 +1348,7 @@ void run_knn_clouds(egt_ctx* h) {
     }
     HIP_CHECK(hipEventRecord(e1, s));
     uint64_t hc[10];
-    HIP_CHECK(hipMemcpyAsync(hc, P.counters, sizeof(hc), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    read_stats(P, hc, s);
     HIP_CHECK(hipEventElapsedTime(&h->stats.knn_ms, e0, e1));
     h->stats.learned_bound_retries = handed_back - (int64_t)hc[9];
     h->stats.knn_insertions = (int64_t)hc[7];
@@ -1336,7 +1382,7 @@ void run_knn_query(egt_ctx* h, const float* dqx, const float* dqy, const float* 
     h->qvcell.alloc((size_t)std::max<int64_t>(nq, 1));
     KnnParams P = knn_params(h);
     P.long_cap = 0;
-    HIP_CHECK(hipMemsetAsync(P.counters, 0, 10 * sizeof(uint64_t), s));
+    clear_stats(P, s);
     Event e0, e1;
     HIP_CHECK(hipEventRecord(e0, s));
     CloudDev qcd{};
@@ -1375,9 +1421,8 @@ void run_knn_query(egt_ctx* h, const float* dqx, const float* dqy, const float* 
         launch_any(P, kclass(k), s, true);
     }
     HIP_CHECK(hipEventRecord(e1, s));
-    uint64_t hc[5];
-    HIP_CHECK(hipMemcpyAsync(hc, P.counters, sizeof(hc), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));  // also keeps qcd alive until its copy has run
+    uint64_t hc[10];
+    read_stats(P, hc, s);  // the wait also keeps qcd alive until its copy has run
     HIP_CHECK(hipEventElapsedTime(&h->stats.query_ms, e0, e1));
     h->stats.query_count = nq;
     h->stats.query_k = k;
@@ -1397,14 +1442,8 @@ void run_knn_query_original(egt_ctx* h, int32_t* out) {
     HIP_CHECK(hipStreamSynchronize(s));
 }
 
-// Counters of the search kernel (KnnParams::counters) in the allocation-free query search's scratch.
-constexpr int QNA_COUNTERS = 16;
-static_assert(QNA_COUNTERS >= 9, "every counter k_knn writes");
-
-// Clears the counters and writes the query set's cloud entry (kernel arguments, so the sequence holds no host
-// copy and no memset).
-__global__ void k_qna_init(unsigned long long* __restrict__ counters, CloudDev* __restrict__ cloud, CloudDev c) {
-    if (threadIdx.x < QNA_COUNTERS) counters[threadIdx.x] = 0ull;
+// Writes the query set's cloud entry (a kernel argument, so the sequence holds no host copy).
+__global__ void k_qna_init(CloudDev* __restrict__ cloud, CloudDev c) {
     if (threadIdx.x == 0) *cloud = c;
 }
 
@@ -1441,13 +1480,13 @@ uint32_t* qna_scratch(int dev) {
 // no host copy and no synchronization; the work is queued on the handle's stream. Layout in 32-bit words,
 // NQ = QNA_MAX_QUERIES: normalized queries (4 NQ), their virtual cells (2 NQ), sort keys (NQ) and values
 // (NQ), the queries in Morton order (4 NQ; the radix sort's workspace before they are written), their cells
-// (2 NQ), then the counters and the query set's cloud entry.
+// (2 NQ), then the query set's cloud entry. It keeps no statistics.
 void run_knn_query_noalloc(egt_ctx* h, const float* dqx, const float* dqy, const float* dqz, int64_t nq, int k,
                            float thres_n, int32_t* rows) {
     if (nq <= 0) return;
     if (nq > QNA_MAX_QUERIES) throw ArgError{EGT_ERR_UNSUPPORTED, "more queries than the scratch holds"};
     constexpr size_t NQ = (size_t)QNA_MAX_QUERIES;
-    static_assert(QNA_WORDS >= 14 * NQ + 2 * QNA_COUNTERS + (sizeof(CloudDev) + 3) / 4, "scratch layout");
+    static_assert(QNA_WORDS >= 14 * NQ + (sizeof(CloudDev) + 3) / 4, "scratch layout");
     if (radix_sort_workspace_words(nq) > 4 * NQ) throw ArgError{EGT_ERR_UNSUPPORTED, "sort workspace"};
     uint32_t* w = qna_scratch(h->device);
     float4* qn = reinterpret_cast<float4*>(w);
@@ -1456,8 +1495,7 @@ void run_knn_query_noalloc(egt_ctx* h, const float* dqx, const float* dqy, const
     uint32_t* idx = w + 7 * NQ;
     float4* qpts = reinterpret_cast<float4*>(w + 8 * NQ);
     uint64_t* qcell = reinterpret_cast<uint64_t*>(w + 12 * NQ);
-    unsigned long long* counters = reinterpret_cast<unsigned long long*>(w + 14 * NQ);
-    CloudDev* qcloud = reinterpret_cast<CloudDev*>(w + 14 * NQ + 2 * QNA_COUNTERS);
+    CloudDev* qcloud = reinterpret_cast<CloudDev*>(w + 14 * NQ);
     hipStream_t s = h->stream;
     KnnParams P = knn_params(h, false);
     P.long_cap = 0;
@@ -1467,7 +1505,7 @@ void run_knn_query_noalloc(egt_ctx* h, const float* dqx, const float* dqy, const
     qcd.row_off = 0;
     qcd.k = k;
     qcd.thres_n = thres_n;
-    k_qna_init<<<1, 64, 0, s>>>(counters, qcloud, qcd);
+    k_qna_init<<<1, 64, 0, s>>>(qcloud, qcd);
     LAUNCH_CHECK();
     const int g = ceil_div(nq, KBLK);
     k_query_prep<<<g, KBLK, 0, s>>>(dqx, dqy, dqz, nq, h->min_extent, h->max_extent, P.a, P.ba, h->B, qn, cellp,
@@ -1480,7 +1518,6 @@ void run_knn_query_noalloc(egt_ctx* h, const float* dqx, const float* dqy, const
     P.qvcell = reinterpret_cast<const unsigned long long*>(qcell);
     P.knn = rows;
     P.kth = nullptr;
-    P.counters = counters;
     P.clouds = qcloud;
     P.mcloud = nullptr;
     P.qlevel = nullptr;
@@ -1515,7 +1552,7 @@ int autotune_shape(egt_ctx* h, int k, float thres_n, float* shape_ms) {
     h->clouds[0].thres_n = thres_n;
     prepare_clouds(h);
     KnnParams P = knn_params(h);
-    HIP_CHECK(hipMemsetAsync(P.counters, 0, 10 * sizeof(uint64_t), s));  // scratch holds earlier contents
+    clear_stats(P, s);  // scratch holds earlier contents
     const int64_t total = (h->n + 63) / 64;
     KnnParams W = P;  // warm-up: the autotuner's sample
     W.stride = (int)std::max<int64_t>(1, total / 8192);
@@ -1559,7 +1596,7 @@ int64_t autotune_class_shapes(egt_ctx* h, float* ms) {
     hipStream_t s = h->stream;
     prepare_clouds(h);
     KnnParams P = knn_params(h);
-    HIP_CHECK(hipMemsetAsync(P.counters, 0, 10 * sizeof(uint64_t), s));  // scratch holds earlier contents
+    clear_stats(P, s);  // scratch holds earlier contents
     const std::vector<WorkClass> classes = build_work_lists(h, h->work_lists);
     for (int i = 0; i < 24; ++i) ms[i] = -1.0f;
     Event e0, e1;
@@ -1614,7 +1651,7 @@ void autotune_learned(egt_ctx* h, int k, float thres_n, int* best_off, int* best
             h->learned_level_offset = off;
             h->learned_mode = mi == 0 ? 1 : 3;
             KnnParams P = knn_params(h);
-            HIP_CHECK(hipMemsetAsync(P.counters, 0, 10 * sizeof(uint64_t), s));
+            clear_stats(P, s);
             KnnParams W = P;
             W.stride = (int)std::max<int64_t>(1, total / 8192);
             W.nchunks = (total + W.stride - 1) / W.stride;
@@ -1668,13 +1705,12 @@ int autotune_start_level(egt_ctx* h, int k, float thres_n, float* trial_ms, floa
     double best_cost = 0.0;
     for (int l = -SUB; l <= top; ++l) {
         P.start_level = l + SUB;
-        HIP_CHECK(hipMemsetAsync(P.counters, 0, 10 * sizeof(uint64_t), s));
+        clear_stats(P, s);
         HIP_CHECK(hipEventRecord(e0, s));
         launch_any(P, K, s);
         HIP_CHECK(hipEventRecord(e1, s));
-        uint64_t hc[5];
-        HIP_CHECK(hipMemcpyAsync(hc, P.counters, sizeof(hc), hipMemcpyDeviceToHost, s));
-        HIP_CHECK(hipStreamSynchronize(s));
+        uint64_t hc[10];
+        read_stats(P, hc, s);
         float ms = 0.0f;
         HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
         const double q = (double)std::min<int64_t>(h->n, P.nchunks * 64);
