@@ -109,8 +109,11 @@ typedef enum {
                                     Which is faster depends on the cloud and k (try both with
                                     egt_autotune_shape). Rows do not depend on it */
     EGT_OPT_KNN_LANES = 8,       /* kNN self search: lanes per query, 1 = one lane per query with the list in its
-                                    registers (default), 64 = one wave per query with the list spread over the
-                                    lanes. Rows do not depend on it */
+                                    registers (default; where that shape leaves the GPU idle or short of
+                                    registers, few queries or k > 40, the library runs a wave per query, unless
+                                    EGT_OPT_KNN_LONG_QUERY is changed, a tuner chose the shape or
+                                    EGT_OPT_KNN_CLASS_SHAPES names it), 64 = one wave per query with the list
+                                    spread over the lanes. Rows do not depend on it */
     EGT_OPT_KNN_LONG_QUERY = 9,  /* kNN self search with one lane per query: a query that has tested more
                                     candidates than this is handed on to a wave-per-query pass (its wave no
                                     longer waits for it); 0 = never; default 2048. Rows do not depend on it */

@@ -344,6 +344,7 @@ egt_status egt_set_option(egt_handle h, egt_option opt, int64_t value) {
             return EGT_OK;
         case EGT_OPT_KNN_PERSISTENT:
             h->knn_persistent = value ? 1 : 0;
+            h->knn_shape_tuned = false;
             return EGT_OK;
         case EGT_OPT_TAUBIN_TILE:
             if (value != 0 && value != 1024 && value != 2048)
@@ -360,6 +361,7 @@ egt_status egt_set_option(egt_handle h, egt_option opt, int64_t value) {
         case EGT_OPT_KNN_LANES:
             if (value != 1 && value != 64) return fail(EGT_ERR_INVALID_ARG, "kNN lanes per query must be 1 or 64");
             h->knn_lanes = (int)value;
+            h->knn_shape_tuned = false;
             return EGT_OK;
         case EGT_OPT_KNN_LONG_QUERY:
             if (value < 0 || value > UINT32_MAX) return fail(EGT_ERR_INVALID_ARG, "long-query cap must be in [0, 2^32)");

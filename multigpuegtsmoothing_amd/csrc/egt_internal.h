@@ -137,6 +137,8 @@ struct CloudDev {
     float max_extent;          // bounding cube upper end (as computed, not min_extent + extent)
 };
 
+constexpr int64_t KNN_LONG_CAP = 2048;  // default of EGT_OPT_KNN_LONG_QUERY
+
 // A neighbour-count class of a batch: its K template and its range in the chunk work list.
 struct WorkClass {
     int K;
@@ -233,7 +235,8 @@ struct egt_ctx {
     int learned_level_offset = 0;  // added to the proposed start levels
     int class_shape[8] = {-1, -1, -1, -1, -1, -1, -1, -1};  // per neighbour-count class (k <= 8, 16, .., 64):
                                                            // 0 lane, 1 persistent, 2 wave; -1 handle-wide
-    int64_t knn_long_cap = 2048;  // lane-per-query search: candidates after which a query goes to a wave
+    bool knn_shape_tuned = false;  // a tuner chose the handle-wide shape: it holds for every size
+    int64_t knn_long_cap = egt::KNN_LONG_CAP;  // lane-per-query search: candidates after which a query goes to a wave
                                   // (0 = never)
     int taubin_graph = 1;
     int taubin_tile = 1024;  // Taubin tile width: 1024 or 2048 points; 0 = tune on the next smoothing call

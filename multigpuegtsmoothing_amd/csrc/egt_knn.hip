@@ -104,6 +104,7 @@ struct KnnParams {
     const float4* __restrict__ qpts;       // query search: queries in Morton order (x', y', z', bits(index))
     const unsigned long long* __restrict__ qvcell;  // query search: virtual cell, clamped to the grid
     int64_t nchunks;   // chunks in the work list (after sampling)
+    int qpw;           // wave-per-query search: queries a wave serves one after another (1, 2, 4, 8 or 16)
     int stride;        // 1 = every chunk; s > 1 = every s-th chunk of the list (sampled trial runs)
     int B, log2B, stages, maxc;
     int Bv;            // cells per axis at internal level 0 (B << SUB)
@@ -777,23 +778,27 @@ __device__ inline int wave_cell_test(const KnnParams& P, int lv, const int (&c)[
 // (387 v_readlane), and the search runs faster with the same rows: the mixture at k=64 from learned starts
 // 68.7 -> 62.7 ms, from the own cell 97.2 -> 89.6; k=40 from the own cell 82.1 -> 75.8 (learned starts 55.9 ->
 // 56.3); a 4M-point torus at level 2 11.2 -> 10.2 (k=40) and 13.4 -> 12.0 ms (k=64). 7 waves: in between.
-template <bool LIST>
+// QUERY: the query search (see k_knn for where it differs).
+template <bool LIST, bool QUERY = false>
 __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) k_knn_wave(KnnParams P) {
+    static_assert(!(LIST && QUERY), "a list holds queries of the self search");
     const int lane = __lane_id();
     const int64_t v = blockIdx.x;
-    if (v >= P.nchunks) return;
     // wave index made uniform for the compiler, so the query's values live in scalar registers
     const int wv_id = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     __shared__ int wmark[KBLK / 64][64];  // per wave: the entry whose run starts at each slot of a batch
     int64_t m0, m1;
     if (LIST) {
-        m0 = v * (KBLK / 64) + wv_id;
-        m1 = min<int64_t>(m0 + 1, P.nlist);
+        m0 = (v * (KBLK / 64) + wv_id) * P.qpw;
+        m1 = min<int64_t>(m0 + P.qpw, P.nlist);
     } else {
-        const int64_t start = P.chunks ? P.chunks[v * P.stride] : v * P.stride * 64;
+        const int per = 16 / P.qpw;  // workgroups per chunk of 64 queries
+        const int64_t chunk = v / per;
+        if (chunk >= P.nchunks) return;
+        const int64_t start = P.chunks ? P.chunks[chunk * P.stride] : chunk * P.stride * 64;
         const CloudDev& c0 = P.clouds[P.mcloud ? (uint32_t)P.mcloud[start] : 0u];
-        m0 = start + (int64_t)wv_id * 16;
-        m1 = min<int64_t>(min<int64_t>(m0 + 16, start + 64), c0.base + c0.n);
+        m0 = start + ((v - chunk * per) * (KBLK / 64) + wv_id) * P.qpw;
+        m1 = min<int64_t>(m0 + P.qpw, c0.base + c0.n);
     }
     uint64_t ncand = 0;
     uint32_t ncells = 0, nins = 0, ninvalid = 0, nlearned = 0, nfallback = 0, most = 0;
@@ -811,11 +816,17 @@ __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) 
         const float thres_n = cd.thres_n;
         const int64_t cend = cd.base + cd.n;
         const uint64_t cand0 = ncand;
-        const float4 q = P.mpts[m];
+        const float4 q = QUERY ? P.qpts[m] : P.mpts[m];
         const int32_t jq = __float_as_int(q.w);
-        const uint64_t qvc = P.mvcell[m];
+        const uint64_t qvc = QUERY ? P.qvcell[m] : P.mvcell[m];
         const int vq[3] = {vcell_axis(qvc, 0), vcell_axis(qvc, 1), vcell_axis(qvc, 2)};
         const float qv[3] = {q.x, q.y, q.z};
+        bool outside = false;  // query search: the query's own (unclamped) cell lies outside the grid
+        if (QUERY) {
+            const int ux = cell_of(q.x, P.a, P.ba, P.B), uy = cell_of(q.y, P.a, P.ba, P.B),
+                      uz = cell_of(q.z, P.a, P.ba, P.B);
+            outside = ux < 0 || uy < 0 || uz < 0 || ux >= P.B || uy >= P.B || uz >= P.B;
+        }
         int own_level = P.start_level;
         if (P.qlevel) {
             own_level = (int)P.qlevel[m] + SUB + P.level_offset;
@@ -837,7 +848,7 @@ __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) 
             const bool in_grid = lane < 27 && c3[0] >= 0 && c3[1] >= 0 && c3[2] >= 0 && c3[0] < Bl &&
                                  c3[1] < Bl && c3[2] < Bl;
             // early exit of k_knn: the reference's next stage does not exist or meets a cell of >= maxc points
-            if (level > first_level && level > SUB) {
+            if (level > first_level && level > SUB && !outside) {
                 const int rl = level - SUB;
                 if (rl >= P.stages) break;
                 if ((P.bigmask >> rl) & 1u) {
@@ -936,10 +947,10 @@ __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) 
                     rem -= (uint32_t)take;
                     uint64_t kk = KEY_EMPTY;
                     bool tested = false;
-                    if (p >= cd.base && p < cend) {
+                    if (QUERY ? p >= 0 : (p >= cd.base && p < cend)) {
                         const float4 e4 = P.mpts[p];
                         const int32_t j = __float_as_int(e4.w);
-                        bool ok = j != jq;
+                        bool ok = QUERY || j != jq;
                         if (ok && eo) {
                             const uint32_t cc = P.mcell[p];
                             const int ex0 = (int)(cc & 1023u) << SUB, ey0 = (int)((cc >> 10) & 1023u) << SUB,
@@ -951,7 +962,8 @@ __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) 
                         if (ok) {
                             tested = true;
                             const float d = sqd(q.x, q.y, q.z, e4.x, e4.y, e4.z);
-                            if (d <= thres_n) kk = ((uint64_t)__float_as_uint(d) << 32) | (uint32_t)j;
+                            if (QUERY ? d < thres_n : d <= thres_n)
+                                kk = ((uint64_t)__float_as_uint(d) << 32) | (uint32_t)j;
                         }
                     }
                     ncand += (uint64_t)__builtin_popcountll(__ballot(tested));
@@ -1020,7 +1032,12 @@ __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) 
         for (int s = 0; s <= P.stages; ++s) {
             const int lvl = s == 0 ? 0 : s - 1;
             const int off = s == 0 ? 0 : 1;
-            const int cx = vq[0] >> (SUB + lvl), cy = vq[1] >> (SUB + lvl), cz = vq[2] >> (SUB + lvl);
+            int cx = vq[0] >> (SUB + lvl), cy = vq[1] >> (SUB + lvl), cz = vq[2] >> (SUB + lvl);
+            if (QUERY) {  // the reference's cell of the query at this level (GridKNNCuda.cu:351-353)
+                cx = cell_of(q.x, P.a, P.ba, P.B >> lvl);
+                cy = cell_of(q.y, P.a, P.ba, P.B >> lvl);
+                cz = cell_of(q.z, P.a, P.ba, P.B >> lvl);
+            }
             if ((P.bigmask >> lvl) & 1u) {
                 bool big = false;
                 if (s == 0) {
@@ -1034,14 +1051,15 @@ __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) 
                                          (my >> lvl) <= cy + off && (mz >> lvl) >= cz - off && (mz >> lvl) <= cz + off);
             const bool inside = __ballot(out) == 0;
             const int cst[3] = {cx, cy, cz};
-            if (inside && !ref_continue<false>(P, kq, thres_n, s, q.x, q.y, q.z, cst, c, kthd)) {
+            if (inside && !ref_continue<QUERY>(P, kq, thres_n, s, q.x, q.y, q.z, cst, c, kthd)) {
                 valid = true;
                 break;
             }
         }
         int32_t* row = P.knn + cd.row_off + (int64_t)(jq - cd.base) * kq;
-        if (lane < kq) row[lane] = (valid && listed) ? (int32_t)(uint32_t)mykey - (int32_t)cd.base : -1;
-        if (lane == 0) P.kth[jq] = (valid && c > 0) ? kthd : -1.0f;
+        const int32_t rbase = QUERY ? 0 : (int32_t)cd.base;  // query rows hold reference sorted indices
+        if (lane < kq) row[lane] = (valid && listed) ? (int32_t)(uint32_t)mykey - rbase : -1;
+        if (!QUERY && lane == 0) P.kth[jq] = (valid && c > 0) ? kthd : -1.0f;
         ninvalid += valid ? 0u : 1u;
         nfallback += fallback_q;
     }
@@ -1063,12 +1081,15 @@ __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) 
 // Query preparation: each query normalized with the reference cloud's extent (normalize_points
 // GridKNNCuda.cu:841-849: x' = (x - min) / (max - min)), its fine cell clamped to the grid and its virtual
 // cell inside that (the search boxes start there), and the Morton code of the fine cell as the sort key, so
-// a wave's 64 queries are spatial neighbours.
+// a wave's 64 queries are spatial neighbours (code null: queries searched in their own order). With qcloud, also
+// writes the query set's cloud entry.
 __global__ void __launch_bounds__(KBLK) k_query_prep(const float* __restrict__ qx, const float* __restrict__ qy,
                                                       const float* __restrict__ qz, int64_t nq, float mn, float mx,
                                                       float a, float ba, int B, float4* __restrict__ qn,
                                                       uint64_t* __restrict__ cellp, uint32_t* __restrict__ code,
-                                                      uint32_t* __restrict__ idx) {
+                                                      uint32_t* __restrict__ idx, CloudDev qcd,
+                                                      CloudDev* __restrict__ qcloud) {
+    if (qcloud && blockIdx.x == 0 && threadIdx.x == 0) *qcloud = qcd;
     const int64_t i = (int64_t)blockIdx.x * KBLK + threadIdx.x;
     if (i >= nq) return;
     const float d = mx - mn;
@@ -1076,10 +1097,12 @@ __global__ void __launch_bounds__(KBLK) k_query_prep(const float* __restrict__ q
     const int cx = min(max(cell_of(x, a, ba, B), 0), B - 1);
     const int cy = min(max(cell_of(y, a, ba, B), 0), B - 1);
     const int cz = min(max(cell_of(z, a, ba, B), 0), B - 1);
-    qn[i] = make_float4(x, y, z, 0.0f);
+    qn[i] = make_float4(x, y, z, __int_as_float((int32_t)i));
     cellp[i] = vcell_pack(vcoord(x, a, ba, B, cx), vcoord(y, a, ba, B, cy), vcoord(z, a, ba, B, cz));
-    code[i] = morton_code(cx, cy, cz);
-    idx[i] = (uint32_t)i;
+    if (code) {
+        code[i] = morton_code(cx, cy, cz);
+        idx[i] = (uint32_t)i;
+    }
 }
 
 __global__ void __launch_bounds__(KBLK) k_query_gather(const float4* __restrict__ qn, const uint64_t* __restrict__ cellp,
@@ -1157,13 +1180,65 @@ void launch_any(const KnnParams& P, int K, hipStream_t s, bool query = false, bo
     }
 }
 
-// Launch shape of a neighbour-count class: the handle's per-class choice (from the class tuner or
-// EGT_OPT_KNN_CLASS_SHAPES), else the handle-wide options. 0 = one lane per query, 1 = the same as one
-// persistent launch, 2 = one wave per query.
-int class_shape(const egt_ctx* h, int K) {
+// Queries a wave of the wave-per-query search serves one after another. More of them reuse the ranges of the last
+// box, fewer give more waves: a 10,000-point torus at k=40 0.105 ms with one query a wave against 0.117, 0.169 and
+// 0.513 with 2, 4 and 16; 150,000 points 0.958, 0.939, 0.965 and 1.194; 1.5M points 6.93, 6.65, 6.57 and 6.78;
+// 16M points (4 and 16) 52.1 and 53.3, a 16M-point cluster mixture 67.7 and 70.5.
+int queries_per_wave(int64_t queries) { return queries < 100000 ? 1 : queries < 300000 ? 2 : 4; }
+
+// Wave-per-query search of P.nchunks chunks of 64 queries.
+template <bool QUERY>
+void launch_wave(KnnParams P, hipStream_t s) {
+    P.qpw = queries_per_wave(P.nchunks * 64);
+    hipLaunchKernelGGL((k_knn_wave<false, QUERY>), dim3((unsigned)(P.nchunks * (16 / P.qpw))), dim3(KBLK), 0, s, P);
+    LAUNCH_CHECK();
+}
+
+// Launch shape of a search of `queries` queries in class K where nothing asks for one: a lane per query leaves the
+// GPU idle when the queries are few (its waves then last as long as their costliest lane) and runs two waves per
+// SIMD once the list passes 40 keys. Measured lane / wave in ms, from the own cell:
+//                            2,000          50,000         150,000        500,000        1.5M
+//   sphere   k=8                          0.52 / 0.33    0.64 / 0.80    1.40 / 2.46    3.27 / 5.61
+//   torus    k=16        0.72 / 0.046     0.64 / 0.34    0.66 / 0.76    1.37 / 2.21    3.09 / 5.54
+//   torus    k=40        0.89 / 0.050     0.85 / 0.39    0.96 / 0.94    2.36 / 2.72    5.64 / 6.57
+//   torus    k=48        0.92 / 0.050     0.93 / 0.41    1.49 / 0.97    3.26 / 2.81    8.67 / 6.95
+//   mixture  k=8         0.84 / 0.047     1.19 / 0.25    1.02 / 0.57    1.48 / 1.48    3.54 / 3.93
+//   mixture  k=16        1.01 / 0.047     1.89 / 0.29    1.66 / 0.64    1.98 / 1.73    4.12 / 4.51
+//   mixture  k=40        1.34 / 0.049     2.92 / 0.41    4.61 / 0.78    5.54 / 2.17    9.34 / 5.99
+// (4M-point torus and 16M-point mixture: k=40 14.3 / 16.3 and 57.0 / 67.7, k=48 21.0 / 17.3 and 87.5 / 71.6.)
+// Dense clusters make costly lanes, so an uneven cloud gains up to larger sizes: uneven is a cloud whose fullest
+// cell of 8 fine cells a side holds 64 times the mean of the non-empty ones (sphere and torus: up to 6 times,
+// mixture: over 200 times).
+bool wave_by_size(int K, int64_t queries, bool uneven) {
+    if (K >= 48) return true;
+    if (uneven) return queries <= (K <= 8 ? 400000 : K <= 16 ? 600000 : 2000000);
+    return queries <= (K <= 16 ? 80000 : 150000);
+}
+
+// The query search's shape. Up to QUERY_UNSORTED queries go to a wave each in their own order: the sort that makes
+// neighbours of a wave's queries is a dozen launches, which cost more than the locality gives. Lane / wave sorted /
+// wave unsorted in ms: 300 queries at k=1 in a 100,000-point sphere 0.37 / 0.090 / 0.030; in a 1M to 4M-point torus
+// 16,000 at k=16 0.67 / 0.18 / 0.087, 60,000 at k=1 0.45 / 0.28 / 0.16 and at k=40 1.05 / 0.45 / 0.33; 250,000 at
+// k=16 0.84 / 1.25 (a lane per query wins), at k=40 1.82 / 1.50.
+constexpr int64_t QUERY_UNSORTED = 100000;
+bool query_by_wave(int K, int64_t nq) { return nq <= QUERY_UNSORTED || wave_by_size(K, nq, false); }
+
+bool uneven_cloud(const egt_ctx* h) {
+    const LevelTable& L = h->lev[std::min(3, h->nlev - 1)];
+    return h->nclouds == 1 && (double)L.max_count * (double)L.cells >= 64.0 * (double)h->n;
+}
+
+// Launch shape of a neighbour-count class of `queries` queries: the handle's per-class choice (from the class
+// tuner or EGT_OPT_KNN_CLASS_SHAPES), else the handle-wide options, else (one lane per query by default, the long
+// query cap untouched, no shape tuned) the rule above. 0 = one lane per query, 1 = the same as one persistent
+// launch, 2 = one wave per query.
+int class_shape(const egt_ctx* h, int K, int64_t queries) {
     const int c = h->class_shape[K / 8 - 1];
     if (c >= 0) return c;
-    return h->knn_lanes == 64 ? 2 : (h->knn_persistent ? 1 : 0);
+    if (h->knn_lanes == 64) return 2;
+    if (h->knn_persistent) return 1;
+    if (h->knn_shape_tuned || h->knn_long_cap != KNN_LONG_CAP) return 0;
+    return wave_by_size(K, queries, uneven_cloud(h)) ? 2 : 0;
 }
 
 // One neighbour-count class: the search in the given launch shape, then the queries it handed back (fewer
@@ -1183,8 +1258,7 @@ int64_t search_class(egt_ctx* h, KnnParams P, int K, hipStream_t s, int shape) {
     if (hand_back) HIP_CHECK(hipMemsetAsync(P.counters + 6, 0, sizeof(uint64_t), s));  // the list's length
     if (shape == 2) {
         if (P.nchunks > 0) {
-            hipLaunchKernelGGL(k_knn_wave<false>, dim3((unsigned)P.nchunks), dim3(KBLK), 0, s, P);
-            LAUNCH_CHECK();
+            launch_wave<false>(P, s);
         }
     } else {
         launch_any(P, K, s);
@@ -1210,8 +1284,9 @@ int64_t search_class(egt_ctx* h, KnnParams P, int K, hipStream_t s, int shape) {
     R.nlist = (int64_t)nb;
     R.stride = 1;
     if (P.long_cap || shape == 2) {
-        R.nchunks = ceil_div((int64_t)nb, KBLK / 64);
-        hipLaunchKernelGGL(k_knn_wave<true>, dim3((unsigned)R.nchunks), dim3(KBLK), 0, s, R);
+        R.qpw = queries_per_wave((int64_t)nb);
+        hipLaunchKernelGGL((k_knn_wave<true, false>), dim3((unsigned)ceil_div((int64_t)nb, KBLK / 64 * R.qpw)),
+                           dim3(KBLK), 0, s, R);
         LAUNCH_CHECK();
     } else {
         R.nchunks = ((int64_t)nb + 63) / 64;
@@ -1344,7 +1419,7 @@ void run_knn_clouds(egt_ctx* h) {
     for (const WorkClass& cr : classes) {
         P.chunks = h->nclouds > 1 ? h->work_lists.p + cr.first : nullptr;
         P.nchunks = cr.count;
-        handed_back += search_class(h, P, cr.K, s, class_shape(h, cr.K));
+        handed_back += search_class(h, P, cr.K, s, class_shape(h, cr.K, cr.count * 64));
     }
     HIP_CHECK(hipEventRecord(e1, s));
     uint64_t hc[10];
@@ -1391,20 +1466,27 @@ void run_knn_query(egt_ctx* h, const float* dqx, const float* dqy, const float* 
     qcd.row_off = 0;
     qcd.k = k;
     qcd.thres_n = thres_n;
+    const int K = kclass(k);
+    const bool wave = query_by_wave(K, nq);
     if (nq > 0) {
-        float4* qn = h->scratch.get<float4>(32, nq);
-        uint64_t* cellp = h->scratch.get<uint64_t>(33, nq);
-        uint32_t* code = h->scratch.get<uint32_t>(34, nq);
-        uint32_t* idx = h->scratch.get<uint32_t>(35, nq);
         const int g = ceil_div(nq, KBLK);
-        k_query_prep<<<g, KBLK, 0, s>>>(dqx, dqy, dqz, nq, h->min_extent, h->max_extent, P.a, P.ba, h->B, qn, cellp,
-                                        code, idx);
-        LAUNCH_CHECK();
-        radix_sort_pairs(code, idx, nq, 30, s, h->scratch);
-        k_query_gather<<<g, KBLK, 0, s>>>(qn, cellp, idx, nq, h->qpts.p, h->qvcell.p);
-        LAUNCH_CHECK();
         h->dqcloud.alloc(1);
-        HIP_CHECK(hipMemcpyAsync(h->dqcloud.p, &qcd, sizeof(CloudDev), hipMemcpyHostToDevice, s));
+        if (wave && nq <= QUERY_UNSORTED) {
+            k_query_prep<<<g, KBLK, 0, s>>>(dqx, dqy, dqz, nq, h->min_extent, h->max_extent, P.a, P.ba, h->B, h->qpts.p,
+                                            h->qvcell.p, nullptr, nullptr, qcd, h->dqcloud.p);
+            LAUNCH_CHECK();
+        } else {
+            float4* qn = h->scratch.get<float4>(32, nq);
+            uint64_t* cellp = h->scratch.get<uint64_t>(33, nq);
+            uint32_t* code = h->scratch.get<uint32_t>(34, nq);
+            uint32_t* idx = h->scratch.get<uint32_t>(35, nq);
+            k_query_prep<<<g, KBLK, 0, s>>>(dqx, dqy, dqz, nq, h->min_extent, h->max_extent, P.a, P.ba, h->B, qn, cellp,
+                                            code, idx, qcd, h->dqcloud.p);
+            LAUNCH_CHECK();
+            radix_sort_pairs(code, idx, nq, 30, s, h->scratch);
+            k_query_gather<<<g, KBLK, 0, s>>>(qn, cellp, idx, nq, h->qpts.p, h->qvcell.p);
+            LAUNCH_CHECK();
+        }
         P.qpts = h->qpts.p;
         P.qvcell = reinterpret_cast<const unsigned long long*>(h->qvcell.p);
         P.knn = h->qknn.p;
@@ -1418,11 +1500,12 @@ void run_knn_query(egt_ctx* h, const float* dqx, const float* dqy, const float* 
         P.queue = nullptr;
         P.stride = 1;
         P.nchunks = (nq + 63) / 64;
-        launch_any(P, kclass(k), s, true);
+        if (wave) launch_wave<true>(P, s);
+        else launch_any(P, K, s, true);
     }
     HIP_CHECK(hipEventRecord(e1, s));
     uint64_t hc[10];
-    read_stats(P, hc, s);  // the wait also keeps qcd alive until its copy has run
+    read_stats(P, hc, s);
     HIP_CHECK(hipEventElapsedTime(&h->stats.query_ms, e0, e1));
     h->stats.query_count = nq;
     h->stats.query_k = k;
@@ -1440,11 +1523,6 @@ void run_knn_query_original(egt_ctx* h, int32_t* out) {
     LAUNCH_CHECK();
     HIP_CHECK(hipMemcpyAsync(out, tmp, cnt * sizeof(int32_t), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
-}
-
-// Writes the query set's cloud entry (a kernel argument, so the sequence holds no host copy).
-__global__ void k_qna_init(CloudDev* __restrict__ cloud, CloudDev c) {
-    if (threadIdx.x == 0) *cloud = c;
 }
 
 }  // namespace egt
@@ -1505,15 +1583,21 @@ void run_knn_query_noalloc(egt_ctx* h, const float* dqx, const float* dqy, const
     qcd.row_off = 0;
     qcd.k = k;
     qcd.thres_n = thres_n;
-    k_qna_init<<<1, 64, 0, s>>>(qcloud, qcd);
-    LAUNCH_CHECK();
     const int g = ceil_div(nq, KBLK);
-    k_query_prep<<<g, KBLK, 0, s>>>(dqx, dqy, dqz, nq, h->min_extent, h->max_extent, P.a, P.ba, h->B, qn, cellp,
-                                    code, idx);
-    LAUNCH_CHECK();
-    radix_sort_pairs_ws(code, idx, nq, 30, s, w + 8 * NQ);
-    k_query_gather<<<g, KBLK, 0, s>>>(qn, cellp, idx, nq, qpts, qcell);
-    LAUNCH_CHECK();
+    const int K = kclass(k);
+    const bool wave = query_by_wave(K, nq);
+    if (wave && nq <= QUERY_UNSORTED) {
+        k_query_prep<<<g, KBLK, 0, s>>>(dqx, dqy, dqz, nq, h->min_extent, h->max_extent, P.a, P.ba, h->B, qpts, qcell,
+                                        nullptr, nullptr, qcd, qcloud);
+        LAUNCH_CHECK();
+    } else {
+        k_query_prep<<<g, KBLK, 0, s>>>(dqx, dqy, dqz, nq, h->min_extent, h->max_extent, P.a, P.ba, h->B, qn, cellp,
+                                        code, idx, qcd, qcloud);
+        LAUNCH_CHECK();
+        radix_sort_pairs_ws(code, idx, nq, 30, s, w + 8 * NQ);
+        k_query_gather<<<g, KBLK, 0, s>>>(qn, cellp, idx, nq, qpts, qcell);
+        LAUNCH_CHECK();
+    }
     P.qpts = qpts;
     P.qvcell = reinterpret_cast<const unsigned long long*>(qcell);
     P.knn = rows;
@@ -1527,7 +1611,8 @@ void run_knn_query_noalloc(egt_ctx* h, const float* dqx, const float* dqy, const
     P.queue = nullptr;
     P.stride = 1;
     P.nchunks = (nq + 63) / 64;
-    launch_any(P, kclass(k), s, true);
+    if (wave) launch_wave<true>(P, s);
+    else launch_any(P, K, s, true);
 }
 
 // Autotuner for the search's start level (the cell size of the first search box). For each candidate level
@@ -1583,6 +1668,7 @@ int autotune_shape(egt_ctx* h, int k, float thres_n, float* shape_ms) {
     }
     h->knn_persistent = best == 1 ? 1 : 0;
     h->knn_lanes = best == 2 ? 64 : 1;
+    h->knn_shape_tuned = true;
     h->class_shape[K / 8 - 1] = -1;  // the handle-wide options now say it
     h->have_knn = false;  // the trial rows cover only the sample
     return best;
@@ -1679,6 +1765,7 @@ void autotune_learned(egt_ctx* h, int k, float thres_n, int* best_off, int* best
     h->learned_level_offset = *best_off;
     h->learned_mode = *best_mode;
     h->knn_lanes = *best_shape == 2 ? 64 : 1;
+    h->knn_shape_tuned = true;
     h->knn_persistent = 0;
     h->class_shape[K / 8 - 1] = -1;
     h->have_knn = false;  // as after the other tuners: the caller runs the search for its rows and statistics

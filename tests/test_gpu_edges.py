@@ -35,3 +35,52 @@ def test_batch_clouds_at_tile_edges(egt_mod, oracle_mod):
         og = O.Grid(*pts)
         np.testing.assert_array_equal(b.GetKNNIndexes(c), og.to_original(og.knn(12)[0]), err_msg=f"cloud {c}")
     b.close()
+
+
+@pytest.mark.parametrize("k", [8, 16, 24, 32, 40, 48, 56, 64])
+def test_lane_shape_on_small_clouds(egt_mod, oracle_mod, k):
+    """A lane per query (named through the class shapes) and the default (few queries: a wave per query) give the
+    oracle's rows on a cloud with dense cells."""
+    E, O = egt_mod, oracle_mod
+    print("k", k, flush=True)
+    pts = D.mixture(6_001, seed=500 + k)
+    og = O.Grid(*pts)
+    want = og.to_original(og.knn(k)[0])
+    for packed in (0, 1 << (2 * (k // 8 - 1))):
+        g = E.GridStructure(pts, 1, 1e-6, 1024, 4)
+        g.set_option(E.OPT_KNN_CLASS_SHAPES, packed)
+        g.GRIDCUDAKNNSELF_COMPACT(k, 1e8)
+        np.testing.assert_array_equal(g.GetKNNIndexes(), want, err_msg=f"class shapes {packed}")
+        g.close()
+
+
+@pytest.mark.parametrize("n,k", [(80_000, 16), (80_065, 16), (99_970, 8), (150_017, 40), (299_995, 48)])
+def test_self_search_at_shape_limits(egt_mod, oracle_mod, n, k):
+    """Sizes at the limits of the launch-shape rule and of the queries a wave serves (1, 2, 4)."""
+    E, O = egt_mod, oracle_mod
+    print("n", n, "k", k, flush=True)
+    pts = D.torus(n, seed=31)
+    g = E.GridStructure(pts, 1, 1e-6, 1024, 4)
+    g.set_option(E.OPT_START_LEVEL, E.START_LEVEL_OCCUPANCY)
+    g.GRIDCUDAKNNSELF_COMPACT(k, 1e8)
+    og = O.Grid(*pts)
+    np.testing.assert_array_equal(g.GetKNNIndexes(), og.to_original(og.knn(k)[0]))
+    g.close()
+
+
+@pytest.mark.parametrize("nq,k", [(1, 1), (63, 64), (99_999, 8), (100_000, 1), (100_001, 16), (100_001, 33),
+                                  (150_001, 40), (120_000, 64)])
+def test_query_search_at_shape_limits(egt_mod, oracle_mod, nq, k):
+    """Query counts around the limits of the unsorted, sorted and lane-per-query searches, a tenth of the queries
+    outside the grid and a finite radius."""
+    E, O = egt_mod, oracle_mod
+    print("nq", nq, "k", k, flush=True)
+    ref = D.sphere(20_000, seed=41)
+    q = [a.copy() for a in D.sphere(nq, seed=42)]
+    q[0][::10] *= np.float32(1.3)
+    q = tuple(q)
+    g = E.GridStructure(ref, 1, 1e-6, 1024, 4)
+    g.GRIDCUDAKNNCompact(q, k, 0.2)
+    og = O.Grid(*ref)
+    np.testing.assert_array_equal(g.GetKNNIndexesQuery(), og.ref_to_original(og.knn_query(*q, k, thres=0.2)[0]))
+    g.close()
