@@ -93,11 +93,13 @@ typedef enum {
                                     1/4, 1/8 of a grid cell; EGT_START_LEVEL_OCCUPANCY = one level from the
                                     mean cell occupancy */
     EGT_OPT_LEARNED = 1,         /* kNN: 1 = start each query from the learned radius proposal */
-    EGT_OPT_TAUBIN_GRAPH = 2,    /* Taubin: 1 = replay the lambda/mu loop as a captured hipGraph (default) */
+    EGT_OPT_TAUBIN_GRAPH = 2,    /* Taubin: 1 = replay the lambda/mu loop as a captured hipGraph (default; clouds of
+                                    up to 262,144 points run every pass in one launch), 0 = a launch per pass */
     EGT_OPT_MAX_PTS_IN_CUBE = 3, /* kNN validity rule: cell population that invalidates a query (1e5) */
     EGT_OPT_KNN_PERSISTENT = 4,  /* kNN: 1 = one persistent work-queue launch per neighbour-count class,
                                     0 = one workgroup per 256 queries (default) */
-    EGT_OPT_TAUBIN_TILE = 5,     /* Taubin: points per LDS tile, 1024 (default) or 2048; 0 = autotune on the
+    EGT_OPT_TAUBIN_TILE = 5,     /* Taubin: points per LDS tile, 1024 (default; small clouds whose passes run in one
+                                    launch use 256 unless this option is set) or 2048; 0 = autotune on the
                                     next smoothing call (times both on copies, keeps the faster; the
                                     per-pass times land in egt_stats.taubin_tile_ms) */
     EGT_OPT_TAUBIN_REGULARIZED = 6, /* Taubin weights: 0 = exp(-d^2) (default, as the reference runs); 1 = the

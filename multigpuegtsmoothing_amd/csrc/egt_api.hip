@@ -350,6 +350,7 @@ egt_status egt_set_option(egt_handle h, egt_option opt, int64_t value) {
             if (value != 0 && value != 1024 && value != 2048)
                 return fail(EGT_ERR_INVALID_ARG, "Taubin tile width must be 1024, 2048 or 0 (autotune)");
             h->taubin_tile = (int)value;
+            h->taubin_tile_set = true;
             return EGT_OK;
         case EGT_OPT_TAUBIN_REGULARIZED:
             h->taubin_regularized = value ? 1 : 0;

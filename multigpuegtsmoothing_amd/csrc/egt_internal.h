@@ -240,6 +240,7 @@ struct egt_ctx {
                                   // (0 = never)
     int taubin_graph = 1;
     int taubin_tile = 1024;  // Taubin tile width: 1024 or 2048 points; 0 = tune on the next smoothing call
+    bool taubin_tile_set = false;  // the width was set by option: no other tiling
     int taubin_regularized = 0;  // isRegularized weights (1 / inverse-square), off as in the reference
     int maxc = 100000;
 

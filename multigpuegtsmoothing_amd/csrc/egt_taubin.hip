@@ -62,10 +62,10 @@ constexpr int tile_threads() { return TILE == 1024 ? 512 : 1024; }
 // of the CU's 160 KiB, so two 1024-thread or four 512-thread blocks still fit per CU. In
 // volumetric regions a 2048-point Morton range has a halo of 2000-3000 points at 16 kept neighbours a point.
 template <int TILE>
-constexpr int halo_cap() { return TILE == 1024 ? 1456 : 2992; }
+constexpr int halo_cap() { return TILE == 256 ? 1024 : TILE == 1024 ? 1456 : 2992; }
 // Longest halo list of a tile (the list's stride per tile); beyond it the tile uses CSR rows.
 template <int TILE>
-constexpr int halo_max() { return TILE == 1024 ? 4096 : 8192; }
+constexpr int halo_max() { return TILE == 256 ? 1024 : TILE == 1024 ? 4096 : 8192; }
 static_assert((2048 + halo_cap<2048>() + 1) * 16 <= 160 * 1024 / 2 - 1024, "two tile blocks per CU");
 static_assert((1024 + halo_cap<1024>() + 1) * 16 <= 160 * 1024 / 4 - 1024, "four tile blocks per CU");
 __device__ inline void block_bitonic_sort(uint32_t* a, int n2) {
@@ -121,19 +121,31 @@ __device__ inline void block_sort(uint32_t* a, int n2) {
     __syncthreads();
 }
 
-// LDS hash set of a tile's external columns: open addressing, linear probing, 2 * halo_max slots. An insert
+// LDS hash set of a tile's external columns: open addressing, linear probing, 2 or 4 * halo_max slots. An insert
 // is only started while the count is at most halo_max, so the set never holds more than halo_max + PBLK
 // entries and every probe sequence reaches an empty slot.
 template <int TILE>
-constexpr int hset_size() { return 2 * halo_max<TILE>(); }
+constexpr int hset_size() { return (TILE == 256 ? 4 : 2) * halo_max<TILE>(); }
 constexpr uint32_t HS_EMPTY = 0xFFFFFFFFu;
 
+// With R.flag (the resident passes below), the tile also reserves its column block, lists the tiles its halo lies
+// in, marks the points it reads and clears its exchange entries.
+struct Resident {
+    uint32_t* flag;    // bit 0: a tile cannot run resident, bit 1: a wait ran out
+    uint32_t* cursor;  // next free column slot
+    uint32_t* reads;   // bit matrix: row t holds the tiles that tile t reads
+    uint32_t* readby;  // its transpose
+    uint32_t* pub;     // bit per Morton position: some other tile reads the point
+    uint64_t* xch;     // exchange: per parity x, y, z arrays of ntiles * RT entries, a version in each high word
+    int words;         // row length of the bit matrices
+};
 template <int TILE>
 __global__ void __launch_bounds__(PBLK) k_tile_prep(const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
                                                      int64_t n, uint16_t* __restrict__ col16,
                                                      int32_t* __restrict__ halo, int32_t* __restrict__ hcount,
                                                      uint16_t* __restrict__ perm, uint32_t* __restrict__ width,
-                                                     uint32_t* __restrict__ padded) {
+                                                     uint32_t* __restrict__ padded, uint64_t* __restrict__ toff,
+                                                     Resident R) {
     constexpr int HS = hset_size<TILE>(), HMAX = halo_max<TILE>();
     static_assert((HS & (HS - 1)) == 0 && HS >= TILE && HS >= HMAX + PBLK, "hash set size");
     __shared__ uint32_t hs[HS];      // hash set, then the row-sort keys
@@ -177,6 +189,7 @@ __global__ void __launch_bounds__(PBLK) k_tile_prep(const int32_t* __restrict__ 
         if (threadIdx.x == 0) {
             hcount[t] = -1;
             padded[t] = 0;
+            if (R.flag) atomicOr(R.flag, 1u);
         }
         return;
     }
@@ -204,7 +217,21 @@ __global__ void __launch_bounds__(PBLK) k_tile_prep(const int32_t* __restrict__ 
     for (int i = (int)H + threadIdx.x; i < n2; i += PBLK) uniq[i] = HS_EMPTY;
     __syncthreads();
     block_sort(uniq, n2);
-    for (uint32_t h = threadIdx.x; h < H; h += PBLK) halo[t * halo_max<TILE>() + h] = (int32_t)uniq[h];
+    for (uint32_t h = threadIdx.x; h < H; h += PBLK) {
+        const uint32_t c = uniq[h];
+        halo[t * halo_max<TILE>() + h] = (int32_t)c;
+        if (R.flag) {
+            atomicOr(&R.pub[c >> 5], 1u << (c & 31));
+            const uint32_t t2 = c / TILE;
+            if (h == 0 || uniq[h - 1] / TILE != t2) {
+                atomicOr(&R.reads[t * R.words + (t2 >> 5)], 1u << (t2 & 31));
+                atomicOr(&R.readby[(int64_t)t2 * R.words + (t >> 5)], 1u << (t & 31));
+            }
+        }
+    }
+    if (R.flag)  // versions no pass produces
+        for (int i = threadIdx.x; i < 6 * TILE; i += PBLK)
+            R.xch[(i / TILE) * ((int64_t)gridDim.x * TILE) + base + i % TILE] = ~0ull;
     for (int32_t e = eb + threadIdx.x; e < ee; e += PBLK) {
         const uint32_t c = (uint32_t)col[e];
         uint16_t loc;
@@ -244,6 +271,7 @@ __global__ void __launch_bounds__(PBLK) k_tile_prep(const int32_t* __restrict__ 
         for (int s = 0; s < TILE / 64; ++s) tot += 128u * ((swid[s] + 1u) >> 1);
         padded[t] = tot;
         hcount[t] = (int32_t)H;
+        if (R.flag) toff[t] = atomicAdd(R.cursor, tot);
     }
 }
 
@@ -503,12 +531,254 @@ __global__ void __launch_bounds__(tile_threads<TILE>()) __attribute__((amdgpu_wa
     for (int i = threadIdx.x; i < np; i += TBLK_TILE) out[base + i] = *reinterpret_cast<const Pt3*>(&lds[i]);
 }
 
-// Writes the smoothed points back to the sorted-space SoA arrays and refreshes the Morton copy.
+// ---------------------------------------------------------------------------------------------------
+// Resident passes (small clouds). All passes run in one launch: a tile of RT points stays in one workgroup's LDS,
+// a row per lane with its columns in registers, and only the points that other tiles read travel, through an
+// exchange buffer in global memory. A coordinate goes out as one 64-bit word that carries its version (the number
+// of passes it has been through), by relaxed agent-scope atomics, so a reader that finds the version it waits for
+// has the value: no flag, fence or barrier across workgroups. Two buffers alternate by parity. A tile may overwrite
+// version v with v + 2 once every reader of v is past it; a reader is past it when it publishes v + 1, so the
+// tiles' reads are made symmetric (k_tile_tokens): a tile that is read by another one reads a point of it too.
+// Every workgroup must be resident, so the tiles are limited to what fits on the GPU at once; should they not be
+// (other work holds the CUs), a wait ends after RWAIT ticks, raises the flag, every workgroup leaves, and the caller
+// runs the passes launch by launch. The points are untouched until k_writeback, which looks at the flag first.
+//
+// Bound: the chain of one pass (publish, find the neighbours' points, two chunks of slots), where a launch per pass
+// costs its start, two dependent rounds of staging loads and its end, with most CUs idle below 256 tiles. Us a pass,
+// resident / a launch per pass, sphere at k=40: 1,000 points 1.1 / 4.6, 20,000 3.2 / 7.1, 100,000 4.3 / 8.3, 262,144
+// 5.9 / 9.0; set-up 20-80 us / 190-240 (no graph, no wait for the host). Exchange entries at the points' own
+// positions, 32 bytes each, took 14.3 us at 262,144 points: every coordinate was a memory request of its own.
+constexpr int RT = 256;            // points per tile, one row per thread
+constexpr int RHP = halo_cap<RT>() / RT;
+constexpr int RCW = 16;            // column words of a row held in registers (32 slots); the rest is read per pass
+constexpr int64_t RWAIT = 2000000;  // 20 ms of the 100 MHz wall clock
+static_assert(halo_cap<RT>() == halo_max<RT>(), "a resident halo lies in LDS");
+
+// Symmetric reads: tile t, read by t2 but not reading it, appends t2's first point to its halo.
+__global__ void __launch_bounds__(64) k_tile_tokens(int32_t* __restrict__ halo, int32_t* __restrict__ hcount,
+                                                     Resident R) {
+    const int64_t t = blockIdx.x;
+    int H = hcount[t];
+    if (H < 0) return;
+    const int lane = threadIdx.x;
+    for (int w0 = 0; w0 < R.words; w0 += 64) {
+        const int w = w0 + lane;
+        uint32_t need = w < R.words ? R.readby[t * R.words + w] & ~R.reads[t * R.words + w] : 0u;
+        int c = __popc(need), incl = c;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += o;
+        }
+        int at = H + incl - c;
+        while (need) {
+            const uint32_t p = ((uint32_t)w * 32 + (uint32_t)__builtin_ctz(need)) * RT;
+            need &= need - 1;
+            if (at < halo_max<RT>()) {
+                halo[t * halo_max<RT>() + at] = (int32_t)p;
+                atomicOr(&R.pub[p >> 5], 1u << (p & 31));
+            }
+            ++at;
+        }
+        H += __shfl(incl, 63, 64);
+    }
+    if (lane == 0) {
+        hcount[t] = H;
+        if (H > halo_max<RT>()) atomicOr(R.flag, 1u);
+    }
+}
+
+// Exchange entry of a published point: its tile's published points lie side by side, in position order, from the
+// tile's first entry on, so a reader's sorted halo becomes a few runs of consecutive entries.
+__device__ inline int64_t xch_entry(const uint32_t* __restrict__ pub, int64_t c) {
+    const int64_t t0 = c / RT * RT;
+    const uint32_t* w = pub + (t0 >> 5);
+    const int r = (int)(c - t0);
+    int at = 0;
+#pragma unroll
+    for (int i = 0; i < RT / 32; ++i) {
+        const uint32_t below = 32 * i + 32 <= r ? ~0u : (32 * i >= r ? 0u : (1u << (r & 31)) - 1u);
+        at += __popc(w[i] & below);
+    }
+    return t0 + at;
+}
+__device__ inline uint64_t xch_load(const uint64_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void xch_store(uint64_t* p, float v, uint32_t version) {
+    __hip_atomic_store(p, (uint64_t)__float_as_uint(v) | ((uint64_t)version << 32), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <bool REG>
+__global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) k_taubin_resident(const float4* __restrict__ mpts, Pt3* __restrict__ out,
+                                                         const uint16_t* __restrict__ scol,
+                                                         const uint64_t* __restrict__ toff,
+                                                         const uint32_t* __restrict__ width,
+                                                         const uint16_t* __restrict__ perm,
+                                                         const int32_t* __restrict__ halo,
+                                                         const int32_t* __restrict__ hcount, int64_t n, int iters,
+                                                         float lambda, float mu, Resident R) {
+    constexpr int S = RT / 64;
+    __shared__ float4 pts[RT + halo_cap<RT>()];
+    __shared__ uint16_t publist[RT];  // the tile's published rows, in position order
+    __shared__ int stop;
+    const int64_t t = blockIdx.x;
+    const int64_t base = t * RT;
+    const int np = (int)(min<int64_t>(base + RT, n) - base);
+    if (threadIdx.x == 0) stop = __hip_atomic_load(R.flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    __syncthreads();
+    if (stop) return;
+    const int H = hcount[t];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t at = 0;
+    for (int i = 0; i < wv; ++i) at += 128u * ((width[t * S + i] + 1u) >> 1);
+    const uint32_t* sb = reinterpret_cast<const uint32_t*>(scol + toff[t] + at);
+    const int W = (int)width[t * S + wv];
+    const int j = wv * 64 + lane;
+    const int row = j < np ? (int)perm[t * RT + j] : -1;
+    const uint32_t self = (uint32_t)row;  // as the padding slots hold it; lanes past the last row match no column
+    const int P = (W + 1) >> 1;
+    uint32_t cw[RCW];
+#pragma unroll
+    for (int q = 0; q < RCW; ++q) cw[q] = q < P ? sb[q * 64 + lane] : 0u;
+    const int64_t own = base + (row < 0 ? 0 : row), xn = (int64_t)gridDim.x * RT;
+    const bool pub = row >= 0 && ((R.pub[own >> 5] >> (own & 31)) & 1u);
+    const int own_x = (int)(xch_entry(R.pub, own) - base);
+    if (pub) publist[own_x] = (uint16_t)row;
+    int npub = 0;
+#pragma unroll
+    for (int i = 0; i < RT / 32; ++i) npub += __popc(R.pub[t * (RT / 32) + i]);
+    const int32_t* hal = halo + t * halo_max<RT>();
+    int64_t hx[RHP];
+#pragma unroll
+    for (int k = 0; k < RHP; ++k) {
+        const int h = (int)threadIdx.x + k * RT;
+        hx[k] = h < H ? (int64_t)hal[h] : -1;
+    }
+    if ((int)threadIdx.x < np) pts[threadIdx.x] = mpts[base + threadIdx.x];
+#pragma unroll
+    for (int k = 0; k < RHP; ++k)
+        if (hx[k] >= 0) {
+            pts[RT + (int)threadIdx.x + k * RT] = mpts[hx[k]];
+            hx[k] = xch_entry(R.pub, hx[k]);
+        }
+    __syncthreads();
+    float4 p = pts[row < 0 ? 0 : row];
+    const int passes = 2 * iters;
+    // Each lane publishes its own row (scattered words), or, with more than a workgroup per CU, the rows go through
+    // LDS and out in entry order, whole lines at a time: 20,000 points 2.50 against 2.65 us a pass, 262,144 points
+    // 4.78 against 3.89 (k=8).
+    const bool direct = gridDim.x <= 256;
+    for (int pass = 0; pass < passes; ++pass) {
+        const float scale = pass & 1 ? mu : lambda;
+        float cgx = 0.0f, cgy = 0.0f, cgz = 0.0f, sum = 0.0f;
+        // slots of one column word pair group, as taubin_two_rows does them
+        auto chunk = [&](const uint32_t(&w4)[TCH / 2], int u0) {
+            uint32_t c[TCH];
+            float4 qs[TCH];
+#pragma unroll
+            for (int u = 0; u < TCH; ++u) c[u] = (u & 1) ? w4[u >> 1] >> 16 : w4[u >> 1] & 0xFFFFu;
+#pragma unroll
+            for (int u = 0; u < TCH; ++u)
+                if (u0 + u < W) qs[u] = pts[c[u]];
+#pragma unroll
+            for (int u = 0; u < TCH; ++u) {
+                if (u0 + u < W) {  // wave-uniform
+                    const float dx = p.x - qs[u].x, dy = p.y - qs[u].y, dz = p.z - qs[u].z;
+                    const float dist = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+                    float w = taubin_weight<REG>(dist, scale);
+                    w = c[u] != self ? w : 0.0f;
+                    cgx = __builtin_fmaf(-w, dx, cgx);
+                    cgy = __builtin_fmaf(-w, dy, cgy);
+                    cgz = __builtin_fmaf(-w, dz, cgz);
+                    sum += w;
+                }
+            }
+        };
+#pragma unroll
+        for (int q = 0; q < RCW; q += TCH / 2)
+            if (2 * q < W) chunk({cw[q], cw[q + 1], cw[q + 2], cw[q + 3]}, 2 * q);
+        for (int q = RCW; 2 * q < W; q += TCH / 2) {
+            uint32_t w4[TCH / 2];
+#pragma unroll
+            for (int i = 0; i < TCH / 2; ++i) w4[i] = sb[min(q + i, P - 1) * 64 + lane];
+            chunk(w4, 2 * q);
+        }
+        p = taubin_result(p, cgx, cgy, cgz, sum, scale);
+        if (pass + 1 == passes) break;
+        const uint32_t version = (uint32_t)pass + 1u;
+        uint64_t* const xb = R.xch + (version & 1u) * 3 * xn;
+        if (direct && pub) {
+            uint64_t* x = xb + base + own_x;
+            xch_store(x, p.x, version);
+            xch_store(x + xn, p.y, version);
+            xch_store(x + 2 * xn, p.z, version);
+        }
+        __syncthreads();  // every lane has read this pass's points
+        if (row >= 0) pts[row] = p;
+        if (!direct) {
+            __syncthreads();
+            if ((int)threadIdx.x < npub) {
+                const float4 v = pts[publist[threadIdx.x]];
+                uint64_t* x = xb + base + threadIdx.x;
+                xch_store(x, v.x, version);
+                xch_store(x + xn, v.y, version);
+                xch_store(x + 2 * xn, v.z, version);
+            }
+        }
+        uint32_t pend = 0;
+#pragma unroll
+        for (int k = 0; k < RHP; ++k) pend |= hx[k] >= 0 ? 1u << k : 0u;
+        int64_t t0 = 0;
+        while (pend) {
+            uint64_t v[RHP][3];
+#pragma unroll
+            for (int k = 0; k < RHP; ++k) {
+                if ((pend >> k) & 1u) {
+                    const uint64_t* x = xb + hx[k];
+                    v[k][0] = xch_load(x);
+                    v[k][1] = xch_load(x + xn);
+                    v[k][2] = xch_load(x + 2 * xn);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < RHP; ++k) {
+                if (((pend >> k) & 1u) && (uint32_t)(v[k][0] >> 32) == version &&
+                    (uint32_t)(v[k][1] >> 32) == version && (uint32_t)(v[k][2] >> 32) == version) {
+                    pts[RT + (int)threadIdx.x + k * RT] =
+                        make_float4(__uint_as_float((uint32_t)v[k][0]), __uint_as_float((uint32_t)v[k][1]),
+                                    __uint_as_float((uint32_t)v[k][2]), 0.0f);
+                    pend &= ~(1u << k);
+                }
+            }
+            if (pend) {
+                const int64_t now = (int64_t)wall_clock64();
+                if (t0 == 0) t0 = now;
+                if (now - t0 > RWAIT) atomicOr(R.flag, 2u);
+                // another workgroup's wait may have run out: looked at now and then, this one's own at once
+                if (now - t0 > RWAIT || ((now - t0) & 0xFF) == 0xFF) {
+                    if (__hip_atomic_load(R.flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                        stop = 1;
+                        pend = 0;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        if (stop) return;  // every thread of the workgroup
+    }
+    if (row >= 0) st3(out, own, p);
+}
+
+// Writes the smoothed points back to the sorted-space SoA arrays and refreshes the Morton copy (not when flag, if
+// given, is raised: the passes did not complete).
 __global__ void __launch_bounds__(TBLK) k_writeback(const Pt3* __restrict__ p, int64_t n,
                                                      float4* __restrict__ mpts, float* __restrict__ x,
-                                                     float* __restrict__ y, float* __restrict__ z) {
+                                                     float* __restrict__ y, float* __restrict__ z,
+                                                     const uint32_t* __restrict__ flag) {
     const int64_t m = (int64_t)blockIdx.x * TBLK + threadIdx.x;
-    if (m >= n) return;
+    if (m >= n || (flag && *flag)) return;
     const float4 v = ld3(p, m);
     const int32_t s = __float_as_int(mpts[m].w);
     mpts[m] = make_float4(v.x, v.y, v.z, __int_as_float(s));
@@ -557,7 +827,7 @@ TilePlan prepare_tiles(egt_ctx* h) {
     uint32_t* padded = h->scratch.get<uint32_t>(30, tp.ntiles);
     tp.toff = h->scratch.get<uint64_t>(31, tp.ntiles);
     k_tile_prep<TILE><<<tp.ntiles, PBLK, 0, s>>>(h->rowptr.p, h->col.p, n, tp.col16, tp.halo, tp.hcount, tp.perm,
-                                                 tp.width, padded);
+                                                 tp.width, padded, tp.toff, Resident{});
     LAUNCH_CHECK();
     std::vector<int32_t> hc(tp.ntiles);
     std::vector<uint32_t> pad(tp.ntiles);
@@ -635,9 +905,96 @@ int tune_tile(egt_ctx* h, const Pt3* A, float lambda, float mu) {
     return best;
 }
 
+__global__ void __launch_bounds__(TBLK) k_zero_u32(uint32_t* __restrict__ p, int64_t n) {
+    for (int64_t i = (int64_t)blockIdx.x * TBLK + threadIdx.x; i < n; i += (int64_t)gridDim.x * TBLK) p[i] = 0u;
+}
+
+// Largest tile count of the resident passes: four workgroups on each CU (their LDS and registers allow more).
+int resident_tiles() {
+    static const int tiles = [] {
+        int dev = 0, cus = 0, a = 0, b = 0;
+        HIP_CHECK(hipGetDevice(&dev));
+        HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_taubin_resident<false>, RT, 0));
+        HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_taubin_resident<true>, RT, 0));
+        return cus * std::min(4, std::min(a, b));
+    }();
+    return tiles;
+}
+
+// All passes in one launch (see k_taubin_resident). Returns false, with the points untouched, when a tile does not
+// fit (halo too long, a row that lists itself) or a wait ran out: the caller then runs the passes launch by launch.
+bool run_resident(egt_ctx* h, int iters, float lambda, float mu) {
+    const int64_t n = h->n;
+    const int nt = ceil_div(n, RT);
+    if (iters < 1 || h->taubin_tile != 1024 || h->taubin_tile_set || !h->taubin_graph || nt > resident_tiles())
+        return false;
+    hipStream_t s = h->stream;
+    Scratch& sc = h->scratch;
+    int kmax = 1;
+    for (const CloudDev& c : h->clouds) kmax = std::max(kmax, c.k);
+    uint16_t* col16 = sc.get<uint16_t>(19, std::max<int64_t>(h->nnz, 1));
+    int32_t* halo = sc.get<int32_t>(20, (size_t)nt * halo_max<RT>());
+    int32_t* hcount = sc.get<int32_t>(21, nt);
+    uint16_t* scol = sc.get<uint16_t>(27, (size_t)nt * RT * (kmax + 1));  // no slice is wider than the longest row
+    uint16_t* perm = sc.get<uint16_t>(28, (size_t)nt * RT);
+    uint32_t* width = sc.get<uint32_t>(29, (size_t)nt * (RT / 64));
+    uint32_t* padded = sc.get<uint32_t>(30, nt);
+    uint64_t* toff = sc.get<uint64_t>(31, nt);
+    Pt3* out = sc.get<Pt3>(12, n);
+    Resident R{};
+    R.words = (nt + 31) / 32;
+    R.xch = sc.get<uint64_t>(22, 6 * (size_t)nt * RT);
+    const size_t zeros = 2 + 2 * (size_t)nt * R.words + (size_t)nt * (RT / 32);
+    uint32_t* z = sc.get<uint32_t>(23, zeros);
+    R.flag = z;
+    R.cursor = z + 1;
+    R.reads = z + 2;
+    R.readby = R.reads + (size_t)nt * R.words;
+    R.pub = R.readby + (size_t)nt * R.words;
+    Event e0, ep, e1;
+    HIP_CHECK(hipEventRecord(e0, s));
+    k_zero_u32<<<(int)std::min<size_t>(256, (zeros + TBLK - 1) / TBLK), TBLK, 0, s>>>(z, (int64_t)zeros);
+    LAUNCH_CHECK();
+    k_tile_prep<RT><<<nt, PBLK, 0, s>>>(h->rowptr.p, h->col.p, n, col16, halo, hcount, perm, width, padded, toff, R);
+    LAUNCH_CHECK();
+    k_tile_sell<RT><<<nt, PBLK, 0, s>>>(h->rowptr.p, col16, n, perm, width, toff, hcount, scol);
+    LAUNCH_CHECK();
+    k_tile_tokens<<<nt, 64, 0, s>>>(halo, hcount, R);
+    LAUNCH_CHECK();
+    HIP_CHECK(hipEventRecord(ep, s));
+    if (h->taubin_regularized)
+        k_taubin_resident<true><<<nt, RT, 0, s>>>(h->mpts.p, out, scol, toff, width, perm, halo, hcount, n, iters,
+                                                  lambda, mu, R);
+    else
+        k_taubin_resident<false><<<nt, RT, 0, s>>>(h->mpts.p, out, scol, toff, width, perm, halo, hcount, n, iters,
+                                                   lambda, mu, R);
+    LAUNCH_CHECK();
+    HIP_CHECK(hipEventRecord(e1, s));
+    k_writeback<<<ceil_div(n, TBLK), TBLK, 0, s>>>(out, n, h->mpts.p, h->x.p, h->y.p, h->z.p, R.flag);
+    LAUNCH_CHECK();
+    uint32_t flag = 0;
+    HIP_CHECK(hipMemcpyAsync(&flag, R.flag, sizeof(flag), hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipStreamSynchronize(s));
+    if (flag) return false;
+    float total = 0.0f, passes = 0.0f;
+    HIP_CHECK(hipEventElapsedTime(&total, e0, e1));
+    HIP_CHECK(hipEventElapsedTime(&passes, ep, e1));
+    h->taubin_fallback_tiles = 0;
+    h->stats.taubin_tile = RT;
+    h->stats.taubin_fallback_tiles = 0;
+    h->stats.taubin_overflow_tiles = 0;
+    h->stats.taubin_ms = total;
+    h->stats.taubin_pass_ms = passes / (2.0f * iters);
+    h->stats.taubin_setup_ms = total - passes;
+    h->search_stale = true;
+    return true;
+}
+
 }  // namespace
 
 void run_taubin(egt_ctx* h, int iters, float lambda, float mu) {
+    if (run_resident(h, iters, lambda, mu)) return;
     const int64_t n = h->n;
     hipStream_t s = h->stream;
     Pt3* A = h->scratch.get<Pt3>(12, n);
@@ -690,7 +1047,7 @@ void run_taubin(egt_ctx* h, int iters, float lambda, float mu) {
         HIP_CHECK(hipEventRecord(ep, s));
     }
     HIP_CHECK(hipEventRecord(e1, s));
-    k_writeback<<<ceil_div(n, TBLK), TBLK, 0, s>>>(A, n, h->mpts.p, h->x.p, h->y.p, h->z.p);
+    k_writeback<<<ceil_div(n, TBLK), TBLK, 0, s>>>(A, n, h->mpts.p, h->x.p, h->y.p, h->z.p, nullptr);
     LAUNCH_CHECK();
     HIP_CHECK(hipEventSynchronize(e1));
     HIP_CHECK(hipEventElapsedTime(&h->stats.taubin_ms, e0, e1));

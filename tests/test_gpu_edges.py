@@ -84,3 +84,59 @@ def test_query_search_at_shape_limits(egt_mod, oracle_mod, nq, k):
     og = O.Grid(*ref)
     np.testing.assert_array_equal(g.GetKNNIndexesQuery(), og.ref_to_original(og.knn_query(*q, k, thres=0.2)[0]))
     g.close()
+
+
+@pytest.mark.parametrize("n,k,alpha,regularized", [(1, 4, 0.65, False), (255, 8, 0.65, False), (256, 8, 0.65, True),
+                                                   (257, 40, 0.65, False), (511, 16, 1e-8, False),
+                                                   (4_097, 64, 1e-8, False), (9_000, 40, 1e-8, True),
+                                                   (65_537, 16, 0.65, False), (262_144, 8, 0.65, False),
+                                                   (262_145, 8, 0.65, False)])
+def test_resident_taubin_sizes(egt_mod, oracle_mod, n, k, alpha, regularized):
+    """Small clouds run every Taubin pass in one launch (tiles of 256 points, up to 1024 of them): tile edges, rows
+    past the 32 slots held in registers (alpha 1e-8 keeps nearly every neighbour), both limits, three calls on a
+    handle (the exchange entries of the call before must not be taken for this one's)."""
+    E, O = egt_mod, oracle_mod
+    print("n", n, "k", k, "alpha", alpha, "regularized", regularized, flush=True)
+    pts = D.mixture(n, seed=600) if n > 16 else D.sphere(n, seed=601)
+    og = O.Grid(*pts)
+    g = E.GridStructure(pts, 1, 1e-6, 1024, 4)
+    g.set_option(E.OPT_TAUBIN_REGULARIZED, int(regularized))
+    g.GRIDCUDAKNNSELF_COMPACT(k, 1e8)
+    x, y, z = og.xs, og.ys, og.zs
+    rows = og.knn(k)[0]
+    for iters in (1, 7, 2):
+        E.EGT_CUDA(g).PerformSmoothing(iters, 0.5, -0.53, alpha)
+        rows = O.egg(x, y, z, rows, alpha)
+        x, y, z = O.taubin_f32(x, y, z, rows, iters, 0.5, -0.53, regularized=regularized)
+        want = og.output(x, y, z)
+        for a, b in zip(E.getOutputPoints(g), want):
+            np.testing.assert_array_equal(a, b, err_msg=f"{iters} iterations")
+    g.close()
+
+
+def test_resident_taubin_from_threads(egt_mod):
+    """Four handles smoothed at once from four threads give what they give one after another."""
+    import threading
+
+    E = egt_mod
+    clouds = [D.torus(30_000 + 7_001 * i, seed=700 + i) for i in range(4)]
+
+    def smooth(i, out):
+        for rep in range(3):
+            g = E.GridStructure(clouds[i], 1, 1e-6, 1024, 4)
+            g.GRIDCUDAKNNSELF_COMPACT(16, 1e8)
+            E.EGT_CUDA(g).PerformSmoothing(40, 0.5, -0.53, 0.65)
+            out[i, rep] = E.getOutputPoints(g)
+            g.close()
+
+    alone, together = {}, {}
+    for i in range(4):
+        smooth(i, alone)
+    threads = [threading.Thread(target=smooth, args=(i, together)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for key in alone:
+        for a, b in zip(alone[key], together[key]):
+            np.testing.assert_array_equal(a, b, err_msg=str(key))
