@@ -551,7 +551,7 @@ void sort_into_sorted_space(egt_ctx* h, const float* dx, const float* dy, const 
         uint32_t* cl = sc.get<uint32_t>(22, n);
         k_gather_cloud<<<ceil_div(n, BLK), BLK, 0, s>>>(icloud, sidx, n, cl);
         LAUNCH_CHECK();
-        radix_sort_pairs(cl, sidx, n, std::max(1, ceil_log2(h->nclouds)), s, sc);
+        radix_sort_pairs(cl, sidx, n, std::max(1, ceil_log2(h->nclouds)), s, sc, false);
         h->scloud.alloc(n);
     }
     h->x.alloc(n);
@@ -682,7 +682,7 @@ void build_search_structure(egt_ctx* h) {
         k_morton_keys<<<ceil_div(n, BLK), BLK, 0, s>>>(h->x.p, h->y.p, h->z.p, h->key.p, n, a, ba, h->B, log2B,
                                                        cell, sub, order.p, spts);
         LAUNCH_CHECK();
-        radix_sort_pairs(sub, order.p, n, 3 * SUB, s, sc);
+        radix_sort_pairs(sub, order.p, n, 3 * SUB, s, sc, false);
         k_gather_u32<<<ceil_div(n, BLK), BLK, 0, s>>>(cell, order.p, n, code.p);
         LAUNCH_CHECK();
     }
@@ -692,7 +692,7 @@ void build_search_structure(egt_ctx* h) {
         uint32_t* cl = sc.get<uint32_t>(22, n);
         k_gather_cloud<<<ceil_div(n, BLK), BLK, 0, s>>>(h->scloud.p, order.p, n, cl);
         LAUNCH_CHECK();
-        radix_sort_pairs(cl, order.p, n, std::max(1, ceil_log2(h->nclouds)), s, sc);
+        radix_sort_pairs(cl, order.p, n, std::max(1, ceil_log2(h->nclouds)), s, sc, false);
         h->mcloud.alloc(n);
     }
     h->mpts.alloc(n);

@@ -270,7 +270,9 @@ void exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t n, hipStream_
 // Same, with the total written to device memory and no synchronization.
 void exclusive_scan_u32_dev(const uint32_t* in, uint32_t* out, int64_t n, hipStream_t s, Scratch& sc,
                             uint32_t* total_dev);
-void radix_sort_pairs(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, Scratch& sc);
+// Stable sort of (key, value) pairs by the low key_bits bits. With keep_keys false the keys end up undefined.
+void radix_sort_pairs(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, Scratch& sc,
+                      bool keep_keys = true);
 // The same sort over a caller's workspace of radix_sort_workspace_words(n) 32-bit words (no allocation).
 size_t radix_sort_workspace_words(int64_t n);
 void radix_sort_pairs_ws(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, uint32_t* ws);

@@ -125,7 +125,19 @@ void scan_rec(const uint32_t* in, uint32_t* out, int64_t n, hipStream_t s, PartF
 // per-wave per-digit LDS counter advanced by the lowest such lane.
 constexpr int RADIX_BITS = 8;
 
-template <int BITS>
+// Three forms by size:
+//  - up to SMALL_MAX keys: every pass in one workgroup's LDS, one launch;
+//  - up to DIRECT_TILES tiles (of 1024 keys, then of 4096): a histogram per tile (tile-major), then a scatter whose
+//    workgroups sum the histograms below their own tile themselves, two launches per pass;
+//  - above: the counts are digit-major and scanned in launches of their own.
+// A key of exactly 9 bits is one pass of 512 values. Bound: launches and a few dependent rounds up to about a
+// million keys, the scattered stores above. Grid build (three sorts) with a scan per pass / now, in ms: 2,000 points
+// 0.30 / 0.19, 16,384 0.40 / 0.26 (0.32 with one workgroup), 100,000 0.50 / 0.34, 1M 0.72 / 0.66, 4M 1.41 / 1.42.
+constexpr int SMALL_BLOCK = 1024;
+constexpr int SMALL_MAX = 8 * SMALL_BLOCK;
+constexpr int DIRECT_TILES = 256;
+
+template <int BITS, int ITEMS, bool TILE_MAJOR>
 __global__ void __launch_bounds__(SORT_BLOCK) k_sort_hist(const uint32_t* __restrict__ keys, int64_t n, int shift,
                                                            uint32_t* __restrict__ counts, int nblocks) {
     constexpr int BINS = 1 << BITS;
@@ -133,40 +145,29 @@ __global__ void __launch_bounds__(SORT_BLOCK) k_sort_hist(const uint32_t* __rest
     __shared__ uint32_t hist[BINS];
     for (int d = threadIdx.x; d < BINS; d += SORT_BLOCK) hist[d] = 0;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * SORT_TILE;
+    const int64_t base = (int64_t)blockIdx.x * SORT_BLOCK * ITEMS;
 #pragma unroll 4
-    for (int r = 0; r < SORT_ITEMS; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const int64_t i = base + (int64_t)r * SORT_BLOCK + threadIdx.x;
         if (i < n) atomicAdd(&hist[(keys[i] >> shift) & MASK], 1u);
     }
     __syncthreads();
-    for (int d = threadIdx.x; d < BINS; d += SORT_BLOCK) counts[(int64_t)d * nblocks + blockIdx.x] = hist[d];
+    for (int d = threadIdx.x; d < BINS; d += SORT_BLOCK)
+        counts[TILE_MAJOR ? (int64_t)blockIdx.x * BINS + d : (int64_t)d * nblocks + blockIdx.x] = hist[d];
 }
 
-template <int BITS>
-__global__ void __launch_bounds__(SORT_BLOCK) k_sort_scatter(const uint32_t* __restrict__ kin,
-                                                              const uint32_t* __restrict__ vin,
-                                                              uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
-                                                              int64_t n, int shift,
-                                                              const uint32_t* __restrict__ offsets, int nblocks) {
-    constexpr int BINS = 1 << BITS;
-    constexpr uint32_t MASK = BINS - 1;
-    __shared__ uint32_t wcnt[SORT_BLOCK / WAVE][BINS];
-    __shared__ uint32_t goff[BINS];
-    const int lane = __lane_id(), wid = threadIdx.x / WAVE;
-    for (int d = threadIdx.x; d < BINS; d += SORT_BLOCK) {
-        for (int w = 0; w < SORT_BLOCK / WAVE; ++w) wcnt[w][d] = 0;
-        goff[d] = offsets[(int64_t)d * nblocks + blockIdx.x];
-    }
-    __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * SORT_TILE + (int64_t)wid * (WAVE * SORT_ITEMS);
-    uint32_t kk[SORT_ITEMS], vv[SORT_ITEMS], pos[SORT_ITEMS];
+// Stable rank of each of a wave's keys (ITEMS rounds of 64 consecutive keys) among the wave's keys with its digit;
+// cnt (the wave's own row, zeroed) ends as the wave's digit counts. load runs ahead of round r.
+template <int BITS, int ITEMS, class Load>
+__device__ inline void wave_ranks(const uint32_t (&kk)[ITEMS], int64_t first, int64_t n, int shift, uint32_t* cnt,
+                                  uint32_t (&pos)[ITEMS], Load&& load) {
+    constexpr uint32_t MASK = (1u << BITS) - 1u;
+    const int lane = __lane_id();
 #pragma unroll
-    for (int r = 0; r < SORT_ITEMS; ++r) {
-        const int64_t i = base + (int64_t)r * WAVE + lane;
+    for (int r = 0; r < ITEMS; ++r) {
+        const int64_t i = first + (int64_t)r * WAVE + lane;
         const bool valid = i < n;
-        kk[r] = valid ? kin[i] : 0u;
-        vv[r] = valid ? vin[i] : 0u;
+        load(r, i, valid);
         const uint32_t digit = (kk[r] >> shift) & MASK;
         uint64_t peers = __ballot(valid);
 #pragma unroll
@@ -178,10 +179,77 @@ __global__ void __launch_bounds__(SORT_BLOCK) k_sort_scatter(const uint32_t* __r
                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)peers, 0u));
         const int leader = __ffsll((unsigned long long)peers) - 1;
         uint32_t old = 0;
-        if (valid && lane == leader) old = atomicAdd(&wcnt[wid][digit], (uint32_t)__popcll(peers));
+        if (valid && lane == leader) old = atomicAdd(&cnt[digit], (uint32_t)__popcll(peers));
         old = __shfl(old, leader < 0 ? 0 : leader, WAVE);
         pos[r] = old + rank;
     }
+}
+
+// table: DIRECT, the tile-major histograms; else the scanned digit-major offsets.
+template <int BITS, int ITEMS, bool DIRECT>
+__global__ void __launch_bounds__(SORT_BLOCK) k_sort_scatter(const uint32_t* __restrict__ kin,
+                                                              const uint32_t* __restrict__ vin,
+                                                              uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
+                                                              int64_t n, int shift,
+                                                              const uint32_t* __restrict__ table, int nblocks) {
+    constexpr int BINS = 1 << BITS, DPT = BINS / SORT_BLOCK;  // digits per thread
+    static_assert(DPT * SORT_BLOCK == BINS, "whole digits per thread");
+    constexpr uint32_t MASK = BINS - 1;
+    __shared__ uint32_t wcnt[SORT_BLOCK / WAVE][BINS];
+    __shared__ uint32_t goff[BINS];
+    __shared__ uint32_t lds4[4];
+    const int lane = __lane_id(), wid = threadIdx.x / WAVE;
+    const int64_t base = (int64_t)blockIdx.x * SORT_BLOCK * ITEMS + (int64_t)wid * (WAVE * ITEMS);
+    uint32_t kk[ITEMS], vv[ITEMS], pos[ITEMS];
+    // the direct form fetches everything beside the histograms; the other one round by round, each used before the
+    // next is fetched (4M keys: 36 us a pass against 47 with the loads hoisted to the front)
+    auto load = [&](int r, int64_t i, bool valid) {
+        kk[r] = valid ? kin[i] : 0u;
+        vv[r] = valid ? vin[i] : 0u;
+    };
+    if (DIRECT) {
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            const int64_t i = base + (int64_t)r * WAVE + lane;
+            load(r, i, i < n);
+        }
+        // digits DPT t .. DPT t + DPT - 1 of every tile, 16 tiles' counts in flight
+        uint32_t below[DPT] = {}, total[DPT] = {};
+        for (int b0 = 0; b0 < nblocks; b0 += 16) {
+            uint32_t c[16][DPT];
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+#pragma unroll
+                for (int e = 0; e < DPT; ++e)
+                    c[u][e] = table[(int64_t)min(b0 + u, nblocks - 1) * BINS + threadIdx.x * DPT + e];
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+#pragma unroll
+                for (int e = 0; e < DPT; ++e) {
+                    if (b0 + u < (int)blockIdx.x) below[e] += c[u][e];
+                    if (b0 + u < nblocks) total[e] += c[u][e];
+                }
+        }
+        uint32_t sum = 0, all;
+#pragma unroll
+        for (int e = 0; e < DPT; ++e) sum += total[e];
+        uint32_t run = block_excl_scan(sum, lds4, &all);
+#pragma unroll
+        for (int e = 0; e < DPT; ++e) {
+            goff[threadIdx.x * DPT + e] = run + below[e];
+            run += total[e];
+        }
+    } else {
+        for (int d = threadIdx.x; d < BINS; d += SORT_BLOCK) goff[d] = table[(int64_t)d * nblocks + blockIdx.x];
+    }
+    for (int d = threadIdx.x; d < BINS; d += SORT_BLOCK)
+        for (int w = 0; w < SORT_BLOCK / WAVE; ++w) wcnt[w][d] = 0;
+    __syncthreads();
+    wave_ranks<BITS, ITEMS>(kk, base, n, shift, wcnt[wid], pos, [&](int r, int64_t i, bool valid) {
+        if (DIRECT) return;
+        load(r, i, valid);
+        asm volatile("" ::"v"(kk[r]), "v"(vv[r]) : "memory");  // used here: the rounds' loads stay apart
+    });
     __syncthreads();
     for (int d = threadIdx.x; d < BINS; d += SORT_BLOCK) {  // per digit: exclusive prefix over the waves
         uint32_t run = 0;
@@ -194,7 +262,7 @@ __global__ void __launch_bounds__(SORT_BLOCK) k_sort_scatter(const uint32_t* __r
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < SORT_ITEMS; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const int64_t i = base + (int64_t)r * WAVE + lane;
         if (i < n) {
             const uint32_t digit = (kk[r] >> shift) & MASK;
@@ -205,27 +273,135 @@ __global__ void __launch_bounds__(SORT_BLOCK) k_sort_scatter(const uint32_t* __r
     }
 }
 
+// Every pass of up to SMALL_BLOCK * ITEMS keys in one workgroup: keys and values stay in LDS between passes.
+template <int ITEMS>
+__global__ void __launch_bounds__(SMALL_BLOCK) k_sort_small(uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                                                             int n, int key_bits) {
+    constexpr int NW = SMALL_BLOCK / WAVE, BINS = 256;
+    __shared__ uint32_t sk[SMALL_BLOCK * ITEMS], sv[SMALL_BLOCK * ITEMS];
+    __shared__ uint32_t wcnt[NW][BINS];
+    __shared__ uint32_t goff[BINS];
+    __shared__ uint32_t ws[BINS / WAVE];
+    const int lane = __lane_id(), wid = threadIdx.x / WAVE;
+    const int base = wid * WAVE * ITEMS;
+    uint32_t kk[ITEMS], vv[ITEMS], pos[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const int i = base + r * WAVE + lane;
+        kk[r] = i < n ? keys[i] : 0u;
+        vv[r] = i < n ? vals[i] : 0u;
+    }
+    for (int shift = 0; shift < key_bits; shift += 8) {
+        for (int i = threadIdx.x; i < NW * BINS; i += SMALL_BLOCK) (&wcnt[0][0])[i] = 0;
+        __syncthreads();
+        wave_ranks<8, ITEMS>(kk, base, n, shift, wcnt[wid], pos, [](int, int64_t, bool) {});
+        __syncthreads();
+        uint32_t total = 0, incl = 0;
+        if (threadIdx.x < BINS) {
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const uint32_t c = wcnt[w][threadIdx.x];
+                wcnt[w][threadIdx.x] = total;
+                total += c;
+            }
+            incl = wave_incl_scan(total);
+            if (lane == WAVE - 1) ws[wid] = incl;
+        }
+        __syncthreads();
+        if (threadIdx.x < BINS) {
+            uint32_t off = incl - total;
+            for (int w = 0; w < wid; ++w) off += ws[w];
+            goff[threadIdx.x] = off;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            if (base + r * WAVE + lane < n) {
+                const uint32_t digit = (kk[r] >> shift) & (BINS - 1);
+                const uint32_t dst = goff[digit] + wcnt[wid][digit] + pos[r];
+                sk[dst] = kk[r];
+                sv[dst] = vv[r];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            const int i = base + r * WAVE + lane;
+            if (i < n) {
+                kk[r] = sk[i];
+                vv[r] = sv[i];
+            }
+        }
+        // the next pass writes sk, sv and goff only after barriers that follow these reads
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const int i = base + r * WAVE + lane;
+        if (i < n) {
+            keys[i] = kk[r];
+            vals[i] = vv[r];
+        }
+    }
+}
+
+// Tiles of the sort at n keys: 1024 keys while the direct form has few enough of them, else 4096.
+bool sort_small_tiles(int64_t n) { return n <= (int64_t)DIRECT_TILES * SORT_BLOCK * 4; }
+int sort_tiles(int64_t n) { return ceil_div(n, sort_small_tiles(n) ? SORT_BLOCK * 4 : SORT_TILE); }
+
+template <int BITS, class PartFn>
+void radix_pass(const uint32_t* ki, const uint32_t* vi, uint32_t* ko, uint32_t* vo, int64_t n, int shift,
+                hipStream_t s, uint32_t* cnt, uint32_t* off, PartFn&& part) {
+    const int nb = sort_tiles(n);
+    if (sort_small_tiles(n)) {
+        k_sort_hist<BITS, 4, true><<<nb, SORT_BLOCK, 0, s>>>(ki, n, shift, cnt, nb);
+        LAUNCH_CHECK();
+        k_sort_scatter<BITS, 4, true><<<nb, SORT_BLOCK, 0, s>>>(ki, vi, ko, vo, n, shift, cnt, nb);
+    } else if (nb <= DIRECT_TILES) {
+        k_sort_hist<BITS, SORT_ITEMS, true><<<nb, SORT_BLOCK, 0, s>>>(ki, n, shift, cnt, nb);
+        LAUNCH_CHECK();
+        k_sort_scatter<BITS, SORT_ITEMS, true><<<nb, SORT_BLOCK, 0, s>>>(ki, vi, ko, vo, n, shift, cnt, nb);
+    } else {
+        k_sort_hist<BITS, SORT_ITEMS, false><<<nb, SORT_BLOCK, 0, s>>>(ki, n, shift, cnt, nb);
+        LAUNCH_CHECK();
+        scan_rec(cnt, off, ((int64_t)1 << BITS) * nb, s, part, 0, nullptr);
+        k_sort_scatter<BITS, SORT_ITEMS, false><<<nb, SORT_BLOCK, 0, s>>>(ki, vi, ko, vo, n, shift, off, nb);
+    }
+    LAUNCH_CHECK();
+}
+
 // One stable LSD pass structure over explicit buffers (ak, av: n keys and values; cnt, off: one count per digit
 // value and sort tile).
 template <class PartFn>
 void radix_passes(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, uint32_t* ak,
-                  uint32_t* av, uint32_t* cnt, uint32_t* off, PartFn&& part) {
-    const int nb = ceil_div(n, SORT_TILE);
+                  uint32_t* av, uint32_t* cnt, uint32_t* off, PartFn&& part, bool keep_keys) {
     uint32_t *ki = keys, *vi = vals, *ko = ak, *vo = av;
     int passes = 0;
-    for (int shift = 0; shift < key_bits; shift += RADIX_BITS, ++passes) {
-        k_sort_hist<RADIX_BITS><<<nb, SORT_BLOCK, 0, s>>>(ki, n, shift, cnt, nb);
-        LAUNCH_CHECK();
-        scan_rec(cnt, off, ((int64_t)1 << RADIX_BITS) * nb, s, part, 0, nullptr);
-        k_sort_scatter<RADIX_BITS><<<nb, SORT_BLOCK, 0, s>>>(ki, vi, ko, vo, n, shift, off, nb);
-        LAUNCH_CHECK();
+    if (key_bits == 9) {
+        radix_pass<9>(ki, vi, ko, vo, n, 0, s, cnt, off, part);
         std::swap(ki, ko);
         std::swap(vi, vo);
+        ++passes;
+    } else {
+        for (int shift = 0; shift < key_bits; shift += RADIX_BITS, ++passes) {
+            radix_pass<RADIX_BITS>(ki, vi, ko, vo, n, shift, s, cnt, off, part);
+            std::swap(ki, ko);
+            std::swap(vi, vo);
+        }
     }
     if (passes & 1) {
-        HIP_CHECK(hipMemcpyAsync(keys, ki, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
+        if (keep_keys) HIP_CHECK(hipMemcpyAsync(keys, ki, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
         HIP_CHECK(hipMemcpyAsync(vals, vi, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
     }
+}
+
+// Sorts up to SMALL_MAX pairs in one launch; false above.
+bool radix_small(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s) {
+    if (n > SMALL_MAX) return false;
+    if (n <= 2 * SMALL_BLOCK) k_sort_small<2><<<1, SMALL_BLOCK, 0, s>>>(keys, vals, (int)n, key_bits);
+    else if (n <= 4 * SMALL_BLOCK) k_sort_small<4><<<1, SMALL_BLOCK, 0, s>>>(keys, vals, (int)n, key_bits);
+    else k_sort_small<8><<<1, SMALL_BLOCK, 0, s>>>(keys, vals, (int)n, key_bits);
+    LAUNCH_CHECK();
+    return true;
 }
 
 __global__ void __launch_bounds__(SCAN_BLOCK) k_sum_u64(const uint32_t* __restrict__ in, int64_t n,
@@ -290,32 +466,33 @@ void exclusive_scan_u32_dev(const uint32_t* in, uint32_t* out, int64_t n, hipStr
     scan_rec(in, out, n, s, scratch_parts(sc), 0, total_dev);
 }
 
-void radix_sort_pairs(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, Scratch& sc) {
-    if (n <= 1) return;
-    const int nb = ceil_div(n, SORT_TILE);
+void radix_sort_pairs(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, Scratch& sc,
+                      bool keep_keys) {
+    if (n <= 1 || radix_small(keys, vals, n, key_bits, s)) return;
+    const int nb = sort_tiles(n);
     DBuf<uint32_t>& ak = part_buf(sc, 4);
     DBuf<uint32_t>& av = part_buf(sc, 5);
     DBuf<uint32_t>& cnt = part_buf(sc, 6);
     DBuf<uint32_t>& off = part_buf(sc, 7);
-    const size_t bins = (size_t)1 << RADIX_BITS;
+    const size_t bins = (size_t)1 << (key_bits == 9 ? 9 : RADIX_BITS);
     ak.alloc(n);
     av.alloc(n);
     cnt.alloc(bins * nb);
     off.alloc(bins * nb);
-    radix_passes(keys, vals, n, key_bits, s, ak.p, av.p, cnt.p, off.p, scratch_parts(sc));
+    radix_passes(keys, vals, n, key_bits, s, ak.p, av.p, cnt.p, off.p, scratch_parts(sc), keep_keys);
 }
 
 size_t radix_sort_workspace_words(int64_t n) {
-    const int64_t nb = (n + SORT_TILE - 1) / SORT_TILE;
-    const int64_t c = ((int64_t)1 << RADIX_BITS) * nb;  // count and offset tables
+    const int64_t nb = sort_tiles(n);
+    const int64_t c = ((int64_t)1 << (RADIX_BITS + 1)) * nb;  // count and offset tables, a 9-bit digit's at most
     const int64_t p0 = (c + SCAN_TILE - 1) / SCAN_TILE, p1 = (p0 + SCAN_TILE - 1) / SCAN_TILE;
     const int64_t p2 = (p1 + SCAN_TILE - 1) / SCAN_TILE;
     return (size_t)(2 * n + 2 * c + 2 * (p0 + p1 + p2));
 }
 
 void radix_sort_pairs_ws(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, uint32_t* ws) {
-    if (n <= 1) return;
-    const int64_t nb = (n + SORT_TILE - 1) / SORT_TILE, c = ((int64_t)1 << RADIX_BITS) * nb;
+    if (n <= 1 || radix_small(keys, vals, n, key_bits, s)) return;
+    const int64_t nb = sort_tiles(n), c = ((int64_t)1 << (RADIX_BITS + 1)) * nb;
     const int64_t p0 = (c + SCAN_TILE - 1) / SCAN_TILE, p1 = (p0 + SCAN_TILE - 1) / SCAN_TILE;
     uint32_t* ak = ws;
     uint32_t* av = ak + n;
@@ -325,7 +502,7 @@ void radix_sort_pairs_ws(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits
     auto part = [parts, p0, p1](int depth, size_t) {
         return depth == 0 ? parts : (depth == 1 ? parts + 2 * p0 : parts + 2 * (p0 + p1));
     };
-    radix_passes(keys, vals, n, key_bits, s, ak, av, cnt, off, part);
+    radix_passes(keys, vals, n, key_bits, s, ak, av, cnt, off, part, true);
 }
 
 static DBuf<uint32_t>& part_buf(Scratch& sc, int i) { return sc.bufs[i]; }

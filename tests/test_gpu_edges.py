@@ -140,3 +140,24 @@ def test_resident_taubin_from_threads(egt_mod):
     for key in alone:
         for a, b in zip(alone[key], together[key]):
             np.testing.assert_array_equal(a, b, err_msg=str(key))
+
+
+@pytest.mark.parametrize("n", [2, 1_024, 2_048, 2_049, 4_096, 4_097, 8_192, 8_193, 262_144, 262_145, 1_048_576, 1_048_577])
+def test_sorts_at_form_limits(egt_mod, n):
+    """Sizes at the limits of the sort's forms (one workgroup with 2, 4 or 8 keys a thread; tiles of 1024 and of 4096
+    keys; scanned counts): the sorted order is numpy's stable sort by cell key, on keys with many duplicates."""
+    E = egt_mod
+    print("n", n, flush=True)
+    r = np.random.default_rng(n)
+    pts = [r.uniform(0, 1, n).astype(np.float32) for _ in range(3)]
+    for a in pts:
+        a[: n // 2] = np.float32(0.5) + (a[: n // 2] - np.float32(0.5)) * np.float32(0.02)  # crowded cells
+    g = E.GridStructure(tuple(pts), 1, 1e-6, 256, 4)
+    mn, mx = np.float32(g.GetMinExtent()), np.float32(g.GetMaxExtent())
+    eps = np.float32(1e-6)
+    a, ba = -eps, (np.float32(1) + eps) + eps
+    c = [(((p - mn) / (mx - mn) - a) / ba * np.float32(256)).astype(np.int64) for p in pts]
+    order = np.argsort(c[0] | (c[1] << 8) | (c[2] << 16), kind="stable")
+    perm = E.device_array(g.GetOriginalRefIndexesDevice(), n, np.int32)
+    np.testing.assert_array_equal(perm, order)
+    g.close()
