@@ -161,3 +161,24 @@ def test_sorts_at_form_limits(egt_mod, n):
     perm = E.device_array(g.GetOriginalRefIndexesDevice(), n, np.int32)
     np.testing.assert_array_equal(perm, order)
     g.close()
+
+
+@pytest.mark.parametrize("n,k", [(1, 4), (2, 1), (63, 6), (1_025, 8), (8_192, 16), (8_193, 16), (30_000, 40), (70_001, 8)])
+def test_normals_at_forest_forms(egt_mod, oracle_mod, n, k):
+    """The spanning forest in one workgroup (up to 8192 points) and in launches per round, with several trees (two
+    separate spheres): normals, trees and edges equal the oracle's."""
+    E, O = egt_mod, oracle_mod
+    print("n", n, "k", k, flush=True)
+    a = D.sphere(max(n // 2, 1), seed=801)
+    b = D.sphere(n - n // 2, seed=802) if n > 1 else a
+    pts = a if n == 1 else tuple(np.concatenate([u, v + np.float32(3 * (ax == 0))]) for ax, (u, v) in enumerate(zip(a, b)))
+    ref = O.pipeline(*pts, k, 2, 0.5, -0.53, 0.65, normals=True)
+    g = E.GridStructure(pts, 1, 1e-6, 1024, 4)
+    g.GRIDCUDAKNNSELF_COMPACT(k, 1e8)
+    E.EGT_CUDA(g).PerformSmoothing(2, 0.5, -0.53, 0.65)
+    got = E.Normal_CUDA(g).GetNormals()
+    st = g.stats()
+    g.close()
+    assert st["msf_edges"] == ref["orient_stats"][1] and st["msf_trees"] == ref["orient_stats"][2]
+    for u, v in zip(got, ref["normals"]):
+        np.testing.assert_array_equal(u, v)
