@@ -89,7 +89,10 @@ typedef struct {
 /* Options set through egt_set_option (no reference counterpart). */
 typedef enum {
     EGT_OPT_START_LEVEL = 0,     /* kNN: pyramid level of the first search box; 0 = the query's own cell, as
-                                    in the reference (default); > 0 coarser cells; -1, -2, -3 = cells of 1/2,
+                                    in the reference (default; on small clouds and clouds of even density the
+                                    library starts at the occupancy level below instead, unless
+                                    EGT_OPT_KNN_LONG_QUERY is changed or egt_autotune chose the level); > 0
+                                    coarser cells; -1, -2, -3 = cells of 1/2,
                                     1/4, 1/8 of a grid cell; EGT_START_LEVEL_OCCUPANCY = one level from the
                                     mean cell occupancy */
     EGT_OPT_LEARNED = 1,         /* kNN: 1 = start each query from the learned radius proposal */

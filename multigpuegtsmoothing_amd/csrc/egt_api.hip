@@ -331,6 +331,7 @@ egt_status egt_set_option(egt_handle h, egt_option opt, int64_t value) {
             if (value != EGT_START_LEVEL_OCCUPANCY && (value < -egt::SUB || value >= h->nlev))
                 return fail(EGT_ERR_INVALID_ARG, "start level out of range");
             h->start_level = (int)value;
+            h->start_tuned = false;
             return EGT_OK;
         case EGT_OPT_LEARNED:
             h->learned = value ? 1 : 0;

@@ -135,6 +135,8 @@ struct CloudDev {
     float min_extent, extent;  // de-normalization: x = x' * extent + min_extent
     int32_t ref_level;         // learned proposal: feature level
     float max_extent;          // bounding cube upper end (as computed, not min_extent + extent)
+    int32_t start_level;       // level of the cloud's first search box where the launch names none
+    int32_t pad;
 };
 
 constexpr int64_t KNN_LONG_CAP = 2048;  // default of EGT_OPT_KNN_LONG_QUERY
@@ -225,6 +227,7 @@ struct egt_ctx {
     bool have_query = false;
 
     // options
+    bool start_tuned = false;  // a tuner chose start_level: 0 then means the own cell
     int start_level = 0;  // reference schedule: every query starts at its own level-0 cell; -SUB..-1 sub-cell
                           // boxes; EGT_START_LEVEL_OCCUPANCY = from the mean cell occupancy
     int learned = 0;

@@ -109,7 +109,7 @@ struct KnnParams {
     int B, log2B, stages, maxc;
     int Bv;            // cells per axis at internal level 0 (B << SUB)
     int nlev;          // internal levels: SUB sub-cell levels + the reference pyramid
-    int start_level;   // internal level of the first box (SUB = the query's own fine cell)
+    int start_level;   // internal level of the first box (SUB = the query's own fine cell); -1: each cloud's own
     int level_offset;  // added to every proposed start level
     uint32_t long_cap; // lane-per-query search: a query that has tested more candidates than this is handed
                        // back to a wave-per-query pass (0 = never)
@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(KBLK)
     const bool active = LIST ? m >= 0 : m < cd.base + cd.n;
     // Learned start: every lane of a wave starts at the smallest level proposed in the wave, so the wave's
     // 64 neighbouring queries scan the same cells in step; lanes whose proposal is higher expand from there.
-    int own_level = P.start_level;
+    int own_level = P.start_level >= 0 ? P.start_level : SUB + cd.start_level;
     int wave_level = own_level;
     if (P.qlevel) {
         own_level = active ? (int)P.qlevel[m] + SUB + P.level_offset : 127;
@@ -827,7 +827,7 @@ __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) 
                       uz = cell_of(q.z, P.a, P.ba, P.B);
             outside = ux < 0 || uy < 0 || uz < 0 || ux >= P.B || uy >= P.B || uz >= P.B;
         }
-        int own_level = P.start_level;
+        int own_level = P.start_level >= 0 ? P.start_level : SUB + cd.start_level;
         if (P.qlevel) {
             own_level = (int)P.qlevel[m] + SUB + P.level_offset;
             ++nlearned;
@@ -1205,6 +1205,8 @@ void launch_wave(KnnParams P, hipStream_t s) {
 //   mixture  k=8         0.84 / 0.047     1.19 / 0.25    1.02 / 0.57    1.48 / 1.48    3.54 / 3.93
 //   mixture  k=16        1.01 / 0.047     1.89 / 0.29    1.66 / 0.64    1.98 / 1.73    4.12 / 4.51
 //   mixture  k=40        1.34 / 0.049     2.92 / 0.41    4.61 / 0.78    5.54 / 2.17    9.34 / 5.99
+// From the occupancy level (below), torus: k=16 150,000 0.35 / 0.32, 500,000 0.54 / 0.92; k=40 150,000 0.52 / 0.39,
+// 500,000 1.10 / 1.14; k=32 500,000 0.91 / 1.08.
 // (4M-point torus and 16M-point mixture: k=40 14.3 / 16.3 and 57.0 / 67.7, k=48 21.0 / 17.3 and 87.5 / 71.6.)
 // Dense clusters make costly lanes, so an uneven cloud gains up to larger sizes: uneven is a cloud whose fullest
 // cell of 8 fine cells a side holds 64 times the mean of the non-empty ones (sphere and torus: up to 6 times,
@@ -1212,7 +1214,7 @@ void launch_wave(KnnParams P, hipStream_t s) {
 bool wave_by_size(int K, int64_t queries, bool uneven) {
     if (K >= 48) return true;
     if (uneven) return queries <= (K <= 8 ? 400000 : K <= 16 ? 600000 : 2000000);
-    return queries <= (K <= 16 ? 80000 : 150000);
+    return queries <= (K <= 16 ? 80000 : 250000);
 }
 
 // The query search's shape. Up to QUERY_UNSORTED queries go to a wave each in their own order: the sort that makes
@@ -1295,9 +1297,27 @@ int64_t search_class(egt_ctx* h, KnnParams P, int K, hipStream_t s, int shape) {
     return (int64_t)nb;
 }
 
-// Search parameters of the handle; with scratch, the per-point k-th distance, the counters and the bounded
+// Where nothing asks for a start level (the option at 0, no tuner, the long query cap untouched), a search of a cloud
+// of even density starts at the occupancy level: from its own cell a query climbs through boxes that cannot hold k
+// points, 27 lookups each. From the own cell / the occupancy level, the search shape of the size, in ms:
+//   sphere  2,000 k=8 0.045 / 0.019    100,000 k=40 0.78 / 0.31    500,000 k=8 1.40 / 0.43    1.5M k=40 6.2 / 3.0
+//   torus   50,000 k=16 0.34 / 0.13    1.5M k=16 3.1 / 1.5    4M k=40 14.3 / 8.2, k=64 18.7 / 10.8    16M k=40 51.5 / 38.7
+//   mixture 2,000 k=40 0.049 / 0.020   50,000 k=16 0.29 / 0.19    150,000 k=40 0.83 / 0.80    500,000 k=40 2.3 / 2.4
+//           4M k=40 14.5 / 30.3    16M k=40 57.0 / 89.1
+// (one level does not fit an uneven cloud, whose dense cells it overfills: beyond START_ANY points such a cloud keeps
+// the own cell, and so do the larger clouds of a batch, whose evenness is not known one by one).
+constexpr int64_t START_ANY = 100000;
+bool own_cell_by_default(const egt_ctx* h) {
+    return h->start_level == 0 && !h->start_tuned && h->knn_long_cap == KNN_LONG_CAP;
+}
+int default_start_level(const egt_ctx* h, int k, int cloud = 0) {
+    if (h->clouds[cloud].n > START_ANY && (h->nclouds > 1 || uneven_cloud(h))) return 0;
+    return auto_start_level(h, k, cloud);
+}
+
+// Search parameters of the handle for neighbour count k (of its first cloud); with scratch, the per-point k-th distance, the counters and the bounded
 // search's hand-back list come from the handle's scratch (else they are left null for the caller).
-KnnParams knn_params(egt_ctx* h, bool scratch = true) {
+KnnParams knn_params(egt_ctx* h, int k, bool scratch = true) {
     KnnParams P{};
     P.mpts = h->mpts.p;
     P.mcell = h->mcell.p;
@@ -1333,8 +1353,11 @@ KnnParams knn_params(egt_ctx* h, bool scratch = true) {
     P.log2B = log2B;
     P.Bv = h->B << SUB;
     P.nlev = h->nlev + SUB;
-    P.start_level = SUB + (h->start_level == EGT_START_LEVEL_OCCUPANCY ? auto_start_level(h, h->clouds[0].k)
-                                                                         : std::min(h->start_level, h->nlev - 1));
+    if (own_cell_by_default(h))
+        P.start_level = h->nclouds > 1 ? -1 : SUB + default_start_level(h, k);
+    else
+        P.start_level = SUB + (h->start_level == EGT_START_LEVEL_OCCUPANCY ? auto_start_level(h, h->clouds[0].k)
+                                                                             : std::min(h->start_level, h->nlev - 1));
     int stages = 0;
     for (int b = h->B; b >= 8; b >>= 1) ++stages;
     P.stages = std::max(stages, 1);
@@ -1382,9 +1405,11 @@ std::vector<WorkClass> build_work_lists(egt_ctx* h, DBuf<int64_t>& lists) {
 // Lays out the rows (cloud after cloud, n_c x k_c) and uploads the per-cloud parameters.
 void prepare_clouds(egt_ctx* h) {
     int64_t off = 0;
-    for (CloudDev& c : h->clouds) {
+    for (int i = 0; i < h->nclouds; ++i) {
+        CloudDev& c = h->clouds[i];
         c.row_off = off;
         off += c.n * c.k;
+        c.start_level = default_start_level(h, c.k, i);
     }
     h->knn.alloc((size_t)std::max<int64_t>(off, 1));
     h->dclouds.alloc(h->clouds.size());
@@ -1409,7 +1434,7 @@ int auto_start_level(const egt_ctx* h, int k, int cloud) {
 void run_knn_clouds(egt_ctx* h) {
     hipStream_t s = h->stream;
     prepare_clouds(h);
-    KnnParams P = knn_params(h);
+    KnnParams P = knn_params(h, h->clouds[0].k);
     const std::vector<WorkClass> classes = build_work_lists(h, h->work_lists);
     h->work_classes = classes;
     clear_stats(P, s);
@@ -1455,7 +1480,7 @@ void run_knn_query(egt_ctx* h, const float* dqx, const float* dqy, const float* 
     h->qknn.alloc((size_t)std::max<int64_t>(nq * k, 1));
     h->qpts.alloc((size_t)std::max<int64_t>(nq, 1));
     h->qvcell.alloc((size_t)std::max<int64_t>(nq, 1));
-    KnnParams P = knn_params(h);
+    KnnParams P = knn_params(h, k);
     P.long_cap = 0;
     clear_stats(P, s);
     Event e0, e1;
@@ -1575,7 +1600,7 @@ void run_knn_query_noalloc(egt_ctx* h, const float* dqx, const float* dqy, const
     uint64_t* qcell = reinterpret_cast<uint64_t*>(w + 12 * NQ);
     CloudDev* qcloud = reinterpret_cast<CloudDev*>(w + 14 * NQ);
     hipStream_t s = h->stream;
-    KnnParams P = knn_params(h, false);
+    KnnParams P = knn_params(h, k, false);
     P.long_cap = 0;
     CloudDev qcd{};
     qcd.base = 0;
@@ -1636,7 +1661,7 @@ int autotune_shape(egt_ctx* h, int k, float thres_n, float* shape_ms) {
     h->clouds[0].k = k;
     h->clouds[0].thres_n = thres_n;
     prepare_clouds(h);
-    KnnParams P = knn_params(h);
+    KnnParams P = knn_params(h, k);
     clear_stats(P, s);  // scratch holds earlier contents
     const int64_t total = (h->n + 63) / 64;
     KnnParams W = P;  // warm-up: the autotuner's sample
@@ -1681,7 +1706,7 @@ int autotune_shape(egt_ctx* h, int k, float thres_n, float* shape_ms) {
 int64_t autotune_class_shapes(egt_ctx* h, float* ms) {
     hipStream_t s = h->stream;
     prepare_clouds(h);
-    KnnParams P = knn_params(h);
+    KnnParams P = knn_params(h, h->clouds[0].k);
     clear_stats(P, s);  // scratch holds earlier contents
     const std::vector<WorkClass> classes = build_work_lists(h, h->work_lists);
     for (int i = 0; i < 24; ++i) ms[i] = -1.0f;
@@ -1736,7 +1761,7 @@ void autotune_learned(egt_ctx* h, int k, float thres_n, int* best_off, int* best
         for (int mi = 0; mi < 2; ++mi) {
             h->learned_level_offset = off;
             h->learned_mode = mi == 0 ? 1 : 3;
-            KnnParams P = knn_params(h);
+            KnnParams P = knn_params(h, k);
             clear_stats(P, s);
             KnnParams W = P;
             W.stride = (int)std::max<int64_t>(1, total / 8192);
@@ -1778,7 +1803,7 @@ int autotune_start_level(egt_ctx* h, int k, float thres_n, float* trial_ms, floa
     prepare_clouds(h);
     const int saved_learned = h->learned;
     h->learned = 0;
-    KnnParams P = knn_params(h);
+    KnnParams P = knn_params(h, k);
     h->learned = saved_learned;
     P.long_cap = 0;  // every query's whole work counts
     const int64_t total = (h->n + 63) / 64;
@@ -1810,6 +1835,7 @@ int autotune_start_level(egt_ctx* h, int k, float thres_n, float* trial_ms, floa
         }
     }
     h->start_level = best;
+    h->start_tuned = true;
     h->have_knn = false;  // the trial rows cover only the sample
     return best;
 }

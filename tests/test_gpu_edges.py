@@ -54,7 +54,8 @@ def test_lane_shape_on_small_clouds(egt_mod, oracle_mod, k):
         g.close()
 
 
-@pytest.mark.parametrize("n,k", [(80_000, 16), (80_065, 16), (99_970, 8), (150_017, 40), (299_995, 48)])
+@pytest.mark.parametrize("n,k", [(80_000, 16), (80_065, 16), (99_970, 8), (150_017, 40), (250_000, 33), (250_049, 40),
+                                 (299_995, 48)])
 def test_self_search_at_shape_limits(egt_mod, oracle_mod, n, k):
     """Sizes at the limits of the launch-shape rule and of the queries a wave serves (1, 2, 4)."""
     E, O = egt_mod, oracle_mod
@@ -69,7 +70,7 @@ def test_self_search_at_shape_limits(egt_mod, oracle_mod, n, k):
 
 
 @pytest.mark.parametrize("nq,k", [(1, 1), (63, 64), (99_999, 8), (100_000, 1), (100_001, 16), (100_001, 33),
-                                  (150_001, 40), (120_000, 64)])
+                                  (250_001, 40), (120_000, 64)])
 def test_query_search_at_shape_limits(egt_mod, oracle_mod, nq, k):
     """Query counts around the limits of the unsorted, sorted and lane-per-query searches, a tenth of the queries
     outside the grid and a finite radius."""
