@@ -52,11 +52,10 @@ constexpr uint32_t SPLIT_COUNT = 96;
 // most of the gain from the own cell.
 constexpr uint32_t WAVE_SPLIT_COUNT = 384;
 // Wave-per-query search: a batch with more survivors than this is sorted and merged into the list, fewer are
-// inserted one at a time. Measured on a 16M-point cluster mixture at 16 / 8 / 32 / never: k=64 from learned
-// starts 59.0 / 60.0 / 60.0 / 75.4 ms, from the own cell 81.7 / 82.4 / 82.4 / 89.9; k=40 from the own cell
-// 69.7 / 70.1 / 70.1 / 72.8, from learned starts 60.4 / 60.0 / 59.9 / 56.6 (there a lane per query is faster
-// still); a 4M-point torus at level 2, k=64: 11.0 / 11.2 / 11.2 / 15.2 ms.
-constexpr int WAVE_SORT_MIN = 16;
+// inserted one at a time. At 8 / 11 / 16: a 4M-point cluster mixture at k=40 12.83 / 12.85 / 12.94 ms, at k=64 15.28 /
+// 15.29 / 15.41; a 1M-point torus at k=48 2.01 / 2.03 / 2.04; never sorting took a 16M-point mixture at k=64 from 59 to
+// 75 ms.
+constexpr int WAVE_SORT_MIN = 8;
 // Keys (distance bits << 32 | sorted index) of non-negative distances, read as IEEE doubles, are positive
 // and order exactly as the integers do, so the list is held as doubles and merged with FP64 min / max (full
 // rate on gfx950; keys of zero distance are denormal doubles, which compute kernels keep). The empty key is
@@ -663,55 +662,64 @@ __device__ inline double shfl_xor_d(double x, int j) {
     const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(u >> 32), j, 64);
     return key_d(((uint64_t)hi << 32) | lo);
 }
-// Value of lane ^ J: quad_perm for 1 and 2, row_shl / row_shr inside rows of 16 for 4 and 8, else ds_bpermute.
-template <int J>
+// Value of lane ^ M: quad_perm for 1, 2 and 3, row_half_mirror (7), row_ror:8 (8), row_mirror (15), 7 then 3 for 4;
+// across rows of 16 a swizzle (16, 31), across halves ds_bpermute (32, 63).
+template <int M>
 __device__ inline int xor_lane(int x) {
-    if constexpr (J == 1) {
-        return dpp<0xB1, 0xf, true>(x);
-    } else if constexpr (J == 2) {
-        return dpp<0x4E, 0xf, true>(x);
-    } else if constexpr (J == 4 || J == 8) {
-        const int a = dpp<0x100 + J, 0xf, true>(x), b = dpp<0x110 + J, 0xf, true>(x);
-        return (__lane_id() & J) ? b : a;
-    } else {
-        return __shfl_xor(x, J, 64);
-    }
+    if constexpr (M == 1) return dpp<0xB1, 0xf, true>(x);
+    else if constexpr (M == 2) return dpp<0x4E, 0xf, true>(x);
+    else if constexpr (M == 3) return dpp<0x1B, 0xf, true>(x);
+    else if constexpr (M == 4) return dpp<0x1B, 0xf, true>(dpp<0x141, 0xf, true>(x));
+    else if constexpr (M == 7) return dpp<0x141, 0xf, true>(x);
+    else if constexpr (M == 8) return dpp<0x128, 0xf, true>(x);
+    else if constexpr (M == 15) return dpp<0x140, 0xf, true>(x);
+    else if constexpr (M == 16) return __builtin_amdgcn_ds_swizzle(x, 0x401F);
+    else if constexpr (M == 31) return __builtin_amdgcn_ds_swizzle(x, 0x7C1F);
+    else return __shfl_xor(x, M, 64);
 }
-template <int J>
-__device__ inline double xor_lane_d(double x) {
+// One compare-exchange stage with the partner lane ^ M: the lane whose bit J is clear keeps the smaller key. The
+// keys are held negated in lanes whose bit J is set, so both lanes keep min(own, -partner's): one FP64 instruction
+// instead of a min, a max and two selects. flip<A, B> moves the signs from bit A to bit B (0: not negated). With
+// direction bits, two-step exchanges at 4 and 8 and min / max / select the search took 14.75 against 12.99 ms on a
+// 4M-point cluster mixture at k=40, 17.6 / 15.4 at k=64, 2.49 / 2.02 on a 1M-point torus at k=48.
+template <int M>
+__device__ inline double stage(double x) {
     const uint64_t u = key_u(x);
-    const uint32_t lo = (uint32_t)xor_lane<J>((int)(uint32_t)u), hi = (uint32_t)xor_lane<J>((int)(uint32_t)(u >> 32));
-    return key_d(((uint64_t)hi << 32) | lo);
+    const uint32_t lo = (uint32_t)xor_lane<M>((int)(uint32_t)u), hi = (uint32_t)xor_lane<M>((int)(uint32_t)(u >> 32));
+    const double p = key_d(((uint64_t)hi << 32) | lo);
+    double r;
+    asm("v_min_f64 %0, %1, -%2" : "=v"(r) : "v"(x), "v"(p));
+    return r;
 }
-// One compare-exchange stage of a bitonic network: partner lane ^ J; the lane keeps the smaller key when its
-// J bit equals its K2 bit (ascending blocks of K2; K2 = 64 and above sorts the whole wave ascending).
-template <int K2, int J>
-__device__ inline double bstage(double x) {
-    const int lane = __lane_id();
-    const double p = xor_lane_d<J>(x);
-    const bool up = K2 >= 64 || (lane & K2) == 0;
-    const bool low = (lane & J) == 0;
-    const double mn = dmin(x, p), mx = dmax(x, p);  // both, then a select: no exec-mask branch
-    return (low == up) ? mn : mx;
+template <int A, int B>
+__device__ inline double flip(double x) {
+    const uint32_t lane = __lane_id();
+    const uint32_t m = ((lane & A) != 0) != ((lane & B) != 0) ? 0x80000000u : 0u;
+    const uint64_t u = key_u(x);
+    return key_d((uint64_t)(uint32_t)u | ((uint64_t)((uint32_t)(u >> 32) ^ m) << 32));
 }
-// Bitonic sort of the 64 lanes' keys, ascending by lane.
+// Stages 8, 4, 2, 1 (each a half-cleaner) after a stage on bit A.
+template <int A, int FROM>
+__device__ inline double clean(double x) {
+    if constexpr (FROM == 1) return stage<1>(flip<A, 1>(x));
+    else return clean<FROM, FROM / 2>(stage<FROM>(flip<A, FROM>(x)));
+}
+// Bitonic sort of the 64 lanes' keys, ascending by lane: blocks of 2, 4, .. 64 keys are merged by a stage against
+// the mirrored lane (every block ascending, no direction bits) and half-cleaners.
 __device__ inline double sort64(double x) {
-    x = bstage<2, 1>(x);
-    x = bstage<4, 2>(x); x = bstage<4, 1>(x);
-    x = bstage<8, 4>(x); x = bstage<8, 2>(x); x = bstage<8, 1>(x);
-    x = bstage<16, 8>(x); x = bstage<16, 4>(x); x = bstage<16, 2>(x); x = bstage<16, 1>(x);
-    x = bstage<32, 16>(x); x = bstage<32, 8>(x); x = bstage<32, 4>(x); x = bstage<32, 2>(x); x = bstage<32, 1>(x);
-    x = bstage<64, 32>(x); x = bstage<64, 16>(x); x = bstage<64, 8>(x); x = bstage<64, 4>(x); x = bstage<64, 2>(x);
-    x = bstage<64, 1>(x);
-    return x;
+    x = stage<1>(flip<0, 1>(x));
+    x = clean<2, 1>(stage<3>(flip<1, 2>(x)));
+    x = clean<4, 2>(stage<7>(flip<1, 4>(x)));
+    x = clean<8, 4>(stage<15>(flip<1, 8>(x)));
+    x = clean<16, 8>(stage<31>(flip<1, 16>(x)));
+    x = clean<32, 16>(stage<63>(flip<1, 32>(x)));
+    return flip<1, 0>(x);
 }
 // The 64 smallest of the ascending list L and the ascending batch S, ascending: min(L[i], S[63 - i]) is a
-// bitonic sequence holding them, then a bitonic merge.
+// bitonic sequence holding them, then half-cleaners.
 __device__ inline double merge64(double L, double S) {
-    double x = dmin(L, shfl_xor_d(S, 63));
-    x = bstage<64, 32>(x); x = bstage<64, 16>(x); x = bstage<64, 8>(x); x = bstage<64, 4>(x); x = bstage<64, 2>(x);
-    x = bstage<64, 1>(x);
-    return x;
+    const double x = dmin(L, shfl_xor_d(S, 63));
+    return flip<1, 0>(clean<0, 32>(x));
 }
 // Running maximum over the wave of non-negative values (the same DPP steps as scan_add).
 __device__ inline int scan_max(int x) {
