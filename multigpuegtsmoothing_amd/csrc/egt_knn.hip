@@ -1203,26 +1203,33 @@ void launch_wave(KnnParams P, hipStream_t s) {
 }
 
 // Launch shape of a search of `queries` queries in class K where nothing asks for one: a lane per query leaves the
-// GPU idle when the queries are few (its waves then last as long as their costliest lane) and runs two waves per
-// SIMD once the list passes 40 keys. Measured lane / wave in ms, from the own cell:
-//                            2,000          50,000         150,000        500,000        1.5M
-//   sphere   k=8                          0.52 / 0.33    0.64 / 0.80    1.40 / 2.46    3.27 / 5.61
-//   torus    k=16        0.72 / 0.046     0.64 / 0.34    0.66 / 0.76    1.37 / 2.21    3.09 / 5.54
-//   torus    k=40        0.89 / 0.050     0.85 / 0.39    0.96 / 0.94    2.36 / 2.72    5.64 / 6.57
-//   torus    k=48        0.92 / 0.050     0.93 / 0.41    1.49 / 0.97    3.26 / 2.81    8.67 / 6.95
-//   mixture  k=8         0.84 / 0.047     1.19 / 0.25    1.02 / 0.57    1.48 / 1.48    3.54 / 3.93
-//   mixture  k=16        1.01 / 0.047     1.89 / 0.29    1.66 / 0.64    1.98 / 1.73    4.12 / 4.51
-//   mixture  k=40        1.34 / 0.049     2.92 / 0.41    4.61 / 0.78    5.54 / 2.17    9.34 / 5.99
-// From the occupancy level (below), torus: k=16 150,000 0.35 / 0.32, 500,000 0.54 / 0.92; k=40 150,000 0.52 / 0.39,
-// 500,000 1.10 / 1.14; k=32 500,000 0.91 / 1.08.
-// (4M-point torus and 16M-point mixture: k=40 14.3 / 16.3 and 57.0 / 67.7, k=48 21.0 / 17.3 and 87.5 / 71.6.)
+// GPU idle when the queries are few (its waves then last as long as their costliest lane) and has fewer waves the
+// longer the list (three per SIMD above 16 keys, two above 40). Measured lane / wave in ms, each from its default
+// start level (see START_ANY):
+//                            100,000         150,000        300,000        500,000         1M             4M
+//   sphere   k=8          0.14 / 0.17    0.26 / 0.30
+//   torus    k=16         0.25 / 0.19    0.37 / 0.28    0.41 / 0.48
+//   torus    k=24                        0.34 / 0.29    0.59 / 0.52    0.76 / 0.84                  6.13 / 6.57
+//   torus    k=32                                       0.72 / 0.58    0.92 / 0.89    1.75 / 1.77   7.15 / 7.04
+//   torus    k=40                                       0.81 / 0.61    1.10 / 0.93    2.07 / 1.85   8.25 / 7.52
+//   (16M-point torus: k=32 32.8 / 29.6, k=40 38.7 / 32.0; 2,000 points: 0.2-1.0 / 0.02-0.05 at every k)
+//                           500,000          1M             2M             4M              8M            16M
+//   mixture  k=8          1.47 / 1.30    2.20 / 2.27    3.80 / 4.56
+//   mixture  k=16         1.98 / 1.50    3.14 / 2.65    4.61 / 5.33    7.76 / 10.0
+//   mixture  k=24                                       6.41 / 5.86    11.1 / 11.2    21.1 / 23.6   43.1 / 55.3
+//   mixture  k=40         5.46 / 2.04                                  14.4 / 12.9    27.6 / 27.6   57.0 / 61.7
 // Dense clusters make costly lanes, so an uneven cloud gains up to larger sizes: uneven is a cloud whose fullest
 // cell of 8 fine cells a side holds 64 times the mean of the non-empty ones (sphere and torus: up to 6 times,
-// mixture: over 200 times).
-bool wave_by_size(int K, int64_t queries, bool uneven) {
+// mixture: over 200 times). Above 40 keys the wave wins on every cloud. Learned starts keep the lane shape at smaller
+// sizes (16M-point mixture, k=40: 61.4 / 66.4; 4M-point torus 8.6 / 9.6), and so do the mixed clouds of a batch
+// (192 clouds, k=40: 32.7 / 36.5).
+enum class Density { even, uneven, mixed };
+bool wave_by_size(int K, int64_t queries, Density d, bool learned) {
     if (K >= 48) return true;
-    if (uneven) return queries <= (K <= 8 ? 400000 : K <= 16 ? 600000 : 2000000);
-    return queries <= (K <= 16 ? 80000 : 250000);
+    if (d == Density::mixed || learned) return queries <= (K <= 16 ? 80000 : 250000);
+    if (d == Density::uneven)
+        return queries <= (K <= 8 ? 800000 : K <= 16 ? 1500000 : K <= 24 ? 3000000 : K <= 32 ? 6000000 : 8000000);
+    return K >= 32 || queries <= (K <= 8 ? 100000 : K <= 16 ? 120000 : 300000);
 }
 
 // The query search's shape. Up to QUERY_UNSORTED queries go to a wave each in their own order: the sort that makes
@@ -1231,7 +1238,7 @@ bool wave_by_size(int K, int64_t queries, bool uneven) {
 // 16,000 at k=16 0.67 / 0.18 / 0.087, 60,000 at k=1 0.45 / 0.28 / 0.16 and at k=40 1.05 / 0.45 / 0.33; 250,000 at
 // k=16 0.84 / 1.25 (a lane per query wins), at k=40 1.82 / 1.50.
 constexpr int64_t QUERY_UNSORTED = 100000;
-bool query_by_wave(int K, int64_t nq) { return nq <= QUERY_UNSORTED || wave_by_size(K, nq, false); }
+bool query_by_wave(int K, int64_t nq) { return nq <= QUERY_UNSORTED || wave_by_size(K, nq, Density::even, false); }
 
 bool uneven_cloud(const egt_ctx* h) {
     const LevelTable& L = h->lev[std::min(3, h->nlev - 1)];
@@ -1248,7 +1255,8 @@ int class_shape(const egt_ctx* h, int K, int64_t queries) {
     if (h->knn_lanes == 64) return 2;
     if (h->knn_persistent) return 1;
     if (h->knn_shape_tuned || h->knn_long_cap != KNN_LONG_CAP) return 0;
-    return wave_by_size(K, queries, uneven_cloud(h)) ? 2 : 0;
+    const Density d = h->nclouds > 1 ? Density::mixed : uneven_cloud(h) ? Density::uneven : Density::even;
+    return wave_by_size(K, queries, d, h->learned != 0) ? 2 : 0;
 }
 
 // One neighbour-count class: the search in the given launch shape, then the queries it handed back (fewer

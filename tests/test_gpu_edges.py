@@ -54,8 +54,8 @@ def test_lane_shape_on_small_clouds(egt_mod, oracle_mod, k):
         g.close()
 
 
-@pytest.mark.parametrize("n,k", [(80_000, 16), (80_065, 16), (99_970, 8), (150_017, 40), (250_000, 33), (250_049, 40),
-                                 (299_995, 48)])
+@pytest.mark.parametrize("n,k", [(99_970, 8), (100_033, 8), (120_000, 16), (120_065, 16), (299_995, 24), (300_033, 24),
+                                 (150_017, 40), (299_995, 48)])
 def test_self_search_at_shape_limits(egt_mod, oracle_mod, n, k):
     """Sizes at the limits of the launch-shape rule and of the queries a wave serves (1, 2, 4)."""
     E, O = egt_mod, oracle_mod
