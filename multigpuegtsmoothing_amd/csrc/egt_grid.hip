@@ -13,12 +13,20 @@ namespace egt {
 namespace {
 
 constexpr int BLK = 256;
+constexpr int MM_WORDS = 7;  // six extremes and the count of non-finite points
+// Cells, over all levels, up to which the level tables are sized by their bound (every point a cell of its own, or
+// every cell of the level's grid): 2 million points at the default grid, 0.5 GB of tables. Saves the trip to the host,
+// and coarse levels, whose bound is far above their count on a surface, get short probe chains. Whole build / search,
+// k=16, by count -> by bound, us: sphere 1,500 points 187 / 49 -> 165 / 49, 100,000 379 / 211 -> 357 / 208, 700,000
+// 873 / 805 -> 859 / 771, 1.9M 1678 / 2068 -> 1806 / 2023; mixture 700,000 799 / 2153 -> 797 / 1904, 1.9M 1500 / 4457
+// -> 1524 / 4085. Beyond, emptying and caching the larger tables costs more than it gives.
+constexpr size_t TABLE_BOUND = (size_t)1 << 23;
 
 // Per-block min/max of x, y, z (thrust reduce with minimum/maximum, GridKNNCuda.cu:1042-1059) plus a
 // count of non-finite inputs.
 __global__ void __launch_bounds__(BLK) k_minmax_partial(const float* __restrict__ x, const float* __restrict__ y,
                                                          const float* __restrict__ z, int64_t n,
-                                                         float* __restrict__ part, uint32_t* __restrict__ bad) {
+                                                         float* __restrict__ part) {
     float v[6] = {1e8f, -1e8f, 1e8f, -1e8f, 1e8f, -1e8f};
     uint32_t nb = 0;
     for (int64_t i = (int64_t)blockIdx.x * BLK + threadIdx.x; i < n; i += (int64_t)gridDim.x * BLK) {
@@ -53,29 +61,84 @@ __global__ void __launch_bounds__(BLK) k_minmax_partial(const float* __restrict_
             }
         uint32_t t = 0;
         for (int w = 0; w < BLK / 64; ++w) t += sb[w];
-        for (int c = 0; c < 6; ++c) part[blockIdx.x * 6 + c] = s[0][c];
-        if (t) atomicAdd(bad, t);
+        for (int c = 0; c < 6; ++c) part[blockIdx.x * MM_WORDS + c] = s[0][c];
+        part[blockIdx.x * MM_WORDS + 6] = __uint_as_float(t);
+    }
+}
+
+// Bounding cube of one cloud from the per-axis min/max, GridKNNCuda.cu:1042-1077.
+__device__ inline void cube_from_minmax(const float (&v)[6], float& mn, float& mx) {
+    const float minx = v[0] - 1e-6f, maxx = v[1] + 1e-6f, miny = v[2] - 1e-6f, maxy = v[3] + 1e-6f;
+    const float minz = v[4] - 1e-6f, maxz = v[5] + 1e-6f;
+    mn = fminf(fminf(minx, miny), minz);
+    mx = fmaxf(fmaxf(maxx, maxy), maxz);
+}
+
+// The cube goes to the cloud's table entry, where the next kernels read it, and to the report, which the host
+// reads once at the end of the build.
+__device__ inline void write_cloud(CloudDev* __restrict__ cloud, uint32_t* __restrict__ cube, int64_t base, int64_t n,
+                                   const float (&v)[6]) {
+    float mn, mx;
+    cube_from_minmax(v, mn, mx);
+    CloudDev c{};
+    c.base = base;
+    c.n = n;
+    c.min_extent = mn;
+    c.extent = mx - mn;
+    c.max_extent = mx;
+    *cloud = c;
+    cube[0] = __float_as_uint(mn);
+    cube[1] = __float_as_uint(mx);
+}
+
+// One cloud: the blocks' partials to its entry and the count of non-finite points.
+__global__ void __launch_bounds__(64) k_cloud_cube(const float* __restrict__ part, int nb, int64_t n,
+                                                    CloudDev* __restrict__ cloud, uint32_t* __restrict__ bad,
+                                                    uint32_t* __restrict__ cube) {
+    float v[6] = {1e8f, -1e8f, 1e8f, -1e8f, 1e8f, -1e8f};
+    uint32_t t = 0;
+    for (int b = (int)threadIdx.x; b < nb; b += 64) {
+        const float* p = part + (size_t)b * MM_WORDS;
+#pragma unroll
+        for (int c = 0; c < 6; c += 2) {
+            v[c] = fminf(v[c], p[c]);
+            v[c + 1] = fmaxf(v[c + 1], p[c + 1]);
+        }
+        t += __float_as_uint(p[6]);
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+#pragma unroll
+        for (int c = 0; c < 6; c += 2) {
+            v[c] = fminf(v[c], __shfl_xor(v[c], d, 64));
+            v[c + 1] = fmaxf(v[c + 1], __shfl_xor(v[c + 1], d, 64));
+        }
+        t += __shfl_xor(t, d, 64);
+    }
+    if (threadIdx.x == 0) {
+        write_cloud(cloud, cube, 0, n, v);
+        *bad = t;
     }
 }
 
 // normalize_points GridKNNCuda.cu:840-849 fused with get_buckets_no_binary :74-88. With icloud (batch) each
 // point uses its own cloud's cube. The normalized point and its key go out as one 16-byte record in input
 // order (the gather into sorted order then reads one record per point), the key and index also as the sort's
-// key and value arrays.
+// key and value arrays. Where a point is not finite the build goes on with every point at one place, and the host,
+// which reads the count at its end, throws: no value reaches a cell index or a table.
 __global__ void __launch_bounds__(BLK) k_normalize_key(const float* __restrict__ x, const float* __restrict__ y,
-                                                        const float* __restrict__ z, int64_t n, float mn, float d,
+                                                        const float* __restrict__ z, int64_t n,
                                                         const int32_t* __restrict__ icloud,
-                                                        const CloudDev* __restrict__ clouds, float a, float ba, int B,
+                                                        const CloudDev* __restrict__ clouds,
+                                                        const uint32_t* __restrict__ bad, float a, float ba, int B,
                                                         int log2B, float4* __restrict__ tp, uint32_t* __restrict__ key,
                                                         uint32_t* __restrict__ idx) {
     const int64_t i = (int64_t)blockIdx.x * BLK + threadIdx.x;
     if (i >= n) return;
-    if (icloud) {
-        const CloudDev& c = clouds[icloud[i]];
-        mn = c.min_extent;
-        d = c.extent;
-    }
-    const float xn = (x[i] - mn) / d, yn = (y[i] - mn) / d, zn = (z[i] - mn) / d;
+    const CloudDev& c = clouds[icloud ? icloud[i] : 0];
+    const float mn = c.min_extent, d = c.extent;
+    float xn = (x[i] - mn) / d, yn = (y[i] - mn) / d, zn = (z[i] - mn) / d;
+    if (*bad) xn = yn = zn = 0.5f;
     const uint32_t cx = (uint32_t)cell_of(xn, a, ba, B), cy = (uint32_t)cell_of(yn, a, ba, B),
                    cz = (uint32_t)cell_of(zn, a, ba, B);
     const uint32_t k = cx | (cy << log2B) | (cz << (2 * log2B));
@@ -172,9 +235,25 @@ __global__ void __launch_bounds__(BLK) k_cloud_minmax(const float* __restrict__ 
     }
 }
 
-__global__ void __launch_bounds__(BLK) k_minmax_init(int* __restrict__ mm, int nclouds) {
+__global__ void __launch_bounds__(BLK) k_minmax_init(int* __restrict__ mm, int nclouds, uint32_t* __restrict__ bad) {
     const int i = blockIdx.x * BLK + threadIdx.x;
     if (i < nclouds * 6) mm[i] = f2o((i & 1) ? -1e8f : 1e8f);
+    if (i == 0) *bad = 0;
+}
+
+// A batch: the entry of every cloud.
+__global__ void __launch_bounds__(BLK) k_cloud_cubes(const int* __restrict__ mm, const int64_t* __restrict__ off,
+                                                      int nclouds, CloudDev* __restrict__ clouds,
+                                                      uint32_t* __restrict__ cubes) {
+    const int c = blockIdx.x * BLK + threadIdx.x;
+    if (c >= nclouds) return;
+    float v[6];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+        const int iv = mm[c * 6 + j];
+        v[j] = __int_as_float(iv >= 0 ? iv : iv ^ 0x7FFFFFFF);
+    }
+    write_cloud(clouds + c, cubes + 2 * c, off[c], off[c + 1] - off[c], v);
 }
 
 // Cloud of each element of an index list (second, stable sort pass by cloud).
@@ -398,15 +477,16 @@ __global__ void __launch_bounds__(64) k_cells_at_bases(const uint32_t* __restric
         if (l < nl && lane == 0) out[(int64_t)l * (nclouds + 2) + 1 + c] = pre[(int64_t)l * nb + t0 / LV_TILE] + v[l];
 }
 
-// Inserts the cells of every level (thread i: cell i - first[l] of the level l whose range holds i), one CAS
-// per cell into a random slot. The level's largest cell is kept by one atomic per wave, and only by a wave that
+// Inserts the cells of every level (thread i: cell i - first[l] of the level l whose range holds i; ranges may be
+// longer than the level's cell count count[l * stride]), one CAS per cell into a random slot. The level's largest cell is kept by one atomic per wave, and only by a wave that
 // exceeds the value read first: with one unconditional atomic per wave, every wave of a level queued at one
 // address (1M points: 411 us for the 11 levels, 158 us now; 4M points: 905 -> 347).
 struct LevelInsert {
-    int64_t first[EGT_MAX_LEVELS + 1];  // first thread of each level; first[nl] = all cells
+    int64_t first[EGT_MAX_LEVELS + 1];  // first thread of each level; first[nl] = all
     uint64_t soff[EGT_MAX_LEVELS];      // the level's cell starts
     uint64_t offset[EGT_MAX_LEVELS];    // the level's table
     uint32_t log2cap[EGT_MAX_LEVELS];
+    uint64_t slots;                     // of all tables
     int nl;
 };
 __device__ inline void max_if_larger(int* p, int v) {
@@ -414,17 +494,18 @@ __device__ inline void max_if_larger(int* p, int v) {
 }
 __global__ void __launch_bounds__(BLK) k_level_insert(LevelInsert P, const uint32_t* __restrict__ starts, int64_t n,
                                                        const uint32_t* __restrict__ code,
-                                                       const int32_t* __restrict__ mcloud, uint4* __restrict__ tab,
-                                                       int* __restrict__ maxc) {
+                                                       const int32_t* __restrict__ mcloud,
+                                                       const uint32_t* __restrict__ count, int stride,
+                                                       uint4* __restrict__ tab, LevelDev* __restrict__ lev) {
     const int64_t i = (int64_t)blockIdx.x * BLK + threadIdx.x;
     int l = 0;
     for (int j = 1; j < P.nl; ++j) l += i >= P.first[j] ? 1 : 0;
     int cnt = 0;
-    if (i < P.first[P.nl]) {
-        const int64_t c = i - P.first[l];
+    const int64_t c = i - P.first[l], cells = count[(int64_t)l * stride];
+    if (c < cells) {
         const uint32_t* st_l = starts + P.soff[l];
         const uint32_t st = st_l[c];
-        const uint32_t en = i + 1 < P.first[l + 1] ? st_l[c + 1] : (uint32_t)n;
+        const uint32_t en = c + 1 < cells ? st_l[c + 1] : (uint32_t)n;
         const unsigned long long cc = cell_key(mcloud ? (uint32_t)mcloud[st] : 0u, code[st] >> (3 * l));
         const uint32_t log2cap = P.log2cap[l], mask = (1u << log2cap) - 1u;
         uint32_t s = hash_slot(cc, log2cap);
@@ -446,14 +527,18 @@ __global__ void __launch_bounds__(BLK) k_level_insert(LevelInsert P, const uint3
     if (__shfl(l, 63, 64) == l0) {
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) cnt = max(cnt, __shfl_xor(cnt, d, 64));
-        if (__lane_id() == 0) max_if_larger(&maxc[l0], cnt);
+        if (__lane_id() == 0) max_if_larger(&lev[l0].max_count, cnt);
     } else {
-        max_if_larger(&maxc[l], cnt);
+        max_if_larger(&lev[l].max_count, cnt);
     }
 }
 
-__global__ void __launch_bounds__(BLK) k_fill_u64(uint64_t* __restrict__ p, uint64_t n, uint64_t v) {
-    for (uint64_t i = (uint64_t)blockIdx.x * BLK + threadIdx.x; i < n; i += (uint64_t)gridDim.x * BLK) p[i] = v;
+// Empties the tables and writes their descriptors.
+__global__ void __launch_bounds__(BLK) k_level_init(LevelInsert P, uint64_t* __restrict__ tab, LevelDev* __restrict__ lev) {
+    for (uint64_t i = (uint64_t)blockIdx.x * BLK + threadIdx.x; i < 2 * P.slots; i += (uint64_t)gridDim.x * BLK)
+        tab[i] = HASH_EMPTY;
+    if (blockIdx.x == 0 && (int)threadIdx.x < P.nl)
+        lev[threadIdx.x] = LevelDev{P.offset[threadIdx.x], P.log2cap[threadIdx.x], 0};
 }
 
 // produce_output_GKNN + rearrange_output, getOutputPoints.cu:9-30, into separate output buffers.
@@ -517,19 +602,21 @@ int ceil_log2(int64_t v) {
     return l;
 }
 
-void upload_clouds(egt_ctx* h) {
-    h->dclouds.alloc(h->clouds.size());
-    HIP_CHECK(hipMemcpyAsync(h->dclouds.p, h->clouds.data(), h->clouds.size() * sizeof(CloudDev),
-                             hipMemcpyHostToDevice, h->stream));
-}
-
-// Bounding cube of one cloud from the per-axis min/max, GridKNNCuda.cu:1042-1077.
-void cube_from_minmax(const float v[6], float& mn, float& mx) {
-    const float minx = v[0] - 1e-6f, maxx = v[1] + 1e-6f, miny = v[2] - 1e-6f, maxy = v[3] + 1e-6f;
-    const float minz = v[4] - 1e-6f, maxz = v[5] + 1e-6f;
-    mn = std::min(std::min(minx, miny), minz);
-    mx = std::max(std::max(maxx, maxy), maxz);
-}
+// What a build tells the host, behind the level descriptors in one buffer, so that one copy brings it over: the count
+// of non-finite input points, the cubes of the clouds, and per level the cell count and the running counts at each
+// cloud's first position.
+struct Report {
+    int nc, nl;
+    size_t bad() const { return EGT_MAX_LEVELS * sizeof(LevelDev) / sizeof(uint32_t); }
+    size_t cubes() const { return bad() + 2; }
+    size_t counts() const { return cubes() + 2 * (size_t)nc; }
+    size_t words() const { return counts() + (size_t)nl * (nc + 2); }
+    uint32_t* dev(egt_ctx* h) const {
+        h->dlev.alloc((words() * sizeof(uint32_t) + sizeof(LevelDev) - 1) / sizeof(LevelDev));
+        return reinterpret_cast<uint32_t*>(h->dlev.p);
+    }
+};
+Report report_of(const egt_ctx* h) { return Report{h->nclouds, ilog2(h->B) + 1}; }
 
 // Normalize, key, stable sort (by cloud, then key) and gather into sorted space. icloud is null for one
 // cloud.
@@ -542,8 +629,9 @@ void sort_into_sorted_space(egt_ctx* h, const float* dx, const float* dy, const 
     float4* tp = sc.get<float4>(9, n);
     uint32_t* skey = sc.get<uint32_t>(12, n);
     uint32_t* sidx = sc.get<uint32_t>(13, n);
-    k_normalize_key<<<ceil_div(n, BLK), BLK, 0, s>>>(dx, dy, dz, n, h->min_extent, h->max_extent - h->min_extent,
-                                                      icloud, h->dclouds.p, a, ba, h->B, log2B, tp, skey, sidx);
+    const Report R = report_of(h);
+    k_normalize_key<<<ceil_div(n, BLK), BLK, 0, s>>>(dx, dy, dz, n, icloud, h->dclouds.p, R.dev(h) + R.bad(), a, ba,
+                                                      h->B, log2B, tp, skey, sidx);
     LAUNCH_CHECK();
     radix_sort_pairs(skey, sidx, n, 3 * log2B, s, sc);
     if (icloud) {
@@ -564,6 +652,30 @@ void sort_into_sorted_space(egt_ctx* h, const float* dx, const float* dy, const 
     LAUNCH_CHECK();
 }
 
+void check_finite(const egt_ctx* h, const std::vector<uint32_t>& rep) {
+    if (rep[report_of(h).bad()]) throw ArgError{EGT_ERR_INVALID_ARG, "input coordinates contain NaN or Inf"};
+}
+
+// The host's cloud table from a build's report.
+void set_clouds(egt_ctx* h, const std::vector<uint32_t>& rep, const int64_t* offsets) {
+    const uint32_t* cube = rep.data() + report_of(h).cubes();
+    h->clouds.assign(h->nclouds, CloudDev{});
+    for (int c = 0; c < h->nclouds; ++c) {
+        float mm[2];
+        std::memcpy(mm, cube + 2 * c, sizeof(mm));
+        CloudDev& cd = h->clouds[c];
+        cd.base = offsets[c];
+        cd.n = offsets[c + 1] - offsets[c];
+        cd.min_extent = mm[0];
+        cd.extent = mm[1] - mm[0];
+        cd.max_extent = mm[1];
+    }
+    h->min_extent = h->clouds[0].min_extent;
+    h->max_extent = h->clouds[0].max_extent;
+}
+
+void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t done);
+
 }  // namespace
 
 void build_grid(egt_ctx* h, const float* dx, const float* dy, const float* dz) {
@@ -574,40 +686,21 @@ void build_grid(egt_ctx* h, const float* dx, const float* dy, const float* dz) {
     HIP_CHECK(hipEventRecord(e0, s));
 
     // bounding cube
-    const int nbp = std::min<int64_t>(1024, std::max<int64_t>(1, ceil_div(n, BLK)));
-    float* dpart = sc.get<float>(8, (size_t)nbp * 6 + 1);
-    uint32_t* dbad = reinterpret_cast<uint32_t*>(dpart + (size_t)nbp * 6);
-    HIP_CHECK(hipMemsetAsync(dbad, 0, sizeof(uint32_t), s));
-    k_minmax_partial<<<nbp, BLK, 0, s>>>(dx, dy, dz, n, dpart, dbad);
-    LAUNCH_CHECK();
-    std::vector<float> hp((size_t)nbp * 6 + 1);
-    HIP_CHECK(hipMemcpyAsync(hp.data(), dpart, hp.size() * sizeof(float), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    uint32_t bad;
-    std::memcpy(&bad, &hp[(size_t)nbp * 6], 4);
-    if (bad) throw ArgError{EGT_ERR_INVALID_ARG, "input coordinates contain NaN or Inf"};
-    float v[6] = {1e8f, -1e8f, 1e8f, -1e8f, 1e8f, -1e8f};
-    for (int b = 0; b < nbp; ++b)
-        for (int c = 0; c < 6; c += 2) {
-            v[c] = std::min(v[c], hp[(size_t)b * 6 + c]);
-            v[c + 1] = std::max(v[c + 1], hp[(size_t)b * 6 + c + 1]);
-        }
-    float mn, mx;
-    cube_from_minmax(v, mn, mx);
-    h->min_extent = mn;
-    h->max_extent = mx;
     h->nclouds = 1;
-    h->clouds.assign(1, CloudDev{});
-    h->clouds[0].base = 0;
-    h->clouds[0].n = n;
-    h->clouds[0].min_extent = mn;
-    h->clouds[0].extent = mx - mn;
-    h->clouds[0].max_extent = mx;
-    upload_clouds(h);
+    h->dclouds.alloc(1);
+    const Report R = report_of(h);
+    uint32_t* rep = R.dev(h);
+    const int nbp = std::min<int64_t>(1024, std::max<int64_t>(1, ceil_div(n, BLK)));
+    float* dpart = sc.get<float>(8, (size_t)nbp * MM_WORDS);
+    k_minmax_partial<<<nbp, BLK, 0, s>>>(dx, dy, dz, n, dpart);
+    LAUNCH_CHECK();
+    k_cloud_cube<<<1, 64, 0, s>>>(dpart, nbp, n, h->dclouds.p, rep + R.bad(), rep + R.cubes());
+    LAUNCH_CHECK();
     sort_into_sorted_space(h, dx, dy, dz, nullptr);
-    build_search_structure(h);
-    HIP_CHECK(hipEventRecord(e1, s));
-    HIP_CHECK(hipEventSynchronize(e1));
+    std::vector<uint32_t> hr;
+    build_search_structure(h, hr, e1);
+    const int64_t offsets[2] = {0, n};
+    set_clouds(h, hr, offsets);
     HIP_CHECK(hipEventElapsedTime(&h->stats.grid_ms, e0, e1));
 }
 
@@ -624,45 +717,28 @@ void build_grid_batch(egt_ctx* h, const float* dx, const float* dy, const float*
     int32_t* icloud = sc.get<int32_t>(21, n);
     k_cloud_of<<<ceil_div(n, BLK), BLK, 0, s>>>(h->in_off.p, nclouds, n, icloud);
     LAUNCH_CHECK();
-    int* mm = sc.get<int>(8, (size_t)nclouds * 6 + 1);
-    uint32_t* dbad = reinterpret_cast<uint32_t*>(mm + (size_t)nclouds * 6);
-    k_minmax_init<<<ceil_div(nclouds * 6, BLK), BLK, 0, s>>>(mm, nclouds);
+    h->dclouds.alloc(nclouds);
+    const Report R = report_of(h);
+    uint32_t* rep = R.dev(h);
+    int* mm = sc.get<int>(8, (size_t)nclouds * 6);
+    k_minmax_init<<<ceil_div(nclouds * 6, BLK), BLK, 0, s>>>(mm, nclouds, rep + R.bad());
     LAUNCH_CHECK();
-    HIP_CHECK(hipMemsetAsync(dbad, 0, sizeof(uint32_t), s));
-    k_cloud_minmax<<<std::max(1, ceil_div(n, (int64_t)BLK * MM_PER)), BLK, 0, s>>>(dx, dy, dz, icloud, n, mm, dbad);
+    k_cloud_minmax<<<std::max(1, ceil_div(n, (int64_t)BLK * MM_PER)), BLK, 0, s>>>(dx, dy, dz, icloud, n, mm,
+                                                                                    rep + R.bad());
     LAUNCH_CHECK();
-    std::vector<int> hm((size_t)nclouds * 6 + 1);
-    HIP_CHECK(hipMemcpyAsync(hm.data(), mm, hm.size() * sizeof(int), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    if (hm[(size_t)nclouds * 6]) throw ArgError{EGT_ERR_INVALID_ARG, "input coordinates contain NaN or Inf"};
-    h->clouds.assign(nclouds, CloudDev{});
-    for (int c = 0; c < nclouds; ++c) {
-        float v[6];
-        for (int j = 0; j < 6; ++j) {
-            int iv = hm[(size_t)c * 6 + j];
-            iv = iv >= 0 ? iv : iv ^ 0x7FFFFFFF;
-            std::memcpy(&v[j], &iv, 4);
-        }
-        float mn, mx;
-        cube_from_minmax(v, mn, mx);
-        CloudDev& cd = h->clouds[c];
-        cd.base = offsets[c];
-        cd.n = offsets[c + 1] - offsets[c];
-        cd.min_extent = mn;
-        cd.extent = mx - mn;
-        cd.max_extent = mx;
-    }
-    h->min_extent = h->clouds[0].min_extent;
-    h->max_extent = h->clouds[0].max_extent;
-    upload_clouds(h);
+    k_cloud_cubes<<<ceil_div(nclouds, BLK), BLK, 0, s>>>(mm, h->in_off.p, nclouds, h->dclouds.p, rep + R.cubes());
+    LAUNCH_CHECK();
     sort_into_sorted_space(h, dx, dy, dz, icloud);
-    build_search_structure(h);
-    HIP_CHECK(hipEventRecord(e1, s));
-    HIP_CHECK(hipEventSynchronize(e1));
+    std::vector<uint32_t> hr;
+    build_search_structure(h, hr, e1);
+    set_clouds(h, hr, offsets);
     HIP_CHECK(hipEventElapsedTime(&h->stats.grid_ms, e0, e1));
 }
 
-void build_search_structure(egt_ctx* h) {
+namespace {
+// The Morton order and the level tables of the sorted points; rep: the report, done: recorded when the work is queued
+// (if not null). Synchronizes the stream.
+void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t done) {
     const int64_t n = h->n;
     hipStream_t s = h->stream;
     Scratch& sc = h->scratch;
@@ -708,9 +784,9 @@ void build_search_structure(egt_ctx* h) {
     LAUNCH_CHECK();
     const int32_t* mcl = batch ? h->mcloud.p : nullptr;
 
-    // level tables: every level's cells are counted, ranked and (below) inserted together; one read-back of the
-    // counts of the levels (and, in a batch, of the running counts at each cloud's first position) sizes the tables
-    h->nlev = log2B + 1;
+    // level tables: every level's cells are counted, ranked and (below) inserted together
+    const Report R = report_of(h);
+    h->nlev = R.nl;
     const int nc = h->nclouds, nl = h->nlev;
     // room for the starts of every level: at most min(n, cells of the level's grid over all clouds) each
     std::vector<size_t> soff(nl + 1, 0);
@@ -723,7 +799,8 @@ void build_search_structure(egt_ctx* h) {
     uint32_t* starts = sc.get<uint32_t>(38, soff[nl]);
     const int nb = ceil_div(n, LV_TILE);
     uint32_t* tiles = sc.get<uint32_t>(9, (size_t)nl * nb);
-    uint32_t* dtot = sc.get<uint32_t>(23, (size_t)nl * (nc + 2));  // per level: total, then the cloud bases
+    uint32_t* drep = R.dev(h);
+    uint32_t* dtot = drep + R.counts();  // per level: total, then the cloud bases
     k_level_count<<<nb, BLK, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles);
     LAUNCH_CHECK();
     k_level_scan<<<nl, LVS_BLK, 0, s>>>(tiles, nb, dtot, nc + 2);
@@ -734,57 +811,53 @@ void build_search_structure(egt_ctx* h) {
         k_cells_at_bases<<<nc + 1, 64, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles, h->dclouds.p, nc, dtot);
         LAUNCH_CHECK();
     }
-    std::vector<uint32_t> ht((size_t)nl * (nc + 2));
-    HIP_CHECK(hipMemcpyAsync(ht.data(), dtot, ht.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    h->cloud_cells.assign((size_t)nc * nl, 0);
-    std::vector<uint32_t> cells(nl);
-    uint64_t total = 0;
-    LevelDev lv[EGT_MAX_LEVELS];
-    for (int l = 0; l < nl; ++l) {
-        const uint32_t* tl = &ht[(size_t)l * (nc + 2)];
-        cells[l] = tl[0];
-        if (batch) {
-            for (int c = 0; c < nc; ++c) h->cloud_cells[(size_t)c * nl + l] = tl[1 + c + 1] - tl[1 + c];
-        } else {
-            h->cloud_cells[l] = cells[l];
-        }
-        uint32_t log2cap = 6;
-        while ((1ull << log2cap) < 2ull * cells[l]) ++log2cap;
-        h->lev[l].log2cap = log2cap;
-        h->lev[l].offset = total;
-        h->lev[l].cells = cells[l];
-        lv[l] = LevelDev{total, log2cap, 0};
-        total += 1ull << log2cap;
-    }
-    h->htab.alloc(total);
-    k_fill_u64<<<1024, BLK, 0, s>>>(reinterpret_cast<uint64_t*>(h->htab.p), 2 * total, HASH_EMPTY);
-    LAUNCH_CHECK();
-    DBuf<uint32_t>& dmax = sc.bufs[14];
-    dmax.alloc(nl);
-    HIP_CHECK(hipMemsetAsync(dmax.p, 0, nl * sizeof(uint32_t), s));
+    // The tables are sized by the levels' cell counts, which takes one trip to the host, or, up to TABLE_BOUND cells,
+    // by the bounds above, which takes none.
+    rep.resize(R.words());
+    auto read_back = [&](size_t words) {
+        HIP_CHECK(hipMemcpyAsync(rep.data(), drep, words * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        HIP_CHECK(hipStreamSynchronize(s));
+        check_finite(h, rep);
+    };
+    const bool by_bound = soff[nl] <= TABLE_BOUND;
+    if (!by_bound) read_back(R.words());
     LevelInsert li{};
     li.nl = nl;
     for (int l = 0; l < nl; ++l) {
-        li.first[l + 1] = li.first[l] + cells[l];
+        const uint64_t cells = by_bound ? soff[l + 1] - soff[l] : rep[R.counts() + (size_t)l * (nc + 2)];
+        // Twice the cells at least, and eight times on the coarse levels, whose tables are small beside the fine ones:
+        // a wave's search waits for its longest probe chain. Search, us, twice everywhere -> eight times on coarse
+        // levels: torus 1M k=16 1122 -> 1047, 16M k=40 32300 -> 31890; mixture 4M k=40 12976 -> 12776, 16M 57136 ->
+        // 55434; builds unchanged (eight times on all levels: the same searches, builds 3-10% slower).
+        const uint64_t room = by_bound || 4 * cells > (uint64_t)n ? 2 : 8;
+        uint32_t log2cap = 6;
+        while ((1ull << log2cap) < room * cells) ++log2cap;
+        h->lev[l].log2cap = li.log2cap[l] = log2cap;
+        h->lev[l].offset = li.offset[l] = li.slots;
+        li.first[l + 1] = li.first[l] + (int64_t)cells;
         li.soff[l] = soff[l];
-        li.offset[l] = h->lev[l].offset;
-        li.log2cap[l] = h->lev[l].log2cap;
+        li.slots += 1ull << log2cap;
     }
-    k_level_insert<<<ceil_div(li.first[nl], BLK), BLK, 0, s>>>(li, starts, n, h->mcode.p, mcl, h->htab.p,
-                                                               reinterpret_cast<int*>(dmax.p));
+    h->htab.alloc(li.slots);
+    k_level_init<<<(int)std::min<uint64_t>(1024, (2 * li.slots + BLK - 1) / BLK), BLK, 0, s>>>(
+        li, reinterpret_cast<uint64_t*>(h->htab.p), h->dlev.p);
     LAUNCH_CHECK();
-    std::vector<int32_t> mx(nl);
-    HIP_CHECK(hipMemcpyAsync(mx.data(), dmax.p, nl * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    k_level_insert<<<ceil_div(li.first[nl], BLK), BLK, 0, s>>>(li, starts, n, h->mcode.p, mcl, dtot, nc + 2, h->htab.p,
+                                                               h->dlev.p);
+    LAUNCH_CHECK();
+    if (done) HIP_CHECK(hipEventRecord(done, s));
+    read_back(by_bound ? R.words() : R.bad() + 1);
+    h->cloud_cells.assign((size_t)nc * nl, 0);
     for (int l = 0; l < nl; ++l) {
-        h->lev[l].max_count = mx[l];
-        lv[l].max_count = mx[l];
+        const uint32_t* tl = &rep[R.counts() + (size_t)l * (nc + 2)];
+        for (int c = 0; c < nc; ++c) h->cloud_cells[(size_t)c * nl + l] = batch ? tl[1 + c + 1] - tl[1 + c] : tl[0];
+        LevelDev d;
+        std::memcpy(&d, &rep[l * (sizeof(LevelDev) / sizeof(uint32_t))], sizeof(d));
+        h->lev[l].cells = tl[0];
+        h->lev[l].max_count = d.max_count;
     }
-    h->dlev.alloc(EGT_MAX_LEVELS);
-    HIP_CHECK(hipMemcpyAsync(h->dlev.p, lv, nl * sizeof(LevelDev), hipMemcpyHostToDevice, s));
-    HIP_CHECK(hipStreamSynchronize(s));
 }
+}  // namespace
 
 namespace {
 __global__ void __launch_bounds__(BLK) k_rekey(const float* __restrict__ x, const float* __restrict__ y,
@@ -805,7 +878,8 @@ void refresh_search_structure(egt_ctx* h) {
     k_rekey<<<ceil_div(h->n, BLK), BLK, 0, h->stream>>>(h->x.p, h->y.p, h->z.p, h->n, a, ba, h->B, ilog2(h->B),
                                                         h->key.p);
     LAUNCH_CHECK();
-    build_search_structure(h);
+    std::vector<uint32_t> rep;
+    build_search_structure(h, rep, nullptr);
     h->search_stale = false;
 }
 

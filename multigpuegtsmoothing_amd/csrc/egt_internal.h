@@ -190,7 +190,7 @@ struct egt_ctx {
     egt::DBuf<uint4> htab;       // all level tables: (key = cell_key(cloud, level code), start, count) per slot
     egt::LevelTable lev[EGT_MAX_LEVELS];
     int nlev = 0;
-    egt::DBuf<egt::LevelDev> dlev;  // device copy of the level descriptors
+    egt::DBuf<egt::LevelDev> dlev;  // the level descriptors, then the build's report (egt_grid.hip)
     std::vector<int64_t> cloud_cells;  // non-empty cells per cloud and level [cloud * nlev + level]
 
     // clouds (a batch handle holds several independent clouds; a plain handle holds one)
@@ -287,7 +287,6 @@ uint32_t morton3(uint32_t x, uint32_t y, uint32_t z);
 void build_grid(egt_ctx* h, const float* dx, const float* dy, const float* dz);
 void build_grid_batch(egt_ctx* h, const float* dx, const float* dy, const float* dz, const int64_t* offsets,
                       int nclouds);
-void build_search_structure(egt_ctx* h);
 void refresh_search_structure(egt_ctx* h);
 
 // kNN (egt_knn.hip)

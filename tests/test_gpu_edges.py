@@ -183,3 +183,23 @@ def test_normals_at_forest_forms(egt_mod, oracle_mod, n, k):
     assert st["msf_edges"] == ref["orient_stats"][1] and st["msf_trees"] == ref["orient_stats"][2]
     for u, v in zip(got, ref["normals"]):
         np.testing.assert_array_equal(u, v)
+
+
+@pytest.mark.parametrize("n", [2_022_253, 2_022_254])
+def test_level_tables_by_bound_and_by_count(egt_mod, oracle_mod, n):
+    """The largest cloud whose level tables are sized by their bound and the smallest sized by the cell counts; a point
+    that is not finite is refused in both."""
+    E, O = egt_mod, oracle_mod
+    print("n", n, flush=True)
+    pts = D.mixture(n, seed=37)
+    g = E.GridStructure(pts, 1, 1e-6, 1024, 4)
+    g.GRIDCUDAKNNSELF_COMPACT(3, 1e8)
+    og = O.Grid(*pts)
+    np.testing.assert_array_equal(g.GetKNNIndexes(), og.to_original(og.knn(3)[0]))
+    g.close()
+    bad = tuple(c.copy() for c in pts)
+    bad[1][n - 1] = np.inf
+    with pytest.raises(E.EGTError, match="NaN or Inf"):
+        E.GridStructure(bad, 1, 1e-6, 1024, 4)
+    with pytest.raises(E.EGTError, match="NaN or Inf"):
+        E.BatchGrid([tuple(c[:500] for c in pts), tuple(c[-500:] for c in bad)])
