@@ -236,7 +236,8 @@ egt_status egt_set_option(egt_handle h, egt_option opt, int64_t value);
 
 /* Device memory cache (no reference counterpart; the reference allocates and frees per call). Memory a
  * destroyed handle held stays cached per device for later handles, up to EGT_DEVICE_CACHE_MB (environment,
- * default 32768) per device. This call returns every cached block to the driver; *released (optional)
+ * default 32768) per device, and so do up to 16 idle streams with 256 KB of pinned host memory each. This call
+ * returns every cached block, and these, to the driver; *released (optional)
  * receives the bytes returned. *cached (optional) receives the bytes cached before the call. */
 egt_status egt_release_cached_memory(uint64_t* released, uint64_t* cached);
 

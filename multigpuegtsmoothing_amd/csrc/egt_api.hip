@@ -47,7 +47,8 @@ egt_status make_handle(const float* x, const float* y, const float* z, int64_t n
     if (!h) return fail(EGT_ERR_OOM, "host allocation failed");
     egt_status st = guarded([&] {
         HIP_CHECK(hipGetDevice(&h->device));
-        HIP_CHECK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
+        h->lane = egt::lane_acquire();
+        h->stream = h->lane.stream;
         h->kind = kind;
         h->n = n;
         h->B = bucket_count;
@@ -65,8 +66,7 @@ egt_status make_handle(const float* x, const float* y, const float* z, int64_t n
         }
     });
     if (st != EGT_OK) {
-        if (h->stream) (void)hipStreamDestroy(h->stream);
-        delete h;
+        egt_destroy(h);
         return st;
     }
     *out = h;
@@ -439,7 +439,8 @@ egt_status batch_create(const float* x, const float* y, const float* z, const in
     if (!h) return fail(EGT_ERR_OOM, "host allocation failed");
     egt_status st = guarded([&] {
         HIP_CHECK(hipGetDevice(&h->device));
-        HIP_CHECK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
+        h->lane = egt::lane_acquire();
+        h->stream = h->lane.stream;
         h->kind = 2;
         h->n = n;
         h->B = bucket_count;
@@ -458,8 +459,7 @@ egt_status batch_create(const float* x, const float* y, const float* z, const in
         }
     });
     if (st != EGT_OK) {
-        if (h->stream) (void)hipStreamDestroy(h->stream);
-        delete h;
+        egt_destroy(h);
         return st;
     }
     *out = h;
@@ -576,11 +576,10 @@ egt_status egt_batch_cloud_info(egt_handle h, int32_t cloud, int64_t* n, int32_t
 
 egt_status egt_destroy(egt_handle h) {
     if (!h) return EGT_OK;
-    if (h->stream) {
-        (void)hipStreamSynchronize(h->stream);
-        (void)hipStreamDestroy(h->stream);
-    }
+    if (h->stream) (void)hipStreamSynchronize(h->stream);
+    const egt::Lane lane = h->lane;
     delete h;
+    egt::lane_release(lane);
     return EGT_OK;
 }
 

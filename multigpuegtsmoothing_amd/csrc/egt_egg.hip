@@ -299,12 +299,12 @@ void finish_csr(egt_ctx* h, const int32_t* mrow, const uint64_t* keepm, const ui
     // is the exact kept count needed (a 64-bit sum; a 512-cloud batch of 54.7M points at mean k 40 holds
     // 2.19G slots, of which the EGG filter keeps far fewer).
     if (row_elems(h) > CSR_MAX_ENTRIES) {
-        if (const char* err = csr_total_error(sum_u32(kept, n, h->stream, h->scratch)))
+        if (const char* err = csr_total_error(sum_u32(h, kept, n)))
             throw ArgError{EGT_ERR_UNSUPPORTED, err};
     }
     uint32_t* off = h->scratch.get<uint32_t>(10, n);
     uint32_t total = 0;
-    exclusive_scan_u32(kept, off, n, h->stream, h->scratch, &total);
+    exclusive_scan_u32(h, kept, off, n, &total);
     h->rowptr.alloc(n + 1);
     h->col.alloc(std::max<uint32_t>(total, 1));
     k_csr_fill<<<ceil_div(n, 4 * CSR_ROWS), 256, 0, h->stream>>>(mrow, keepm, n, h->dclouds.p,

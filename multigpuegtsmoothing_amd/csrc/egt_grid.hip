@@ -815,8 +815,7 @@ void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t d
     // by the bounds above, which takes none.
     rep.resize(R.words());
     auto read_back = [&](size_t words) {
-        HIP_CHECK(hipMemcpyAsync(rep.data(), drep, words * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        HIP_CHECK(hipStreamSynchronize(s));
+        fetch(h->lane, {{rep.data(), drep, words * sizeof(uint32_t)}});
         check_finite(h, rep);
     };
     const bool by_bound = soff[nl] <= TABLE_BOUND;
@@ -891,10 +890,8 @@ void run_output(egt_ctx* h, float* x, float* y, float* z) {
                                               h->nclouds > 1 ? h->scloud.p : nullptr, h->dclouds.p, n,
                                               h->min_extent, h->max_extent - h->min_extent, ox, ox + n, ox + 2 * n);
     LAUNCH_CHECK();
-    HIP_CHECK(hipMemcpyAsync(x, ox, n * sizeof(float), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(y, ox + n, n * sizeof(float), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(z, ox + 2 * n, n * sizeof(float), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    const size_t bytes = n * sizeof(float);
+    fetch(h->lane, {{x, ox, bytes}, {y, ox + n, bytes}, {z, ox + 2 * n, bytes}});
 }
 
 void run_knn_original(egt_ctx* h, int32_t* out) {
@@ -903,8 +900,7 @@ void run_knn_original(egt_ctx* h, int32_t* out) {
     int32_t* tmp = h->scratch.get<int32_t>(9, n * k);
     k_knn_original<<<ceil_div(n * k, BLK), BLK, 0, s>>>(h->knn.p, h->perm.p, n, (int)k, tmp);
     LAUNCH_CHECK();
-    HIP_CHECK(hipMemcpyAsync(out, tmp, n * k * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    fetch(h->lane, {{out, tmp, n * k * sizeof(int32_t)}});
 }
 
 void run_knn_original_cloud(egt_ctx* h, int cloud, int32_t* out) {
@@ -914,8 +910,7 @@ void run_knn_original_cloud(egt_ctx* h, int cloud, int32_t* out) {
     int32_t* tmp = h->scratch.get<int32_t>(9, std::max<int64_t>(cnt, 1));
     k_knn_original_cloud<<<std::max(1, ceil_div(cnt, BLK)), BLK, 0, s>>>(h->knn.p, h->perm.p, c, c.base, tmp);
     LAUNCH_CHECK();
-    HIP_CHECK(hipMemcpyAsync(out, tmp, cnt * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    fetch(h->lane, {{out, tmp, cnt * sizeof(int32_t)}});
 }
 
 uint32_t morton3(uint32_t x, uint32_t y, uint32_t z) { return morton_code(x, y, z); }

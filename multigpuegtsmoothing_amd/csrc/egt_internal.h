@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <initializer_list>
 #include <string>
 #include <vector>
 #include "../../include/egt.h"
@@ -90,6 +91,25 @@ void device_release(void* p, size_t capacity);
 size_t device_cache_release_all();
 size_t device_cache_bytes();
 
+// A handle's stream and a pinned block for its small read-backs, taken from the idle ones of the current device or
+// made, and given back when the handle ends (no work in flight).
+struct Lane {
+    hipStream_t stream = nullptr;
+    void* pinned = nullptr;  // PINNED_BYTES, or null
+    int device = 0;
+};
+constexpr size_t PINNED_BYTES = (size_t)256 << 10;
+Lane lane_acquire();
+void lane_release(const Lane& l);
+
+// Device memory to the host, through the pinned block what fits there; synchronizes the stream.
+struct HostCopy {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+void fetch(const Lane& l, std::initializer_list<HostCopy> copies);
+
 // Device allocation owned by a handle.
 template <typename T>
 struct DBuf {
@@ -164,7 +184,8 @@ struct Scratch {
 
 struct egt_ctx {
     int kind = 0;  // 0 cloud, 1 mesh
-    hipStream_t stream = nullptr;
+    egt::Lane lane;
+    hipStream_t stream = nullptr;  // the lane's
     int device = 0;
     int64_t n = 0;
     int k = 0;
@@ -268,8 +289,7 @@ struct egt_model_s {
 
 namespace egt {
 // scan / sort / reduce utilities (egt_prims.hip)
-void exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t n, hipStream_t s, Scratch& sc,
-                        uint32_t* total_host);
+void exclusive_scan_u32(egt_ctx* h, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total_host);
 // Same, with the total written to device memory and no synchronization.
 void exclusive_scan_u32_dev(const uint32_t* in, uint32_t* out, int64_t n, hipStream_t s, Scratch& sc,
                             uint32_t* total_dev);
@@ -280,7 +300,7 @@ void radix_sort_pairs(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, h
 size_t radix_sort_workspace_words(int64_t n);
 void radix_sort_pairs_ws(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, uint32_t* ws);
 // Sum of n uint32 values in 64 bits (synchronizes the stream).
-uint64_t sum_u32(const uint32_t* in, int64_t n, hipStream_t s, Scratch& sc);
+uint64_t sum_u32(egt_ctx* h, const uint32_t* in, int64_t n);
 uint32_t morton3(uint32_t x, uint32_t y, uint32_t z);
 
 // grid (egt_grid.hip)

@@ -1283,8 +1283,7 @@ int64_t search_class(egt_ctx* h, KnnParams P, int K, hipStream_t s, int shape) {
     }
     if (!hand_back) return 0;
     uint64_t nb = 0;
-    HIP_CHECK(hipMemcpyAsync(&nb, P.counters + 6, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    fetch(h->lane, {{&nb, P.counters + 6, sizeof(nb)}});
     if (nb == 0) return 0;
     if ((int64_t)nb > P.retry_cap) throw std::runtime_error("kNN hand-back list longer than its buffer");
     int bits = 1;
@@ -1388,11 +1387,10 @@ KnnParams knn_params(egt_ctx* h, int k, bool scratch = true) {
 void clear_stats(const KnnParams& P, hipStream_t s) {
     HIP_CHECK(hipMemsetAsync(P.counters, 0, (size_t)STAT_WORDS * (STAT_SLOTS + 1) * sizeof(uint64_t), s));
 }
-void read_stats(const KnnParams& P, uint64_t (&hc)[10], hipStream_t s) {
-    k_stats_sum<<<1, STAT_SLOTS, 0, s>>>(P.counters + STAT_WORDS, P.counters);
+void read_stats(const egt_ctx* h, const KnnParams& P, uint64_t (&hc)[10]) {
+    k_stats_sum<<<1, STAT_SLOTS, 0, h->stream>>>(P.counters + STAT_WORDS, P.counters);
     LAUNCH_CHECK();
-    HIP_CHECK(hipMemcpyAsync(hc, P.counters, sizeof(hc), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    fetch(h->lane, {{hc, P.counters, sizeof(hc)}});
 }
 
 // Work lists per neighbour-count class: chunks of 64 Morton-consecutive queries that never straddle two
@@ -1464,7 +1462,7 @@ void run_knn_clouds(egt_ctx* h) {
     }
     HIP_CHECK(hipEventRecord(e1, s));
     uint64_t hc[10];
-    read_stats(P, hc, s);
+    read_stats(h, P, hc);
     HIP_CHECK(hipEventElapsedTime(&h->stats.knn_ms, e0, e1));
     h->stats.learned_bound_retries = handed_back - (int64_t)hc[9];
     h->stats.knn_insertions = (int64_t)hc[7];
@@ -1546,7 +1544,7 @@ void run_knn_query(egt_ctx* h, const float* dqx, const float* dqy, const float* 
     }
     HIP_CHECK(hipEventRecord(e1, s));
     uint64_t hc[10];
-    read_stats(P, hc, s);
+    read_stats(h, P, hc);
     HIP_CHECK(hipEventElapsedTime(&h->stats.query_ms, e0, e1));
     h->stats.query_count = nq;
     h->stats.query_k = k;
@@ -1562,8 +1560,7 @@ void run_knn_query_original(egt_ctx* h, int32_t* out) {
     int32_t* tmp = h->scratch.get<int32_t>(9, cnt);
     k_query_original<<<ceil_div(cnt, KBLK), KBLK, 0, s>>>(h->qknn.p, h->perm.p, cnt, tmp);
     LAUNCH_CHECK();
-    HIP_CHECK(hipMemcpyAsync(out, tmp, cnt * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    fetch(h->lane, {{out, tmp, cnt * sizeof(int32_t)}});
 }
 
 }  // namespace egt
@@ -1838,7 +1835,7 @@ int autotune_start_level(egt_ctx* h, int k, float thres_n, float* trial_ms, floa
         launch_any(P, K, s);
         HIP_CHECK(hipEventRecord(e1, s));
         uint64_t hc[10];
-        read_stats(P, hc, s);
+        read_stats(h, P, hc);
         float ms = 0.0f;
         HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
         const double q = (double)std::min<int64_t>(h->n, P.nchunks * 64);

@@ -691,7 +691,7 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
     k_edges<0><<<gn, blk, 0, s>>>(h->rowptr.p, h->col.p, h->morder.p, n, cnt, own, lcount, nullptr);
     LAUNCH_CHECK();
     uint32_t m = 0;
-    exclusive_scan_u32(cnt, off, n, s, h->scratch, &m);
+    exclusive_scan_u32(h, cnt, off, n, &m);
     HIP_CHECK(hipMemcpyAsync(cnt, off, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
     DBuf<uint8_t> pool;
     const size_t mm = std::max<uint32_t>(m, 1);
@@ -759,8 +759,7 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
             std::swap(count[0], count[1]);
             if (round >= first_look && ((round - first_look) & 1) == 0) {
                 uint32_t hs[3];
-                HIP_CHECK(hipMemcpyAsync(hs, state, sizeof(hs), hipMemcpyDeviceToHost, s));
-                HIP_CHECK(hipStreamSynchronize(s));
+                fetch(h->lane, {{hs, state, sizeof(hs)}});
                 if (hs[0]) throw ArgError{EGT_ERR_STATE, "spanning forest: hook walk exceeded n steps"};
                 bound = hs[count[0] - state];
             }
@@ -785,18 +784,18 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
     std::vector<double> hw(sb);
     std::vector<uint32_t> hc(sb);
     uint32_t trees = 0;
-    HIP_CHECK(hipMemcpyAsync(hw.data(), part_w, sb * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(hc.data(), part_c, sb * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(&trees, trees_d, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
 
     // original order
     float* on = nrm + 3 * n;
     k_scatter_normals<<<gn, blk, 0, s>>>(nx, ny, nz, h->perm.p, n, on, on + n, on + 2 * n);
     LAUNCH_CHECK();
-    HIP_CHECK(hipMemcpyAsync(nxh, on, n * sizeof(float), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(nyh, on + n, n * sizeof(float), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(nzh, on + 2 * n, n * sizeof(float), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    const size_t bytes = n * sizeof(float);
+    fetch(h->lane, {{hw.data(), part_w, sb * sizeof(double)},
+                    {hc.data(), part_c, sb * sizeof(uint32_t)},
+                    {&trees, trees_d, sizeof(uint32_t)},
+                    {nxh, on, bytes},
+                    {nyh, on + n, bytes},
+                    {nzh, on + 2 * n, bytes}});
     HIP_CHECK(hipEventElapsedTime(&h->stats.normals_ms, ev0, ev1));
     double W = 0.0;
     int64_t C = 0;

@@ -418,17 +418,17 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_sum_u64(const uint32_t* __restri
 
 static DBuf<uint32_t>& part_buf(Scratch& sc, int i);
 
-uint64_t sum_u32(const uint32_t* in, int64_t n, hipStream_t s, Scratch& sc) {
-    unsigned long long* t = reinterpret_cast<unsigned long long*>(sc.get<uint64_t>(36, 1));
+uint64_t sum_u32(egt_ctx* h, const uint32_t* in, int64_t n) {
+    hipStream_t s = h->stream;
+    unsigned long long* t = reinterpret_cast<unsigned long long*>(h->scratch.get<uint64_t>(36, 1));
     HIP_CHECK(hipMemsetAsync(t, 0, sizeof(uint64_t), s));
     if (n > 0) {
         k_sum_u64<<<(int)std::min<int64_t>(2048, ceil_div(n, SCAN_BLOCK)), SCAN_BLOCK, 0, s>>>(in, n, t);
         LAUNCH_CHECK();
     }
-    uint64_t h = 0;
-    HIP_CHECK(hipMemcpyAsync(&h, t, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    return h;
+    uint64_t total = 0;
+    fetch(h->lane, {{&total, t, sizeof(total)}});
+    return total;
 }
 
 namespace {
@@ -442,19 +442,13 @@ auto scratch_parts(Scratch& sc) {
 }
 }  // namespace
 
-void exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t n, hipStream_t s, Scratch& sc,
-                        uint32_t* total_host) {
-    if (n <= 0) {
-        if (total_host) *total_host = 0;
-        return;
-    }
-    DBuf<uint32_t>& tot = part_buf(sc, 3);
+void exclusive_scan_u32(egt_ctx* h, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total_host) {
+    *total_host = 0;
+    if (n <= 0) return;
+    DBuf<uint32_t>& tot = part_buf(h->scratch, 3);
     tot.alloc(1);
-    scan_rec(in, out, n, s, scratch_parts(sc), 0, tot.p);
-    if (total_host) {
-        HIP_CHECK(hipMemcpyAsync(total_host, tot.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        HIP_CHECK(hipStreamSynchronize(s));
-    }
+    scan_rec(in, out, n, h->stream, scratch_parts(h->scratch), 0, tot.p);
+    fetch(h->lane, {{total_host, tot.p, sizeof(uint32_t)}});
 }
 
 void exclusive_scan_u32_dev(const uint32_t* in, uint32_t* out, int64_t n, hipStream_t s, Scratch& sc,

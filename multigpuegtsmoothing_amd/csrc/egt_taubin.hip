@@ -831,9 +831,8 @@ TilePlan prepare_tiles(egt_ctx* h) {
     LAUNCH_CHECK();
     std::vector<int32_t> hc(tp.ntiles);
     std::vector<uint32_t> pad(tp.ntiles);
-    HIP_CHECK(hipMemcpyAsync(hc.data(), tp.hcount, tp.ntiles * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(pad.data(), padded, tp.ntiles * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    fetch(h->lane, {{hc.data(), tp.hcount, tp.ntiles * sizeof(int32_t)},
+                    {pad.data(), padded, tp.ntiles * sizeof(uint32_t)}});
     std::vector<uint64_t> off(tp.ntiles);
     uint64_t tot = 0;
     for (int t = 0; t < tp.ntiles; ++t) {
@@ -974,8 +973,7 @@ bool run_resident(egt_ctx* h, int iters, float lambda, float mu) {
     k_writeback<<<ceil_div(n, TBLK), TBLK, 0, s>>>(out, n, h->mpts.p, h->x.p, h->y.p, h->z.p, R.flag);
     LAUNCH_CHECK();
     uint32_t flag = 0;
-    HIP_CHECK(hipMemcpyAsync(&flag, R.flag, sizeof(flag), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    fetch(h->lane, {{&flag, R.flag, sizeof(flag)}});
     if (flag) return false;
     float total = 0.0f, passes = 0.0f;
     HIP_CHECK(hipEventElapsedTime(&total, e0, e1));
