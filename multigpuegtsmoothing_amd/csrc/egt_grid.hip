@@ -168,51 +168,35 @@ __device__ inline int f2o(float f) {
 }
 
 // Per-cloud min/max of x, y, z (fold starting at +-1e8, as the reference's thrust reductions
-// GridKNNCuda.cu:1042-1059) plus a count of non-finite inputs. A wave whose 64 points share one cloud
-// reduces first and issues one atomic per value.
-// Each thread folds MM_PER points (stride BLK, so loads stay coalesced) into running extremes of the cloud it
-// is in, flushing them with atomics only when the cloud changes (clouds are contiguous in the input); the
-// final extremes are reduced over the wave when the wave ends in one cloud. Every point of a wave used to
-// hit the same six addresses of its cloud: 5.5 ms on 54.7M points against a fraction of that now.
-constexpr int MM_PER = 16;
+// GridKNNCuda.cu:1042-1059) plus a count of non-finite inputs. A wave takes groups of 64 MM_ROUNDS consecutive points,
+// the loads of a group in flight together. Rounds that lie in the running cloud fold into registers; where the cloud
+// changes the wave reduces what it holds and one lane sends it, and a round that straddles clouds sends its points one
+// by one. (With 16 points a thread, a stride of the block apart, a block of small clouds straddled in every thread:
+// 110 us for 24 clouds of 100,000 points in all, the longest step of their build; now 17, and 140 for 20M points in
+// 192 clouds, 560 with one group a wave.)
+constexpr int MM_ROUNDS = 4;
 __device__ inline void minmax_flush(int* __restrict__ mm, int c, const float (&v)[6]) {
+    // atomics only where they change something: the waves of a large cloud would queue at its six words
+    int seen[6];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) seen[j] = __hip_atomic_load(&mm[c * 6 + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
     for (int j = 0; j < 6; j += 2) {
-        atomicMin(&mm[c * 6 + j], f2o(v[j]));
-        atomicMax(&mm[c * 6 + j + 1], f2o(v[j + 1]));
+        if (f2o(v[j]) < seen[j]) atomicMin(&mm[c * 6 + j], f2o(v[j]));
+        if (f2o(v[j + 1]) > seen[j + 1]) atomicMax(&mm[c * 6 + j + 1], f2o(v[j + 1]));
     }
 }
 __global__ void __launch_bounds__(BLK) k_cloud_minmax(const float* __restrict__ x, const float* __restrict__ y,
                                                        const float* __restrict__ z, const int32_t* __restrict__ icloud,
-                                                       int64_t n, int* __restrict__ mm, uint32_t* __restrict__ bad) {
-    const int64_t first = (int64_t)blockIdx.x * BLK * MM_PER + threadIdx.x;
-    int c = -1;
+                                                       int64_t n, int groups, int* __restrict__ mm,
+                                                       uint32_t* __restrict__ bad) {
+    const int lane = __lane_id();
+    const int64_t w = (int64_t)blockIdx.x * (BLK / 64) + threadIdx.x / 64;
     float v[6] = {1e8f, -1e8f, 1e8f, -1e8f, 1e8f, -1e8f};
     uint32_t nb = 0;
-    for (int r = 0; r < MM_PER; ++r) {
-        const int64_t i = first + (int64_t)r * BLK;
-        if (i >= n) break;
-        const int ci = icloud[i];
-        if (ci != c) {
-            if (c >= 0) minmax_flush(mm, c, v);
-            c = ci;
-#pragma unroll
-            for (int j = 0; j < 6; j += 2) {
-                v[j] = 1e8f;
-                v[j + 1] = -1e8f;
-            }
-        }
-        const float p[3] = {x[i], y[i], z[i]};
-        nb += !(__builtin_isfinite(p[0]) && __builtin_isfinite(p[1]) && __builtin_isfinite(p[2]));
-        for (int ax = 0; ax < 3; ++ax) {
-            v[2 * ax] = fminf(v[2 * ax], p[ax]);
-            v[2 * ax + 1] = fmaxf(v[2 * ax + 1], p[ax]);
-        }
-    }
-    const bool act = c >= 0;
-    const int c0 = __shfl(c, 0, 64);
-    // uniform with c0 < 0: a wave past the end with no point (nothing to add)
-    const bool uniform = __ballot(c == c0) == ~0ull;
-    if (uniform && c0 >= 0) {
+    int run = -1;  // cloud of v
+    auto flush = [&] {
+        if (run < 0) return;
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) {
 #pragma unroll
@@ -220,19 +204,55 @@ __global__ void __launch_bounds__(BLK) k_cloud_minmax(const float* __restrict__ 
                 v[j] = fminf(v[j], __shfl_xor(v[j], d, 64));
                 v[j + 1] = fmaxf(v[j + 1], __shfl_xor(v[j + 1], d, 64));
             }
-            nb += __shfl_xor(nb, d, 64);
         }
-        if (__lane_id() == 0) {
-            for (int j = 0; j < 6; j += 2) {
-                atomicMin(&mm[c0 * 6 + j], f2o(v[j]));
-                atomicMax(&mm[c0 * 6 + j + 1], f2o(v[j + 1]));
+        if (lane == 0) minmax_flush(mm, run, v);
+        run = -1;
+#pragma unroll
+        for (int j = 0; j < 6; j += 2) {
+            v[j] = 1e8f;
+            v[j + 1] = -1e8f;
+        }
+    };
+    for (int g = 0; g < groups; ++g) {
+        const int64_t first = (w * groups + g) * (64 * MM_ROUNDS);
+        if (first >= n) break;  // wave-uniform
+        float p[MM_ROUNDS][3];
+        int ci[MM_ROUNDS];
+#pragma unroll
+        for (int r = 0; r < MM_ROUNDS; ++r) {
+            const int64_t i = min(first + r * 64 + lane, n - 1);  // past the end: the last point again
+            ci[r] = icloud[i];
+            p[r][0] = x[i];
+            p[r][1] = y[i];
+            p[r][2] = z[i];
+        }
+#pragma unroll
+        for (int r = 0; r < MM_ROUNDS; ++r) {
+            nb += first + r * 64 + lane < n &&
+                  !(__builtin_isfinite(p[r][0]) && __builtin_isfinite(p[r][1]) && __builtin_isfinite(p[r][2]));
+            const int c0 = __builtin_amdgcn_readfirstlane(ci[r]);
+            const bool uniform = __ballot(ci[r] == c0) == ~0ull;
+            if (!uniform || c0 != run) flush();
+            if (uniform) {
+                run = c0;
+#pragma unroll
+                for (int ax = 0; ax < 3; ++ax) {
+                    v[2 * ax] = fminf(v[2 * ax], p[r][ax]);
+                    v[2 * ax + 1] = fmaxf(v[2 * ax + 1], p[r][ax]);
+                }
+            } else {
+                float q[6];
+#pragma unroll
+                for (int ax = 0; ax < 3; ++ax) {
+                    q[2 * ax] = fminf(1e8f, p[r][ax]);
+                    q[2 * ax + 1] = fmaxf(-1e8f, p[r][ax]);
+                }
+                minmax_flush(mm, ci[r], q);
             }
-            if (nb) atomicAdd(bad, nb);
         }
-    } else if (!uniform && act) {
-        minmax_flush(mm, c, v);
-        if (nb) atomicAdd(bad, nb);
     }
+    flush();
+    if (nb) atomicAdd(bad, nb);
 }
 
 __global__ void __launch_bounds__(BLK) k_minmax_init(int* __restrict__ mm, int nclouds, uint32_t* __restrict__ bad) {
@@ -409,14 +429,17 @@ __global__ void __launch_bounds__(LVS_BLK) k_level_scan(uint32_t* __restrict__ c
     if (threadIdx.x == 0) total[(int64_t)blockIdx.x * stride] = run;
 }
 
-// First position of every cell of every level: starts + soff[l], in Morton order.
+// First position of every cell of every level: starts + soff[l], in Morton order. In a batch also the running cell
+// count of every level at each cloud's first position, which is the rank of the cell that begins there:
+// out[l * stride + 1 + c] (entry 0 of a level holds its total).
 struct LevelStarts {
     uint64_t soff[EGT_MAX_LEVELS];
 };
 __global__ void __launch_bounds__(BLK) k_level_starts(const uint32_t* __restrict__ code,
                                                        const int32_t* __restrict__ mcloud, int64_t n, int nl, int nb,
                                                        const uint32_t* __restrict__ pre, LevelStarts S,
-                                                       uint32_t* __restrict__ starts) {
+                                                       uint32_t* __restrict__ starts, uint32_t* __restrict__ out,
+                                                       int stride) {
     __shared__ uint32_t g[EGT_MAX_LEVELS][LV_GROUPS];
     const int lane = __lane_id(), wid = threadIdx.x / 64;
     const int64_t base = (int64_t)blockIdx.x * LV_TILE + threadIdx.x;
@@ -441,46 +464,32 @@ __global__ void __launch_bounds__(BLK) k_level_starts(const uint32_t* __restrict
     }
     __syncthreads();
     const uint64_t lt = (1ull << lane) - 1ull;
+    int first_of[LV_ITEMS];  // the cloud whose first position it is, or -1
+    if (mcloud) {
+#pragma unroll
+        for (int r = 0; r < LV_ITEMS; ++r) {
+            const int64_t m = base + r * BLK;
+            first_of[r] = fl[r] == nl && (m == 0 || mcloud[m] != mcloud[m - 1]) ? mcloud[m] : -1;
+        }
+    }
     for (int l = 0; l < nl; ++l) {
 #pragma unroll
         for (int r = 0; r < LV_ITEMS; ++r) {
             const uint64_t b = __ballot(fl[r] > l);
-            if (fl[r] > l)
-                starts[S.soff[l] + g[l][r * (BLK / 64) + wid] + (uint32_t)__popcll(b & lt)] =
-                    (uint32_t)(base + r * BLK);
+            if (fl[r] > l) {
+                const uint32_t rank = g[l][r * (BLK / 64) + wid] + (uint32_t)__popcll(b & lt);
+                starts[S.soff[l] + rank] = (uint32_t)(base + r * BLK);
+                if (mcloud && first_of[r] >= 0) out[(int64_t)l * stride + 1 + first_of[r]] = rank;
+            }
         }
     }
 }
 
-// Running cell count of every level at each cloud's first position, one wave per cloud:
-// out[l * (nclouds + 2) + 1 + c] (entry 0 of a level holds its total, entry nclouds + 1 gets it again).
-__global__ void __launch_bounds__(64) k_cells_at_bases(const uint32_t* __restrict__ code,
-                                                        const int32_t* __restrict__ mcloud, int64_t n, int nl, int nb,
-                                                        const uint32_t* __restrict__ pre,
-                                                        const CloudDev* __restrict__ clouds, int nclouds,
-                                                        uint32_t* __restrict__ out) {
-    const int c = blockIdx.x, lane = threadIdx.x;
-    if (c == nclouds) {
-        if (lane < nl) out[(int64_t)lane * (nclouds + 2) + 1 + c] = out[(int64_t)lane * (nclouds + 2)];
-        return;
-    }
-    const int64_t base = clouds[c].base, t0 = base / LV_TILE * LV_TILE;
-    uint32_t v[EGT_MAX_LEVELS] = {};
-    for (int64_t m0 = t0; m0 < base; m0 += 64) {
-        const int64_t m = m0 + lane;
-        const int fl = m < base ? first_levels(code, mcloud, m, n, nl) : 0;
-#pragma unroll
-        for (int l = 0; l < EGT_MAX_LEVELS; ++l) v[l] += (uint32_t)__popcll(__ballot(fl > l));
-    }
-#pragma unroll
-    for (int l = 0; l < EGT_MAX_LEVELS; ++l)
-        if (l < nl && lane == 0) out[(int64_t)l * (nclouds + 2) + 1 + c] = pre[(int64_t)l * nb + t0 / LV_TILE] + v[l];
-}
-
 // Inserts the cells of every level (thread i: cell i - first[l] of the level l whose range holds i; ranges may be
-// longer than the level's cell count count[l * stride]), one CAS per cell into a random slot. The level's largest cell is kept by one atomic per wave, and only by a wave that
-// exceeds the value read first: with one unconditional atomic per wave, every wave of a level queued at one
-// address (1M points: 411 us for the 11 levels, 158 us now; 4M points: 905 -> 347).
+// longer than the level's cell count count[l * stride]), one CAS per cell into a random slot. The level's largest cell
+// is kept by one atomic per wave, and only by a wave that exceeds the value read first: with one unconditional atomic
+// per wave, every wave of a level queued at one address (1M points: 411 us for the 11 levels, 158 us now; 4M points:
+// 905 -> 347).
 struct LevelInsert {
     int64_t first[EGT_MAX_LEVELS + 1];  // first thread of each level; first[nl] = all
     uint64_t soff[EGT_MAX_LEVELS];      // the level's cell starts
@@ -610,13 +619,21 @@ struct Report {
     size_t bad() const { return EGT_MAX_LEVELS * sizeof(LevelDev) / sizeof(uint32_t); }
     size_t cubes() const { return bad() + 2; }
     size_t counts() const { return cubes() + 2 * (size_t)nc; }
-    size_t words() const { return counts() + (size_t)nl * (nc + 2); }
+    size_t words() const { return counts() + (size_t)nl * (nc + 1); }
     uint32_t* dev(egt_ctx* h) const {
         h->dlev.alloc((words() * sizeof(uint32_t) + sizeof(LevelDev) - 1) / sizeof(LevelDev));
         return reinterpret_cast<uint32_t*>(h->dlev.p);
     }
 };
 Report report_of(const egt_ctx* h) { return Report{h->nclouds, ilog2(h->B) + 1}; }
+
+// Points of the largest cloud: where they fit a workgroup's sort, each cloud is sorted by one, in one launch (24 clouds
+// of 100,000 points in all: 22 launches of passes over all points before).
+int64_t max_cloud(const egt_ctx* h) {
+    int64_t m = 0;
+    for (const CloudDev& c : h->clouds) m = std::max(m, c.n);
+    return m;
+}
 
 // Normalize, key, stable sort (by cloud, then key) and gather into sorted space. icloud is null for one
 // cloud.
@@ -633,14 +650,16 @@ void sort_into_sorted_space(egt_ctx* h, const float* dx, const float* dy, const 
     k_normalize_key<<<ceil_div(n, BLK), BLK, 0, s>>>(dx, dy, dz, n, icloud, h->dclouds.p, R.dev(h) + R.bad(), a, ba,
                                                       h->B, log2B, tp, skey, sidx);
     LAUNCH_CHECK();
-    radix_sort_pairs(skey, sidx, n, 3 * log2B, s, sc);
-    if (icloud) {
+    const bool by_cloud = sort_segments(skey, sidx, max_cloud(h), 3 * log2B, icloud ? h->in_off.p : nullptr, h->nclouds,
+                                        nullptr, 0, s);
+    if (!by_cloud) radix_sort_pairs(skey, sidx, n, 3 * log2B, s, sc);
+    if (icloud) h->scloud.alloc(n);
+    if (icloud && !by_cloud) {
         // second stable pass by cloud: sorted by (cloud, key), ties in input order
         uint32_t* cl = sc.get<uint32_t>(22, n);
         k_gather_cloud<<<ceil_div(n, BLK), BLK, 0, s>>>(icloud, sidx, n, cl);
         LAUNCH_CHECK();
         radix_sort_pairs(cl, sidx, n, std::max(1, ceil_log2(h->nclouds)), s, sc, false);
-        h->scloud.alloc(n);
     }
     h->x.alloc(n);
     h->y.alloc(n);
@@ -656,16 +675,22 @@ void check_finite(const egt_ctx* h, const std::vector<uint32_t>& rep) {
     if (rep[report_of(h).bad()]) throw ArgError{EGT_ERR_INVALID_ARG, "input coordinates contain NaN or Inf"};
 }
 
-// The host's cloud table from a build's report.
-void set_clouds(egt_ctx* h, const std::vector<uint32_t>& rep, const int64_t* offsets) {
+// The host's cloud table: places and sizes, before a build, and the cubes from its report.
+void place_clouds(egt_ctx* h, int nclouds, const int64_t* offsets) {
+    h->nclouds = nclouds;
+    h->clouds.assign(nclouds, CloudDev{});
+    for (int c = 0; c < nclouds; ++c) {
+        h->clouds[c].base = offsets[c];
+        h->clouds[c].n = offsets[c + 1] - offsets[c];
+    }
+    h->dclouds.alloc(nclouds);
+}
+void set_cubes(egt_ctx* h, const std::vector<uint32_t>& rep) {
     const uint32_t* cube = rep.data() + report_of(h).cubes();
-    h->clouds.assign(h->nclouds, CloudDev{});
     for (int c = 0; c < h->nclouds; ++c) {
         float mm[2];
         std::memcpy(mm, cube + 2 * c, sizeof(mm));
         CloudDev& cd = h->clouds[c];
-        cd.base = offsets[c];
-        cd.n = offsets[c + 1] - offsets[c];
         cd.min_extent = mm[0];
         cd.extent = mm[1] - mm[0];
         cd.max_extent = mm[1];
@@ -686,8 +711,8 @@ void build_grid(egt_ctx* h, const float* dx, const float* dy, const float* dz) {
     HIP_CHECK(hipEventRecord(e0, s));
 
     // bounding cube
-    h->nclouds = 1;
-    h->dclouds.alloc(1);
+    const int64_t offsets[2] = {0, n};
+    place_clouds(h, 1, offsets);
     const Report R = report_of(h);
     uint32_t* rep = R.dev(h);
     const int nbp = std::min<int64_t>(1024, std::max<int64_t>(1, ceil_div(n, BLK)));
@@ -699,8 +724,7 @@ void build_grid(egt_ctx* h, const float* dx, const float* dy, const float* dz) {
     sort_into_sorted_space(h, dx, dy, dz, nullptr);
     std::vector<uint32_t> hr;
     build_search_structure(h, hr, e1);
-    const int64_t offsets[2] = {0, n};
-    set_clouds(h, hr, offsets);
+    set_cubes(h, hr);
     HIP_CHECK(hipEventElapsedTime(&h->stats.grid_ms, e0, e1));
 }
 
@@ -711,27 +735,28 @@ void build_grid_batch(egt_ctx* h, const float* dx, const float* dy, const float*
     Scratch& sc = h->scratch;
     Event e0, e1;
     HIP_CHECK(hipEventRecord(e0, s));
-    h->nclouds = nclouds;
+    place_clouds(h, nclouds, offsets);
     h->in_off.alloc(nclouds + 1);
     HIP_CHECK(hipMemcpyAsync(h->in_off.p, offsets, (nclouds + 1) * sizeof(int64_t), hipMemcpyHostToDevice, s));
     int32_t* icloud = sc.get<int32_t>(21, n);
     k_cloud_of<<<ceil_div(n, BLK), BLK, 0, s>>>(h->in_off.p, nclouds, n, icloud);
     LAUNCH_CHECK();
-    h->dclouds.alloc(nclouds);
     const Report R = report_of(h);
     uint32_t* rep = R.dev(h);
     int* mm = sc.get<int>(8, (size_t)nclouds * 6);
     k_minmax_init<<<ceil_div(nclouds * 6, BLK), BLK, 0, s>>>(mm, nclouds, rep + R.bad());
     LAUNCH_CHECK();
-    k_cloud_minmax<<<std::max(1, ceil_div(n, (int64_t)BLK * MM_PER)), BLK, 0, s>>>(dx, dy, dz, icloud, n, mm,
-                                                                                    rep + R.bad());
+    // one group a wave while that leaves few waves, then more groups and fewer sends
+    const int groups = (int)std::min<int64_t>(16, std::max<int64_t>(1, n / ((int64_t)8192 * 64 * MM_ROUNDS)));
+    k_cloud_minmax<<<ceil_div(n, (int64_t)BLK * MM_ROUNDS * groups), BLK, 0, s>>>(dx, dy, dz, icloud, n, groups, mm,
+                                                                                 rep + R.bad());
     LAUNCH_CHECK();
     k_cloud_cubes<<<ceil_div(nclouds, BLK), BLK, 0, s>>>(mm, h->in_off.p, nclouds, h->dclouds.p, rep + R.cubes());
     LAUNCH_CHECK();
     sort_into_sorted_space(h, dx, dy, dz, icloud);
     std::vector<uint32_t> hr;
     build_search_structure(h, hr, e1);
-    set_clouds(h, hr, offsets);
+    set_cubes(h, hr);
     HIP_CHECK(hipEventElapsedTime(&h->stats.grid_ms, e0, e1));
 }
 
@@ -750,6 +775,7 @@ void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t d
     order.alloc(n);
     const float a = -h->eps, ba = (1.0f + h->eps) - a;
     float4* spts = sc.get<float4>(11, n);  // sorted-space records (x, y, z, key)
+    bool by_cloud = false;
     {
         // Morton order of the fine cells, points of a cell in sub-code order: stable sort by sub code, then
         // stable sort by cell code
@@ -758,18 +784,22 @@ void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t d
         k_morton_keys<<<ceil_div(n, BLK), BLK, 0, s>>>(h->x.p, h->y.p, h->z.p, h->key.p, n, a, ba, h->B, log2B,
                                                        cell, sub, order.p, spts);
         LAUNCH_CHECK();
-        radix_sort_pairs(sub, order.p, n, 3 * SUB, s, sc, false);
-        k_gather_u32<<<ceil_div(n, BLK), BLK, 0, s>>>(cell, order.p, n, code.p);
-        LAUNCH_CHECK();
+        by_cloud = sort_segments(sub, order.p, max_cloud(h), 3 * SUB, batch ? h->in_off.p : nullptr, h->nclouds, cell,
+                                 3 * log2B, s);
+        if (!by_cloud) {
+            radix_sort_pairs(sub, order.p, n, 3 * SUB, s, sc, false);
+            k_gather_u32<<<ceil_div(n, BLK), BLK, 0, s>>>(cell, order.p, n, code.p);
+            LAUNCH_CHECK();
+            radix_sort_pairs(code.p, order.p, n, 3 * log2B, s, sc);
+        }
     }
-    radix_sort_pairs(code.p, order.p, n, 3 * log2B, s, sc);
-    if (batch) {
+    if (batch) h->mcloud.alloc(n);
+    if (batch && !by_cloud) {
         // second stable pass by cloud: Morton order within each cloud, clouds in input order
         uint32_t* cl = sc.get<uint32_t>(22, n);
         k_gather_cloud<<<ceil_div(n, BLK), BLK, 0, s>>>(h->scloud.p, order.p, n, cl);
         LAUNCH_CHECK();
         radix_sort_pairs(cl, order.p, n, std::max(1, ceil_log2(h->nclouds)), s, sc, false);
-        h->mcloud.alloc(n);
     }
     h->mpts.alloc(n);
     h->mcell.alloc(n);
@@ -803,14 +833,10 @@ void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t d
     uint32_t* dtot = drep + R.counts();  // per level: total, then the cloud bases
     k_level_count<<<nb, BLK, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles);
     LAUNCH_CHECK();
-    k_level_scan<<<nl, LVS_BLK, 0, s>>>(tiles, nb, dtot, nc + 2);
+    k_level_scan<<<nl, LVS_BLK, 0, s>>>(tiles, nb, dtot, nc + 1);
     LAUNCH_CHECK();
-    k_level_starts<<<nb, BLK, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles, ls, starts);
+    k_level_starts<<<nb, BLK, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles, ls, starts, dtot, nc + 1);
     LAUNCH_CHECK();
-    if (batch) {
-        k_cells_at_bases<<<nc + 1, 64, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles, h->dclouds.p, nc, dtot);
-        LAUNCH_CHECK();
-    }
     // The tables are sized by the levels' cell counts, which takes one trip to the host, or, up to TABLE_BOUND cells,
     // by the bounds above, which takes none.
     rep.resize(R.words());
@@ -823,7 +849,7 @@ void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t d
     LevelInsert li{};
     li.nl = nl;
     for (int l = 0; l < nl; ++l) {
-        const uint64_t cells = by_bound ? soff[l + 1] - soff[l] : rep[R.counts() + (size_t)l * (nc + 2)];
+        const uint64_t cells = by_bound ? soff[l + 1] - soff[l] : rep[R.counts() + (size_t)l * (nc + 1)];
         // Twice the cells at least, and eight times on the coarse levels, whose tables are small beside the fine ones:
         // a wave's search waits for its longest probe chain. Search, us, twice everywhere -> eight times on coarse
         // levels: torus 1M k=16 1122 -> 1047, 16M k=40 32300 -> 31890; mixture 4M k=40 12976 -> 12776, 16M 57136 ->
@@ -841,15 +867,18 @@ void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t d
     k_level_init<<<(int)std::min<uint64_t>(1024, (2 * li.slots + BLK - 1) / BLK), BLK, 0, s>>>(
         li, reinterpret_cast<uint64_t*>(h->htab.p), h->dlev.p);
     LAUNCH_CHECK();
-    k_level_insert<<<ceil_div(li.first[nl], BLK), BLK, 0, s>>>(li, starts, n, h->mcode.p, mcl, dtot, nc + 2, h->htab.p,
+    k_level_insert<<<ceil_div(li.first[nl], BLK), BLK, 0, s>>>(li, starts, n, h->mcode.p, mcl, dtot, nc + 1, h->htab.p,
                                                                h->dlev.p);
     LAUNCH_CHECK();
     if (done) HIP_CHECK(hipEventRecord(done, s));
     read_back(by_bound ? R.words() : R.bad() + 1);
     h->cloud_cells.assign((size_t)nc * nl, 0);
     for (int l = 0; l < nl; ++l) {
-        const uint32_t* tl = &rep[R.counts() + (size_t)l * (nc + 2)];
-        for (int c = 0; c < nc; ++c) h->cloud_cells[(size_t)c * nl + l] = batch ? tl[1 + c + 1] - tl[1 + c] : tl[0];
+        const uint32_t* tl = &rep[R.counts() + (size_t)l * (nc + 1)];
+        for (int c = 0; c < nc; ++c) {
+            const uint32_t end = c + 1 < nc ? tl[1 + c + 1] : tl[0];
+            h->cloud_cells[(size_t)c * nl + l] = end - (c > 0 ? tl[1 + c] : 0);
+        }
         LevelDev d;
         std::memcpy(&d, &rep[l * (sizeof(LevelDev) / sizeof(uint32_t))], sizeof(d));
         h->lev[l].cells = tl[0];

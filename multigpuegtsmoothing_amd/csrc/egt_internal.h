@@ -296,7 +296,12 @@ void exclusive_scan_u32_dev(const uint32_t* in, uint32_t* out, int64_t n, hipStr
 // Stable sort of (key, value) pairs by the low key_bits bits. With keep_keys false the keys end up undefined.
 void radix_sort_pairs(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, Scratch& sc,
                       bool keep_keys = true);
-// The same sort over a caller's workspace of radix_sort_workspace_words(n) 32-bit words (no allocation).
+// Stable sorts of the segments [seg[b], seg[b + 1]) (null: one of max_len pairs), each in one workgroup, by the low
+// key_bits bits of keys and then, where keys2 is given, by the low key_bits2 bits of keys2[value]. False, with nothing
+// done, where max_len is beyond a workgroup's. With keys2 the keys end up undefined.
+bool sort_segments(uint32_t* keys, uint32_t* vals, int64_t max_len, int key_bits, const int64_t* seg, int nseg,
+                   const uint32_t* keys2, int key_bits2, hipStream_t s);
+// radix_sort_pairs over a caller's workspace of radix_sort_workspace_words(n) 32-bit words (no allocation).
 size_t radix_sort_workspace_words(int64_t n);
 void radix_sort_pairs_ws(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, uint32_t* ws);
 // Sum of n uint32 values in 64 bits (synchronizes the stream).

@@ -273,10 +273,12 @@ __global__ void __launch_bounds__(SORT_BLOCK) k_sort_scatter(const uint32_t* __r
     }
 }
 
-// Every pass of up to SMALL_BLOCK * ITEMS keys in one workgroup: keys and values stay in LDS between passes.
+// Every pass of up to SMALL_BLOCK * ITEMS keys in one workgroup: keys and values stay in LDS between passes. With
+// seg, workgroup b sorts the keys [seg[b], seg[b + 1]). With keys2, a second stable sort follows, by keys2[value].
 template <int ITEMS>
 __global__ void __launch_bounds__(SMALL_BLOCK) k_sort_small(uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
-                                                             int n, int key_bits) {
+                                                             int n, int key_bits, const int64_t* __restrict__ seg,
+                                                             const uint32_t* __restrict__ keys2, int key_bits2) {
     constexpr int NW = SMALL_BLOCK / WAVE, BINS = 256;
     __shared__ uint32_t sk[SMALL_BLOCK * ITEMS], sv[SMALL_BLOCK * ITEMS];
     __shared__ uint32_t wcnt[NW][BINS];
@@ -284,6 +286,12 @@ __global__ void __launch_bounds__(SMALL_BLOCK) k_sort_small(uint32_t* __restrict
     __shared__ uint32_t ws[BINS / WAVE];
     const int lane = __lane_id(), wid = threadIdx.x / WAVE;
     const int base = wid * WAVE * ITEMS;
+    if (seg) {
+        const int64_t first = seg[blockIdx.x];
+        keys += first;
+        vals += first;
+        n = (int)(seg[blockIdx.x + 1] - first);
+    }
     uint32_t kk[ITEMS], vv[ITEMS], pos[ITEMS];
 #pragma unroll
     for (int r = 0; r < ITEMS; ++r) {
@@ -291,7 +299,15 @@ __global__ void __launch_bounds__(SMALL_BLOCK) k_sort_small(uint32_t* __restrict
         kk[r] = i < n ? keys[i] : 0u;
         vv[r] = i < n ? vals[i] : 0u;
     }
-    for (int shift = 0; shift < key_bits; shift += 8) {
+    for (int shift = 0;; shift += 8) {
+        if (shift >= key_bits) {
+            if (!keys2) break;
+#pragma unroll
+            for (int r = 0; r < ITEMS; ++r) kk[r] = base + r * WAVE + lane < n ? keys2[vv[r]] : 0u;
+            keys2 = nullptr;
+            key_bits = key_bits2;
+            shift = 0;
+        }
         for (int i = threadIdx.x; i < NW * BINS; i += SMALL_BLOCK) (&wcnt[0][0])[i] = 0;
         __syncthreads();
         wave_ranks<8, ITEMS>(kk, base, n, shift, wcnt[wid], pos, [](int, int64_t, bool) {});
@@ -394,13 +410,23 @@ void radix_passes(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipSt
     }
 }
 
+// Sorts of at most max_len <= SMALL_MAX pairs each, in one launch.
+void sort_small(uint32_t* keys, uint32_t* vals, int64_t max_len, int key_bits, const int64_t* seg, int nseg,
+                const uint32_t* keys2, int key_bits2, hipStream_t s) {
+    const int n = (int)max_len;
+    if (n <= 2 * SMALL_BLOCK)
+        k_sort_small<2><<<nseg, SMALL_BLOCK, 0, s>>>(keys, vals, n, key_bits, seg, keys2, key_bits2);
+    else if (n <= 4 * SMALL_BLOCK)
+        k_sort_small<4><<<nseg, SMALL_BLOCK, 0, s>>>(keys, vals, n, key_bits, seg, keys2, key_bits2);
+    else
+        k_sort_small<8><<<nseg, SMALL_BLOCK, 0, s>>>(keys, vals, n, key_bits, seg, keys2, key_bits2);
+    LAUNCH_CHECK();
+}
+
 // Sorts up to SMALL_MAX pairs in one launch; false above.
 bool radix_small(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s) {
     if (n > SMALL_MAX) return false;
-    if (n <= 2 * SMALL_BLOCK) k_sort_small<2><<<1, SMALL_BLOCK, 0, s>>>(keys, vals, (int)n, key_bits);
-    else if (n <= 4 * SMALL_BLOCK) k_sort_small<4><<<1, SMALL_BLOCK, 0, s>>>(keys, vals, (int)n, key_bits);
-    else k_sort_small<8><<<1, SMALL_BLOCK, 0, s>>>(keys, vals, (int)n, key_bits);
-    LAUNCH_CHECK();
+    sort_small(keys, vals, n, key_bits, nullptr, 1, nullptr, 0, s);
     return true;
 }
 
@@ -458,6 +484,13 @@ void exclusive_scan_u32_dev(const uint32_t* in, uint32_t* out, int64_t n, hipStr
         return;
     }
     scan_rec(in, out, n, s, scratch_parts(sc), 0, total_dev);
+}
+
+bool sort_segments(uint32_t* keys, uint32_t* vals, int64_t max_len, int key_bits, const int64_t* seg, int nseg,
+                   const uint32_t* keys2, int key_bits2, hipStream_t s) {
+    if (max_len > SMALL_MAX) return false;
+    sort_small(keys, vals, max_len, key_bits, seg, nseg, keys2, key_bits2, s);
+    return true;
 }
 
 void radix_sort_pairs(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, Scratch& sc,

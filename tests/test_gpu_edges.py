@@ -203,3 +203,30 @@ def test_level_tables_by_bound_and_by_count(egt_mod, oracle_mod, n):
         E.GridStructure(bad, 1, 1e-6, 1024, 4)
     with pytest.raises(E.EGTError, match="NaN or Inf"):
         E.BatchGrid([tuple(c[:500] for c in pts), tuple(c[-500:] for c in bad)])
+
+
+@pytest.mark.parametrize("sizes", [[2_048, 1, 7, 2_047], [4_096, 2_049, 300], [8_192, 4_097, 1], [8_193, 5_000, 64],
+                                   [1] * 200 + [500]])
+def test_batch_sorts_at_form_limits(egt_mod, oracle_mod, sizes):
+    """Clouds up to 8,192 points are sorted a workgroup each (2, 4 or 8 keys a thread), larger ones by passes over all
+    points; clouds of one point put many cloud changes into one wave of the extents kernel. After a smoothing call
+    the search structure is rebuilt the same way: rows as a handle of one cloud gives them."""
+    E, O = egt_mod, oracle_mod
+    print("sizes", sizes[:4], flush=True)
+    clouds = [tuple(c * (1 + i % 5) + 10 * i for c in D.sphere(n, seed=600 + i)) for i, n in enumerate(sizes)]
+    clouds = [tuple(c.astype(np.float32) for c in cl) for cl in clouds]
+    b = E.BatchGrid(clouds)
+    b.knn(9)
+    grids = [O.Grid(*cl) for cl in clouds]
+    for c in [i for i in range(len(clouds)) if i < 3 or i > len(clouds) - 3]:
+        np.testing.assert_array_equal(b.GetKNNIndexes(c), grids[c].to_original(grids[c].knn(9)[0]), err_msg=f"cloud {c}")
+    E.EGT_CUDA(b).PerformSmoothing(2, 0.5, -0.53, 0.65)
+    b.knn(9)
+    for c in (0, 1, len(clouds) - 1):
+        g = E.GridStructure(clouds[c], 1, 1e-6, 1024, 4)
+        g.GRIDCUDAKNNSELF_COMPACT(9, 1e8)
+        E.EGT_CUDA(g).PerformSmoothing(2, 0.5, -0.53, 0.65)
+        g.GRIDCUDAKNNSELF_COMPACT(9, 1e8)
+        np.testing.assert_array_equal(b.GetKNNIndexes(c), g.GetKNNIndexes(), err_msg=f"smoothed cloud {c}")
+        g.close()
+    b.close()
