@@ -284,12 +284,33 @@ __global__ void __launch_bounds__(BLK) k_gather_cloud(const int32_t* __restrict_
     if (i < n) out[i] = (uint32_t)cloud_of[idx[i]];
 }
 
-// thrust::gather into sorted order, GridKNNCuda.cu:1114-1128: one 16-byte record per point.
+// Sort keys of the Morton order: the fine cell's Morton code and the Morton code of the point's position
+// inside the cell (sorted first, stably, so that points of a cell end up in sub-code order); also the point as
+// one 16-byte record (x, y, z, key) in sorted order for the gather into Morton order.
+struct MortonKeys {
+    float a, ba;
+    int B, log2B;
+    uint32_t *code, *sub, *idx;
+    float4* spts;
+};
+__device__ inline void morton_keys(const MortonKeys& K, int64_t s, float px, float py, float pz, uint32_t k) {
+    const uint32_t m = (1u << K.log2B) - 1u;
+    const uint32_t cx = k & m, cy = (k >> K.log2B) & m, cz = k >> (2 * K.log2B);
+    K.code[s] = morton_code(cx, cy, cz);
+    K.sub[s] = vcell_sub(vcell_pack(vcoord(px, K.a, K.ba, K.B, (int)cx), vcoord(py, K.a, K.ba, K.B, (int)cy),
+                                    vcoord(pz, K.a, K.ba, K.B, (int)cz)));
+    K.idx[s] = (uint32_t)s;
+    K.spts[s] = make_float4(px, py, pz, __int_as_float((int32_t)k));
+}
+
+// thrust::gather into sorted order, GridKNNCuda.cu:1114-1128: one 16-byte record per point; its Morton sort keys
+// while it is at hand.
 __global__ void __launch_bounds__(BLK) k_gather_sorted(const float4* __restrict__ tp, const int32_t* __restrict__ icloud,
                                                         const uint32_t* __restrict__ sidx, int64_t n,
                                                         float* __restrict__ x, float* __restrict__ y,
                                                         float* __restrict__ z, int32_t* __restrict__ perm,
-                                                        int32_t* __restrict__ key, int32_t* __restrict__ scloud) {
+                                                        int32_t* __restrict__ key, int32_t* __restrict__ scloud,
+                                                        MortonKeys K) {
     const int64_t s = (int64_t)blockIdx.x * BLK + threadIdx.x;
     if (s >= n) return;
     const uint32_t o = sidx[s];
@@ -300,26 +321,7 @@ __global__ void __launch_bounds__(BLK) k_gather_sorted(const float4* __restrict_
     x[s] = v.x;
     y[s] = v.y;
     z[s] = v.z;
-}
-
-// Sort keys of the Morton order: the fine cell's Morton code and the Morton code of the point's position
-// inside the cell (sorted first, stably, so that points of a cell end up in sub-code order); also the point as
-// one 16-byte record (x, y, z, key) in sorted order for the gather into Morton order.
-__global__ void __launch_bounds__(BLK) k_morton_keys(const float* __restrict__ x, const float* __restrict__ y,
-                                                      const float* __restrict__ z, const int32_t* __restrict__ key,
-                                                      int64_t n, float a, float ba, int B, int log2B,
-                                                      uint32_t* __restrict__ code, uint32_t* __restrict__ sub,
-                                                      uint32_t* __restrict__ idx, float4* __restrict__ spts) {
-    const int64_t s = (int64_t)blockIdx.x * BLK + threadIdx.x;
-    if (s >= n) return;
-    const uint32_t k = (uint32_t)key[s], m = (1u << log2B) - 1u;
-    const uint32_t cx = k & m, cy = (k >> log2B) & m, cz = k >> (2 * log2B);
-    const float px = x[s], py = y[s], pz = z[s];
-    code[s] = morton_code(cx, cy, cz);
-    sub[s] = vcell_sub(vcell_pack(vcoord(px, a, ba, B, (int)cx), vcoord(py, a, ba, B, (int)cy),
-                                  vcoord(pz, a, ba, B, (int)cz)));
-    idx[s] = (uint32_t)s;
-    spts[s] = make_float4(px, py, pz, __int_as_float((int32_t)k));
+    morton_keys(K, s, v.x, v.y, v.z, __float_as_uint(v.w));
 }
 
 __global__ void __launch_bounds__(BLK) k_gather_u32(const uint32_t* __restrict__ src,
@@ -431,7 +433,8 @@ __global__ void __launch_bounds__(LVS_BLK) k_level_scan(uint32_t* __restrict__ c
 
 // First position of every cell of every level: starts + soff[l], in Morton order. In a batch also the running cell
 // count of every level at each cloud's first position, which is the rank of the cell that begins there:
-// out[l * stride + 1 + c] (entry 0 of a level holds its total).
+// out[l * stride + 1 + c] (entry 0 of a level holds its total). A single tile needs no prefix (pre null): it writes the
+// totals itself.
 struct LevelStarts {
     uint64_t soff[EGT_MAX_LEVELS];
 };
@@ -455,12 +458,13 @@ __global__ void __launch_bounds__(BLK) k_level_starts(const uint32_t* __restrict
     }
     __syncthreads();
     if ((int)threadIdx.x < nl) {
-        uint32_t run = pre[(int64_t)threadIdx.x * nb + blockIdx.x];
+        uint32_t run = pre ? pre[(int64_t)threadIdx.x * nb + blockIdx.x] : 0u;
         for (int i = 0; i < LV_GROUPS; ++i) {
             const uint32_t c = g[threadIdx.x][i];
             g[threadIdx.x][i] = run;
             run += c;
         }
+        if (!pre) out[(int64_t)threadIdx.x * stride] = run;
     }
     __syncthreads();
     const uint64_t lt = (1ull << lane) - 1ull;
@@ -635,9 +639,18 @@ int64_t max_cloud(const egt_ctx* h) {
     return m;
 }
 
+// Sort keys and values of the Morton order (buffers apart from those of the first sort).
+MortonKeys morton_buffers(egt_ctx* h) {
+    const int64_t n = h->n;
+    Scratch& sc = h->scratch;
+    const float a = -h->eps;
+    return MortonKeys{a, (1.0f + h->eps) - a, h->B, ilog2(h->B), sc.get<uint32_t>(8, n), sc.get<uint32_t>(22, n),
+                      sc.get<uint32_t>(10, n), sc.get<float4>(11, n)};
+}
+
 // Normalize, key, stable sort (by cloud, then key) and gather into sorted space. icloud is null for one
 // cloud.
-void sort_into_sorted_space(egt_ctx* h, const float* dx, const float* dy, const float* dz, const int32_t* icloud) {
+MortonKeys sort_into_sorted_space(egt_ctx* h, const float* dx, const float* dy, const float* dz, const int32_t* icloud) {
     const int64_t n = h->n;
     hipStream_t s = h->stream;
     Scratch& sc = h->scratch;
@@ -666,9 +679,11 @@ void sort_into_sorted_space(egt_ctx* h, const float* dx, const float* dy, const 
     h->z.alloc(n);
     h->perm.alloc(n);
     h->key.alloc(n);
+    const MortonKeys K = morton_buffers(h);
     k_gather_sorted<<<ceil_div(n, BLK), BLK, 0, s>>>(tp, icloud, sidx, n, h->x.p, h->y.p, h->z.p, h->perm.p,
-                                                      h->key.p, icloud ? h->scloud.p : nullptr);
+                                                      h->key.p, icloud ? h->scloud.p : nullptr, K);
     LAUNCH_CHECK();
+    return K;
 }
 
 void check_finite(const egt_ctx* h, const std::vector<uint32_t>& rep) {
@@ -699,7 +714,7 @@ void set_cubes(egt_ctx* h, const std::vector<uint32_t>& rep) {
     h->max_extent = h->clouds[0].max_extent;
 }
 
-void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t done);
+void build_search_structure(egt_ctx* h, const MortonKeys& K, std::vector<uint32_t>& rep, hipEvent_t done);
 
 }  // namespace
 
@@ -716,14 +731,14 @@ void build_grid(egt_ctx* h, const float* dx, const float* dy, const float* dz) {
     const Report R = report_of(h);
     uint32_t* rep = R.dev(h);
     const int nbp = std::min<int64_t>(1024, std::max<int64_t>(1, ceil_div(n, BLK)));
-    float* dpart = sc.get<float>(8, (size_t)nbp * MM_WORDS);
+    float* dpart = sc.get<float>(8, std::max<size_t>((size_t)nbp * MM_WORDS, n));  // the Morton keys' size
     k_minmax_partial<<<nbp, BLK, 0, s>>>(dx, dy, dz, n, dpart);
     LAUNCH_CHECK();
     k_cloud_cube<<<1, 64, 0, s>>>(dpart, nbp, n, h->dclouds.p, rep + R.bad(), rep + R.cubes());
     LAUNCH_CHECK();
-    sort_into_sorted_space(h, dx, dy, dz, nullptr);
+    const MortonKeys K = sort_into_sorted_space(h, dx, dy, dz, nullptr);
     std::vector<uint32_t> hr;
-    build_search_structure(h, hr, e1);
+    build_search_structure(h, K, hr, e1);
     set_cubes(h, hr);
     HIP_CHECK(hipEventElapsedTime(&h->stats.grid_ms, e0, e1));
 }
@@ -743,7 +758,7 @@ void build_grid_batch(egt_ctx* h, const float* dx, const float* dy, const float*
     LAUNCH_CHECK();
     const Report R = report_of(h);
     uint32_t* rep = R.dev(h);
-    int* mm = sc.get<int>(8, (size_t)nclouds * 6);
+    int* mm = sc.get<int>(8, std::max<size_t>((size_t)nclouds * 6, n));  // the Morton keys' size
     k_minmax_init<<<ceil_div(nclouds * 6, BLK), BLK, 0, s>>>(mm, nclouds, rep + R.bad());
     LAUNCH_CHECK();
     // one group a wave while that leaves few waves, then more groups and fewer sends
@@ -753,53 +768,40 @@ void build_grid_batch(egt_ctx* h, const float* dx, const float* dy, const float*
     LAUNCH_CHECK();
     k_cloud_cubes<<<ceil_div(nclouds, BLK), BLK, 0, s>>>(mm, h->in_off.p, nclouds, h->dclouds.p, rep + R.cubes());
     LAUNCH_CHECK();
-    sort_into_sorted_space(h, dx, dy, dz, icloud);
+    const MortonKeys K = sort_into_sorted_space(h, dx, dy, dz, icloud);
     std::vector<uint32_t> hr;
-    build_search_structure(h, hr, e1);
+    build_search_structure(h, K, hr, e1);
     set_cubes(h, hr);
     HIP_CHECK(hipEventElapsedTime(&h->stats.grid_ms, e0, e1));
 }
 
 namespace {
-// The Morton order and the level tables of the sorted points; rep: the report, done: recorded when the work is queued
+// The Morton order (from the sort keys K) and the level tables of the sorted points; rep: the report, done: recorded when the work is queued
 // (if not null). Synchronizes the stream.
-void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t done) {
+void build_search_structure(egt_ctx* h, const MortonKeys& K, std::vector<uint32_t>& rep, hipEvent_t done) {
     const int64_t n = h->n;
     hipStream_t s = h->stream;
     Scratch& sc = h->scratch;
     const int log2B = ilog2(h->B);
     const bool batch = h->nclouds > 1;
-    DBuf<uint32_t>& code = sc.bufs[12];
-    DBuf<uint32_t>& order = sc.bufs[13];
-    code.alloc(n);
-    order.alloc(n);
-    const float a = -h->eps, ba = (1.0f + h->eps) - a;
-    float4* spts = sc.get<float4>(11, n);  // sorted-space records (x, y, z, key)
-    bool by_cloud = false;
-    {
-        // Morton order of the fine cells, points of a cell in sub-code order: stable sort by sub code, then
-        // stable sort by cell code
-        uint32_t* sub = sc.get<uint32_t>(22, n);
-        uint32_t* cell = sc.get<uint32_t>(8, n);
-        k_morton_keys<<<ceil_div(n, BLK), BLK, 0, s>>>(h->x.p, h->y.p, h->z.p, h->key.p, n, a, ba, h->B, log2B,
-                                                       cell, sub, order.p, spts);
+    uint32_t* order = K.idx;
+    // Morton order of the fine cells, points of a cell in sub-code order: stable sort by sub code, then by cell code
+    const bool by_cloud = sort_segments(K.sub, order, max_cloud(h), 3 * SUB, batch ? h->in_off.p : nullptr, h->nclouds,
+                                        K.code, 3 * log2B, s);
+    if (!by_cloud) {
+        uint32_t* code = sc.get<uint32_t>(12, n);
+        radix_sort_pairs(K.sub, order, n, 3 * SUB, s, sc, false);
+        k_gather_u32<<<ceil_div(n, BLK), BLK, 0, s>>>(K.code, order, n, code);
         LAUNCH_CHECK();
-        by_cloud = sort_segments(sub, order.p, max_cloud(h), 3 * SUB, batch ? h->in_off.p : nullptr, h->nclouds, cell,
-                                 3 * log2B, s);
-        if (!by_cloud) {
-            radix_sort_pairs(sub, order.p, n, 3 * SUB, s, sc, false);
-            k_gather_u32<<<ceil_div(n, BLK), BLK, 0, s>>>(cell, order.p, n, code.p);
-            LAUNCH_CHECK();
-            radix_sort_pairs(code.p, order.p, n, 3 * log2B, s, sc);
-        }
+        radix_sort_pairs(code, order, n, 3 * log2B, s, sc);
     }
     if (batch) h->mcloud.alloc(n);
     if (batch && !by_cloud) {
         // second stable pass by cloud: Morton order within each cloud, clouds in input order
         uint32_t* cl = sc.get<uint32_t>(22, n);
-        k_gather_cloud<<<ceil_div(n, BLK), BLK, 0, s>>>(h->scloud.p, order.p, n, cl);
+        k_gather_cloud<<<ceil_div(n, BLK), BLK, 0, s>>>(h->scloud.p, order, n, cl);
         LAUNCH_CHECK();
-        radix_sort_pairs(cl, order.p, n, std::max(1, ceil_log2(h->nclouds)), s, sc, false);
+        radix_sort_pairs(cl, order, n, std::max(1, ceil_log2(h->nclouds)), s, sc, false);
     }
     h->mpts.alloc(n);
     h->mcell.alloc(n);
@@ -807,8 +809,8 @@ void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t d
     h->mcode.alloc(n);
     h->morder.alloc(n);
     h->minv.alloc(n);
-    k_morton_points<<<ceil_div(n, BLK), BLK, 0, s>>>(spts, batch ? h->scloud.p : nullptr,
-                                                      order.p, n, a, ba, h->B, log2B, h->mpts.p, h->mcell.p,
+    k_morton_points<<<ceil_div(n, BLK), BLK, 0, s>>>(K.spts, batch ? h->scloud.p : nullptr,
+                                                      order, n, K.a, K.ba, h->B, log2B, h->mpts.p, h->mcell.p,
                                                       reinterpret_cast<unsigned long long*>(h->mvcell.p), h->mcode.p,
                                                       batch ? h->mcloud.p : nullptr, h->morder.p, h->minv.p);
     LAUNCH_CHECK();
@@ -828,13 +830,15 @@ void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t d
     }
     uint32_t* starts = sc.get<uint32_t>(38, soff[nl]);
     const int nb = ceil_div(n, LV_TILE);
-    uint32_t* tiles = sc.get<uint32_t>(9, (size_t)nl * nb);
+    uint32_t* tiles = nb > 1 ? sc.get<uint32_t>(9, (size_t)nl * nb) : nullptr;
     uint32_t* drep = R.dev(h);
     uint32_t* dtot = drep + R.counts();  // per level: total, then the cloud bases
-    k_level_count<<<nb, BLK, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles);
-    LAUNCH_CHECK();
-    k_level_scan<<<nl, LVS_BLK, 0, s>>>(tiles, nb, dtot, nc + 1);
-    LAUNCH_CHECK();
+    if (nb > 1) {
+        k_level_count<<<nb, BLK, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles);
+        LAUNCH_CHECK();
+        k_level_scan<<<nl, LVS_BLK, 0, s>>>(tiles, nb, dtot, nc + 1);
+        LAUNCH_CHECK();
+    }
     k_level_starts<<<nb, BLK, 0, s>>>(h->mcode.p, mcl, n, nl, nb, tiles, ls, starts, dtot, nc + 1);
     LAUNCH_CHECK();
     // The tables are sized by the levels' cell counts, which takes one trip to the host, or, up to TABLE_BOUND cells,
@@ -889,25 +893,27 @@ void build_search_structure(egt_ctx* h, std::vector<uint32_t>& rep, hipEvent_t d
 
 namespace {
 __global__ void __launch_bounds__(BLK) k_rekey(const float* __restrict__ x, const float* __restrict__ y,
-                                                const float* __restrict__ z, int64_t n, float a, float ba, int B,
-                                                int log2B, int32_t* __restrict__ key) {
+                                                const float* __restrict__ z, int64_t n, int32_t* __restrict__ key,
+                                                MortonKeys K) {
     const int64_t s = (int64_t)blockIdx.x * BLK + threadIdx.x;
     if (s >= n) return;
-    const uint32_t cx = (uint32_t)cell_of(x[s], a, ba, B), cy = (uint32_t)cell_of(y[s], a, ba, B),
-                   cz = (uint32_t)cell_of(z[s], a, ba, B);
-    key[s] = (int32_t)(cx | (cy << log2B) | (cz << (2 * log2B)));
+    const float px = x[s], py = y[s], pz = z[s];
+    const uint32_t cx = (uint32_t)cell_of(px, K.a, K.ba, K.B), cy = (uint32_t)cell_of(py, K.a, K.ba, K.B),
+                   cz = (uint32_t)cell_of(pz, K.a, K.ba, K.B);
+    const uint32_t k = cx | (cy << K.log2B) | (cz << (2 * K.log2B));
+    key[s] = (int32_t)k;
+    morton_keys(K, s, px, py, pz, k);
 }
 }  // namespace
 
 // After smoothing moved the points: recompute each point's fine cell and rebuild the Morton search
 // structure (the sorted-space order itself is kept).
 void refresh_search_structure(egt_ctx* h) {
-    const float a = -h->eps, ba = (1.0f + h->eps) - a;
-    k_rekey<<<ceil_div(h->n, BLK), BLK, 0, h->stream>>>(h->x.p, h->y.p, h->z.p, h->n, a, ba, h->B, ilog2(h->B),
-                                                        h->key.p);
+    const MortonKeys K = morton_buffers(h);
+    k_rekey<<<ceil_div(h->n, BLK), BLK, 0, h->stream>>>(h->x.p, h->y.p, h->z.p, h->n, h->key.p, K);
     LAUNCH_CHECK();
     std::vector<uint32_t> rep;
-    build_search_structure(h, rep, nullptr);
+    build_search_structure(h, K, rep, nullptr);
     h->search_stale = false;
 }
 

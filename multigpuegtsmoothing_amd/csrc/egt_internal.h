@@ -289,10 +289,8 @@ struct egt_model_s {
 
 namespace egt {
 // scan / sort / reduce utilities (egt_prims.hip)
-void exclusive_scan_u32(egt_ctx* h, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total_host);
-// Same, with the total written to device memory and no synchronization.
-void exclusive_scan_u32_dev(const uint32_t* in, uint32_t* out, int64_t n, hipStream_t s, Scratch& sc,
-                            uint32_t* total_dev);
+// Exclusive prefix sums of n > 0 values; returns where the total lies in device memory (until the next scan).
+const uint32_t* exclusive_scan_u32(egt_ctx* h, const uint32_t* in, uint32_t* out, int64_t n);
 // Stable sort of (key, value) pairs by the low key_bits bits. With keep_keys false the keys end up undefined.
 void radix_sort_pairs(uint32_t* keys, uint32_t* vals, int64_t n, int key_bits, hipStream_t s, Scratch& sc,
                       bool keep_keys = true);

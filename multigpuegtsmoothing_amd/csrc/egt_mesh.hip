@@ -103,7 +103,7 @@ void run_mesh_adjacency(egt_ctx* h, int k) {
         LAUNCH_CHECK();
     }
     uint32_t total = 0;
-    exclusive_scan_u32(h, cnt, off, n, &total);
+    fetch(h->lane, {{&total, exclusive_scan_u32(h, cnt, off, n), sizeof(total)}});
     int32_t* adj = h->scratch.get<int32_t>(11, std::max<uint32_t>(total, 1));
     HIP_CHECK(hipMemcpyAsync(cnt, off, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
     if (ntri > 0) {

@@ -149,11 +149,12 @@ __global__ void __launch_bounds__(NBLK) k_edges(const int32_t* __restrict__ rowp
     }
 }
 
-__global__ void __launch_bounds__(NBLK) k_edge_sort(const uint32_t* __restrict__ off, int64_t n, uint32_t m,
+__global__ void __launch_bounds__(NBLK) k_edge_sort(const uint32_t* __restrict__ off, int64_t n,
+                                                     const uint32_t* __restrict__ m,
                                                      int32_t* __restrict__ ev, int32_t* __restrict__ eu) {
     const int64_t u = (int64_t)blockIdx.x * NBLK + threadIdx.x;
     if (u >= n) return;
-    const uint32_t b = off[u], e = u + 1 < n ? off[u + 1] : m;
+    const uint32_t b = off[u], e = u + 1 < n ? off[u + 1] : *m;
     if (e - b <= 16) {  // the common case: sorted in registers by a 16-wide bitonic network, padded with INT_MAX
         int32_t r[16];
 #pragma unroll
@@ -195,12 +196,12 @@ __global__ void __launch_bounds__(NBLK) k_edge_sort(const uint32_t* __restrict__
 }
 
 __global__ void __launch_bounds__(NBLK) k_edge_attr(const int32_t* __restrict__ eu, const int32_t* __restrict__ ev,
-                                                     uint32_t m, const float* __restrict__ nx,
+                                                     const uint32_t* __restrict__ m, const float* __restrict__ nx,
                                                      const float* __restrict__ ny, const float* __restrict__ nz,
                                                      uint64_t* __restrict__ ekey, uint8_t* __restrict__ erel,
                                                      float* __restrict__ ew) {
     const uint32_t e = blockIdx.x * NBLK + threadIdx.x;
-    if (e >= m) return;
+    if (e >= *m) return;
     const int32_t u = eu[e], v = ev[e];
     const float dot = __builtin_fmaf(nz[u], nz[v], __builtin_fmaf(ny[u], ny[v], nx[u] * nx[v]));
     const float w = fmaxf(0.0f, 1.0f - __builtin_fabsf(dot));
@@ -492,13 +493,14 @@ __global__ void __launch_bounds__(NBLK) k_orient(int64_t n, const int32_t* __res
 // 8,192; with four launches a round 0.68 -> 0.33 at 20,000, 1.92 -> 1.55 at 1M.
 constexpr int BVS_BLOCK = 1024, BVS_PER = 8, BVS_MAX = BVS_BLOCK * BVS_PER;  // vertices
 constexpr size_t bvs_lds(int64_t n) { return (size_t)n * (sizeof(uint64_t) + 2 * sizeof(uint32_t)); }
-__global__ void __launch_bounds__(BVS_BLOCK) k_bv_small(int n, uint32_t m, const int32_t* __restrict__ eu,
+__global__ void __launch_bounds__(BVS_BLOCK) k_bv_small(int n, const uint32_t* __restrict__ mcount, const int32_t* __restrict__ eu,
                                                          const int32_t* __restrict__ ev,
                                                          const uint64_t* __restrict__ ekey,
                                                          const uint8_t* __restrict__ erel, uint8_t* __restrict__ msf,
                                                          float* __restrict__ nx, float* __restrict__ ny,
                                                          float* __restrict__ nz, uint32_t* __restrict__ trees) {
     extern __shared__ uint64_t lds[];
+    const uint32_t m = *mcount;
     uint64_t* best = lds;
     uint32_t* comp = reinterpret_cast<uint32_t*>(lds + n);  // root << 1 | parity to it
     uint32_t* H = comp + n;                                 // hook word of a root: target << 1 | parity
@@ -613,13 +615,15 @@ __global__ void __launch_bounds__(BVS_BLOCK) k_bv_small(int n, uint32_t m, const
 
 // deterministic forest statistics: per-block partial sums, summed on the host in block order
 __global__ void __launch_bounds__(NBLK) k_msf_stats(const uint8_t* __restrict__ msf, const float* __restrict__ ew,
-                                                     uint32_t m, double* __restrict__ part_w,
+                                                     const uint32_t* __restrict__ mcount, double* __restrict__ part_w,
                                                      uint32_t* __restrict__ part_c) {
     __shared__ double sw[NBLK];
     __shared__ uint32_t scnt[NBLK];
     double w = 0.0;
     uint32_t c = 0;
-    for (uint32_t e = blockIdx.x * NBLK + threadIdx.x; e < m; e += gridDim.x * NBLK)
+    // as many blocks as the edges fill, whatever the launch allowed for: the partial sums stay the same
+    const uint32_t m = *mcount, stride = min(gridDim.x, max(1u, (m + NBLK - 1) / NBLK)) * NBLK;
+    for (uint32_t e = blockIdx.x * NBLK + threadIdx.x; e < m && blockIdx.x * NBLK < stride; e += stride)
         if (msf[e]) {
             w += (double)ew[e];
             ++c;
@@ -690,8 +694,11 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
     HIP_CHECK(hipMemsetAsync(cnt, 0, n * sizeof(uint32_t), s));
     k_edges<0><<<gn, blk, 0, s>>>(h->rowptr.p, h->col.p, h->morder.p, n, cnt, own, lcount, nullptr);
     LAUNCH_CHECK();
-    uint32_t m = 0;
-    exclusive_scan_u32(h, cnt, off, n, &m);
+    // the edges' exact number sizes their arrays, or, where one workgroup builds the forest, the number of columns
+    // does, which spares a trip to the host; the kernels read it where it lies
+    const uint32_t* md = exclusive_scan_u32(h, cnt, off, n);
+    uint32_t m = (uint32_t)h->nnz;
+    if (n > BVS_MAX) fetch(h->lane, {{&m, md, sizeof(m)}});
     HIP_CHECK(hipMemcpyAsync(cnt, off, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
     DBuf<uint8_t> pool;
     const size_t mm = std::max<uint32_t>(m, 1);
@@ -718,16 +725,16 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
 
     k_edges<1><<<gn, blk, 0, s>>>(h->rowptr.p, h->col.p, h->morder.p, n, cnt, own, lcount, ev);
     LAUNCH_CHECK();
-    k_edge_sort<<<gn, blk, 0, s>>>(off, n, m, ev, eu);
+    k_edge_sort<<<gn, blk, 0, s>>>(off, n, md, ev, eu);
     LAUNCH_CHECK();
     const dim3 gm(std::max(1, ceil_div(m, NBLK)));
     if (m > 0) {
-        k_edge_attr<<<gm, blk, 0, s>>>(eu, ev, m, nx, ny, nz, ekey, erel, ew);
+        k_edge_attr<<<gm, blk, 0, s>>>(eu, ev, md, nx, ny, nz, ekey, erel, ew);
         LAUNCH_CHECK();
     }
     uint32_t* trees_d = state + 3;
     if (n <= BVS_MAX) {
-        k_bv_small<<<1, BVS_BLOCK, bvs_lds(n), s>>>((int)n, m, eu, ev, ekey, erel, msf, nx, ny, nz, trees_d);
+        k_bv_small<<<1, BVS_BLOCK, bvs_lds(n), s>>>((int)n, md, eu, ev, ekey, erel, msf, nx, ny, nz, trees_d);
         LAUNCH_CHECK();
     } else {
         // Boruvka with parity. The alive-edge counts live in device memory, so rounds follow one another without a
@@ -779,7 +786,7 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
 
     // statistics
     const int sb = std::min(1024, std::max(1, ceil_div(m, NBLK)));
-    k_msf_stats<<<sb, blk, 0, s>>>(msf, ew, m, part_w, part_c);
+    k_msf_stats<<<sb, blk, 0, s>>>(msf, ew, md, part_w, part_c);
     LAUNCH_CHECK();
     std::vector<double> hw(sb);
     std::vector<uint32_t> hc(sb);

@@ -468,22 +468,11 @@ auto scratch_parts(Scratch& sc) {
 }
 }  // namespace
 
-void exclusive_scan_u32(egt_ctx* h, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total_host) {
-    *total_host = 0;
-    if (n <= 0) return;
+const uint32_t* exclusive_scan_u32(egt_ctx* h, const uint32_t* in, uint32_t* out, int64_t n) {
     DBuf<uint32_t>& tot = part_buf(h->scratch, 3);
     tot.alloc(1);
     scan_rec(in, out, n, h->stream, scratch_parts(h->scratch), 0, tot.p);
-    fetch(h->lane, {{total_host, tot.p, sizeof(uint32_t)}});
-}
-
-void exclusive_scan_u32_dev(const uint32_t* in, uint32_t* out, int64_t n, hipStream_t s, Scratch& sc,
-                            uint32_t* total_dev) {
-    if (n <= 0) {
-        HIP_CHECK(hipMemsetAsync(total_dev, 0, sizeof(uint32_t), s));
-        return;
-    }
-    scan_rec(in, out, n, s, scratch_parts(sc), 0, total_dev);
+    return tot.p;
 }
 
 bool sort_segments(uint32_t* keys, uint32_t* vals, int64_t max_len, int key_bits, const int64_t* seg, int nseg,
