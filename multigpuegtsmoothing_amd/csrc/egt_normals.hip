@@ -85,30 +85,32 @@ __global__ void __launch_bounds__(NBLK) k_pca(const float4* __restrict__ mpts, c
 // CSR row for that and stores the answer in own[], which pass 1 reads). Edges with u = i go to the row's own
 // bucket: one atomic per row reserves them (order within a bucket is free: k_edge_sort sorts it; pass 0 keeps
 // their count per row in lcount[]); only the edges owned by another row (u = nb) take an atomic each.
+// EDGE_LANES lanes share a row, entry by entry: a row's scans of other rows are chains of three dependent loads, and a
+// thread a row ran about four of them one after the other. Normals with 1 / 4 / 8 lanes: 4M-point torus 6.83 / 6.36 /
+// 6.42 ms, cluster mixture 8.23 / 7.68 / 7.71, 100,000 points 0.39 / 0.38 / 0.40.
+constexpr int EDGE_LANES = 4;
 template <int PASS>
 __global__ void __launch_bounds__(NBLK) k_edges(const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
                                                  const int32_t* __restrict__ morder, int64_t n,
                                                  uint32_t* __restrict__ cnt, uint8_t* __restrict__ own,
                                                  uint8_t* __restrict__ lcount, int32_t* __restrict__ ev) {
-    const int64_t m = (int64_t)blockIdx.x * NBLK + threadIdx.x;
-    if (m >= n) return;
-    const int32_t i = morder[m];
-    const int32_t e0 = rowptr[m], e1 = rowptr[m + 1];
-    uint32_t local = 0;  // edges of this row with u = i
-    // the row is walked four entries per step, their loads issued together (indices clamped to the row)
+    const int64_t m = ((int64_t)blockIdx.x * NBLK + threadIdx.x) / EDGE_LANES;
+    const int r = (int)threadIdx.x % EDGE_LANES, g0 = (__lane_id() / EDGE_LANES) * EDGE_LANES;
+    const bool row = m < n;
+    const int32_t i = row ? morder[m] : 0;
+    const int32_t e0 = row ? rowptr[m] : 0, len = row ? rowptr[m + 1] - e0 : 0;
+    // the lanes' flags of one row, as a mask of EDGE_LANES bits
+    auto row_mask = [&](bool f) { return (uint32_t)(__ballot(f) >> g0) & ((1u << EDGE_LANES) - 1u); };
     if (PASS == 0) {
-        for (int32_t e = e0; e < e1; e += 4) {
-            int32_t m2v[4], nbv[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) m2v[u] = col[min(e + u, e1 - 1)];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) nbv[u] = morder[m2v[u]];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (e + u >= e1) continue;
-                const int32_t m2 = m2v[u], nb = nbv[u];
-                bool emit = nb != i;
-                if (emit && i > nb) {
+        uint32_t local = 0;  // edges of this row with u = i
+        for (int b = 0; __ballot(b < len); b += EDGE_LANES) {
+            const bool act = b + r < len;
+            bool emit = false, mine = false;
+            if (act) {
+                const int32_t m2 = col[e0 + b + r], nb = morder[m2];
+                emit = nb != i;
+                mine = emit && nb > i;
+                if (emit && !mine) {
                     bool listed = false;  // does row nb list i? then row nb owns the edge
                     const int32_t f1 = rowptr[m2 + 1];
                     for (int32_t f = rowptr[m2]; f < f1; f += 4) {
@@ -120,31 +122,27 @@ __global__ void __launch_bounds__(NBLK) k_edges(const int32_t* __restrict__ rowp
                     }
                     emit = !listed;
                     if (emit) atomicAdd(&cnt[nb], 1u);
-                } else if (emit) {
-                    ++local;
                 }
-                own[e + u] = emit ? 1 : 0;
+                own[e0 + b + r] = emit ? 1 : 0;
             }
+            local += (uint32_t)__popc(row_mask(mine));
         }
-        lcount[m] = (uint8_t)local;  // a row has at most 64 entries
-        if (local) atomicAdd(&cnt[i], local);
+        if (row && r == 0) {
+            lcount[m] = (uint8_t)local;  // a row has at most 64 entries
+            if (local) atomicAdd(&cnt[i], local);
+        }
     } else {
-        local = lcount[m];
-        uint32_t p = local ? atomicAdd(&cnt[i], local) : 0u;
-        for (int32_t e = e0; e < e1; e += 4) {
-            uint8_t ow[4];
-            int32_t nbv[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) ow[u] = own[min(e + u, e1 - 1)];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) nbv[u] = morder[col[min(e + u, e1 - 1)]];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (e + u >= e1 || !ow[u]) continue;
-                const int32_t nb = nbv[u];
-                if (nb > i) ev[p++] = nb;
-                else ev[atomicAdd(&cnt[nb], 1u)] = i;
-            }
+        const uint32_t local = row ? lcount[m] : 0u;
+        uint32_t p = r == 0 && local ? atomicAdd(&cnt[i], local) : 0u;
+        p = __shfl(p, g0, 64);
+        for (int b = 0; __ballot(b < len); b += EDGE_LANES) {
+            const int32_t e = e0 + b + r;
+            const bool ow = b + r < len && own[e];
+            const int32_t nb = ow ? morder[col[e]] : i;
+            const uint32_t mask = row_mask(nb > i);
+            if (nb > i) ev[p + __popc(mask & ((1u << r) - 1u))] = nb;
+            else if (ow) ev[atomicAdd(&cnt[nb], 1u)] = i;
+            p += (uint32_t)__popc(mask);
         }
     }
 }
@@ -323,11 +321,20 @@ __device__ inline void block_atomic_min(uint64_t* base, int32_t idx, uint64_t va
 // The alive-edge count is read from device memory (*mcount). The edge kernels of a round loop over it with a
 // grid capped at BV_GRID blocks, so a round with few edges left costs a few microseconds, not a launch over
 // the host's stale bound.
+// After the first round the alive edges are 16-byte records of their key (whose low word is the edge) and the roots at
+// their ends, which the merge that keeps them knows: a round then reads each edge in one piece, where an index into
+// the edge arrays led to five more reads, two of them random. Normals of a
+// torus / a cluster mixture: 100,000 points 0.38 -> 0.34 ms, 1M 1.45 -> 1.40, 4M 6.37 -> 6.07 / 7.71 -> 7.24.
 constexpr int BV_GRID = 4096;
+__device__ inline uint4 bv_record(const uint4* __restrict__ alive, uint32_t t, const int32_t* __restrict__ eu,
+                                  const int32_t* __restrict__ ev, const uint64_t* __restrict__ ekey) {
+    if (alive) return alive[t];
+    const uint64_t key = ekey[t];  // first round: every vertex is its own root
+    return make_uint4((uint32_t)key, (uint32_t)(key >> 32), (uint32_t)eu[t], (uint32_t)ev[t]);
+}
 __global__ void __launch_bounds__(NBLK) k_bv_best(const int32_t* __restrict__ eu, const int32_t* __restrict__ ev,
-                                                   const uint64_t* __restrict__ ekey, const uint32_t* __restrict__ alive,
-                                                   const uint32_t* __restrict__ mcount, const int32_t* __restrict__ comp,
-                                                   uint64_t* __restrict__ best) {
+                                                   const uint64_t* __restrict__ ekey, const uint4* __restrict__ alive,
+                                                   const uint32_t* __restrict__ mcount, uint64_t* __restrict__ best) {
     const uint32_t m = *mcount;
     for (uint32_t t0 = blockIdx.x * NBLK; t0 < m; t0 += gridDim.x * NBLK) {  // block-uniform bound
         const uint32_t t = t0 + threadIdx.x;
@@ -335,11 +342,11 @@ __global__ void __launch_bounds__(NBLK) k_bv_best(const int32_t* __restrict__ eu
         uint64_t key = 0;
         bool act = t < m;
         if (act) {
-            const uint32_t e = alive ? alive[t] : t;
-            cu = comp[eu[e]];
-            cv = comp[ev[e]];
+            const uint4 a = bv_record(alive, t, eu, ev, ekey);
+            cu = (int32_t)a.z;
+            cv = (int32_t)a.w;
             act = cu != cv;
-            key = ekey[e];
+            key = ((uint64_t)a.y << 32) | a.x;
         }
         wave_atomic_min(best, cu, key, act);
         wave_atomic_min(best, cv, key, act);
@@ -397,25 +404,25 @@ __global__ void __launch_bounds__(NBLK) k_bv_jump(int64_t n, const int32_t* __re
 }
 
 // Relabels every vertex to its new root and keeps the edges that still join two components (the rest can never be
-// chosen again) for the next round. The edge half does not wait for the vertex half: a vertex's component word is
-// its old root or already the new one, and H leads from either to the new root. A workgroup filters BV_CHUNK edges
+// chosen again) for the next round, with their new roots. The edge half does not wait for the vertex half: H leads
+// from an old root to the new one. A workgroup filters BV_CHUNK edges
 // at a time and reserves its place in the output with one atomic, so the kept edges stay in id order within a
 // chunk only; the minima do not depend on the order, and runs of equal endpoints survive.
 constexpr int BV_CHUNK = 8 * NBLK;
 __global__ void __launch_bounds__(NBLK) k_bv_merge(int64_t n, int32_t* __restrict__ comp, uint8_t* __restrict__ par,
                                                     const uint32_t* __restrict__ H, uint64_t* __restrict__ best,
                                                     const int32_t* __restrict__ eu, const int32_t* __restrict__ ev,
-                                                    const uint32_t* __restrict__ alive,
-                                                    const uint32_t* __restrict__ mcount, uint32_t* __restrict__ out,
+                                                    const uint64_t* __restrict__ ekey, const uint4* __restrict__ alive,
+                                                    const uint32_t* __restrict__ mcount, uint4* __restrict__ out,
                                                     uint32_t* __restrict__ out_count, int vblocks) {
     __shared__ uint32_t wcount[NBLK / 64][8];
     __shared__ uint32_t base;
     if ((int)blockIdx.x < vblocks) {
         const int64_t v = (int64_t)blockIdx.x * NBLK + threadIdx.x;
         if (v >= n) return;
-        const uint32_t w = H[__hip_atomic_load(&comp[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)];
+        const uint32_t w = H[comp[v]];
         const int32_t root = (int32_t)(w >> 1);
-        __hip_atomic_store(&comp[v], root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        comp[v] = root;
         par[v] ^= (uint8_t)(w & 1u);
         if (root == (int32_t)v) best[v] = KEY_EMPTY;
         return;
@@ -424,22 +431,19 @@ __global__ void __launch_bounds__(NBLK) k_bv_merge(int64_t n, int32_t* __restric
     const int lane = __lane_id(), wid = threadIdx.x / 64;
     const uint32_t nblk = gridDim.x - (uint32_t)vblocks;
     for (uint32_t t0 = (blockIdx.x - (uint32_t)vblocks) * BV_CHUNK; t0 < m; t0 += nblk * BV_CHUNK) {
-        uint32_t ed[8];
+        uint4 ed[8];
         uint64_t keep[8];
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
             const uint32_t t = t0 + r * NBLK + threadIdx.x;
-            ed[r] = t < m ? (alive ? alive[t] : t) : 0u;
+            ed[r] = bv_record(alive, min(t, m - 1), eu, ev, ekey);
         }
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
             const uint32_t t = t0 + r * NBLK + threadIdx.x;
-            bool k = false;
-            if (t < m) {
-                const int32_t cu = __hip_atomic_load(&comp[eu[ed[r]]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const int32_t cv = __hip_atomic_load(&comp[ev[ed[r]]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                k = (H[cu] >> 1) != (H[cv] >> 1);
-            }
+            ed[r].z = H[ed[r].z] >> 1;
+            ed[r].w = H[ed[r].w] >> 1;
+            const bool k = t < m && ed[r].z != ed[r].w;
             keep[r] = __ballot(k);
             if (lane == 0) wcount[wid][r] = (uint32_t)__popcll(keep[r]);
         }
@@ -493,7 +497,8 @@ __global__ void __launch_bounds__(NBLK) k_orient(int64_t n, const int32_t* __res
 // 8,192; with four launches a round 0.68 -> 0.33 at 20,000, 1.92 -> 1.55 at 1M.
 constexpr int BVS_BLOCK = 1024, BVS_PER = 8, BVS_MAX = BVS_BLOCK * BVS_PER;  // vertices
 constexpr size_t bvs_lds(int64_t n) { return (size_t)n * (sizeof(uint64_t) + 2 * sizeof(uint32_t)); }
-__global__ void __launch_bounds__(BVS_BLOCK) k_bv_small(int n, const uint32_t* __restrict__ mcount, const int32_t* __restrict__ eu,
+__global__ void __launch_bounds__(BVS_BLOCK) k_bv_small(int n, const uint32_t* __restrict__ mcount,
+                                                         const int32_t* __restrict__ eu,
                                                          const int32_t* __restrict__ ev,
                                                          const uint64_t* __restrict__ ekey,
                                                          const uint8_t* __restrict__ erel, uint8_t* __restrict__ msf,
@@ -692,7 +697,8 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
     uint8_t* own = h->scratch.get<uint8_t>(11, std::max<int64_t>(h->nnz, 1) + n);
     uint8_t* lcount = own + std::max<int64_t>(h->nnz, 1);  // per Morton position: edges the row owns
     HIP_CHECK(hipMemsetAsync(cnt, 0, n * sizeof(uint32_t), s));
-    k_edges<0><<<gn, blk, 0, s>>>(h->rowptr.p, h->col.p, h->morder.p, n, cnt, own, lcount, nullptr);
+    const dim3 ge(ceil_div(n, NBLK / EDGE_LANES));
+    k_edges<0><<<ge, blk, 0, s>>>(h->rowptr.p, h->col.p, h->morder.p, n, cnt, own, lcount, nullptr);
     LAUNCH_CHECK();
     // the edges' exact number sizes their arrays, or, where one workgroup builds the forest, the number of columns
     // does, which spares a trip to the host; the kernels read it where it lies
@@ -702,7 +708,7 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
     HIP_CHECK(hipMemcpyAsync(cnt, off, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
     DBuf<uint8_t> pool;
     const size_t mm = std::max<uint32_t>(m, 1);
-    pool.alloc(mm * (4 + 4 + 8 + 1 + 1 + 4 + 8) + (size_t)n * (4 + 1 + 8 + 4 + 8 + 8) + 24 * 256 + 4096 * 12);
+    pool.alloc(mm * (4 + 4 + 8 + 1 + 1 + 4 + 32) + (size_t)n * (4 + 1 + 8 + 4 + 8 + 8) + 24 * 256 + 4096 * 12);
     size_t po = 0;
     int32_t* ev = dalloc<int32_t>(pool, po, mm);
     int32_t* eu = dalloc<int32_t>(pool, po, mm);
@@ -716,14 +722,14 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
     uint32_t* H = dalloc<uint32_t>(pool, po, n);
     uint64_t* tmin = dalloc<uint64_t>(pool, po, n);
     uint64_t* best1 = dalloc<uint64_t>(pool, po, n);
-    uint32_t* alive_a = dalloc<uint32_t>(pool, po, mm);
-    uint32_t* alive_b = dalloc<uint32_t>(pool, po, mm);
+    uint4* alive_a = dalloc<uint4>(pool, po, mm);
+    uint4* alive_b = dalloc<uint4>(pool, po, mm);
     uint32_t* state = dalloc<uint32_t>(pool, po, 4);  // hook-walk overflow, alive-edge counts (two), trees
     double* part_w = dalloc<double>(pool, po, 1024);
     uint32_t* part_c = dalloc<uint32_t>(pool, po, 1024);
     if (po > pool.n) throw ArgError{EGT_ERR_STATE, "normals pool overflow"};
 
-    k_edges<1><<<gn, blk, 0, s>>>(h->rowptr.p, h->col.p, h->morder.p, n, cnt, own, lcount, ev);
+    k_edges<1><<<ge, blk, 0, s>>>(h->rowptr.p, h->col.p, h->morder.p, n, cnt, own, lcount, ev);
     LAUNCH_CHECK();
     k_edge_sort<<<gn, blk, 0, s>>>(off, n, md, ev, eu);
     LAUNCH_CHECK();
@@ -749,18 +755,18 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
         while ((1ll << first_look) < n) ++first_look;
         first_look = (int)(first_look / 2.4);
         uint32_t* count[2] = {state + 2, state + 1};  // alive edges, this round and next; state[0]: overflow flag
-        uint32_t* alive = nullptr;                    // null = all edges
+        uint4* alive = nullptr;                       // null = all edges
         uint32_t bound = m;                           // host-side upper bound of the alive count
         for (int round = 0; round < 64 && bound > 0; ++round) {
             const int gb = std::min(BV_GRID, std::max(1, ceil_div(bound, NBLK)));
-            const int ge = std::min(BV_GRID, std::max(1, ceil_div(bound, BV_CHUNK)));
-            k_bv_best<<<gb, blk, 0, s>>>(eu, ev, ekey, alive, count[0], comp, best);
+            const int gm2 = std::min(BV_GRID, std::max(1, ceil_div(bound, BV_CHUNK)));
+            k_bv_best<<<gb, blk, 0, s>>>(eu, ev, ekey, alive, count[0], best);
             k_bv_hook<<<gn, blk, 0, s>>>(n, eu, ev, erel, comp, par, best, H, msf, round == 0 ? best1 : nullptr,
                                          count[1]);
             k_bv_jump<<<gn, blk, 0, s>>>(n, comp, H, state);
-            uint32_t* out = alive == alive_a ? alive_b : alive_a;
-            k_bv_merge<<<(int)gn.x + ge, blk, 0, s>>>(n, comp, par, H, best, eu, ev, alive, count[0], out, count[1],
-                                                     (int)gn.x);
+            uint4* out = alive == alive_a ? alive_b : alive_a;
+            k_bv_merge<<<(int)gn.x + gm2, blk, 0, s>>>(n, comp, par, H, best, eu, ev, ekey, alive, count[0], out,
+                                                       count[1], (int)gn.x);
             LAUNCH_CHECK();
             alive = out;
             std::swap(count[0], count[1]);
