@@ -1220,13 +1220,24 @@ void launch_wave(KnnParams P, hipStream_t s) {
 //   mixture  k=40         5.46 / 2.04                                  14.4 / 12.9    27.6 / 27.6   57.0 / 61.7
 // Dense clusters make costly lanes, so an uneven cloud gains up to larger sizes: uneven is a cloud whose fullest
 // cell of 8 fine cells a side holds 64 times the mean of the non-empty ones (sphere and torus: up to 6 times,
-// mixture: over 200 times). Above 40 keys the wave wins on every cloud. Learned starts keep the lane shape at smaller
-// sizes (16M-point mixture, k=40: 61.4 / 66.4; 4M-point torus 8.6 / 9.6), and so do the mixed clouds of a batch
-// (192 clouds, k=40: 32.7 / 36.5).
+// mixture: over 200 times). Above 40 keys the wave wins on every cloud. Mixed clouds of a batch keep the lane shape at
+// smaller sizes (192 clouds, k=40: 32.7 / 36.5), and so do learned starts, by level and bound at the proposed level
+// and one coarser (lane / wave, lane / wave):
+//                  100,000                   600,000                   4M                        16M
+//   torus    k=8   0.26 / 0.21, 0.20 / 0.21  0.51 / 0.88, 0.47 / 0.92
+//   torus    k=16  0.26 / 0.21, 0.31 / 0.22  0.68 / 0.97, 0.72 / 1.16  5.33 / 6.26, 4.33 / 7.68
+//   torus    k=24                            0.89 / 1.04, 1.10 / 1.26
+//   torus    k=40  0.45 / 0.24, 0.51 / 0.29  1.31 / 1.15, 1.45 / 1.45  10.2 / 8.0, 8.6 / 9.7
+//   mixture  k=8   0.84 / 0.26, 0.80 / 0.30  1.29 / 1.05, 0.97 / 1.18  5.86 / 6.65, 4.55 / 7.17
+//   mixture  k=16  1.77 / 0.29, 1.92 / 0.36  1.61 / 1.22, 1.58 / 1.55  6.66 / 7.00, 6.02 / 8.80  24.9 / 27.5, 24.3 / 35.1
+//   mixture  k=24                            1.96 / 1.45, 2.97 / 1.93  8.74 / 8.64, 9.71 / 10.5  33.8 / 35.1, 39.2 / 47.7
+//   mixture  k=40  4.26 / 0.45, 3.94 / 0.57  4.82 / 2.33, 4.94 / 3.65  12.3 / 11.4, 17.9 / 17.1  47.7 / 50.9, 61.0 / 65.9
 enum class Density { even, uneven, mixed };
 bool wave_by_size(int K, int64_t queries, Density d, bool learned) {
     if (K >= 48) return true;
-    if (d == Density::mixed || learned) return queries <= (K <= 16 ? 80000 : 250000);
+    if (d == Density::mixed) return queries <= (K <= 16 ? 80000 : 250000);
+    if (learned && d == Density::even) return queries <= (K <= 16 ? 100000 : K <= 24 ? 250000 : 600000);
+    if (learned) return queries <= (K <= 8 ? 300000 : K <= 16 ? 500000 : K <= 24 ? 2000000 : 6000000);
     if (d == Density::uneven)
         return queries <= (K <= 8 ? 800000 : K <= 16 ? 1500000 : K <= 24 ? 3000000 : K <= 32 ? 6000000 : 8000000);
     return K >= 32 || queries <= (K <= 8 ? 100000 : K <= 16 ? 120000 : 300000);

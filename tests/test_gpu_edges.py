@@ -230,3 +230,21 @@ def test_batch_sorts_at_form_limits(egt_mod, oracle_mod, sizes):
         np.testing.assert_array_equal(b.GetKNNIndexes(c), g.GetKNNIndexes(), err_msg=f"smoothed cloud {c}")
         g.close()
     b.close()
+
+
+@pytest.mark.parametrize("shape,n,k", [("torus", 99_968, 16), ("torus", 100_033, 16), ("mixture", 299_968, 8),
+                                       ("mixture", 300_033, 8)])
+def test_learned_search_at_shape_limits(egt_mod, oracle_mod, shape, n, k):
+    """Sizes at the limits of the launch-shape rule of a learned search, even and uneven clouds."""
+    E, O = egt_mod, oracle_mod
+    print(shape, "n", n, "k", k, flush=True)
+    pts = getattr(D, shape)(n, seed=41)
+    g = E.GridStructure(pts, 1, 1e-6, 1024, 4)
+    model = E.RadiusModel(seed=4)
+    model.propose(g, k)
+    g.set_option(E.OPT_LEARNED_MODE, 3)
+    g.GRIDCUDAKNNSELF_COMPACT(k, 1e8)
+    og = O.Grid(*pts)
+    np.testing.assert_array_equal(g.GetKNNIndexes(), og.to_original(og.knn(k)[0]))
+    g.close()
+    model.close()
