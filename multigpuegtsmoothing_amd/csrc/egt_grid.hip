@@ -172,7 +172,7 @@ __device__ inline int f2o(float f) {
 // the loads of a group in flight together. Rounds that lie in the running cloud fold into registers; where the cloud
 // changes the wave reduces what it holds and one lane sends it, and a round that straddles clouds sends its points one
 // by one. (With 16 points a thread, a stride of the block apart, a block of small clouds straddled in every thread:
-// 110 us for 24 clouds of 100,000 points in all, the longest step of their build; now 17, and 140 for 20M points in
+// 110 us for 24 clouds of 38,000 points in all, the longest step of their build; now 17, and 140 for 20M points in
 // 192 clouds, 560 with one group a wave.)
 constexpr int MM_ROUNDS = 4;
 __device__ inline void minmax_flush(int* __restrict__ mm, int c, const float (&v)[6]) {
@@ -632,7 +632,7 @@ struct Report {
 Report report_of(const egt_ctx* h) { return Report{h->nclouds, ilog2(h->B) + 1}; }
 
 // Points of the largest cloud: where they fit a workgroup's sort, each cloud is sorted by one, in one launch (24 clouds
-// of 100,000 points in all: 22 launches of passes over all points before).
+// of 38,000 points in all: 22 launches of passes over all points before).
 int64_t max_cloud(const egt_ctx* h) {
     int64_t m = 0;
     for (const CloudDev& c : h->clouds) m = std::max(m, c.n);

@@ -167,9 +167,9 @@ struct WorkClass {
     int64_t first, count;
 };
 
-// Reusable temporaries: 0-2 scan partials, 3 scan total, 4-7 radix sort, 8-15 stage code (15 = k-th
-// distance of the last search), 16 host-input staging, 17-23 EGG / Taubin, 24-26 learned proposal,
-// 27-31 Taubin sliced-ELLPACK tiles, 32-35 query-vs-reference search, 36 64-bit totals, 37 queries handed
+// Reusable temporaries: 0-2 scan partials, 3 scan total, 4-7 radix sort, 8-15 stage code (14 = search
+// statistics, 15 = k-th distance of the last search), 16 host-input staging, 17-23 EGG / Taubin (22, 23 also the
+// exchange and flags of the resident passes), 24-26 learned proposal, 27-31 Taubin sliced-ELLPACK tiles, 32-35 query-vs-reference search, 36 64-bit totals, 37 queries handed
 // back by a bounded kNN search, 38 the level tables' cell starts.
 struct Scratch {
     DBuf<uint32_t> bufs[39];

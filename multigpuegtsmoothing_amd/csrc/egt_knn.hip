@@ -20,7 +20,7 @@
 //
 // Two launch shapes run this search: one lane per query (k_knn, the list in the lane's registers) and one
 // wave per query (k_knn_wave, the list spread over the lanes, one key per lane), chosen per neighbour-count
-// class by the options or the tuners below. A lane-per-query search hands queries that exceed a candidate
+// class by the options or the tuners below, else by size (wave_by_size). A lane-per-query search hands queries that exceed a candidate
 // cap, and queries with fewer than k points inside a learned radius bound, to a wave-per-query pass.
 #include <algorithm>
 #include <mutex>
