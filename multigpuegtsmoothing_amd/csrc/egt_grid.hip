@@ -858,7 +858,8 @@ void build_search_structure(egt_ctx* h, const MortonKeys& K, std::vector<uint32_
         // a wave's search waits for its longest probe chain. Search, us, twice everywhere -> eight times on coarse
         // levels: torus 1M k=16 1122 -> 1047, 16M k=40 32300 -> 31890; mixture 4M k=40 12976 -> 12776, 16M 57136 ->
         // 55434; builds unchanged (eight times on all levels: the same searches, builds 3-10% slower).
-        const uint64_t room = by_bound || 4 * cells > (uint64_t)n ? 2 : 8;
+        // (A slot is a 32-bit number: beyond 2^28 cells there is no room for eight.)
+        const uint64_t room = by_bound || 4 * cells > (uint64_t)n || cells > (1ull << 28) ? 2 : 8;
         uint32_t log2cap = 6;
         while ((1ull << log2cap) < room * cells) ++log2cap;
         h->lev[l].log2cap = li.log2cap[l] = log2cap;
