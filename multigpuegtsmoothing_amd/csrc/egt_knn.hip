@@ -103,7 +103,8 @@ struct KnnParams {
     const float4* __restrict__ qpts;       // query search: queries in Morton order (x', y', z', bits(index))
     const unsigned long long* __restrict__ qvcell;  // query search: virtual cell, clamped to the grid
     int64_t nchunks;   // chunks in the work list (after sampling)
-    int qpw;           // wave-per-query search: queries a wave serves one after another (1, 2, 4, 8 or 16)
+    int qpw;           // wave-per-query search: queries a wave serves one after another (1, 2 or 4)
+    int64_t first;     // wave-per-query search: the launch's first chunk (of a list: its first workgroup)
     int stride;        // 1 = every chunk; s > 1 = every s-th chunk of the list (sampled trial runs)
     int B, log2B, stages, maxc;
     int Bv;            // cells per axis at internal level 0 (B << SUB)
@@ -797,15 +798,15 @@ __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) 
     __shared__ int wmark[KBLK / 64][64];  // per wave: the entry whose run starts at each slot of a batch
     int64_t m0, m1;
     if (LIST) {
-        m0 = (v * (KBLK / 64) + wv_id) * P.qpw;
+        m0 = ((P.first + v) * (KBLK / 64) + wv_id) * P.qpw;
         m1 = min<int64_t>(m0 + P.qpw, P.nlist);
     } else {
         const int per = 16 / P.qpw;  // workgroups per chunk of 64 queries
-        const int64_t chunk = v / per;
+        const int64_t chunk = P.first + v / per;
         if (chunk >= P.nchunks) return;
         const int64_t start = P.chunks ? P.chunks[chunk * P.stride] : chunk * P.stride * 64;
         const CloudDev& c0 = P.clouds[P.mcloud ? (uint32_t)P.mcloud[start] : 0u];
-        m0 = start + ((v - chunk * per) * (KBLK / 64) + wv_id) * P.qpw;
+        m0 = start + ((v - (chunk - P.first) * per) * (KBLK / 64) + wv_id) * P.qpw;
         m1 = min<int64_t>(m0 + P.qpw, c0.base + c0.n);
     }
     uint64_t ncand = 0;
@@ -1188,18 +1189,16 @@ void launch_any(const KnnParams& P, int K, hipStream_t s, bool query = false, bo
     }
 }
 
-// Queries a wave of the wave-per-query search serves one after another. More of them reuse the ranges of the last
-// box, fewer give more waves: a 10,000-point torus at k=40 0.105 ms with one query a wave against 0.117, 0.169 and
-// 0.513 with 2, 4 and 16; 150,000 points 0.958, 0.939, 0.965 and 1.194; 1.5M points 6.93, 6.65, 6.57 and 6.78;
-// 16M points (4 and 16) 52.1 and 53.3, a 16M-point cluster mixture 67.7 and 70.5.
-int queries_per_wave(int64_t queries) { return queries < 100000 ? 1 : queries < 300000 ? 2 : 4; }
-
 // Wave-per-query search of P.nchunks chunks of 64 queries.
 template <bool QUERY>
 void launch_wave(KnnParams P, hipStream_t s) {
     P.qpw = queries_per_wave(P.nchunks * 64);
-    hipLaunchKernelGGL((k_knn_wave<false, QUERY>), dim3((unsigned)(P.nchunks * (16 / P.qpw))), dim3(KBLK), 0, s, P);
-    LAUNCH_CHECK();
+    in_launches(P.nchunks, wave_chunks_per_launch(P.qpw), [&](int64_t first, int64_t chunks) {
+        P.first = first;
+        hipLaunchKernelGGL((k_knn_wave<false, QUERY>), dim3((unsigned)(chunks * wave_groups_per_chunk(P.qpw))),
+                           dim3(KBLK), 0, s, P);
+        LAUNCH_CHECK();
+    });
 }
 
 // Launch shape of a search of `queries` queries in class K where nothing asks for one: a lane per query leaves the
@@ -1313,9 +1312,11 @@ int64_t search_class(egt_ctx* h, KnnParams P, int K, hipStream_t s, int shape) {
     R.stride = 1;
     if (P.long_cap || shape == 2) {
         R.qpw = queries_per_wave((int64_t)nb);
-        hipLaunchKernelGGL((k_knn_wave<true, false>), dim3((unsigned)ceil_div((int64_t)nb, KBLK / 64 * R.qpw)),
-                           dim3(KBLK), 0, s, R);
-        LAUNCH_CHECK();
+        in_launches(ceil_div((int64_t)nb, KBLK / 64 * R.qpw), MAX_GROUPS, [&](int64_t first, int64_t groups) {
+            R.first = first;
+            hipLaunchKernelGGL((k_knn_wave<true, false>), dim3((unsigned)groups), dim3(KBLK), 0, s, R);
+            LAUNCH_CHECK();
+        });
     } else {
         R.nchunks = ((int64_t)nb + 63) / 64;
         launch_any(R, K, s, false, true);

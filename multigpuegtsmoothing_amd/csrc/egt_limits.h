@@ -1,9 +1,13 @@
-// Size limits of the library's 32-bit index spaces (host-only, no HIP: the CPU tests compile it with g++).
+// Size limits of the library's 32-bit index spaces and of its launches (host-only, no HIP: the CPU tests compile it
+// with g++).
 //
 // The EGG-kept adjacency is a CSR with int32 row offsets (Taubin, PCA and the normals' edge list index it
 // with int32), and a mesh's corner lists (two entries per triangle corner) use uint32 offsets. A count past
 // these limits would wrap and make the kernels index out of bounds, so the entry points refuse it with
 // EGT_ERR_UNSUPPORTED instead.
+//
+// A launch's threads are a 32-bit count: HIP refuses 2^32 and more. Kernels with several threads per point reach that
+// before the point count's own limit of 2^31 - 1, so their work goes out in as many launches as it takes.
 #pragma once
 #include <cstdint>
 
@@ -25,5 +29,24 @@ inline const char* csr_total_error(uint64_t total) {
 inline const char* mesh_triangles_error(int64_t ntri) {
     return ntri > MESH_MAX_TRIANGLES ? "more than (2^31 - 1) / 6 triangles (int32 corner-list offsets)" : nullptr;
 }
+
+// Workgroups of 256 threads in one launch.
+constexpr int64_t MAX_GROUPS = ((int64_t)1 << 32) / 256 - 1;
+
+// launch(first, count) for consecutive ranges of at most `most` of `items` items.
+template <class Launch>
+void in_launches(int64_t items, int64_t most, Launch&& launch) {
+    for (int64_t first = 0; first < items; first += most) launch(first, items - first < most ? items - first : most);
+}
+
+// Queries a wave of the wave-per-query search serves one after another. More of them reuse the ranges of the last
+// box, fewer give more waves: a 10,000-point torus at k=40 0.105 ms with one query a wave against 0.117, 0.169 and
+// 0.513 with 2, 4 and 16; 150,000 points 0.958, 0.939, 0.965 and 1.194; 1.5M points 6.93, 6.65, 6.57 and 6.78;
+// 16M points (4 and 16) 52.1 and 53.3, a 16M-point cluster mixture 67.7 and 70.5.
+inline int queries_per_wave(int64_t queries) { return queries < 100000 ? 1 : queries < 300000 ? 2 : 4; }
+
+// Its workgroups (four waves) per chunk of 64 queries, and the chunks of one launch.
+inline int wave_groups_per_chunk(int qpw) { return 16 / qpw; }
+inline int64_t wave_chunks_per_launch(int qpw) { return MAX_GROUPS / wave_groups_per_chunk(qpw); }
 
 }  // namespace egt

@@ -1,0 +1,58 @@
+"""Searches whose threads exceed what one launch takes (2^32 - 1): the split on the host, and a query search that
+needs it."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from multigpuegtsmoothing_amd import datasets as D
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def test_launch_split(tmp_path):
+    exe = str(tmp_path / "launch_check")
+    subprocess.run(["g++", "-std=c++17", "-I", os.path.join(ROOT, "multigpuegtsmoothing_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "native", "launch_check.cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0 and r.stdout.strip() == "0", r.stdout
+
+
+@pytest.mark.gpu
+def test_query_search_in_two_launches(egt_mod, oracle_mod):
+    """2^28 + 65 queries at k=41 (a wave per query, 16 threads each): a set of 131,073 queries over and over, whose
+    rows equal the oracle's for one set and repeat for all others."""
+    import torch
+
+    E, O = egt_mod, oracle_mod
+    nq, base, k = (1 << 28) + 65, 131_073, 41
+    if torch.cuda.mem_get_info()[0] < 120e9:
+        pytest.skip("needs 120 GB of free device memory")
+    ref = D.sphere(2_000, seed=43)
+    q = D.sphere(base, seed=44)
+    print("queries", nq, "k", k, flush=True)
+    dq = []
+    for a in q:
+        t = torch.from_numpy(a).cuda()
+        dq.append(t.repeat((nq + base - 1) // base)[:nq].contiguous())
+    torch.cuda.synchronize()
+    g = E.GridStructure(ref, 1, 1e-6, 1024, 4)
+    g.GRIDCUDAKNNCompact(tuple(dq), k, 1e8)
+    ptr, n, kk = g.GetKNNIndexesQueryDevice()
+    assert (n, kk) == (nq, k)
+
+    class View:
+        __cuda_array_interface__ = {"data": (ptr, False), "shape": (nq, k), "typestr": "<i4", "version": 2}
+
+    rows = torch.as_tensor(View(), device="cuda")
+    og = O.Grid(*ref)
+    np.testing.assert_array_equal(rows[:base].cpu().numpy(), og.knn_query(*q, k)[0])
+    for first in range(0, nq, 64 * base):
+        part = rows[first:first + 64 * base]
+        want = rows[:base].repeat((part.shape[0] + base - 1) // base, 1)[:part.shape[0]]
+        assert torch.equal(part, want), f"queries from {first}"
+    del rows, part, want, dq
+    g.close()
+    torch.cuda.empty_cache()
+    E.release_cached_memory()
