@@ -509,8 +509,9 @@ __global__ void __launch_bounds__(BLK) k_level_insert(LevelInsert P, const uint3
                                                        const uint32_t* __restrict__ code,
                                                        const int32_t* __restrict__ mcloud,
                                                        const uint32_t* __restrict__ count, int stride,
-                                                       uint4* __restrict__ tab, LevelDev* __restrict__ lev) {
-    const int64_t i = (int64_t)blockIdx.x * BLK + threadIdx.x;
+                                                       uint4* __restrict__ tab, LevelDev* __restrict__ lev,
+                                                       int64_t first_group) {
+    const int64_t i = (first_group + blockIdx.x) * BLK + threadIdx.x;
     int l = 0;
     for (int j = 1; j < P.nl; ++j) l += i >= P.first[j] ? 1 : 0;
     int cnt = 0;
@@ -872,9 +873,12 @@ void build_search_structure(egt_ctx* h, const MortonKeys& K, std::vector<uint32_
     k_level_init<<<(int)std::min<uint64_t>(1024, (2 * li.slots + BLK - 1) / BLK), BLK, 0, s>>>(
         li, reinterpret_cast<uint64_t*>(h->htab.p), h->dlev.p);
     LAUNCH_CHECK();
-    k_level_insert<<<ceil_div(li.first[nl], BLK), BLK, 0, s>>>(li, starts, n, h->mcode.p, mcl, dtot, nc + 1, h->htab.p,
-                                                               h->dlev.p);
-    LAUNCH_CHECK();
+    // (a batch of very many points has more cells, over all levels, than one launch takes threads)
+    in_launches(ceil_div(li.first[nl], BLK), MAX_GROUPS, [&](int64_t first, int64_t groups) {
+        k_level_insert<<<(unsigned)groups, BLK, 0, s>>>(li, starts, n, h->mcode.p, mcl, dtot, nc + 1, h->htab.p,
+                                                        h->dlev.p, first);
+        LAUNCH_CHECK();
+    });
     if (done) HIP_CHECK(hipEventRecord(done, s));
     read_back(by_bound ? R.words() : R.bad() + 1);
     h->cloud_cells.assign((size_t)nc * nl, 0);

@@ -93,8 +93,9 @@ template <int PASS>
 __global__ void __launch_bounds__(NBLK) k_edges(const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
                                                  const int32_t* __restrict__ morder, int64_t n,
                                                  uint32_t* __restrict__ cnt, uint8_t* __restrict__ own,
-                                                 uint8_t* __restrict__ lcount, int32_t* __restrict__ ev) {
-    const int64_t m = ((int64_t)blockIdx.x * NBLK + threadIdx.x) / EDGE_LANES;
+                                                 uint8_t* __restrict__ lcount, int32_t* __restrict__ ev,
+                                                 int64_t first_group) {
+    const int64_t m = ((first_group + blockIdx.x) * NBLK + threadIdx.x) / EDGE_LANES;
     const int r = (int)threadIdx.x % EDGE_LANES, g0 = (__lane_id() / EDGE_LANES) * EDGE_LANES;
     const bool row = m < n;
     const int32_t i = row ? morder[m] : 0;
@@ -697,9 +698,13 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
     uint8_t* own = h->scratch.get<uint8_t>(11, std::max<int64_t>(h->nnz, 1) + n);
     uint8_t* lcount = own + std::max<int64_t>(h->nnz, 1);  // per Morton position: edges the row owns
     HIP_CHECK(hipMemsetAsync(cnt, 0, n * sizeof(uint32_t), s));
-    const dim3 ge(ceil_div(n, NBLK / EDGE_LANES));
-    k_edges<0><<<ge, blk, 0, s>>>(h->rowptr.p, h->col.p, h->morder.p, n, cnt, own, lcount, nullptr);
-    LAUNCH_CHECK();
+    auto edges = [&](auto kernel, int32_t* out) {
+        in_launches(ceil_div(n, NBLK / EDGE_LANES), MAX_GROUPS, [&](int64_t first, int64_t groups) {
+            kernel<<<(unsigned)groups, blk, 0, s>>>(h->rowptr.p, h->col.p, h->morder.p, n, cnt, own, lcount, out, first);
+            LAUNCH_CHECK();
+        });
+    };
+    edges(k_edges<0>, nullptr);
     // the edges' exact number sizes their arrays, or, where one workgroup builds the forest, the number of columns
     // does, which spares a trip to the host; the kernels read it where it lies
     const uint32_t* md = exclusive_scan_u32(h, cnt, off, n);
@@ -729,8 +734,7 @@ void run_normals(egt_ctx* h, float* nxh, float* nyh, float* nzh) {
     uint32_t* part_c = dalloc<uint32_t>(pool, po, 1024);
     if (po > pool.n) throw ArgError{EGT_ERR_STATE, "normals pool overflow"};
 
-    k_edges<1><<<ge, blk, 0, s>>>(h->rowptr.p, h->col.p, h->morder.p, n, cnt, own, lcount, ev);
-    LAUNCH_CHECK();
+    edges(k_edges<1>, ev);
     k_edge_sort<<<gn, blk, 0, s>>>(off, n, md, ev, eu);
     LAUNCH_CHECK();
     const dim3 gm(std::max(1, ceil_div(m, NBLK)));

@@ -32,7 +32,8 @@ int main() {
     check(1, egt::MAX_GROUPS, 1, true);
     check(egt::MAX_GROUPS, egt::MAX_GROUPS, 1, true);
     check(egt::MAX_GROUPS + 1, egt::MAX_GROUPS, 1, false);
-    check((int64_t)11 * INT32_MAX / 256, egt::MAX_GROUPS, 1, false);
+    check((int64_t)11 * INT32_MAX / 256, egt::MAX_GROUPS, 1, false);  // level inserts: a thread per cell of 11 levels
+    check((int64_t)4 * INT32_MAX / 256, egt::MAX_GROUPS, 1, false);   // edge list: four threads per row
     egt::in_launches(0, egt::MAX_GROUPS, [&](int64_t, int64_t) { ++bad; });
     std::printf("%d\n", bad);
     return bad;
