@@ -77,10 +77,14 @@ def measured_traffic(which="torus"):
     return None
 
 
+def start_option(E, level):
+    """OPT_START_LEVEL value of a level the tuner chose; None: the query's own cell, as in the reference."""
+    return E.START_LEVEL_OWN_CELL if not level else level
+
+
 def gpu_step(E, torch, dev_xyz, args, start_level):
     g = E.GridStructure(dev_xyz, 1, 1e-6, 1024, 4)
-    if start_level is not None:
-        g.set_option(E.OPT_START_LEVEL, start_level)
+    g.set_option(E.OPT_START_LEVEL, start_option(E, start_level))
     if args.no_graph:
         g.set_option(E.OPT_TAUBIN_GRAPH, 0)
     g.GRIDCUDAKNNSELF_COMPACT(args.k, 1e8)
@@ -116,10 +120,9 @@ def learned_vs_plain(E, dev_xyz, args, start_level=None):
     modes = ("plain", "learned") + (("autotuned",) if start_level is not None else ())
     for mode in modes:
         g = E.GridStructure(dev_xyz, 1, 1e-6, 1024, 4)
-        if mode == "autotuned":
-            g.set_option(E.OPT_START_LEVEL, start_level)
+        g.set_option(E.OPT_START_LEVEL, start_option(E, start_level if mode == "autotuned" else None))
         if mode == "learned":
-            g.set_option(E.OPT_KNN_LANES, 64 if lshape == 2 else 1)
+            g.set_option(E.OPT_KNN_CLASS_SHAPES, E.class_shapes_all(lshape))
         best = None
         for _ in range(3):
             prop = 0.0
@@ -299,8 +302,7 @@ def mixture_main(args):
                 g = E.GridStructure(dev, 1, 1e-6, 1024, 4)
                 if mode == "learned":
                     model.propose(g, k)
-                if mode == "autotuned":
-                    g.set_option(E.OPT_START_LEVEL, lvl)
+                g.set_option(E.OPT_START_LEVEL, start_option(E, lvl if mode == "autotuned" else None))
                 g.GRIDCUDAKNNSELF_COMPACT(k, 1e8)
                 r = g.GetKNNIndexesDevice()
                 E.EGT_CUDA(g).PerformSmoothing(iters, 0.5, -0.53, 0.65)
@@ -379,8 +381,8 @@ def batch_result(args, steps, warmup, per_cloud=True):
     from {16, 40, 64}, alpha 0.65, 100 iterations (lambda 0.5, mu -0.53). One step = batch build (cube, sort,
     cell tables for all clouds) + (learned proposal) + kNN (one launch per neighbour-count class over 64-query
     chunks) + EGG + Taubin (one captured graph over all clouds). Coordinates are resident in HBM before timing.
-    The learned batch (model trained on the GPU on 64 clouds of other seeds) and the plain batch (every query
-    from its own cell), each with the kNN launch shape per neighbour-count class that the class tuner picks
+    The learned batch (model trained on the GPU on 64 clouds of other seeds) and the plain batch (the library's
+    start levels), each with the kNN launch shape per neighbour-count class that the class tuner picks
     for it (outside the timing), are each timed over `steps` steps; beside them, when per_cloud, the plain GPU path of
     the reference interface (one handle per cloud, plain search, EGG, Taubin, cloud after cloud), timed once
     after a warm-up pass."""
@@ -471,7 +473,7 @@ def batch_result(args, steps, warmup, per_cloud=True):
                for ci in range(8) if (packed >> (2 * ci)) & 3}
                for path, (packed, ms) in (("learned", shapes[True]), ("plain", shapes[False]))}}
     if per_cloud:
-        # The plain GPU path on the same clouds: one GridStructure per cloud, the plain (own-cell) search, EGG
+        # The plain GPU path on the same clouds: one GridStructure per cloud, the plain search as it comes, EGG
         # and Taubin, cloud after cloud (what a caller of the reference's interface does with many clouds).
         offs = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
 
@@ -627,7 +629,7 @@ def mixture_modes(args, k=40, steps=5, warmup=2):
     lvl = int(g.autotune(k)[0])
     # launch shape (lane per query / persistent / wave per query) for the tuned level and for the learned
     # starts, each timed on the tuner's sample, outside the timed steps
-    g.set_option(E.OPT_START_LEVEL, lvl)
+    g.set_option(E.OPT_START_LEVEL, start_option(E, lvl))
     shapes = {"plain_own_cell": (0, None), "plain_autotuned": g.autotune_shape(k)}
     g.close()
     # the learned path: level offset, the proposal's level alone or with its radius bound, and the shape,
@@ -651,10 +653,8 @@ def mixture_modes(args, k=40, steps=5, warmup=2):
                 model.propose(g, k)
                 g.set_option(E.OPT_LEARNED_MODE, learned_mode)
                 g.set_option(E.OPT_LEARNED_LEVEL_OFFSET, level_offset)
-            elif mode == "plain_autotuned":
-                g.set_option(E.OPT_START_LEVEL, lvl)
-            g.set_option(E.OPT_KNN_PERSISTENT, 1 if shape == 1 else 0)
-            g.set_option(E.OPT_KNN_LANES, 64 if shape == 2 else 1)
+            g.set_option(E.OPT_START_LEVEL, start_option(E, lvl if mode == "plain_autotuned" else None))
+            g.set_option(E.OPT_KNN_CLASS_SHAPES, E.class_shapes_all(shape))
             g.GRIDCUDAKNNSELF_COMPACT(k, 1e8)
             E.EGT_CUDA(g).PerformSmoothing(iters, 0.5, -0.53, 0.65)
             st = g.stats()

@@ -83,18 +83,22 @@ typedef struct {
 
 /* EGT_OPT_START_LEVEL value: choose the level from the mean cell occupancy. */
 #define EGT_START_LEVEL_OCCUPANCY 127
+/* EGT_OPT_START_LEVEL value: every query's own cell, as in the reference, whatever the cloud. */
+#define EGT_START_LEVEL_OWN_CELL 126
+/* EGT_OPT_KNN_CLASS_SHAPES value: one shape (0, 1 or 2, as the shape tuners report it) for every k. */
+#define EGT_CLASS_SHAPES_ALL(shape) (0x5555 * ((shape) + 1))
 /* Entries of the autotuner's trial arrays: start levels -3 .. 10, entry i = level i - 3. */
 #define EGT_AUTOTUNE_SLOTS 14
 
 /* Options set through egt_set_option (no reference counterpart). */
 typedef enum {
-    EGT_OPT_START_LEVEL = 0,     /* kNN: pyramid level of the first search box; 0 = the query's own cell, as
-                                    in the reference (default; on small clouds and clouds of even density the
-                                    library starts at the occupancy level below instead, unless
-                                    EGT_OPT_KNN_LONG_QUERY is changed or egt_autotune chose the level); > 0
-                                    coarser cells; -1, -2, -3 = cells of 1/2,
-                                    1/4, 1/8 of a grid cell; EGT_START_LEVEL_OCCUPANCY = one level from the
-                                    mean cell occupancy */
+    EGT_OPT_START_LEVEL = 0,     /* kNN: pyramid level of the first search box; 0 = the library's choice
+                                    (default): the occupancy level below on clouds of up to 100,000 points and
+                                    clouds of even density, else the query's own cell;
+                                    EGT_START_LEVEL_OWN_CELL = the query's own cell, as in the reference; > 0
+                                    coarser cells; -1, -2, -3 = cells of 1/2, 1/4, 1/8 of a grid cell;
+                                    EGT_START_LEVEL_OCCUPANCY = one level from the mean cell occupancy. Rows do
+                                    not depend on it */
     EGT_OPT_LEARNED = 1,         /* kNN: 1 = start each query from the learned radius proposal */
     EGT_OPT_TAUBIN_GRAPH = 2,    /* Taubin: 1 = replay the lambda/mu loop as a captured hipGraph (default; clouds of
                                     up to 262,144 points run every pass in one launch), 0 = a launch per pass */
@@ -113,15 +117,16 @@ typedef enum {
                                     inside it are searched again without the bound); default 1 (the level only).
                                     Which is faster depends on the cloud and k (try both with
                                     egt_autotune_shape). Rows do not depend on it */
-    EGT_OPT_KNN_LANES = 8,       /* kNN self search: lanes per query, 1 = one lane per query with the list in its
-                                    registers (default; where that shape leaves the GPU idle or short of
-                                    registers, few queries or k > 40, the library runs a wave per query, unless
-                                    EGT_OPT_KNN_LONG_QUERY is changed, a tuner chose the shape or
-                                    EGT_OPT_KNN_CLASS_SHAPES names it), 64 = one wave per query with the list
-                                    spread over the lanes. Rows do not depend on it */
+    EGT_OPT_KNN_LANES = 8,       /* kNN self search: 1 = the library's choice (default): one lane per query with
+                                    the list in its registers, or one wave per query with the list spread over
+                                    the lanes where a lane per query leaves the GPU idle or short of registers
+                                    (few queries, k > 24 on clouds of even density, k > 40 on all); 64 = one
+                                    wave per query. EGT_OPT_KNN_CLASS_SHAPES names either shape. Rows do not
+                                    depend on it */
     EGT_OPT_KNN_LONG_QUERY = 9,  /* kNN self search with one lane per query: a query that has tested more
                                     candidates than this is handed on to a wave-per-query pass (its wave no
-                                    longer waits for it); 0 = never; default 2048. Rows do not depend on it */
+                                    longer waits for it); 0 = never; default 2048. Setting it asks for a lane
+                                    per query where nothing else names a shape. Rows do not depend on it */
     EGT_OPT_KNN_CLASS_SHAPES = 10, /* kNN self search: launch shape per neighbour-count class (k <= 8, 16, ..,
                                     64 are classes 0..7): bits 2i..2i+1 hold class i's shape + 1 (1 = one lane
                                     per query, 2 = the same as one persistent launch, 3 = one wave per query,
@@ -244,8 +249,9 @@ egt_status egt_release_cached_memory(uint64_t* released, uint64_t* cached);
 /* Autotuner (no reference counterpart): runs the plain search with neighbour count k and radius thres
  * (input units, as egt_grid_knn_self) on an evenly spread sample of queries for each candidate start level
  * (the cell size of the first search box), scores each level by its measured work per query (candidates
- * tested + 3 x cells looked up) and sets EGT_OPT_START_LEVEL to the cheapest. Rows do not depend on the
- * choice. trial_ms and trial_cost (optional, EGT_AUTOTUNE_SLOTS floats each) receive each level's sample time
+ * tested + 3 x cells looked up) and the handle starts at the cheapest. Rows do not depend on the choice.
+ * *start_level (optional) receives it, for later handles: EGT_OPT_START_LEVEL takes it, with
+ * EGT_START_LEVEL_OWN_CELL for level 0. trial_ms and trial_cost (optional, EGT_AUTOTUNE_SLOTS floats each) receive each level's sample time
  * in ms and its score at index level + 3, -1 where untried. The handle's neighbour rows are not valid
  * afterwards: run egt_grid_knn_self. */
 egt_status egt_autotune(egt_handle h, int k, float thres, int32_t* start_level, float* trial_ms,
@@ -255,18 +261,19 @@ egt_status egt_autotune(egt_handle h, int k, float thres, int32_t* start_level, 
  * EGT_OPT_LEARNED, the proposal in place) with neighbour count k and radius thres over all queries in each
  * launch shape: 0 = one lane per query, one workgroup per 256 queries; 1 = one lane per query, one
  * persistent work-queue launch; 2 = one wave per query. Each shape is
- * warmed up on the autotuner's sample, then timed once on the full search; the fastest is kept through
- * EGT_OPT_KNN_PERSISTENT and EGT_OPT_KNN_LANES. Rows do not depend on the choice. *shape (optional) receives
- * it, shape_ms (optional, 3 floats) each shape's time in ms. The handle's neighbour rows
+ * warmed up on the autotuner's sample, then timed once on the full search; the handle keeps the fastest for every
+ * k (until EGT_OPT_KNN_LANES or EGT_OPT_KNN_PERSISTENT is set). Rows do not depend on the choice. *shape
+ * (optional) receives it, for later handles: EGT_OPT_KNN_CLASS_SHAPES with EGT_CLASS_SHAPES_ALL(*shape); shape_ms (optional, 3 floats) each shape's time in ms. The handle's neighbour rows
  * are not valid afterwards: run egt_grid_knn_self. */
 egt_status egt_autotune_shape(egt_handle h, int k, float thres, int32_t* shape, float* shape_ms);
 
 /* Learned-start tuner (no reference counterpart): with a proposal in place (egt_model_propose), times the full
  * search with neighbour count k and radius thres for each level offset (0, +1), each use of the proposal
  * (EGT_OPT_LEARNED_MODE 1 = its level, 3 = its level and radius bound) and each of the lane-per-query and
- * wave-per-query shapes, each after a warm-up on the autotuner's sample, and keeps the fastest through
- * EGT_OPT_LEARNED_LEVEL_OFFSET, EGT_OPT_LEARNED_MODE and EGT_OPT_KNN_LANES. Rows do not depend on the choice.
- * offset, mode, shape (optional) receive it (shape 0 = lane per query, 2 = wave per query); ms (optional, 8
+ * wave-per-query shapes, each after a warm-up on the autotuner's sample, and keeps the fastest. Rows do not depend
+ * on the choice. offset, mode, shape (optional) receive it, for later handles: EGT_OPT_LEARNED_LEVEL_OFFSET,
+ * EGT_OPT_LEARNED_MODE and EGT_OPT_KNN_CLASS_SHAPES with EGT_CLASS_SHAPES_ALL(*shape) (shape 0 = lane per query,
+ * 2 = wave per query); ms (optional, 8
  * floats) the times, index (offset x 2 + (mode == 3)) x 2 + (shape == 2). One-cloud handles. The handle's
  * neighbour rows are not valid afterwards: run egt_grid_knn_self. */
 egt_status egt_autotune_learned(egt_handle h, int k, float thres, int32_t* offset, int32_t* mode, int32_t* shape,

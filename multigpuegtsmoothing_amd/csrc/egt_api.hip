@@ -328,10 +328,10 @@ egt_status egt_set_option(egt_handle h, egt_option opt, int64_t value) {
     if (need(h)) return EGT_ERR_INVALID_ARG;
     switch (opt) {
         case EGT_OPT_START_LEVEL:
-            if (value != EGT_START_LEVEL_OCCUPANCY && (value < -egt::SUB || value >= h->nlev))
+            if (value != EGT_START_LEVEL_OCCUPANCY && value != EGT_START_LEVEL_OWN_CELL &&
+                (value < -egt::SUB || value >= h->nlev))
                 return fail(EGT_ERR_INVALID_ARG, "start level out of range");
             h->start_level = (int)value;
-            h->start_tuned = false;
             return EGT_OK;
         case EGT_OPT_LEARNED:
             h->learned = value ? 1 : 0;
@@ -368,6 +368,7 @@ egt_status egt_set_option(egt_handle h, egt_option opt, int64_t value) {
         case EGT_OPT_KNN_LONG_QUERY:
             if (value < 0 || value > UINT32_MAX) return fail(EGT_ERR_INVALID_ARG, "long-query cap must be in [0, 2^32)");
             h->knn_long_cap = value;
+            h->knn_long_set = true;
             return EGT_OK;
         case EGT_OPT_LEARNED_LEVEL_OFFSET:
             if (value < -3 || value > 3) return fail(EGT_ERR_INVALID_ARG, "learned level offset must be in [-3, 3]");

@@ -248,20 +248,21 @@ struct egt_ctx {
     bool have_query = false;
 
     // options
-    bool start_tuned = false;  // a tuner chose start_level: 0 then means the own cell
-    int start_level = 0;  // reference schedule: every query starts at its own level-0 cell; -SUB..-1 sub-cell
-                          // boxes; EGT_START_LEVEL_OCCUPANCY = from the mean cell occupancy
+    int start_level = 0;  // 0 the library's choice; EGT_START_LEVEL_OWN_CELL the reference schedule: every query
+                          // starts at its own level-0 cell; > 0 coarser; -SUB..-1 sub-cell boxes;
+                          // EGT_START_LEVEL_OCCUPANCY = from the mean cell occupancy
     int learned = 0;
     int learned_mode = 1;  // with learned: 1 = start at the proposed level, 2 = bound the search by the proposed
                            // radius, 3 = both
     int knn_persistent = 0;  // kNN as one persistent work-queue launch per neighbour-count class
-    int knn_lanes = 1;       // kNN self search: 1 = one lane per query, 64 = one wave per query
+    int knn_lanes = 1;       // kNN self search: 1 = by size and density, 64 = one wave per query
     int learned_level_offset = 0;  // added to the proposed start levels
     int class_shape[8] = {-1, -1, -1, -1, -1, -1, -1, -1};  // per neighbour-count class (k <= 8, 16, .., 64):
                                                            // 0 lane, 1 persistent, 2 wave; -1 handle-wide
     bool knn_shape_tuned = false;  // a tuner chose the handle-wide shape: it holds for every size
     int64_t knn_long_cap = egt::KNN_LONG_CAP;  // lane-per-query search: candidates after which a query goes to a wave
                                   // (0 = never)
+    bool knn_long_set = false;  // the cap was set by option: it belongs to the lane shape, which is then asked for
     int taubin_graph = 1;
     int taubin_tile = 1024;  // Taubin tile width: 1024 or 2048 points; 0 = tune on the next smoothing call
     bool taubin_tile_set = false;  // the width was set by option: no other tiling

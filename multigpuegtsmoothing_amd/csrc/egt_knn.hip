@@ -1256,15 +1256,15 @@ bool uneven_cloud(const egt_ctx* h) {
 }
 
 // Launch shape of a neighbour-count class of `queries` queries: the handle's per-class choice (from the class
-// tuner or EGT_OPT_KNN_CLASS_SHAPES), else the handle-wide options, else (one lane per query by default, the long
-// query cap untouched, no shape tuned) the rule above. 0 = one lane per query, 1 = the same as one persistent
-// launch, 2 = one wave per query.
+// tuner or EGT_OPT_KNN_CLASS_SHAPES), else the handle-wide options, else, where nothing asks for a shape (no tuner, no
+// long query cap set), the rule above. 0 = one lane per query, 1 = the same as one persistent launch, 2 = one wave per
+// query.
 int class_shape(const egt_ctx* h, int K, int64_t queries) {
     const int c = h->class_shape[K / 8 - 1];
     if (c >= 0) return c;
     if (h->knn_lanes == 64) return 2;
     if (h->knn_persistent) return 1;
-    if (h->knn_shape_tuned || h->knn_long_cap != KNN_LONG_CAP) return 0;
+    if (h->knn_shape_tuned || h->knn_long_set) return 0;
     const Density d = h->nclouds > 1 ? Density::mixed : uneven_cloud(h) ? Density::uneven : Density::even;
     return wave_by_size(K, queries, d, h->learned != 0) ? 2 : 0;
 }
@@ -1324,9 +1324,8 @@ int64_t search_class(egt_ctx* h, KnnParams P, int K, hipStream_t s, int shape) {
     return (int64_t)nb;
 }
 
-// Where nothing asks for a start level (the option at 0, no tuner, the long query cap untouched), a search of a cloud
-// of even density starts at the occupancy level: from its own cell a query climbs through boxes that cannot hold k
-// points, 27 lookups each. From the own cell / the occupancy level, the search shape of the size, in ms:
+// Where nothing asks for a start level (the option at 0, no tuner), a search of a cloud of even density starts at the
+// occupancy level: from its own cell a query climbs through boxes that cannot hold k points, 27 lookups each. From the own cell / the occupancy level, the search shape of the size, in ms:
 //   sphere  2,000 k=8 0.045 / 0.019    100,000 k=40 0.78 / 0.31    500,000 k=8 1.40 / 0.43    1.5M k=40 6.2 / 3.0
 //   torus   50,000 k=16 0.34 / 0.13    1.5M k=16 3.1 / 1.5    4M k=40 14.3 / 8.2, k=64 18.7 / 10.8    16M k=40 51.5 / 38.7
 //   mixture 2,000 k=40 0.049 / 0.020   50,000 k=16 0.29 / 0.19    150,000 k=40 0.83 / 0.80    500,000 k=40 2.3 / 2.4
@@ -1334,9 +1333,6 @@ int64_t search_class(egt_ctx* h, KnnParams P, int K, hipStream_t s, int shape) {
 // (one level does not fit an uneven cloud, whose dense cells it overfills: beyond START_ANY points such a cloud keeps
 // the own cell, and so do the larger clouds of a batch, whose evenness is not known one by one).
 constexpr int64_t START_ANY = 100000;
-bool own_cell_by_default(const egt_ctx* h) {
-    return h->start_level == 0 && !h->start_tuned && h->knn_long_cap == KNN_LONG_CAP;
-}
 int default_start_level(const egt_ctx* h, int k, int cloud = 0) {
     if (h->clouds[cloud].n > START_ANY && (h->nclouds > 1 || uneven_cloud(h))) return 0;
     return auto_start_level(h, k, cloud);
@@ -1380,11 +1376,14 @@ KnnParams knn_params(egt_ctx* h, int k, bool scratch = true) {
     P.log2B = log2B;
     P.Bv = h->B << SUB;
     P.nlev = h->nlev + SUB;
-    if (own_cell_by_default(h))
+    if (h->start_level == 0)
         P.start_level = h->nclouds > 1 ? -1 : SUB + default_start_level(h, k);
+    else if (h->start_level == EGT_START_LEVEL_OWN_CELL)
+        P.start_level = SUB;
+    else if (h->start_level == EGT_START_LEVEL_OCCUPANCY)
+        P.start_level = SUB + auto_start_level(h, h->clouds[0].k);
     else
-        P.start_level = SUB + (h->start_level == EGT_START_LEVEL_OCCUPANCY ? auto_start_level(h, h->clouds[0].k)
-                                                                             : std::min(h->start_level, h->nlev - 1));
+        P.start_level = SUB + std::min(h->start_level, h->nlev - 1);
     int stages = 0;
     for (int b = h->B; b >= 8; b >>= 1) ++stages;
     P.stages = std::max(stages, 1);
@@ -1859,8 +1858,7 @@ int autotune_start_level(egt_ctx* h, int k, float thres_n, float* trial_ms, floa
             best_cost = cost;
         }
     }
-    h->start_level = best;
-    h->start_tuned = true;
+    h->start_level = best == 0 ? EGT_START_LEVEL_OWN_CELL : best;
     h->have_knn = false;  // the trial rows cover only the sample
     return best;
 }

@@ -27,13 +27,21 @@ STATUS_NAMES = {0: "OK", 1: "INVALID_ARG", 2: "OOM", 3: "HIP_ERROR", 4: "UNSUPPO
 OPT_START_LEVEL, OPT_LEARNED, OPT_TAUBIN_GRAPH, OPT_MAX_PTS_IN_CUBE, OPT_KNN_PERSISTENT, OPT_TAUBIN_TILE = 0, 1, 2, 3, 4, 5
 OPT_TAUBIN_REGULARIZED = 6
 OPT_LEARNED_MODE = 7         # learned proposal: 1 = start level (default), 2 = radius bound, 3 = both
-OPT_KNN_LANES = 8            # kNN self search: 1 = one lane per query (default), 64 = one wave per query
+OPT_KNN_LANES = 8            # kNN self search: 1 = the library's choice (default), 64 = one wave per query
 OPT_KNN_LONG_QUERY = 9       # lane-per-query search: candidates after which a query goes to a wave (2048; 0 = never)
-OPT_KNN_CLASS_SHAPES = 10    # per neighbour-count class launch shapes, as BatchGrid.autotune_shape returns them
+OPT_KNN_CLASS_SHAPES = 10    # per neighbour-count class launch shapes, as BatchGrid.autotune_shape returns them, or
+                             # class_shapes_all(shape)
 OPT_LEARNED_LEVEL_OFFSET = 11  # added to the proposed start levels (-3..3)
-START_LEVEL_OCCUPANCY = 127  # OPT_START_LEVEL value: one level from the mean cell occupancy
+START_LEVEL_OCCUPANCY = 127  # OPT_START_LEVEL values: one level from the mean cell occupancy; every query's own
+START_LEVEL_OWN_CELL = 126   # cell, as in the reference (0, the default, is the library's choice)
 SUB_LEVELS = 3               # start levels -1, -2, -3: boxes of cells 1/2, 1/4, 1/8 of a grid cell
 AUTOTUNE_SLOTS = 14          # autotuner trial arrays: levels -3 .. 10
+
+
+def class_shapes_all(shape):
+    """OPT_KNN_CLASS_SHAPES value: one shape for every k (0 = lane per query, 1 = the same as one persistent launch,
+    2 = wave per query, as autotune_shape and autotune_learned return it)."""
+    return 0x5555 * (shape + 1)
 
 
 class EGTError(RuntimeError):
@@ -295,7 +303,8 @@ class GridStructure(_Provider):
     def autotune(self, k, thres=1e8):
         """Picks the start level with the least measured work per query for this cloud and k, on a sample of
         queries (no reference counterpart). Returns (level, per-level sample times in ms, per-level scores):
-        entry i of the arrays is level i - 3, -1 where untried."""
+        entry i of the arrays is level i - 3, -1 where untried. Later handles take the level through
+        OPT_START_LEVEL (level 0 as START_LEVEL_OWN_CELL)."""
         lvl = ctypes.c_int32()
         ms = np.empty(AUTOTUNE_SLOTS, np.float32)
         cost = np.empty(AUTOTUNE_SLOTS, np.float32)
@@ -305,7 +314,8 @@ class GridStructure(_Provider):
     def autotune_shape(self, k, thres=1e8):
         """Times the current search (start level, learned proposal) in each kNN launch shape over all queries
         and keeps the fastest (no reference counterpart). Returns (shape, ms per shape): 0 = one lane per
-        query, 1 = the same as one persistent launch, 2 = one wave per query."""
+        query, 1 = the same as one persistent launch, 2 = one wave per query. Later handles take the shape
+        through OPT_KNN_CLASS_SHAPES with class_shapes_all(shape)."""
         shape = ctypes.c_int32()
         ms = np.empty(3, np.float32)
         _check(_lib.egt_autotune_shape(self.handle, k, thres, ctypes.byref(shape), ms))
