@@ -132,9 +132,11 @@ typedef enum {
                                     per query, 2 = the same as one persistent launch, 3 = one wave per query,
                                     0 = the handle-wide EGT_OPT_KNN_LANES / EGT_OPT_KNN_PERSISTENT; default 0).
                                     egt_batch_autotune_shape returns such a value. Rows do not depend on it */
-    EGT_OPT_LEARNED_LEVEL_OFFSET = 11 /* kNN with the learned proposal: added to every proposed start level,
+    EGT_OPT_LEARNED_LEVEL_OFFSET = 11, /* kNN with the learned proposal: added to every proposed start level,
                                     -3..3 (default 0; +1 = one level coarser than proposed).
                                     egt_autotune_learned picks it. Rows do not depend on it */
+    EGT_OPT_KNN_QUERY_LANES = 12  /* query search: 1 = one lane per query, 64 = one wave per query, 0 = the
+                                    library's choice by query count and k (default). Rows do not depend on it */
 } egt_option;
 
 const char* egt_last_error_string(void);

@@ -374,6 +374,11 @@ egt_status egt_set_option(egt_handle h, egt_option opt, int64_t value) {
             if (value < -3 || value > 3) return fail(EGT_ERR_INVALID_ARG, "learned level offset must be in [-3, 3]");
             h->learned_level_offset = (int)value;
             return EGT_OK;
+        case EGT_OPT_KNN_QUERY_LANES:
+            if (value != 0 && value != 1 && value != 64)
+                return fail(EGT_ERR_INVALID_ARG, "query lanes must be 0, 1 or 64");
+            h->knn_query_lanes = (int)value;
+            return EGT_OK;
         case EGT_OPT_KNN_CLASS_SHAPES:
             if (value < 0 || value >= (1 << 16)) return fail(EGT_ERR_INVALID_ARG, "class shapes: 8 fields of 2 bits");
             for (int c = 0; c < 8; ++c) h->class_shape[c] = (int)((value >> (2 * c)) & 3) - 1;

@@ -262,6 +262,7 @@ struct egt_ctx {
     bool knn_shape_tuned = false;  // a tuner chose the handle-wide shape: it holds for every size
     int64_t knn_long_cap = egt::KNN_LONG_CAP;  // lane-per-query search: candidates after which a query goes to a wave
                                   // (0 = never)
+    int knn_query_lanes = 0;    // query search: 0 = by query count and k, 1 = one lane per query, 64 = one wave
     bool knn_long_set = false;  // the cap was set by option: it belongs to the lane shape, which is then asked for
     int taubin_graph = 1;
     int taubin_tile = 1024;  // Taubin tile width: 1024 or 2048 points; 0 = tune on the next smoothing call

@@ -1242,13 +1242,16 @@ bool wave_by_size(int K, int64_t queries, Density d, bool learned) {
     return K >= 32 || queries <= (K <= 8 ? 100000 : K <= 16 ? 120000 : 300000);
 }
 
-// The query search's shape. Up to QUERY_UNSORTED queries go to a wave each in their own order: the sort that makes
+// The query search's shape where EGT_OPT_KNN_QUERY_LANES names none. Up to QUERY_UNSORTED queries go to a wave each in their own order: the sort that makes
 // neighbours of a wave's queries is a dozen launches, which cost more than the locality gives. Lane / wave sorted /
 // wave unsorted in ms: 300 queries at k=1 in a 100,000-point sphere 0.37 / 0.090 / 0.030; in a 1M to 4M-point torus
 // 16,000 at k=16 0.67 / 0.18 / 0.087, 60,000 at k=1 0.45 / 0.28 / 0.16 and at k=40 1.05 / 0.45 / 0.33; 250,000 at
 // k=16 0.84 / 1.25 (a lane per query wins), at k=40 1.82 / 1.50.
 constexpr int64_t QUERY_UNSORTED = 100000;
-bool query_by_wave(int K, int64_t nq) { return nq <= QUERY_UNSORTED || wave_by_size(K, nq, Density::even, false); }
+bool query_by_wave(const egt_ctx* h, int K, int64_t nq) {
+    if (h->knn_query_lanes) return h->knn_query_lanes == 64;
+    return nq <= QUERY_UNSORTED || wave_by_size(K, nq, Density::even, false);
+}
 
 bool uneven_cloud(const egt_ctx* h) {
     const LevelTable& L = h->lev[std::min(3, h->nlev - 1)];
@@ -1517,7 +1520,7 @@ void run_knn_query(egt_ctx* h, const float* dqx, const float* dqy, const float* 
     qcd.k = k;
     qcd.thres_n = thres_n;
     const int K = kclass(k);
-    const bool wave = query_by_wave(K, nq);
+    const bool wave = query_by_wave(h, K, nq);
     if (nq > 0) {
         const int g = ceil_div(nq, KBLK);
         h->dqcloud.alloc(1);
@@ -1634,7 +1637,7 @@ void run_knn_query_noalloc(egt_ctx* h, const float* dqx, const float* dqy, const
     qcd.thres_n = thres_n;
     const int g = ceil_div(nq, KBLK);
     const int K = kclass(k);
-    const bool wave = query_by_wave(K, nq);
+    const bool wave = query_by_wave(h, K, nq);
     if (wave && nq <= QUERY_UNSORTED) {
         k_query_prep<<<g, KBLK, 0, s>>>(dqx, dqy, dqz, nq, h->min_extent, h->max_extent, P.a, P.ba, h->B, qpts, qcell,
                                         nullptr, nullptr, qcd, qcloud);

@@ -32,6 +32,7 @@ OPT_KNN_LONG_QUERY = 9       # lane-per-query search: candidates after which a q
 OPT_KNN_CLASS_SHAPES = 10    # per neighbour-count class launch shapes, as BatchGrid.autotune_shape returns them, or
                              # class_shapes_all(shape)
 OPT_LEARNED_LEVEL_OFFSET = 11  # added to the proposed start levels (-3..3)
+OPT_KNN_QUERY_LANES = 12     # query search: 0 = the library's choice (default), 1 = one lane, 64 = one wave per query
 START_LEVEL_OCCUPANCY = 127  # OPT_START_LEVEL values: one level from the mean cell occupancy; every query's own
 START_LEVEL_OWN_CELL = 126   # cell, as in the reference (0, the default, is the library's choice)
 SUB_LEVELS = 3               # start levels -1, -2, -3: boxes of cells 1/2, 1/4, 1/8 of a grid cell

@@ -68,3 +68,83 @@ def test_tuned_start_level_replayed(egt_mod):
         print("level", level, flush=True)
         _, st = _search(E, pts, k, START_LEVEL=level if level else E.START_LEVEL_OWN_CELL)
         assert st["knn_cells"] == tuned["knn_cells"] and st["knn_candidates"] == tuned["knn_candidates"]
+
+
+class _Named:
+    """The package with every GridStructure made under the given options (a test of another file then runs in the shape
+    that these name; a start level 0 in it means the own cell)."""
+
+    def __init__(self, E, **options):
+        class Grid(E.GridStructure):
+            def __init__(self, *args, **kwargs):
+                super().__init__(*args, **kwargs)
+                for name, value in options.items():
+                    super().set_option(getattr(E, "OPT_" + name), value)
+
+            def set_option(self, opt, value):
+                own = opt == E.OPT_START_LEVEL and value == 0
+                super().set_option(opt, E.START_LEVEL_OWN_CELL if own else value)
+
+        self._E, self.GridStructure = E, Grid
+
+    def __getattr__(self, name):
+        return getattr(self._E, name)
+
+
+@pytest.mark.parametrize("k", [8, 16, 24])
+@pytest.mark.parametrize("lanes", [0, 1, 64])
+def test_query_shapes_at_300001(egt_mod, oracle_mod, k, lanes):
+    """More queries than the library gives to a wave each at these k: its own choice is then a lane per query. A tenth of
+    the queries outside the grid and a finite radius."""
+    E, O = egt_mod, oracle_mod
+    ref = D.sphere(20_000, seed=41)
+    q = tuple(a.copy() for a in D.sphere(300_001, seed=42))
+    q[0][::10] *= np.float32(1.3)
+    print("k", k, "lanes", lanes, flush=True)
+    g = E.GridStructure(ref, 1, 1e-6, 1024, 4)
+    g.set_option(E.OPT_KNN_QUERY_LANES, lanes)
+    g.GRIDCUDAKNNCompact(q, k, 0.05)
+    got, st = g.GetKNNIndexesQuery(), g.stats()
+    g.close()
+    og = O.Grid(*ref)
+    rows, _, inv, _ = og.knn_query(*q, k, thres=0.05)
+    np.testing.assert_array_equal(got, og.ref_to_original(rows))
+    assert st["query_invalid_rows"] == int(inv.sum())
+
+
+@pytest.mark.parametrize("case", ["sphere_k16", "torus_k40", "sphere_k64", "mixture_k8", "torus_k1", "sphere_k33",
+                                  "outside", "short", "device", "crowded0", "crowded-2"])
+def test_lane_query_search(egt_mod, oracle_mod, case):
+    """The query tests with a lane per query (so few queries go to a wave each by default)."""
+    import test_gpu_query as Q
+
+    E = _Named(egt_mod, KNN_QUERY_LANES=1)
+    if case == "outside":
+        Q.test_queries_outside_the_grid(E, oracle_mod)
+    elif case == "short":
+        Q.test_short_rows_duplicates_and_big_cells(E, oracle_mod)
+    elif case == "device":
+        Q.test_device_input_and_self_rows_untouched(E, oracle_mod)
+    elif case.startswith("crowded"):
+        Q.test_queries_crowded_cells(E, oracle_mod, int(case[7:]))
+    else:
+        Q.test_query_rows_bit_exact(E, oracle_mod, case)
+
+
+def test_query_lanes_option(egt_mod):
+    """The allocation-free search follows the named shape as well; other values are refused."""
+    import torch
+    from test_zz_no_alloc import _allocating, _noalloc
+
+    E = egt_mod
+    g = E.GridStructure(D.torus(60_000, seed=66), 1, 1e-6, 1024, 4)
+    for nq, k in ((5_000, 40), (150_000, 8)):
+        q = tuple(torch.from_numpy(a).cuda() for a in D.torus(nq, seed=67))
+        want = _allocating(E, g, q, k)
+        for lanes in (1, 64, 0):
+            g.set_option(E.OPT_KNN_QUERY_LANES, lanes)
+            np.testing.assert_array_equal(_noalloc(E, torch, g, q, k), want, err_msg=f"{nq} lanes {lanes}")
+    for bad in (-1, 2, 65):
+        with pytest.raises(E.EGTError):
+            g.set_option(E.OPT_KNN_QUERY_LANES, bad)
+    g.close()
