@@ -71,21 +71,24 @@ def test_tuned_start_level_replayed(egt_mod):
 
 
 class _Named:
-    """The package with every GridStructure made under the given options (a test of another file then runs in the shape
-    that these name; a start level 0 in it means the own cell)."""
+    """The package with every point-cloud handle made under the given options (a test of another file then runs in the
+    shape that these name; a start level 0 in it means the own cell)."""
 
     def __init__(self, E, **options):
-        class Grid(E.GridStructure):
-            def __init__(self, *args, **kwargs):
-                super().__init__(*args, **kwargs)
-                for name, value in options.items():
-                    super().set_option(getattr(E, "OPT_" + name), value)
+        def named(base):
+            class Grid(base):
+                def __init__(self, *args, **kwargs):
+                    super().__init__(*args, **kwargs)
+                    for name, value in options.items():
+                        super().set_option(getattr(E, "OPT_" + name), value)
 
-            def set_option(self, opt, value):
-                own = opt == E.OPT_START_LEVEL and value == 0
-                super().set_option(opt, E.START_LEVEL_OWN_CELL if own else value)
+                def set_option(self, opt, value):
+                    own = opt == E.OPT_START_LEVEL and value == 0
+                    super().set_option(opt, E.START_LEVEL_OWN_CELL if own else value)
 
-        self._E, self.GridStructure = E, Grid
+            return Grid
+
+        self._E, self.GridStructure, self.BatchGrid = E, named(E.GridStructure), named(E.BatchGrid)
 
     def __getattr__(self, name):
         return getattr(self._E, name)
@@ -148,3 +151,40 @@ def test_query_lanes_option(egt_mod):
         with pytest.raises(E.EGTError):
             g.set_option(E.OPT_KNN_QUERY_LANES, bad)
     g.close()
+
+
+LANE_TESTS = ([("test_knn_rows_bit_exact", (c, 1)) for c in ("sphere20k_k40", "torus30k_k16", "sphere5k_k64", "lattice_k18",
+                                                             "dups_k8")]
+              + [("test_lattice_rows_follow_bucket_count", (k,)) for k in (10, 18)]
+              + [("test_knn_independent_of_start_level", (v, 1)) for v in ("occupancy", -3, -2, -1, 0, 2, 5, 9)]
+              + [("test_knn_invalidation_rules", (1,)), ("test_duplicate_points_rows_bit_exact", (1,))]
+              + [("test_knn_crowded_cells_sub_levels", (v, m, 1)) for v in (0, -1, -3) for m in (None, 3750)]
+              + [("test_every_k_class_bit_exact", (k,)) for k in (1, 7, 9, 23, 31, 33, 47, 55, 63)])
+
+
+@pytest.mark.parametrize("start", ["own", "default"])
+@pytest.mark.parametrize("name,args", LANE_TESTS, ids=[f"{n[5:]}-{a}" for n, a in LANE_TESTS])
+def test_lane_search(egt_mod, oracle_mod, name, args, start):
+    """The self search tests with a lane per query (clouds of their sizes go to a wave per query by default), from the
+    own cell, as the reference starts, and from the default level."""
+    import test_gpu_parity as P
+
+    options = {"START_LEVEL": egt_mod.START_LEVEL_OWN_CELL} if start == "own" else {}
+    E = _Named(egt_mod, KNN_CLASS_SHAPES=egt_mod.class_shapes_all(0), **options)
+    getattr(P, name)(E, oracle_mod, *args)
+
+
+@pytest.mark.parametrize("start", ["own", "default"])
+def test_lane_batch(egt_mod, oracle_mod, start):
+    import test_gpu_batch as B
+
+    options = {"START_LEVEL": egt_mod.START_LEVEL_OWN_CELL} if start == "own" else {}
+    E = _Named(egt_mod, KNN_CLASS_SHAPES=egt_mod.class_shapes_all(0), **options)
+    B.test_batch_matches_separate_oracle_runs(E, oracle_mod, 0, 1, None)
+
+
+@pytest.mark.parametrize("n", [1, 64, 2048, 2049, 4097])
+def test_own_cell_at_tile_edges(egt_mod, oracle_mod, n):
+    import test_gpu_edges as T
+
+    T.test_level_tables_at_tile_edges(_Named(egt_mod), oracle_mod, n, 1024)
