@@ -188,3 +188,24 @@ def test_own_cell_at_tile_edges(egt_mod, oracle_mod, n):
     import test_gpu_edges as T
 
     T.test_level_tables_at_tile_edges(_Named(egt_mod), oracle_mod, n, 1024)
+
+
+@pytest.mark.parametrize("n,k,shape", [(99_968, 8, 2), (99_969, 8, 0), (120_000, 16, 2), (120_001, 16, 0),
+                                       (299_968, 24, 2), (299_969, 24, 0), (99_968, 32, 2), (99_969, 32, 2),
+                                       (299_968, 40, 2), (299_969, 40, 2), (99_969, 64, 2), (299_968, 64, 2)])
+def test_both_sides_of_the_shape_limits(egt_mod, oracle_mod, n, k, shape):
+    """The rule counts whole chunks of 64 queries. The largest size of the wave shape and the smallest of the lane shape
+    at short lists, and of 1, 2 and 4 queries a wave at long ones: the search does the work of the named shape, and
+    rows are the oracle's."""
+    E, O = egt_mod, oracle_mod
+    print("n", n, "k", k, flush=True)
+    pts = D.torus(n, seed=31)
+    rows, st = _search(E, pts, k)
+    work = {}
+    for s in (0, 2):
+        named = _search(E, pts, k, KNN_CLASS_SHAPES=E.class_shapes_all(s))[1]
+        work[s] = named["knn_cells"], named["knn_candidates"]
+    print("cells, candidates: lane", work[0], "wave", work[2], flush=True)
+    assert (st["knn_cells"], st["knn_candidates"]) == work[shape] != work[2 - shape]
+    og = O.Grid(*pts)
+    np.testing.assert_array_equal(rows, og.to_original(og.knn(k)[0]))
