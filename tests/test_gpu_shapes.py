@@ -209,3 +209,23 @@ def test_both_sides_of_the_shape_limits(egt_mod, oracle_mod, n, k, shape):
     assert (st["knn_cells"], st["knn_candidates"]) == work[shape] != work[2 - shape]
     og = O.Grid(*pts)
     np.testing.assert_array_equal(rows, og.to_original(og.knn(k)[0]))
+
+
+def test_taubin_graph_replays_match_launches(egt_mod):
+    """The captured Taubin graphs against eager launches, by name (at this size the passes otherwise run in one launch):
+    three smoothing calls of 60 iterations on one handle, two replays of the 25-iteration graph and one of the
+    10-iteration graph each, with an eager search between the calls."""
+    import test_gpu_parity as P
+
+    E = egt_mod
+    P.test_taubin_graph_replays_match_eager(_Named(E, TAUBIN_TILE=1024))
+    g = E.GridStructure(D.sphere(30_000, seed=45), 1, 1e-6, 1024, 4)
+    g.GRIDCUDAKNNSELF_COMPACT(16, 1e8)
+    tiles = []
+    for options in ((), ((E.OPT_TAUBIN_TILE, 1024),)):
+        for o in options:
+            g.set_option(*o)
+        E.EGT_CUDA(g).PerformSmoothing(60, 0.5, -0.53, 0.65)
+        tiles.append(g.stats()["taubin_tile"])
+    g.close()
+    assert tiles == [256, 1024]
