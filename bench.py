@@ -380,7 +380,7 @@ def batch_result(args, steps, warmup, per_cloud=True):
     """Batched uneven workload: args.clouds superquadric clouds, sizes log-uniform in [5k, 500k], k drawn
     from {16, 40, 64}, alpha 0.65, 100 iterations (lambda 0.5, mu -0.53). One step = batch build (cube, sort,
     cell tables for all clouds) + (learned proposal) + kNN (one launch per neighbour-count class over 64-query
-    chunks) + EGG + Taubin (one captured graph over all clouds). Coordinates are resident in HBM before timing.
+    chunks) + EGG + Taubin (one graph over all clouds). Coordinates are resident in HBM before timing.
     The learned batch (model trained on the GPU on 64 clouds of other seeds) and the plain batch (the library's
     start levels), each with the kNN launch shape per neighbour-count class that the class tuner picks
     for it (outside the timing), are each timed over `steps` steps; beside them, when per_cloud, the plain GPU path of
@@ -542,7 +542,7 @@ def torus_result(args):
     # Taubin pass, algorithmic bytes per launch: own xyz read 12 + write 12 + row ptr 4 per point, 4 B per
     # kept neighbour index
     taub_bytes = 28 * n + 4 * nnz
-    # one pass: the captured lambda/mu passes alone, timed by the library with HIP events on its stream (the
+    # one pass: the lambda/mu passes alone, timed by the library with HIP events on its stream (the
     # once-per-call tile set-up and graph build are reported apart as taubin_setup_ms)
     taub_pass_ms = med("taubin_pass_ms") if passes else float("nan")
     # kNN, algorithmic bytes: query xyz 12 + 4k output per query

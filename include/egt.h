@@ -100,7 +100,7 @@ typedef enum {
                                     EGT_START_LEVEL_OCCUPANCY = one level from the mean cell occupancy. Rows do
                                     not depend on it */
     EGT_OPT_LEARNED = 1,         /* kNN: 1 = start each query from the learned radius proposal */
-    EGT_OPT_TAUBIN_GRAPH = 2,    /* Taubin: 1 = replay the lambda/mu loop as a captured hipGraph (default; clouds of
+    EGT_OPT_TAUBIN_GRAPH = 2,    /* Taubin: 1 = replay the lambda/mu loop as a hipGraph (default; clouds of
                                     up to 262,144 points run every pass in one launch), 0 = a launch per pass */
     EGT_OPT_MAX_PTS_IN_CUBE = 3, /* kNN validity rule: cell population that invalidates a query (1e5) */
     EGT_OPT_KNN_PERSISTENT = 4,  /* kNN: 1 = one persistent work-queue launch per neighbour-count class,

@@ -44,43 +44,39 @@ struct Event {
     operator hipEvent_t() const { return e; }
 };
 
-// An instantiated graph owned for one scope.
-struct GraphExec {
+template <class T>
+struct Same {  // a parameter of this type takes no part in template argument deduction
+    using type = T;
+};
+
+// A chain of kernel launches as a graph, owned for one scope. Its nodes are added one by one, not captured from a
+// stream: a capture ends in an error when another thread synchronizes the device meanwhile, as a handle does whose
+// buffers grow.
+struct GraphChain {
     hipGraph_t g = nullptr;
     hipGraphExec_t ge = nullptr;
-    GraphExec() = default;
-    GraphExec(const GraphExec&) = delete;
-    GraphExec& operator=(const GraphExec&) = delete;
-    ~GraphExec() {
+    hipGraphNode_t last = nullptr;
+    GraphChain() { HIP_CHECK(hipGraphCreate(&g, 0)); }
+    GraphChain(const GraphChain&) = delete;
+    GraphChain& operator=(const GraphChain&) = delete;
+    ~GraphChain() {
         if (ge) (void)hipGraphExecDestroy(ge);
         if (g) (void)hipGraphDestroy(g);
     }
-};
-
-// Stream capture for one scope: if anything throws between begin and end, the destructor ends the capture
-// (and drops the partial graph), so the stream leaves capture mode and the handle stays usable.
-struct Capture {
-    hipStream_t s;
-    bool active = false;
-    explicit Capture(hipStream_t st) : s(st) {
-        HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        active = true;
+    template <class... P>
+    void add(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, typename Same<P>::type... args) {
+        void* ptrs[] = {(void*)&args...};  // copied into the node
+        hipKernelNodeParams k{};
+        k.func = reinterpret_cast<void*>(kernel);
+        k.gridDim = grid;
+        k.blockDim = block;
+        k.sharedMemBytes = (unsigned)lds;
+        k.kernelParams = ptrs;
+        hipGraphNode_t node = nullptr;
+        HIP_CHECK(hipGraphAddKernelNode(&node, g, last ? &last : nullptr, last ? 1 : 0, &k));
+        last = node;
     }
-    Capture(const Capture&) = delete;
-    Capture& operator=(const Capture&) = delete;
-    // Ends the capture into out.g and instantiates out.ge.
-    void end(GraphExec& out) {
-        active = false;
-        HIP_CHECK(hipStreamEndCapture(s, &out.g));
-        HIP_CHECK(hipGraphInstantiate(&out.ge, out.g, nullptr, nullptr, 0));
-    }
-    ~Capture() {
-        if (!active) return;
-        hipGraph_t g = nullptr;
-        (void)hipStreamEndCapture(s, &g);
-        if (g) (void)hipGraphDestroy(g);
-        (void)hipGetLastError();
-    }
+    void instantiate() { HIP_CHECK(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0)); }
 };
 
 // Device memory cache (egt_memory.hip): device_alloc returns a block of at least `bytes` (its capacity in

@@ -6,8 +6,8 @@
 // Points live in Morton order as packed x, y, z (12 bytes) in two buffers, so a wave's 64 points are spatial
 // neighbours and their gathers mostly hit the same cache lines; a tile stages them in LDS as float4. Blocks
 // are remapped so each of the 8 XCDs walks chunks of consecutive Morton tiles (workgroups are dealt to XCDs
-// round robin), which keeps a block's neighbours in its own XCD's L2. The 2*iterations passes are recorded
-// into hipGraphs and replayed. The exp is egt_expf, so results match the host oracle bit for bit; the
+// round robin), which keeps a block's neighbours in its own XCD's L2. The 2*iterations passes are replayed as
+// hipGraphs. The exp is egt_expf, so results match the host oracle bit for bit; the
 // per-point arithmetic and neighbour order are those of the reference, only the memory layout differs.
 #include "egt_device.h"
 #include "egt_internal.h"
@@ -852,21 +852,25 @@ TilePlan prepare_tiles(egt_ctx* h) {
     return tp;
 }
 
+// One pass: launched on the handle's stream, or added to a graph.
 template <int TILE, bool REG>
-void launch_tile(egt_ctx* h, const TilePlan& tp, const Pt3* in, Pt3* out, float scale) {
+void launch_tile(egt_ctx* h, const TilePlan& tp, const Pt3* in, Pt3* out, float scale, GraphChain* graph) {
     const size_t lds_bytes = (size_t)(tp.tile + tp.maxH + 1) * sizeof(float4);  // + the halo's spill entry
     const dim3 tgrid(ceil_div(tp.ntiles, NXCD * XCHUNK) * NXCD * XCHUNK), tblk(tile_threads<TILE>());
-    k_taubin_tile<TILE, REG><<<tgrid, tblk, lds_bytes, h->stream>>>(in, out, h->rowptr.p, h->col.p, tp.scol, tp.toff,
-                                                                    tp.width, tp.perm, tp.halo, tp.hcount, h->n, scale,
-                                                                    tp.ntiles);
+    if (graph)
+        graph->add(k_taubin_tile<TILE, REG>, tgrid, tblk, lds_bytes, in, out, h->rowptr.p, h->col.p, tp.scol, tp.toff,
+                   tp.width, tp.perm, tp.halo, tp.hcount, h->n, scale, tp.ntiles);
+    else
+        k_taubin_tile<TILE, REG><<<tgrid, tblk, lds_bytes, h->stream>>>(in, out, h->rowptr.p, h->col.p, tp.scol, tp.toff,
+                                                                        tp.width, tp.perm, tp.halo, tp.hcount, h->n,
+                                                                        scale, tp.ntiles);
 }
 
-void launch_pass(egt_ctx* h, const TilePlan& tp, const Pt3* in, Pt3* out, float scale) {
+void launch_pass(egt_ctx* h, const TilePlan& tp, const Pt3* in, Pt3* out, float scale, GraphChain* graph = nullptr) {
     const bool reg = h->taubin_regularized != 0;
-    if (tp.tile == 2048)
-        reg ? launch_tile<2048, true>(h, tp, in, out, scale) : launch_tile<2048, false>(h, tp, in, out, scale);
-    else
-        reg ? launch_tile<1024, true>(h, tp, in, out, scale) : launch_tile<1024, false>(h, tp, in, out, scale);
+    const auto launch = tp.tile == 2048 ? (reg ? launch_tile<2048, true> : launch_tile<2048, false>)
+                                        : (reg ? launch_tile<1024, true> : launch_tile<1024, false>);
+    launch(h, tp, in, out, scale, graph);
 }
 
 TilePlan prepare(egt_ctx* h, int tile) { return tile == 2048 ? prepare_tiles<2048>(h) : prepare_tiles<1024>(h); }
@@ -1010,23 +1014,21 @@ void run_taubin(egt_ctx* h, int iters, float lambda, float mu) {
     h->stats.taubin_tile = tile;
     h->stats.taubin_fallback_tiles = (int32_t)tp.fallback_tiles;
     h->stats.taubin_overflow_tiles = (int32_t)tp.overflow_tiles;
-    auto pass = [&](const Pt3* in, Pt3* out, float scale) { launch_pass(h, tp, in, out, scale); };
     if (iters > 0) {
         if (h->taubin_graph) {
             // A graph of up to GRAPH_ITERS iterations (2 GRAPH_ITERS passes; each iteration ends back in A) is
             // built once and replayed; the remaining iterations form a second, shorter graph. Building one
             // node per pass for hundreds of iterations costs more host time than the replays save.
             constexpr int GRAPH_ITERS = 25;  // set-up 2.9 ms vs 3.75 ms for one 600-node graph (4M torus)
-            auto build = [&](int its, GraphExec& out) {
-                Capture cap(s);
+            auto build = [&](int its, GraphChain& out) {
                 for (int it = 0; it < its; ++it) {
-                    pass(A, Bf, lambda);
-                    pass(Bf, A, mu);
+                    launch_pass(h, tp, A, Bf, lambda, &out);
+                    launch_pass(h, tp, Bf, A, mu, &out);
                 }
-                cap.end(out);
+                out.instantiate();
             };
             const int full = iters / GRAPH_ITERS, rest = iters % GRAPH_ITERS;
-            GraphExec G0, G1;
+            GraphChain G0, G1;
             if (full > 0) build(GRAPH_ITERS, G0);
             if (rest > 0) build(rest, G1);
             HIP_CHECK(hipEventRecord(ep, s));  // the passes alone: from here to e1
@@ -1036,8 +1038,8 @@ void run_taubin(egt_ctx* h, int iters, float lambda, float mu) {
         } else {
             HIP_CHECK(hipEventRecord(ep, s));
             for (int it = 0; it < iters; ++it) {
-                pass(A, Bf, lambda);
-                pass(Bf, A, mu);
+                launch_pass(h, tp, A, Bf, lambda);
+                launch_pass(h, tp, Bf, A, mu);
             }
             LAUNCH_CHECK();
         }
