@@ -135,8 +135,12 @@ typedef enum {
     EGT_OPT_LEARNED_LEVEL_OFFSET = 11, /* kNN with the learned proposal: added to every proposed start level,
                                     -3..3 (default 0; +1 = one level coarser than proposed).
                                     egt_autotune_learned picks it. Rows do not depend on it */
-    EGT_OPT_KNN_QUERY_LANES = 12  /* query search: 1 = one lane per query, 64 = one wave per query, 0 = the
+    EGT_OPT_KNN_QUERY_LANES = 12, /* query search: 1 = one lane per query, 64 = one wave per query, 0 = the
                                     library's choice by query count and k (default). Rows do not depend on it */
+    EGT_OPT_TAUBIN_WAIT = 13      /* Taubin passes of a small cloud in one launch: microseconds (0 to 10^6, default
+                                    500) in which its workgroups all have to be on the GPU, which other work may
+                                    prevent. The call, and later ones on the handle until this option is set
+                                    again, else run a launch per pass. Results do not depend on it */
 } egt_option;
 
 const char* egt_last_error_string(void);

@@ -374,6 +374,11 @@ egt_status egt_set_option(egt_handle h, egt_option opt, int64_t value) {
             if (value < -3 || value > 3) return fail(EGT_ERR_INVALID_ARG, "learned level offset must be in [-3, 3]");
             h->learned_level_offset = (int)value;
             return EGT_OK;
+        case EGT_OPT_TAUBIN_WAIT:
+            if (value < 0 || value > 1000000) return fail(EGT_ERR_INVALID_ARG, "Taubin wait must be in [0, 10^6] us");
+            h->taubin_wait_us = value;
+            h->taubin_wait_over = false;
+            return EGT_OK;
         case EGT_OPT_KNN_QUERY_LANES:
             if (value != 0 && value != 1 && value != 64)
                 return fail(EGT_ERR_INVALID_ARG, "query lanes must be 0, 1 or 64");

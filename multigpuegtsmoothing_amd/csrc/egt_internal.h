@@ -263,6 +263,8 @@ struct egt_ctx {
     int taubin_graph = 1;
     int taubin_tile = 1024;  // Taubin tile width: 1024 or 2048 points; 0 = tune on the next smoothing call
     bool taubin_tile_set = false;  // the width was set by option: no other tiling
+    int64_t taubin_wait_us = 500;    // resident passes: how long a tile waits for its neighbours to be there
+    bool taubin_wait_over = false;   // such a wait ran out: no resident passes until the option is set again
     int taubin_regularized = 0;  // isRegularized weights (1 / inverse-square), off as in the reference
     int maxc = 100000;
 

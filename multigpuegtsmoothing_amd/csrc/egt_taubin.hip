@@ -9,6 +9,7 @@
 // round robin), which keeps a block's neighbours in its own XCD's L2. The 2*iterations passes are replayed as
 // hipGraphs. The exp is egt_expf, so results match the host oracle bit for bit; the
 // per-point arithmetic and neighbour order are those of the reference, only the memory layout differs.
+#include "egt_budget.h"
 #include "egt_device.h"
 #include "egt_internal.h"
 
@@ -539,9 +540,15 @@ __global__ void __launch_bounds__(tile_threads<TILE>()) __attribute__((amdgpu_wa
 // has the value: no flag, fence or barrier across workgroups. Two buffers alternate by parity. A tile may overwrite
 // version v with v + 2 once every reader of v is past it; a reader is past it when it publishes v + 1, so the
 // tiles' reads are made symmetric (k_tile_tokens): a tile that is read by another one reads a point of it too.
-// Every workgroup must be resident, so the tiles are limited to what fits on the GPU at once; should they not be
-// (other work holds the CUs), a wait ends after RWAIT ticks, raises the flag, every workgroup leaves, and the caller
-// runs the passes launch by launch. The points are untouched until k_writeback, which looks at the flag first.
+// Every workgroup must be resident, so the tiles are limited to what fits on the GPU at once, less those of other
+// handles' resident passes (TileBudget: two clouds of 262,144 points smoothed from two threads held each other's
+// workgroups out, and both waited in vain). Even so some workgroups may not come: with another queue's work waiting
+// for the same places the last ones were seen to stay out until the others left, however long these waited. Then a
+// wait ends, raises the flag, every workgroup leaves, and the caller runs the passes launch by launch, as every later
+// call on the handle does. A tile whose neighbour is not there finds that out in the first exchange, so that one ends
+// after `wait` ticks (EGT_OPT_TAUBIN_WAIT, 500 us) and later ones, which only another process can hold up, after
+// RLATER times as many. Two such clouds from two threads, 20 calls each, launch by launch 66-77 ms; with a wait of
+// 100 us 56-64, 250 us 58-63, 500 us 61-65, 2 ms 72-74, 5 ms 81-82, 20 ms 105-177, 100 ms 164-460. The points are untouched until k_writeback, which looks at the flag first.
 //
 // Bound: the chain of one pass (publish, find the neighbours' points, two chunks of slots), where a launch per pass
 // costs its start, two dependent rounds of staging loads and its end, with most CUs idle below 256 tiles. Us a pass,
@@ -551,7 +558,8 @@ __global__ void __launch_bounds__(tile_threads<TILE>()) __attribute__((amdgpu_wa
 constexpr int RT = 256;            // points per tile, one row per thread
 constexpr int RHP = halo_cap<RT>() / RT;
 constexpr int RCW = 16;            // column words of a row held in registers (32 slots); the rest is read per pass
-constexpr int64_t RWAIT = 2000000;  // 20 ms of the 100 MHz wall clock
+constexpr int RTICKS = 100;        // ticks of the wall clock per us
+constexpr int RLATER = 40;         // later waits, as a multiple of the first
 static_assert(halo_cap<RT>() == halo_max<RT>(), "a resident halo lies in LDS");
 
 // Symmetric reads: tile t, read by t2 but not reading it, appends t2's first point to its halo.
@@ -618,7 +626,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) k_
                                                          const uint16_t* __restrict__ perm,
                                                          const int32_t* __restrict__ halo,
                                                          const int32_t* __restrict__ hcount, int64_t n, int iters,
-                                                         float lambda, float mu, Resident R) {
+                                                         float lambda, float mu, Resident R, int64_t wait) {
     constexpr int S = RT / 64;
     __shared__ float4 pts[RT + halo_cap<RT>()];
     __shared__ uint16_t publist[RT];  // the tile's published rows, in position order
@@ -730,6 +738,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) k_
         uint32_t pend = 0;
 #pragma unroll
         for (int k = 0; k < RHP; ++k) pend |= hx[k] >= 0 ? 1u << k : 0u;
+        const int64_t limit = pass == 0 ? wait : RLATER * wait;
         int64_t t0 = 0;
         while (pend) {
             uint64_t v[RHP][3];
@@ -755,9 +764,9 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) k_
             if (pend) {
                 const int64_t now = (int64_t)wall_clock64();
                 if (t0 == 0) t0 = now;
-                if (now - t0 > RWAIT) atomicOr(R.flag, 2u);
+                if (now - t0 >= limit) atomicOr(R.flag, 2u);
                 // another workgroup's wait may have run out: looked at now and then, this one's own at once
-                if (now - t0 > RWAIT || ((now - t0) & 0xFF) == 0xFF) {
+                if (now - t0 >= limit || ((now - t0) & 0xFF) == 0xFF) {
                     if (__hip_atomic_load(R.flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
                         stop = 1;
                         pend = 0;
@@ -912,26 +921,39 @@ __global__ void __launch_bounds__(TBLK) k_zero_u32(uint32_t* __restrict__ p, int
     for (int64_t i = (int64_t)blockIdx.x * TBLK + threadIdx.x; i < n; i += (int64_t)gridDim.x * TBLK) p[i] = 0u;
 }
 
-// Largest tile count of the resident passes: four workgroups on each CU (their LDS and registers allow more).
-int resident_tiles() {
-    static const int tiles = [] {
-        int dev = 0, cus = 0, a = 0, b = 0;
-        HIP_CHECK(hipGetDevice(&dev));
+// Largest tile count of the resident passes on a device: four workgroups on each CU (their LDS and registers allow
+// more).
+int resident_tiles(int dev) {
+    static std::mutex mu;
+    static std::map<int, int> tiles;
+    std::lock_guard<std::mutex> lock(mu);
+    int& t = tiles[dev];
+    if (t == 0) {
+        int cus = 0, a = 0, b = 0;
         HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
         HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_taubin_resident<false>, RT, 0));
         HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_taubin_resident<true>, RT, 0));
-        return cus * std::min(4, std::min(a, b));
-    }();
-    return tiles;
+        t = cus * std::min(4, std::min(a, b));
+    }
+    return t;
+}
+TileBudget& resident_budget() {
+    static TileBudget b;
+    return b;
 }
 
-// All passes in one launch (see k_taubin_resident). Returns false, with the points untouched, when a tile does not
-// fit (halo too long, a row that lists itself) or a wait ran out: the caller then runs the passes launch by launch.
+// All passes in one launch (see k_taubin_resident). Returns false, with the points untouched, when other handles' passes
+// leave too few places, a tile does not fit (halo too long, a row that lists itself) or a wait ran out: the caller
+// then runs the passes launch by launch.
 bool run_resident(egt_ctx* h, int iters, float lambda, float mu) {
     const int64_t n = h->n;
     const int nt = ceil_div(n, RT);
-    if (iters < 1 || h->taubin_tile != 1024 || h->taubin_tile_set || !h->taubin_graph || nt > resident_tiles())
+    if (iters < 1 || h->taubin_tile != 1024 || h->taubin_tile_set || !h->taubin_graph || h->taubin_wait_over ||
+        n > (int64_t)resident_tiles(h->device) * RT)
         return false;
+    const TileShare share(resident_budget(), h->device, nt, resident_tiles(h->device));
+    if (!share) return false;
+    const int64_t wait = h->taubin_wait_us * RTICKS;
     hipStream_t s = h->stream;
     Scratch& sc = h->scratch;
     int kmax = 1;
@@ -968,16 +990,17 @@ bool run_resident(egt_ctx* h, int iters, float lambda, float mu) {
     HIP_CHECK(hipEventRecord(ep, s));
     if (h->taubin_regularized)
         k_taubin_resident<true><<<nt, RT, 0, s>>>(h->mpts.p, out, scol, toff, width, perm, halo, hcount, n, iters,
-                                                  lambda, mu, R);
+                                                  lambda, mu, R, wait);
     else
         k_taubin_resident<false><<<nt, RT, 0, s>>>(h->mpts.p, out, scol, toff, width, perm, halo, hcount, n, iters,
-                                                   lambda, mu, R);
+                                                   lambda, mu, R, wait);
     LAUNCH_CHECK();
     HIP_CHECK(hipEventRecord(e1, s));
     k_writeback<<<ceil_div(n, TBLK), TBLK, 0, s>>>(out, n, h->mpts.p, h->x.p, h->y.p, h->z.p, R.flag);
     LAUNCH_CHECK();
     uint32_t flag = 0;
-    fetch(h->lane, {{&flag, R.flag, sizeof(flag)}});
+    fetch(h->lane, {{&flag, R.flag, sizeof(flag)}});  // the launch is over: its share may go back
+    if (flag & 2u) h->taubin_wait_over = true;
     if (flag) return false;
     float total = 0.0f, passes = 0.0f;
     HIP_CHECK(hipEventElapsedTime(&total, e0, e1));

@@ -33,6 +33,7 @@ OPT_KNN_CLASS_SHAPES = 10    # per neighbour-count class launch shapes, as Batch
                              # class_shapes_all(shape)
 OPT_LEARNED_LEVEL_OFFSET = 11  # added to the proposed start levels (-3..3)
 OPT_KNN_QUERY_LANES = 12     # query search: 0 = the library's choice (default), 1 = one lane, 64 = one wave per query
+OPT_TAUBIN_WAIT = 13         # Taubin passes in one launch: us in which all workgroups have to be there (500)
 START_LEVEL_OCCUPANCY = 127  # OPT_START_LEVEL values: one level from the mean cell occupancy; every query's own
 START_LEVEL_OWN_CELL = 126   # cell, as in the reference (0, the default, is the library's choice)
 SUB_LEVELS = 3               # start levels -1, -2, -3: boxes of cells 1/2, 1/4, 1/8 of a grid cell
