@@ -740,6 +740,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) k_
         for (int k = 0; k < RHP; ++k) pend |= hx[k] >= 0 ? 1u << k : 0u;
         const int64_t limit = pass == 0 ? wait : RLATER * wait;
         int64_t t0 = 0;
+        uint32_t looks = 0;
         while (pend) {
             uint64_t v[RHP][3];
 #pragma unroll
@@ -765,8 +766,9 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) k_
                 const int64_t now = (int64_t)wall_clock64();
                 if (t0 == 0) t0 = now;
                 if (now - t0 >= limit) atomicOr(R.flag, 2u);
-                // another workgroup's wait may have run out: looked at now and then, this one's own at once
-                if (now - t0 >= limit || ((now - t0) & 0xFF) == 0xFF) {
+                // another workgroup's wait may have run out: looked at every so many looks (by the clock's low bits it
+                // was missed for the whole wait), this one's own at once
+                if (now - t0 >= limit || (++looks & 31u) == 0u) {
                     if (__hip_atomic_load(R.flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
                         stop = 1;
                         pend = 0;

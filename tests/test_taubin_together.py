@@ -23,7 +23,9 @@ def test_launch_budget(tmp_path):
 
 @pytest.mark.gpu
 def test_two_clouds_that_fill_the_gpu(egt_mod):
-    """Two clouds whose tiles fill the GPU each, smoothed from two threads: results are those of each cloud alone."""
+    """Two clouds whose tiles fill the GPU each, smoothed from two threads: results are those of each cloud alone, and
+    the calls together take less than half the time of the waits that two launches holding each other's places out
+    would run into (20 ms in each of 8 rounds; about 2 ms a call)."""
     E = egt_mod
     clouds = [D.torus(262_144, seed=710), D.sphere(262_144, seed=711)]
     rounds = 8
@@ -59,6 +61,7 @@ def test_two_clouds_that_fill_the_gpu(egt_mod):
         for out in together[i][0]:
             for a, b in zip(alone[i][0][0], out):
                 np.testing.assert_array_equal(a, b, err_msg=f"cloud {i}")
+    assert min(together[0][2], together[1][2]) < rounds * 0.010
 
 
 @pytest.mark.gpu
