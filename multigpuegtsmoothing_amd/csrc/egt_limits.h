@@ -30,6 +30,12 @@ inline const char* mesh_triangles_error(int64_t ntri) {
     return ntri > MESH_MAX_TRIANGLES ? "more than (2^31 - 1) / 6 triangles (int32 corner-list offsets)" : nullptr;
 }
 
+// Iterations that the Taubin passes of a small cloud run in one launch, at most: its pass counter is an int (two passes
+// an iteration) and the launch has the GPU to itself for as long as it runs, up to about 10 s here. More iterations
+// run a launch per pass.
+constexpr int MAX_RESIDENT_ITERATIONS = 1 << 20;
+inline bool resident_iterations(int iterations) { return iterations >= 1 && iterations <= MAX_RESIDENT_ITERATIONS; }
+
 // Workgroups of 256 threads in one launch.
 constexpr int64_t MAX_GROUPS = ((int64_t)1 << 32) / 256 - 1;
 

@@ -950,8 +950,8 @@ TileBudget& resident_budget() {
 bool run_resident(egt_ctx* h, int iters, float lambda, float mu) {
     const int64_t n = h->n;
     const int nt = ceil_div(n, RT);
-    if (iters < 1 || h->taubin_tile != 1024 || h->taubin_tile_set || !h->taubin_graph || h->taubin_wait_over ||
-        n > (int64_t)resident_tiles(h->device) * RT)
+    if (!resident_iterations(iters) || h->taubin_tile != 1024 || h->taubin_tile_set || !h->taubin_graph ||
+        h->taubin_wait_over || n > (int64_t)resident_tiles(h->device) * RT)
         return false;
     const TileShare share(resident_budget(), h->device, nt, resident_tiles(h->device));
     if (!share) return false;

@@ -35,6 +35,10 @@ int main() {
     check((int64_t)11 * INT32_MAX / 256, egt::MAX_GROUPS, 1, false);  // level inserts: a thread per cell of 11 levels
     check((int64_t)4 * INT32_MAX / 256, egt::MAX_GROUPS, 1, false);   // edge list: four threads per row
     egt::in_launches(0, egt::MAX_GROUPS, [&](int64_t, int64_t) { ++bad; });
+    // iterations of one launch: none and too many are not for it, and twice the most are an int
+    bad += egt::resident_iterations(0) || egt::resident_iterations(-1) || !egt::resident_iterations(1);
+    bad += !egt::resident_iterations(1000000) || egt::resident_iterations(1 << 30) || egt::resident_iterations(INT32_MAX);
+    bad += 2 * (int64_t)egt::MAX_RESIDENT_ITERATIONS > INT32_MAX;
     std::printf("%d\n", bad);
     return bad;
 }
