@@ -257,20 +257,20 @@ egt_status egt_release_cached_memory(uint64_t* released, uint64_t* cached);
  * (the cell size of the first search box), scores each level by its measured work per query (candidates
  * tested + 3 x cells looked up) and the handle starts at the cheapest. Rows do not depend on the choice.
  * *start_level (optional) receives it, for later handles: EGT_OPT_START_LEVEL takes it, with
- * EGT_START_LEVEL_OWN_CELL for level 0. trial_ms and trial_cost (optional, EGT_AUTOTUNE_SLOTS floats each) receive each level's sample time
- * in ms and its score at index level + 3, -1 where untried. The handle's neighbour rows are not valid
- * afterwards: run egt_grid_knn_self. */
+ * EGT_START_LEVEL_OWN_CELL for level 0. trial_ms and trial_cost (optional, EGT_AUTOTUNE_SLOTS floats each)
+ * receive each level's sample time in ms and its score at index level + 3, -1 where untried. The handle's
+ * neighbour rows are not valid afterwards: run egt_grid_knn_self. */
 egt_status egt_autotune(egt_handle h, int k, float thres, int32_t* start_level, float* trial_ms,
                         float* trial_cost);
 
 /* Launch-shape tuner (no reference counterpart): times the handle's current search (its start level and, with
  * EGT_OPT_LEARNED, the proposal in place) with neighbour count k and radius thres over all queries in each
  * launch shape: 0 = one lane per query, one workgroup per 256 queries; 1 = one lane per query, one
- * persistent work-queue launch; 2 = one wave per query. Each shape is
- * warmed up on the autotuner's sample, then timed once on the full search; the handle keeps the fastest for every
- * k (until EGT_OPT_KNN_LANES or EGT_OPT_KNN_PERSISTENT is set). Rows do not depend on the choice. *shape
- * (optional) receives it, for later handles: EGT_OPT_KNN_CLASS_SHAPES with EGT_CLASS_SHAPES_ALL(*shape); shape_ms (optional, 3 floats) each shape's time in ms. The handle's neighbour rows
- * are not valid afterwards: run egt_grid_knn_self. */
+ * persistent work-queue launch; 2 = one wave per query. Each shape is warmed up on the autotuner's sample, then
+ * timed once on the full search; the handle keeps the fastest for every k (until EGT_OPT_KNN_LANES or
+ * EGT_OPT_KNN_PERSISTENT is set). Rows do not depend on the choice. *shape (optional) receives it, for later
+ * handles: EGT_OPT_KNN_CLASS_SHAPES with EGT_CLASS_SHAPES_ALL(*shape); shape_ms (optional, 3 floats) each shape's
+ * time in ms. The handle's neighbour rows are not valid afterwards: run egt_grid_knn_self. */
 egt_status egt_autotune_shape(egt_handle h, int k, float thres, int32_t* shape, float* shape_ms);
 
 /* Learned-start tuner (no reference counterpart): with a proposal in place (egt_model_propose), times the full
@@ -279,9 +279,8 @@ egt_status egt_autotune_shape(egt_handle h, int k, float thres, int32_t* shape, 
  * wave-per-query shapes, each after a warm-up on the autotuner's sample, and keeps the fastest. Rows do not depend
  * on the choice. offset, mode, shape (optional) receive it, for later handles: EGT_OPT_LEARNED_LEVEL_OFFSET,
  * EGT_OPT_LEARNED_MODE and EGT_OPT_KNN_CLASS_SHAPES with EGT_CLASS_SHAPES_ALL(*shape) (shape 0 = lane per query,
- * 2 = wave per query); ms (optional, 8
- * floats) the times, index (offset x 2 + (mode == 3)) x 2 + (shape == 2). One-cloud handles. The handle's
- * neighbour rows are not valid afterwards: run egt_grid_knn_self. */
+ * 2 = wave per query); ms (optional, 8 floats) the times, index (offset x 2 + (mode == 3)) x 2 + (shape == 2).
+ * One-cloud handles. The handle's neighbour rows are not valid afterwards: run egt_grid_knn_self. */
 egt_status egt_autotune_learned(egt_handle h, int k, float thres, int32_t* offset, int32_t* mode, int32_t* shape,
                                 float* ms);
 

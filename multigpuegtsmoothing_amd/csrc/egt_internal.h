@@ -155,7 +155,11 @@ struct CloudDev {
     int32_t pad;
 };
 
-constexpr int64_t KNN_LONG_CAP = 2048;  // default of EGT_OPT_KNN_LONG_QUERY
+// Default of EGT_OPT_KNN_LONG_QUERY. Two 16M-point cluster mixtures (datasets.mixture seed 4; another scene) at k=40, ms
+// at 512 / 1024 / 2048 / 4096 / never: own cell 70.0 / 59.6 / 59.8 / 60.3 / 64.4 and 74.6 / 61.8 / 55.5 / 54.3 / 53.8;
+// learned level and bound, offset +1, 55.4 / 48.6 / 49.3 / 49.9 / 133.9 and 77.9 / 65.5 / 60.7 / 58.4 / 72.5; offset 0
+// 49.6 / 49.5 / 50.2 / 50.7 / 134.6 and 57.9 / 47.2 / 46.9 / 46.9 / 61.2. No cap is best on both.
+constexpr int64_t KNN_LONG_CAP = 2048;
 
 // A neighbour-count class of a batch: its K template and its range in the chunk work list.
 struct WorkClass {

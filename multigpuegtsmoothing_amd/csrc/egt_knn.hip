@@ -623,7 +623,7 @@ __global__ void __launch_bounds__(KBLK)
 // coalesced). The list is spread over the lanes, lane i holding the i-th smallest key (lanes past k hold the
 // next keys, which never reach a row). A batch's survivors go in one by one as max(L[i-1], min(key, L[i]))
 // with L[i-1] shifted in from the lane below, or, when many survive, by a bitonic sort of the batch and a
-// bitonic merge with the list. Each wave serves 16 Morton-consecutive queries of a 64-query chunk and keeps
+// bitonic merge with the list. Each wave serves 1, 2 or 4 Morton-consecutive queries of a 64-query chunk and keeps
 // the ranges of the last box it looked up for the next query with the same box.
 namespace wv {
 
@@ -1231,6 +1231,11 @@ void launch_wave(KnnParams P, hipStream_t s) {
 //   mixture  k=16  1.77 / 0.29, 1.92 / 0.36  1.61 / 1.22, 1.58 / 1.55  6.66 / 7.00, 6.02 / 8.80  24.9 / 27.5, 24.3 / 35.1
 //   mixture  k=24                            1.96 / 1.45, 2.97 / 1.93  8.74 / 8.64, 9.71 / 10.5  33.8 / 35.1, 39.2 / 47.7
 //   mixture  k=40  4.26 / 0.45, 3.94 / 0.57  4.82 / 2.33, 4.94 / 3.65  12.3 / 11.4, 17.9 / 17.1  47.7 / 50.9, 61.0 / 65.9
+// Size and evenness do not settle the shape of a large uneven cloud: the mixtures above are points of one scene, and
+// on another scene of the same generator (datasets.mixture, seed 4) 16M points at k=40 take 59.8 / 51.3 from the own
+// cell, 50.2 / 35.6 and 49.3 / 50.3 with learned level and bound at offsets 0 and +1, 55.0 / 34.3 with the level
+// alone, where the first scene takes 55.5 / 60.2, 46.9 / 50.2, 60.7 / 64.6 and 47.2 / 51.5. The limits keep the lane
+// shape there, which the shape tuners then change for a cloud where the wave is faster.
 enum class Density { even, uneven, mixed };
 bool wave_by_size(int K, int64_t queries, Density d, bool learned) {
     if (K >= 48) return true;
@@ -1671,7 +1676,10 @@ void run_knn_query_noalloc(egt_ctx* h, const float* dqx, const float* dqy, const
 // it runs the plain search on an evenly spread sample of chunks (about 8192 chunks of 64 Morton-consecutive
 // queries) and reads back the work counters. The score per sampled query is candidates + 3 x cells looked up
 // (a cell lookup costs about three candidate tests on gfx950: a dependent hash probe and range fetch against a
-// coalesced distance test; cells looked up include the binary-search steps of sub-cell ranges). Counters,
+// coalesced distance test; cells looked up include the binary-search steps of sub-cell ranges). The sample runs a lane
+// per query in either shape: the wave's own counters choose the same level or a slower one, since a wave looks a box's
+// cells up at once (full search by a wave at the level its / the lane's counters choose: mixture 4M k=64 12.9 / 11.9
+// ms, 50,000 points k=16 0.150 / 0.129; seven other clouds the same level). Counters,
 // not the sample's wall time, rank the levels: a sample's time is set by its slowest wave (isolated queries
 // next to dense clusters), not by the bulk of the work. Rows do not depend on the choice. Levels -SUB .. top
 // are tried; trial_ms / trial_cost get each level's sample time and score at index level + SUB (-1 for

@@ -548,7 +548,8 @@ __global__ void __launch_bounds__(tile_threads<TILE>()) __attribute__((amdgpu_wa
 // call on the handle does. A tile whose neighbour is not there finds that out in the first exchange, so that one ends
 // after `wait` ticks (EGT_OPT_TAUBIN_WAIT, 500 us) and later ones, which only another process can hold up, after
 // RLATER times as many. Two such clouds from two threads, 20 calls each, launch by launch 66-77 ms; with a wait of
-// 100 us 56-64, 250 us 58-63, 500 us 61-65, 2 ms 72-74, 5 ms 81-82, 20 ms 105-177, 100 ms 164-460. The points are untouched until k_writeback, which looks at the flag first.
+// 100 us 56-64, 250 us 58-63, 500 us 61-65, 2 ms 72-74, 5 ms 81-82, 20 ms 105-177, 100 ms 164-460. The points are
+// untouched until k_writeback, which looks at the flag first.
 //
 // Bound: the chain of one pass (publish, find the neighbours' points, two chunks of slots), where a launch per pass
 // costs its start, two dependent rounds of staging loads and its end, with most CUs idle below 256 tiles. Us a pass,
