@@ -103,8 +103,7 @@ struct KnnParams {
     const float4* __restrict__ qpts;       // query search: queries in Morton order (x', y', z', bits(index))
     const unsigned long long* __restrict__ qvcell;  // query search: virtual cell, clamped to the grid
     int64_t nchunks;   // chunks in the work list (after sampling)
-    int qpw;           // wave-per-query search: queries a wave serves one after another (1, 2 or 4)
-    int64_t first;     // wave-per-query search: the launch's first chunk (of a list: its first workgroup)
+    int qpw;           // wave-per-query search: queries a wave serves one after another (1, 2, 4 or 16)
     int stride;        // 1 = every chunk; s > 1 = every s-th chunk of the list (sampled trial runs)
     int B, log2B, stages, maxc;
     int Bv;            // cells per axis at internal level 0 (B << SUB)
@@ -623,7 +622,7 @@ __global__ void __launch_bounds__(KBLK)
 // coalesced). The list is spread over the lanes, lane i holding the i-th smallest key (lanes past k hold the
 // next keys, which never reach a row). A batch's survivors go in one by one as max(L[i-1], min(key, L[i]))
 // with L[i-1] shifted in from the lane below, or, when many survive, by a bitonic sort of the batch and a
-// bitonic merge with the list. Each wave serves 1, 2 or 4 Morton-consecutive queries of a 64-query chunk and keeps
+// bitonic merge with the list. Each wave serves 1, 2, 4 or 16 Morton-consecutive queries of a 64-query chunk and keeps
 // the ranges of the last box it looked up for the next query with the same box.
 namespace wv {
 
@@ -798,15 +797,15 @@ __global__ void __launch_bounds__(KBLK) __attribute__((amdgpu_waves_per_eu(6))) 
     __shared__ int wmark[KBLK / 64][64];  // per wave: the entry whose run starts at each slot of a batch
     int64_t m0, m1;
     if (LIST) {
-        m0 = ((P.first + v) * (KBLK / 64) + wv_id) * P.qpw;
+        m0 = (v * (KBLK / 64) + wv_id) * P.qpw;
         m1 = min<int64_t>(m0 + P.qpw, P.nlist);
     } else {
         const int per = 16 / P.qpw;  // workgroups per chunk of 64 queries
-        const int64_t chunk = P.first + v / per;
+        const int64_t chunk = v / per;
         if (chunk >= P.nchunks) return;
         const int64_t start = P.chunks ? P.chunks[chunk * P.stride] : chunk * P.stride * 64;
         const CloudDev& c0 = P.clouds[P.mcloud ? (uint32_t)P.mcloud[start] : 0u];
-        m0 = start + ((v - (chunk - P.first) * per) * (KBLK / 64) + wv_id) * P.qpw;
+        m0 = start + ((v - chunk * per) * (KBLK / 64) + wv_id) * P.qpw;
         m1 = min<int64_t>(m0 + P.qpw, c0.base + c0.n);
     }
     uint64_t ncand = 0;
@@ -1193,12 +1192,9 @@ void launch_any(const KnnParams& P, int K, hipStream_t s, bool query = false, bo
 template <bool QUERY>
 void launch_wave(KnnParams P, hipStream_t s) {
     P.qpw = queries_per_wave(P.nchunks * 64);
-    in_launches(P.nchunks, wave_chunks_per_launch(P.qpw), [&](int64_t first, int64_t chunks) {
-        P.first = first;
-        hipLaunchKernelGGL((k_knn_wave<false, QUERY>), dim3((unsigned)(chunks * wave_groups_per_chunk(P.qpw))),
-                           dim3(KBLK), 0, s, P);
-        LAUNCH_CHECK();
-    });
+    hipLaunchKernelGGL((k_knn_wave<false, QUERY>), dim3((unsigned)(P.nchunks * wave_groups_per_chunk(P.qpw))), dim3(KBLK),
+                       0, s, P);
+    LAUNCH_CHECK();
 }
 
 // Launch shape of a search of `queries` queries in class K where nothing asks for one: a lane per query leaves the
@@ -1254,6 +1250,7 @@ bool wave_by_size(int K, int64_t queries, Density d, bool learned) {
 // k=16 0.84 / 1.25 (a lane per query wins), at k=40 1.82 / 1.50.
 constexpr int64_t QUERY_UNSORTED = 100000;
 bool query_by_wave(const egt_ctx* h, int K, int64_t nq) {
+    if (nq > WAVE_MAX_QUERIES) return false;
     if (h->knn_query_lanes) return h->knn_query_lanes == 64;
     return nq <= QUERY_UNSORTED || wave_by_size(K, nq, Density::even, false);
 }
@@ -1283,6 +1280,7 @@ int class_shape(const egt_ctx* h, int K, int64_t queries) {
 // the bound, from the handle's start level: one wave per query when the class ran in the wave shape or the
 // cap is on, else one lane per query. Returns how many were handed back.
 int64_t search_class(egt_ctx* h, KnnParams P, int K, hipStream_t s, int shape) {
+    if (shape == 2 && P.nchunks * 64 > WAVE_MAX_QUERIES) shape = 0;
     if (shape == 1) {  // persistent: the work-queue counter starts at zero
         P.queue = P.counters + 5;
         HIP_CHECK(hipMemsetAsync(P.queue, 0, sizeof(uint64_t), s));
@@ -1320,9 +1318,11 @@ int64_t search_class(egt_ctx* h, KnnParams P, int K, hipStream_t s, int shape) {
     R.stride = 1;
     if (P.long_cap || shape == 2) {
         R.qpw = queries_per_wave((int64_t)nb);
-        in_launches(ceil_div((int64_t)nb, KBLK / 64 * R.qpw), MAX_GROUPS, [&](int64_t first, int64_t groups) {
-            R.first = first;
-            hipLaunchKernelGGL((k_knn_wave<true, false>), dim3((unsigned)groups), dim3(KBLK), 0, s, R);
+        const int64_t per = KBLK / 64 * R.qpw;  // queries per workgroup
+        in_launches((int64_t)nb, MAX_GROUPS * per, [&](int64_t first, int64_t count) {
+            R.qlist = P.retry + first;
+            R.nlist = count;
+            hipLaunchKernelGGL((k_knn_wave<true, false>), dim3((unsigned)ceil_div(count, per)), dim3(KBLK), 0, s, R);
             LAUNCH_CHECK();
         });
     } else {

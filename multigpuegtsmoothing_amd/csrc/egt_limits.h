@@ -7,7 +7,8 @@
 // EGT_ERR_UNSUPPORTED instead.
 //
 // A launch's threads are a 32-bit count: HIP refuses 2^32 and more. Kernels with several threads per point reach that
-// before the point count's own limit of 2^31 - 1, so their work goes out in as many launches as it takes.
+// before the point count's own limit of 2^31 - 1: their work goes out in as many launches as it takes, or in another
+// shape.
 #pragma once
 #include <cstdint>
 
@@ -48,11 +49,15 @@ void in_launches(int64_t items, int64_t most, Launch&& launch) {
 // Queries a wave of the wave-per-query search serves one after another. More of them reuse the ranges of the last
 // box, fewer give more waves: a 10,000-point torus at k=40 0.105 ms with one query a wave against 0.117, 0.169 and
 // 0.513 with 2, 4 and 16; 150,000 points 0.958, 0.939, 0.965 and 1.194; 1.5M points 6.93, 6.65, 6.57 and 6.78;
-// 16M points (4 and 16) 52.1 and 53.3, a 16M-point cluster mixture 67.7 and 70.5.
-inline int queries_per_wave(int64_t queries) { return queries < 100000 ? 1 : queries < 300000 ? 2 : 4; }
-
-// Its workgroups (four waves) per chunk of 64 queries, and the chunks of one launch.
+// 16M points (4 and 16) 52.1 and 53.3, a 16M-point cluster mixture 67.7 and 70.5. Where four would take more threads
+// than a launch, 16 (as a chunk number for the launch in the kernel would: 46 spilled scalars against 42, a 4M-point
+// mixture at k=64 16.35 -> 16.43 ms).
+inline int queries_per_wave(int64_t queries) {
+    return queries < 100000 ? 1 : queries < 300000 ? 2 : queries <= MAX_GROUPS / 4 * 64 ? 4 : 16;
+}
+// Its workgroups (four waves) per chunk of 64 queries, and the queries of one launch; a larger search runs a lane per
+// query, whatever shape is named.
 inline int wave_groups_per_chunk(int qpw) { return 16 / qpw; }
-inline int64_t wave_chunks_per_launch(int qpw) { return MAX_GROUPS / wave_groups_per_chunk(qpw); }
+constexpr int64_t WAVE_MAX_QUERIES = MAX_GROUPS * 64;
 
 }  // namespace egt

@@ -20,8 +20,8 @@ def test_launch_split(tmp_path):
 
 
 @pytest.mark.gpu
-def test_query_search_in_two_launches(egt_mod, oracle_mod):
-    """2^28 + 65 queries at k=41 (a wave per query, 16 threads each): a set of 131,073 queries over and over, whose
+def test_query_search_past_2_28(egt_mod, oracle_mod):
+    """2^28 + 65 queries at k=41 (a wave per query; 16 threads each would not fit a launch): a set of 131,073 queries over and over, whose
     rows equal the oracle's for one set and repeat for all others."""
     import torch
 
